@@ -658,7 +658,8 @@ zc_status zc_hip_moe_forward(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
 namespace {
 struct PrefillSpace {
     Workspace base;
-    uint16_t *xb, *actb, *sactb; float *xsum, *xplain, *asum, *ssum, *xsum16, *asum16, *ssum16;   // xplain: the inputs' sums for affine Q8 gate/up rows
+    // rows of the products: as bf16, as the matrix-core operand, their group sums in pieces (xplain: for affine Q8 gate/up rows), their block sums
+    uint16_t *xb, *actb, *sactb, *xp, *actp, *sactp, *xplanes, *xplain, *aplanes, *splanes; float *xsum16, *asum16, *ssum16;
     int32_t *tile_expert, *tile_first, *tile_rows, *tile_count, *stile_expert, *stile_first, *stile_rows, *stile_count;
     uint32_t max_tiles, max_shared_tiles;
     uint32_t* near_bits;      // one bit per product element: recompute exactly
@@ -672,10 +673,11 @@ PrefillSpace carve_prefill(const zc_moe_config* c, uint32_t T, void* base) {
     uint64_t at = w.base.bytes;
     auto take = [&](uint64_t bytes) { void* p = base ? static_cast<uint8_t*>(base) + at : nullptr; at += align_up(bytes, 256); return p; };
     const uint64_t n = uint64_t(T) * c->topk;
-    w.max_tiles = uint32_t(n / 32 + c->experts); w.max_shared_tiles = (T + 31) / 32;
-    w.xb = (uint16_t*)take(uint64_t(T) * c->hidden * 2); w.xsum = (float*)take(uint64_t(T) * (c->hidden / 64) * 4);
-    w.actb = (uint16_t*)take(n * c->inter * 2); w.asum = (float*)take(n * (c->inter / 64) * 4);
-    w.sactb = (uint16_t*)take(uint64_t(T) * c->inter * 2); w.ssum = (float*)take(uint64_t(T) * (c->inter / 64) * 4);
+    w.max_tiles = (uint32_t(n / 32 + c->experts) + 7) / 8 * 8; w.max_shared_tiles = ((T + 31) / 32 + 7) / 8 * 8;   // (the product kernel deals tiles out eight at a time)
+    const uint64_t xpitch = 3 * 2 * zc::prefill_pitch(c->hidden), apitch = 3 * 2 * zc::prefill_pitch(c->inter);
+    w.xb = (uint16_t*)take(uint64_t(T) * c->hidden * 2); w.xp = (uint16_t*)take(uint64_t(T) * c->hidden * 2); w.xplanes = (uint16_t*)take(T * xpitch);
+    w.actb = (uint16_t*)take(n * c->inter * 2); w.actp = (uint16_t*)take(n * c->inter * 2); w.aplanes = (uint16_t*)take(n * apitch);
+    w.sactb = (uint16_t*)take(uint64_t(T) * c->inter * 2); w.sactp = (uint16_t*)take(uint64_t(T) * c->inter * 2); w.splanes = (uint16_t*)take(T * apitch);
     w.tile_expert = (int32_t*)take(w.max_tiles * 4ull); w.tile_first = (int32_t*)take(w.max_tiles * 4ull); w.tile_rows = (int32_t*)take(w.max_tiles * 4ull);
     w.tile_count = (int32_t*)take(4);
     w.stile_expert = (int32_t*)take(w.max_shared_tiles * 4ull); w.stile_first = (int32_t*)take(w.max_shared_tiles * 4ull);
@@ -684,7 +686,7 @@ PrefillSpace carve_prefill(const zc_moe_config* c, uint32_t T, void* base) {
     w.xsum16 = (float*)take(uint64_t(T) * (c->hidden / 16) * 4); w.asum16 = (float*)take(n * (c->inter / 16) * 4);
     w.ssum16 = (float*)take(uint64_t(T) * (c->inter / 16) * 4);
     w.norms = (float*)take((uint64_t(T) + c->experts) * 4);
-    w.xplain = (float*)take(uint64_t(T) * (c->hidden / 64) * 4);
+    w.xplain = (uint16_t*)take(T * xpitch);
     w.shared_near_bits = (uint32_t*)take(uint64_t(T) * std::max(c->hidden, c->inter) / 8);
     w.bytes = at;
     return w;
@@ -721,7 +723,7 @@ zc_status zc_hip_moe_prefill(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
     // router logits, top-k + softmax, dispatch (model.cpp:434-479), shared gate: the exact kernels, except that a long batch
     // whose logits nobody asks for gets exact logits only where the selection can see the difference (launch_prefill_router)
     const bool x_q4 = c->bits_gate_up == 4 || c->shared_bits_gate_up == 4, x_q8 = c->bits_gate_up == 8 || c->shared_bits_gate_up == 8;
-    zc::launch_prefill_rows(s, x, T, H, w.xb, x_q4 ? w.xsum : nullptr, x_q4 ? w.xsum16 : nullptr, x_q8 ? w.xplain : nullptr, ctx->moe_status);
+    zc::launch_prefill_rows(s, x, T, H, w.xb, w.xp, x_q4 ? w.xplanes : nullptr, x_q8 ? w.xplain : nullptr, x_q4 ? w.xsum16 : nullptr, ctx->moe_status);
     // the shared expert needs the bf16 rows and nothing of the routing: it runs on a stream of its own from here to the combine
     if (!ctx->beside) {
         ZC_HIP(hipStreamCreateWithFlags(&ctx->beside, hipStreamNonBlocking));
@@ -757,7 +759,7 @@ zc_status zc_hip_moe_prefill(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
     {   // routed gate/up + SwiGLU on gathered rows (pipeline.cpp:18-24), then down scattered to the slots (pipeline.cpp:25-29)
         zc::PrefillGemm g{};
         g.bits = c->bits_gate_up;
-        g.a = w.xb; g.asum = g.bits == 4 ? w.xsum : w.xplain; g.asum16 = g.bits == 4 ? w.xsum16 : nullptr; g.a_rows = w.base.slots; g.a_div = k; g.out_rows = nullptr;
+        g.a = w.xp; g.a_plain = w.xb; g.planes = g.bits == 4 ? w.xplanes : w.xplain; g.asum16 = g.bits == 4 ? w.xsum16 : nullptr; g.a_rows = w.base.rows; g.out_rows = nullptr;
         g.records = static_cast<const uint8_t*>(l->expert_records); g.stride = l->record_stride; offsets_of(l->expert_records, 0, g.off, 0, 2);
         g.tile_expert = w.tile_expert; g.tile_first = w.tile_first; g.tile_rows = w.tile_rows; g.tile_count = w.tile_count;
         g.K = H; g.N = I; g.out_b = w.actb;
@@ -767,8 +769,8 @@ zc_status zc_hip_moe_prefill(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
         zc::launch_prefill_patch(s, g, true);
         zc::PrefillGemm d{};
         d.bits = c->bits_down;
-        zc::launch_prefill_sums(s, w.actb, nullptr, uint32_t(n), I, w.asum, table_inter && d.bits == 4 ? w.asum16 : nullptr, d.bits == 8);
-        d.a = w.actb; d.asum = w.asum; d.asum16 = table_inter && d.bits == 4 ? w.asum16 : nullptr; d.a_rows = nullptr; d.a_div = 1; d.out_rows = w.base.slots;
+        zc::launch_prefill_acts(s, w.actb, uint32_t(n), I, w.actp, d.bits == 4 ? w.aplanes : nullptr, d.bits == 8 ? w.aplanes : nullptr, table_inter && d.bits == 4 ? w.asum16 : nullptr);
+        d.a = w.actp; d.a_plain = w.actb; d.planes = w.aplanes; d.asum16 = table_inter && d.bits == 4 ? w.asum16 : nullptr; d.a_rows = nullptr; d.out_rows = w.base.slots;
         d.records = g.records; d.stride = g.stride; offsets_of(l->expert_records, 0, d.off, 2, 1);
         d.tile_expert = w.tile_expert; d.tile_first = w.tile_first; d.tile_rows = w.tile_rows; d.tile_count = w.tile_count;
         d.K = I; d.N = H;
@@ -782,7 +784,7 @@ zc_status zc_hip_moe_prefill(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
     {   // shared expert (model.cpp:482-485): one group of all the tokens, beside the routed experts
         zc::PrefillGemm g{};
         g.bits = c->shared_bits_gate_up;
-        g.a = w.xb; g.asum = g.bits == 4 ? w.xsum : w.xplain; g.asum16 = g.bits == 4 ? w.xsum16 : nullptr; g.a_rows = nullptr; g.a_div = 1;
+        g.a = w.xp; g.a_plain = w.xb; g.planes = g.bits == 4 ? w.xplanes : w.xplain; g.asum16 = g.bits == 4 ? w.xsum16 : nullptr; g.a_rows = nullptr;
         g.records = static_cast<const uint8_t*>(l->shared_record); g.stride = 0; offsets_of(l->shared_record, 1, g.off, 0, 2);
         g.tile_expert = w.stile_expert; g.tile_first = w.stile_first; g.tile_rows = w.stile_rows; g.tile_count = w.stile_count;
         g.K = H; g.N = I; g.out_b = w.sactb;
@@ -791,8 +793,8 @@ zc_status zc_hip_moe_prefill(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
         zc::launch_prefill_patch(s2, g, true);
         zc::PrefillGemm d{};
         d.bits = c->shared_bits_down;
-        zc::launch_prefill_sums(s2, w.sactb, nullptr, T, I, w.ssum, table_inter && d.bits == 4 ? w.ssum16 : nullptr, d.bits == 8);
-        d.a = w.sactb; d.asum = w.ssum; d.asum16 = table_inter && d.bits == 4 ? w.ssum16 : nullptr; d.a_rows = nullptr; d.a_div = 1; d.out_rows = nullptr;
+        zc::launch_prefill_acts(s2, w.sactb, T, I, w.sactp, d.bits == 4 ? w.splanes : nullptr, d.bits == 8 ? w.splanes : nullptr, table_inter && d.bits == 4 ? w.ssum16 : nullptr);
+        d.a = w.sactp; d.a_plain = w.sactb; d.planes = w.splanes; d.asum16 = table_inter && d.bits == 4 ? w.ssum16 : nullptr; d.a_rows = nullptr; d.out_rows = nullptr;
         d.records = g.records; d.stride = 0; offsets_of(l->shared_record, 1, d.off, 2, 1);
         d.tile_expert = w.stile_expert; d.tile_first = w.stile_first; d.tile_rows = w.stile_rows; d.tile_count = w.stile_count;
         d.K = I; d.N = H; d.out_f = w.base.shared;

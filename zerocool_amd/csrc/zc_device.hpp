@@ -36,16 +36,18 @@ __device__ __forceinline__ float exp32(float x) {
     return y * __uint_as_float(uint32_t(a + 127) << 23) * __uint_as_float(uint32_t(b + 127) << 23);
 }
 // BF16 sigmoid with a rounding after the exponential, the sum and the reciprocal
-// (reference: qwen.metal:33-35).
+// (reference: qwen.metal:33-35).  The divisor is a BF16 number of at least 1: its reciprocal lies at least 2^-17 of itself
+// away from every BF16 rounding boundary (|1 - b t| is a multiple of 2^-16 for a boundary t of nine bits and b of eight,
+// and zero for no b), so the hardware's reciprocal, good to one fp32 step, rounds to the same BF16 number as the
+// correctly rounded quotient at a twelfth of the instructions.  Divisors whose reciprocal is subnormal are divided.
 __device__ __forceinline__ float sigmoid_bf(float x) {
-    const float y = bf(1.0f / bf(1.0f + bf(exp32(__builtin_fabsf(x)))));
+    const float b = bf(1.0f + bf(exp32(__builtin_fabsf(x))));
+    const float y = bf(__builtin_expect(b < 0x1p125f, 1) ? __builtin_amdgcn_rcpf(b) : 1.0f / b);
     return x < 0 ? y : bf(1.0f - y);
 }
 // SwiGLU epilogue of the fused gate/up product (reference: qwen.metal:78-80).
-__device__ __forceinline__ float swiglu_bf(float gate_sum, float up_sum) {
-    const float g = bf(gate_sum), u = bf(up_sum);
-    return bf(bf(g * sigmoid_bf(g)) * u);
-}
+__device__ __forceinline__ float swiglu_rounded(float g, float u) { return bf(bf(g * sigmoid_bf(g)) * u); }   // g, u: BF16 values
+__device__ __forceinline__ float swiglu_bf(float gate_sum, float up_sum) { return swiglu_rounded(bf(gate_sum), bf(up_sum)); }
 
 // Sum over the 32 reference lanes as an xor butterfly with strides 16,8,4,2,1.
 // A 64-lane wavefront carries two independent 32-lane groups; strides below 32

@@ -115,17 +115,17 @@ hipError_t decode_wide_occupancy(uint32_t lds_bytes, int* blocks_per_cu);
 
 // ---- prefill: sorted-token grouped GEMM on the bf16 matrix cores (zc_prefill.hip)
 struct PrefillGemm {
-    const uint16_t* a;        // bf16 rows [.][K]
-    const float* asum;        // per (row, group of 64): sum of the blocks' BF16-rounded sum-of-four chains
+    const uint16_t* a;        // rows [.][K] as the product kernel reads them (prefill_rows_kernel's xp)
+    const uint16_t* a_plain;  // the same rows as bf16 in their own order (read by the recomputation)
+    const uint16_t* planes;   // per (row, group of 64): the input sum in three bf16 pieces
     const float* asum16;      // per (row, block of 16): that block's chain sum (read by the recomputation; null: formed there)
-    const int32_t* a_rows;    // row of `a` for sorted position pos: a_rows ? a_rows[pos] / a_div : pos
-    uint32_t a_div;
+    const int32_t* a_rows;    // row of `a` for sorted position pos: a_rows ? a_rows[pos] : pos
     const int32_t* out_rows;  // output row for sorted position pos: out_rows ? out_rows[pos] : pos   (down projection)
     const uint8_t* records; uint64_t stride;   // expert e's record at records + e * stride
     uint64_t off[6];          // byte offsets in a record: codes, scales, biases of the (gate | down) projection, then of up
     const int32_t *tile_expert, *tile_first, *tile_rows, *tile_count;
     uint32_t K, N;            // reduction length, rows of ONE projection
-    uint32_t bits;            // 4: nibble codes, asum = the Q4 lanes' BF16-rounded sum-of-four chains; 8: byte codes, asum = the Q8 lanes' plain sums
+    uint32_t bits;            // 4: nibble codes, planes of the Q4 lanes' BF16-rounded sum-of-four chains; 8: byte codes, planes of the Q8 lanes' plain sums
     uint16_t* out_b;          // gate/up: SwiGLU activations as bf16 [sorted position][N]
     float* out_f;             // down: BF16-rounded fp32 [output row][N]
     uint16_t* out_h;          // down, instead of out_f when not null: the same values as bf16 (what the combine reads is half as long)
@@ -145,11 +145,12 @@ struct PrefillGemm {
 // 2^-23 (the largest distance seen between the two orders of additions, on rows of 8 and of 32 groups, is a quarter of it),
 // beyond that 2^-28 per group (2^-22 again at 64): the distance grows with the number of additions.
 constexpr float prefill_margin(uint32_t K) { return K / 64 < 8 ? 0x1p-22f : (K / 64 <= 32 ? 0x1p-23f : float(K / 64) * 0x1p-28f); }
-void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t K, uint16_t* xb, float* sums, float* sums16, float* plain, int32_t* status);
+constexpr uint32_t prefill_pitch(uint32_t K) { return (K / 64 + 7) / 8 * 8; }   // of a piece's row: sixteen-byte loads
+void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain, float* sums16, int32_t* status);
+void launch_prefill_acts(hipStream_t s, const uint16_t* xb, uint32_t rows, uint32_t K, uint16_t* xp, uint16_t* planes, uint16_t* plain, float* sums16);
 // ids / weights not null (topk <= 64): the selection runs in the same launch and the logits are not written
 void launch_prefill_router(hipStream_t s, const float* x, const uint16_t* xb, const void* w, const float* offsets, uint32_t T, uint32_t K,
                            uint32_t E, uint32_t topk, float* norms, float* logits, int32_t* ids, float* weights);
-void launch_prefill_sums(hipStream_t s, const uint16_t* xb, const int32_t* rows_ptr, uint32_t rows_max, uint32_t K, float* sums, float* sums16, bool plain);
 void launch_prefill_dispatch(hipStream_t s, const int32_t* ids, uint32_t tokens, uint32_t topk, uint32_t E, int32_t* offsets, int32_t* slots, int32_t* rows,
                              int32_t* status, int32_t* tile_expert, int32_t* tile_first, int32_t* tile_rows, int32_t* tile_count);
 bool prefill_dispatch_fits(const int32_t* ids, uint32_t tokens, uint32_t topk, uint32_t E);

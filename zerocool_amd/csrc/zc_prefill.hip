@@ -4,21 +4,30 @@
 //
 // Arithmetic.  The reference evaluates, per 16-element block, scale * sum(x q) + bias * sum'(x) with sum' the
 // BF16-rounded sum-of-four chain (qwen.metal:46-62).  Here the products x * q run on v_mfma_f32_16x16x32_bf16: x is
-// BF16-valued (exact as a bf16 operand), q in 0..15 is exact in bf16, products are exact and accumulate in fp32 over one
-// scale group of 64; per group the accumulator is folded as  total += scale * dot + bias * chain_sum  with the chain
-// sums precomputed per (row, group) exactly as the reference rounds them.  Only the order of the fp32 additions
+// BF16-valued (exact as a bf16 operand), products are exact and accumulate in fp32 over one scale group of 64; per group
+// the accumulator is folded as  total += scale * dot.  The bias half, sum over the groups of bias * chain sum, is a product
+// over the group index and runs on the same instruction before the walk over K, the chain sums cut into three bf16 pieces
+// that add up to them exactly.  Only the order of the fp32 additions
 // differs from the reference, so results agree to a few fp32 steps before the BF16 rounding of the outputs.  Every sum
 // that lands within prefill_margin(K) of its term magnitudes of a BF16 rounding boundary is then recomputed with the reference's exact
 // lane arithmetic (about 2-3 % of the elements), which removes the rounding flips in practice; the path is still
 // specified by a tolerance (max relative error 2e-3 of the layer output), not as bit-exact.  Routing, dispatch and the
 // combine use the exact kernels.
 //
+// Codes as operands.  The matrix cores take subnormal bf16 operands at full precision, and the bit pattern of an integer
+// code 0..255 read as bf16 is the number code * 2^-133: a code needs no conversion, only its place in a 16-bit half, one
+// mask (and shift) per two codes where the conversion to a float and on to bf16 took 3 instructions per two codes, each
+// at half rate.  The token rows carry 2^100 to stay in range, the scales the remaining 2^33: both exact.
+// Nibbles i and i + 4 of a word share one mask, so the rows are stored with every eight elements in the order
+// 0 4 1 5 2 6 3 7.  Groups whose values would leave the exact range (|x| >= 2^26, all below 2^-60, inf, NaN) get a NaN
+// chain sum: every output of such a row is then recomputed with the lane arithmetic.
+//
 // Tiling.  One workgroup (4 waves) owns up to 48 sorted token rows of ONE expert and 128 weight rows (gate/up: 64 gate rows
 // and the 64 up rows of the same indices, so SwiGLU is fused in registers), and walks K in steps of 64 = one scale
-// group.  Each wave multiplies all (two or three) 16-row blocks of the tokens by 2 of the 8 column tiles: the 4-bit codes
-// of its 32 weight rows go from memory straight into the lanes that feed them to the matrix cores and are expanded to
-// bf16 there (once per workgroup and step), the token rows are gathered into LDS as bf16, double-buffered, and the
-// scales, biases and chain sums of all steps are brought into LDS once.  An expert's rows are cut into tiles of 32, except
+// group.  Each wave multiplies all (two or three) 16-row blocks of the tokens by 2 of the 8 column tiles: the codes
+// of its 32 weight rows go from memory straight into the lanes that feed them to the matrix cores, the token rows are
+// gathered into LDS as bf16, double-buffered, and the
+// scales of all steps are brought into LDS once.  An expert's rows are cut into tiles of 32, except
 // that a run of up to 48 rows (a whole expert with few rows, or the last rows of a longer run) is ONE tile: with about
 // forty rows per expert -- an unskewed router at 2048 tokens -- every expert's codes are then expanded once, not twice.
 #include "zc_kernels.hpp"
@@ -33,70 +42,88 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-constexpr uint32_t kTileRows = 32, kTileRowsMax = 48, kTileCols = 128, kPitch = 72;   // LDS row pitch in bf16 elements (144 bytes)
-
-// fp32 rows holding BF16 values -> bf16 rows, plus per (row, group of 64) the sum of the four blocks' BF16-rounded
-// sum-of-four chains.  One thread per (row, group).  status bit 4: a value was not BF16-valued.
-// plain (optional): per (row, group) the sum of the plain fp32 sums of the group's eight 8-element blocks, the affine Q8
-// lanes' input sum (qwen.metal:112-125: sum += v, element by element).
-__global__ __launch_bounds__(256) void prefill_rows_kernel(const float* x, uint32_t rows, uint32_t K, uint16_t* xb, float* sums, float* sums16, float* plain,
-                                                           int32_t* status) {
-    const uint32_t groups = K / 64, i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= rows * groups) return;
-    const uint32_t r = i / groups, g = i % groups;
-    const float4* src = reinterpret_cast<const float4*>(x + uint64_t(r) * K + g * 64);
-    uint32_t low = 0;
-    float total = 0, total_plain = 0;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        float sum = 0, eight[2] = {0, 0};
-        uint32_t packed[8];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float4 v = src[b * 4 + q];
-            sum += bf(bf(bf(v.x + v.y) + v.z) + v.w);
-            eight[q / 2] = (((eight[q / 2] + v.x) + v.y) + v.z) + v.w;
-            const uint32_t u0 = __float_as_uint(v.x), u1 = __float_as_uint(v.y), u2 = __float_as_uint(v.z), u3 = __float_as_uint(v.w);
-            low |= (u0 | u1 | u2 | u3) & 0xffffu;
-            packed[2 * q] = (u0 >> 16) | (u1 & 0xffff0000u); packed[2 * q + 1] = (u2 >> 16) | (u3 & 0xffff0000u);
-        }
-        total += sum;
-        total_plain = (total_plain + eight[0]) + eight[1];
-        if (sums16) sums16[uint64_t(i) * 4 + b] = sum;
-        uint4* dst = reinterpret_cast<uint4*>(xb + uint64_t(r) * K + g * 64 + b * 16);
-        dst[0] = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-        dst[1] = make_uint4(packed[4], packed[5], packed[6], packed[7]);
-    }
-    if (sums) sums[i] = total;
-    if (plain) plain[i] = total_plain;
-    if (low) atomicOr(status, 4);
+// Eight bytes whose address is a multiple of four only.
+__device__ __forceinline__ uint2 ldg_u2_by_words(const void* p) {
+    typedef uint32_t words __attribute__((ext_vector_type(2), aligned(4)));
+    const words v = *as_global<words>(p);
+    return make_uint2(v.x, v.y);
 }
-// The same sums for rows that are already bf16 (the SwiGLU activations).
-// plain: the affine Q8 lanes' sums instead (see prefill_rows_kernel); no per-block table then.
-__global__ __launch_bounds__(256) void prefill_sums_kernel(const uint16_t* xb, const int32_t* rows_ptr, uint32_t rows_max, uint32_t K, float* sums, float* sums16,
-                                                           bool plain) {
-    const uint32_t groups = K / 64, i = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t rows = rows_ptr ? min(uint32_t(*rows_ptr), rows_max) : rows_max;
-    if (i >= rows * groups) return;
-    const uint32_t r = i / groups, g = i % groups;
-    const uint4* src = reinterpret_cast<const uint4*>(xb + uint64_t(r) * K + g * 64);
-    float total = 0;
+constexpr uint32_t kTileRows = 32, kTileRowsMax = 48, kPitch = 136;   // LDS row pitch in bf16 elements: 128 elements of a row, sixteen rows on different banks
+
+// What the matrix-core products and the recomputation need of their token rows, from fp32 rows holding BF16 values (F32)
+// or from bf16 rows (the SwiGLU activations): a thread takes four neighbouring elements, so loads and stores are whole runs.
+//   xb      the row as bf16 (F32 only)
+//   xp      the row times 2^100, every eight elements in the order 0 4 1 5 2 6 3 7: the matrix-core operand
+//   planes  per (row, group of 64) the group's input sum as three bf16 pieces, [row][piece][prefill_pitch(K)]: the four
+//           blocks' BF16-rounded sum-of-four chains (Q4 lanes), NaN where the group leaves the operand's exact range
+//   plain   the same of the plain fp32 sums (Q8 lanes, qwen.metal:112-125: sum += v, element by element in blocks of eight)
+//   sums16  per (row, block of 16) the chain sum itself (read by the recomputation)
+// status bit 4: a value was not BF16-valued.
+__device__ __forceinline__ void store_pieces(uint16_t* at, uint32_t pitch, float v) {
+    const uint32_t hi = __float_as_uint(v) & 0xffff0000u;
+    const float rest = v - __uint_as_float(hi);
+    const uint32_t mid = __float_as_uint(rest) & 0xffff0000u;
+    at[0] = uint16_t(hi >> 16); at[pitch] = uint16_t(mid >> 16); at[2 * pitch] = uint16_t(__float_as_uint(rest - __uint_as_float(mid)) >> 16);
+}
+template <bool F32>
+__global__ __launch_bounds__(256) void prefill_rows_kernel(const void* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain,
+                                                           float* sums16, int32_t* status) {
+    const uint32_t quads = K / 4, i = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63u;
+    if (i >= rows * quads) return;               // (whole groups of sixteen lanes: K is a multiple of 128)
+    const uint32_t r = i / quads, c = i % quads, pitch = prefill_pitch(K);
+    float v[4];
+    if constexpr (F32) {
+        const float4 q = reinterpret_cast<const float4*>(x)[i];
+        v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+        uint32_t low = 0;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        const uint4 lo = src[2 * b], hi = src[2 * b + 1];
-        const uint32_t w[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-        float sum = 0, eight[2] = {0, 0};
+        for (int k = 0; k < 4; ++k) low |= __float_as_uint(v[k]) & 0xffffu;
+        if (low) atomicOr(status, 4);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float a = __uint_as_float(w[2 * q] << 16), c = __uint_as_float(w[2 * q] & 0xffff0000u);
-            const float d = __uint_as_float(w[2 * q + 1] << 16), e = __uint_as_float(w[2 * q + 1] & 0xffff0000u);
-            sum += bf(bf(bf(a + c) + d) + e);
-            eight[q / 2] = (((eight[q / 2] + a) + c) + d) + e;
-        }
-        total = plain ? (total + eight[0]) + eight[1] : total + sum;
-        if (sums16 && !plain) sums16[uint64_t(i) * 4 + b] = sum;
+        for (int k = 0; k < 4; ++k) v[k] = __uint_as_float(__float_as_uint(v[k]) & 0xffff0000u);
+        reinterpret_cast<uint2*>(xb)[i] = make_uint2((__float_as_uint(v[0]) >> 16) | __float_as_uint(v[1]), (__float_as_uint(v[2]) >> 16) | __float_as_uint(v[3]));
+    } else {
+        const uint2 q = reinterpret_cast<const uint2*>(x)[i];
+        v[0] = __uint_as_float(q.x << 16); v[1] = __uint_as_float(q.x & 0xffff0000u); v[2] = __uint_as_float(q.y << 16); v[3] = __uint_as_float(q.y & 0xffff0000u);
     }
-    sums[i] = total;
+    uint32_t largest = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) largest = max(largest, __float_as_uint(v[k]) & 0x7fffffffu);
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) largest = max(largest, uint32_t(__shfl_xor(int(largest), o)));
+    const bool strange = largest >= 0x4c800000u || (largest != 0 && largest < 0x21800000u);   // 2^26, 2^-60
+    {   // lane 2m of a pair holds elements 0..3, lane 2m + 1 elements 4..7: 0 4 1 5 | 2 6 3 7
+        uint32_t mine[2], other[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) mine[k] = (__float_as_uint(v[2 * k] * 0x1p100f) >> 16) | (__float_as_uint(v[2 * k + 1] * 0x1p100f) & 0xffff0000u);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) other[k] = uint32_t(__shfl_xor(int(mine[k]), 1));
+        const bool odd = lane & 1u;
+        const uint32_t a = odd ? other[1] : mine[0], b = odd ? mine[1] : other[0];   // a: elements (2) 0 and (3) 1; b: elements (6) 4 and (7) 5
+        reinterpret_cast<uint2*>(xp)[i] = make_uint2((a & 0xffffu) | (b << 16), (a >> 16) | (b & 0xffff0000u));
+    }
+    const uint32_t group = r * (3 * pitch) + c / 16, base = lane & ~15u;
+    if (planes || sums16) {
+        const float quad = bf(bf(bf(v[0] + v[1]) + v[2]) + v[3]);
+        float sum = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) sum += __shfl(quad, int((lane & ~3u) + uint32_t(k)));
+        if (sums16 && (lane & 3u) == 0) sums16[i / 4] = sum;
+        if (planes) {
+            float total = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) total += __shfl(sum, int(base + 4u * uint32_t(k)));
+            if ((lane & 15u) == 0) store_pieces(planes + group, pitch, strange ? __uint_as_float(0x7fc00000u) : total);
+        }
+    }
+    if (plain) {
+        const float head = (((0.0f + v[0]) + v[1]) + v[2]) + v[3], before = __shfl_xor(head, 1);
+        const float eight = (((before + v[0]) + v[1]) + v[2]) + v[3];       // (of odd lanes)
+        float total = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) total += __shfl(eight, int(base + 2u * uint32_t(k) + 1u));
+        if ((lane & 15u) == 0) store_pieces(plain + group, pitch, strange ? __uint_as_float(0x7fc00000u) : total);
+    }
 }
 
 // Work list: tile t = (expert, first sorted position, rows).  offsets[e] .. offsets[e+1] are the expert's sorted
@@ -242,249 +269,294 @@ __global__ __launch_bounds__(256) void prefill_dispatch_kernel(const int32_t* __
     }
 }
 
-// BITS: 4 (nibble codes, eight bytes of a row per lane and step) or 8 (byte codes, sixteen bytes; the chain sums are then
-// the plain ones of the Q8 lanes).  A byte code is exact in bf16 like a nibble code, and its product with a BF16 value is
-// exact in fp32.
-template <bool GATED, int BITS>
-__global__ __launch_bounds__(256) void prefill_gemm_kernel(PrefillGemm p) {
-    __shared__ __align__(16) uint16_t a_s[2][kTileRowsMax * kPitch];
-    // The scales and biases of the workgroup's 128 weight rows and the chain sums of its token rows, for every step, are
-    // brought in once (whole runs of consecutive bytes: fetched step by step they cost a cache access per row and step
-    // for two or four bytes each, more accesses than the codes and the token rows together).
-    extern __shared__ __align__(16) uint8_t meta_s[];
-    __shared__ uint32_t row_s[kTileRowsMax];
-    const uint32_t tile = blockIdx.y;
-    if (tile >= uint32_t(*p.tile_count)) return;
+// One tile: up to 16 NB rows of one expert x 128 weight rows.  BITS: 4 (nibble codes) or 8 (byte codes; the planes are then
+// the plain sums of the Q8 lanes).  The number of row blocks is a compile-time value, so that the walk over K is straight-line
+// code: as a run-time bound it cut every step into short blocks that each waited for its own LDS reads.
+//
+// The walk goes two scale groups (128 elements) at a time, weights and token rows one such pair ahead.  What bounds it is
+// the SIMDs' issue: per wave and pair 24 matrix-core instructions (7.7 ns each) and about 165 vector ones (1.0 to 1.5 ns),
+// which overlap only in part -- weights and rows read from a warm cache leave the time of the walk unchanged.  A wave
+// alone issues one vector instruction every five clocks, so the registers are kept to what three waves per SIMD allow
+// (Q4: 166 of 168; with a second set of token rows or four pairs of weights in flight two waves fit, and the layer of
+// hidden 2048 took 680 us at 2048 tokens instead of 621).  At that size the routed gate/up product takes 258 us (369 with
+// converted codes, a run-time number of row blocks and the scales staged through LDS), the down product 174 us (258).
+template <bool GATED, int BITS, int NB>
+__device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s, uint16_t* marks_s, uint32_t expert, uint32_t first, uint32_t rows, uint32_t n0) {
+    constexpr int kAhead = 2, kRegs = BITS;       // pairs of groups in flight; dwords of a column tile's pair per lane
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, j = lane & 15u, g4 = lane >> 4;
-    const uint32_t expert = uint32_t(p.tile_expert[tile]), first = uint32_t(p.tile_first[tile]), rows = uint32_t(p.tile_rows[tile]);
-    const uint32_t K = p.K, N = p.N, groups = K / 64;
-    const uint32_t n0 = blockIdx.x * (GATED ? 64u : 128u);
+    const uint32_t K = p.K, N = p.N, groups = K / 64, pairs = K / 128;
     const uint8_t* record = p.records + uint64_t(expert) * p.stride;
-
-    // what this thread fetches every step
-    const uint32_t a_r = tid >> 3, a_c = tid & 7u;                       // token row of the tile, 16-byte chunk of the step
-    const uint32_t a_pos = first + min(a_r, rows - 1);                   // rows past the end repeat the last one (never stored)
-    const uint32_t a_row = p.a_rows ? uint32_t(p.a_rows[a_pos]) / p.a_div : a_pos;
-    const uint16_t* a_src = p.a + uint64_t(a_row) * K + a_c * 8;
-    const bool tall = rows > kTileRows;                                  // a third block of sixteen rows: threads 0..127 fetch it too
-    const uint32_t a_pos2 = first + min(32u + (a_r & 15u), rows - 1);
-    const uint32_t a_row2 = p.a_rows ? uint32_t(p.a_rows[a_pos2]) / p.a_div : a_pos2;
-    const uint16_t* a_src2 = p.a + uint64_t(a_row2) * K + a_c * 8;
     // The wave's two column tiles (rows of the workgroup's 128 weight rows) for every block of sixteen token rows; gate/up:
     // a gate tile and the up tile of the same rows.  The codes go from memory straight into the lanes that feed them to
-    // the matrix cores: lane (j, g4) holds codes 16 g4 .. 16 g4 + 15 of the step for weight row j of each tile (eight
-    // bytes), the first eight for one product and the rest for the next; the token rows are read from LDS in the same
-    // order, and the order of k inside a step is free.
-    uint32_t col_row[2];
-    const uint8_t* b_src[2];
+    // the matrix cores, whole 64-byte pieces of a row per load.
+    // (Bases are the same in every lane, lanes add 32-bit offsets.)
+    const uint8_t *codes_of[2], *scales_of[2], *biases_of[2];
+    uint32_t b_at[2], m_at[2];                   // the lane's weight row: bytes from the bases
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-        col_row[q] = (GATED ? (uint32_t(q) * 64u + wave * 16u) : (2 * wave + uint32_t(q)) * 16u) + j;
-        const uint32_t b_proj = GATED ? col_row[q] >> 6 : 0u, b_n = n0 + (GATED ? (col_row[q] & 63u) : col_row[q]);
-        b_src[q] = record + p.off[b_proj * 3] + uint64_t(b_n) * (K * BITS / 8) + g4 * (2 * BITS);
+        const uint32_t proj = GATED ? uint32_t(q) : 0u, n = n0 + (GATED ? wave * 16u : (2 * wave + uint32_t(q)) * 16u) + j;
+        codes_of[q] = record + p.off[proj * 3]; scales_of[q] = record + p.off[proj * 3 + 1]; biases_of[q] = record + p.off[proj * 3 + 2];
+        b_at[q] = n * (K * BITS / 8) + g4 * 16; m_at[q] = n * groups * 2;
     }
-    // scales then biases as bf16 [128][groups + 2] (the pad keeps sixteen rows on different banks), then the chain sums
-    // [groups][48]
-    const uint32_t pitch = groups + 2;
-    uint16_t* scale_s = reinterpret_cast<uint16_t*>(meta_s);
-    uint16_t* bias_s = scale_s + kTileCols * pitch;
-    float* sum_s = reinterpret_cast<float*>(bias_s + kTileCols * pitch);
-    if (tid < kTileRowsMax) {
-        const uint32_t x_pos = first + min(tid, rows - 1);
-        row_s[tid] = p.a_rows ? uint32_t(p.a_rows[x_pos]) / p.a_div : x_pos;
-    }
-    {   // a projection's 64 (gate/up) or 128 rows are consecutive in the record: groups / 2 dwords per row
-        const uint32_t half = groups / 2, per_proj = (GATED ? 64u : 128u) * half;
-        for (uint32_t i = tid; i < 128u * half; i += 256) {
-            const uint32_t proj = GATED ? i / per_proj : 0u, at = GATED ? i % per_proj : i, r = i / half, g2 = i % half;
-            const uint32_t sv = ldg_u32(record + p.off[proj * 3 + 1] + uint64_t(n0) * groups * 2, at);
-            const uint32_t ov = ldg_u32(record + p.off[proj * 3 + 2] + uint64_t(n0) * groups * 2, at);
-            *reinterpret_cast<uint32_t*>(scale_s + r * pitch + 2 * g2) = sv;
-            *reinterpret_cast<uint32_t*>(bias_s + r * pitch + 2 * g2) = ov;
-        }
-    }
-    __syncthreads();
-    for (uint32_t i = tid; i < kTileRowsMax * groups; i += 256) {
-        const uint32_t r = i / groups, g = i % groups;
-        sum_s[g * kTileRowsMax + r] = p.asum[uint64_t(row_s[r]) * groups + g];
-    }
-
-    // What a step needs is requested two steps ahead and waits in registers (two sets, taken in turn): with one step of
-    // lead the loads' latency, several times a step's arithmetic, was paid at every step.
-    struct Fetched { uint4 a, a2; uint32_t b[2][BITS / 2]; };   // the lane's sixteen codes of a step: two dwords (Q4) or four (Q8)
-    Fetched ahead[2];
-    ahead[0] = ahead[1] = Fetched{make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0), {}};
-    auto fetch = [&](uint32_t g, Fetched& f) {
-        f.a = *reinterpret_cast<const uint4*>(a_src + g * 64);
+    u32x4 ring[kAhead][2][kRegs / 4];
+    auto fetch_b = [&](uint32_t pair, u32x4 (&to)[2][kRegs / 4]) {
+        const uint32_t at = min(pair, pairs - 1) * (16 * BITS);   // (past the end: the last pair again, not used)
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int h = 0; h < kRegs / 4; ++h) to[q][h] = *as_global<u32x4>(codes_of[q] + (b_at[q] + at + 64u * uint32_t(h)));
+    };
+#pragma unroll
+    for (int d = 0; d + 1 < kAhead; ++d) fetch_b(uint32_t(d), ring[d]);
+    auto row_of = [&](uint32_t m) {              // row of `a` for row m of the tile; rows past the end repeat the last one (never stored)
+        const uint32_t pos = first + min(m, rows - 1);
+        return p.a_rows ? uint32_t(p.a_rows[pos]) : pos;
+    };
+    const uint16_t* a_src[NB];                   // thread: sixteen bytes of one row of every block
+    const uint32_t a_at = (tid >> 4) * kPitch + (tid & 15u) * 8;
+#pragma unroll
+    for (int rb = 0; rb < NB; ++rb) a_src[rb] = p.a + uint64_t(row_of(16 * uint32_t(rb) + (tid >> 4))) * K + (tid & 15u) * 8;
+    u32x4 a_next[NB];
+    auto fetch_a = [&](uint32_t pair, u32x4 (&to)[NB]) {
+#pragma unroll
+        for (int rb = 0; rb < NB; ++rb) to[rb] = *as_global<u32x4>(a_src[rb] + min(pair, pairs - 1) * 128);
+    };
+    auto stash_a = [&](uint32_t buf, const u32x4 (&from)[NB]) {
+#pragma unroll
+        for (int rb = 0; rb < NB; ++rb) *reinterpret_cast<u32x4*>(a_s + (buf * kTileRowsMax + 16 * uint32_t(rb)) * kPitch + a_at) = from[rb];
+    };
+    u32x4 a_first[NB];
+    fetch_a(0, a_first); fetch_a(1, a_next);
+    // The scales of the lane's two weight rows, four groups per load (the four lanes of a row fetch the same bytes), one load
+    // ahead.  (In LDS, filled by a loop of dependent loads and stores before the walk, they cost 11 us of a workgroup's
+    // 29: nearly as much as the walk.)  A row's last load may run into the rows behind it, which the biases always follow.
+    uint32_t scales[2][2], scales_next[2][2];
+    auto fetch_s = [&](uint32_t g) {
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-            if constexpr (BITS == 4) { const uint2 v = ldg_u2(b_src[q] + g * 32); f.b[q][0] = v.x; f.b[q][1] = v.y; }
-            else { const uint4 v = ldg_u4(b_src[q] + g * 64); f.b[q][0] = v.x; f.b[q][1] = v.y; f.b[q][2] = v.z; f.b[q][3] = v.w; }
+            const uint2 v = ldg_u2_by_words(scales_of[q] + (m_at[q] + min(g, (groups - 1) / 4 * 4) * 2));
+            scales_next[q][0] = v.x; scales_next[q][1] = v.y;
         }
-        if (tall && tid < 128) f.a2 = *reinterpret_cast<const uint4*>(a_src2 + g * 64);
     };
-    auto stash = [&](uint32_t buf, const Fetched& f) {   // the token rows
-        *reinterpret_cast<uint4*>(&a_s[buf][a_r * kPitch + a_c * 8]) = f.a;
-        if (tall && tid < 128) *reinterpret_cast<uint4*>(&a_s[buf][(32 + a_r) * kPitch + a_c * 8]) = f.a2;
-    };
-    // eight codes -> eight bf16: nibble i of the word is element i
-    auto expand = [](uint32_t word) {
-        uint32_t even = word & 0x0f0f0f0fu, odd = (word >> 4) & 0x0f0f0f0fu;
-        // the masked words are kept from the optimiser, which would otherwise fold mask and shift into a bit-field extract
-        // per element and convert that: with whole bytes every element is one byte-to-float conversion
-        asm volatile("" : "+v"(even), "+v"(odd));
-        uint32_t out[4];
+    fetch_s(0);
+    f32x4 total[NB][2], mag[NB][2];   // mag: sum of the magnitudes of the folded terms, the scale of the rounding error
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const f32x2 pair = {float((even >> (8 * q)) & 0xffu), float((odd >> (8 * q)) & 0xffu)};
-            out[q] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, bf16x2));
-        }
-        return __builtin_bit_cast(bf16x8, make_uint4(out[0], out[1], out[2], out[3]));
-    };
-    // eight byte codes (two words, byte i of the pair is element i) -> eight bf16
-    auto expand_bytes = [](uint32_t lo, uint32_t hi) {
-        uint32_t out[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t word = q < 2 ? lo : hi;
-            const f32x2 pair = {float((word >> (16 * (q & 1))) & 0xffu), float((word >> (16 * (q & 1) + 8)) & 0xffu)};
-            out[q] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, bf16x2));
-        }
-        return __builtin_bit_cast(bf16x8, make_uint4(out[0], out[1], out[2], out[3]));
-    };
-
-    constexpr int kBlocks = int(kTileRowsMax / 16);
-    const int blocks = tall ? kBlocks : 2;
-    f32x4 total[kBlocks][2], mag[kBlocks][2];   // mag: sum of the magnitudes of the folded terms, the scale of the rounding error
-#pragma unroll
-    for (int rb = 0; rb < kBlocks; ++rb)
+    for (int rb = 0; rb < NB; ++rb)
 #pragma unroll
         for (int q = 0; q < 2; ++q) total[rb][q] = mag[rb][q] = f32x4{0, 0, 0, 0};
-
-    fetch(0, ahead[0]);
-    if (groups > 1) fetch(1, ahead[1]);
-    stash(0, ahead[0]);
-    __syncthreads();
-    // The bias half of the magnitudes, sum over the groups of |bias| * |chain sum|, is a product over the group index:
-    // one matrix-core instruction per accumulator tile and 32 groups instead of a multiply-add per element and step (the
-    // chain sums rounded to bf16 for it, made up for by the factor below: the magnitudes only scale a margin).
-    for (uint32_t g0 = 0; g0 < groups; g0 += 32) {
-        bf16x8 bias_abs[2];
+    // The bias half of the totals and of their magnitudes, 32 groups per instruction: three instructions (the pieces of the
+    // chain sums, smallest first) where the fold took a multiply-add per element and group, and one for the magnitudes (the
+    // first piece is the chain sum cut off to bf16, made up for by the factor: the magnitudes only scale a margin).
+    const uint32_t pitch = prefill_pitch(K);
+    const uint16_t* planes_of[NB];
+#pragma unroll
+    for (int rb = 0; rb < NB; ++rb) planes_of[rb] = p.planes + uint64_t(row_of(16 * uint32_t(rb) + j)) * (3 * pitch);
+    uint32_t g0 = 0;
+    do {   // (at least once: the compiler then knows that no load from before it is pending in the walk)
+        const uint32_t mine = g0 + 8 * g4, M = 0x7fff7fffu;
+        bf16x8 bias[2], bias_size[2];
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             uint32_t w[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const uint32_t g = g0 + 8 * g4 + 2 * uint32_t(i);
-                w[i] = g < groups ? *reinterpret_cast<const uint32_t*>(bias_s + col_row[q] * pitch + g) & 0x7fff7fffu : 0u;
+                const uint32_t g = mine + 2 * uint32_t(i), v = ldg_u32(biases_of[q] + (m_at[q] + min(g, groups - 2) * 2));
+                w[i] = g < groups ? v : 0u;
             }
-            bias_abs[q] = __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
+            bias[q] = __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
+            bias_size[q] = __builtin_bit_cast(bf16x8, make_uint4(w[0] & M, w[1] & M, w[2] & M, w[3] & M));
+        }
+        uint4 pieces[NB][3];                     // (all requested before the first is used)
+#pragma unroll
+        for (int rb = 0; rb < NB; ++rb) {
+            const uint16_t* src = planes_of[rb] + min(mine, pitch - 8);
+#pragma unroll
+            for (int w = 0; w < 3; ++w) pieces[rb][w] = ldg_u4(src + uint32_t(w) * pitch);
         }
 #pragma unroll
-        for (int rb = 0; rb < kBlocks; ++rb) {
-            if (rb >= blocks) break;
-            uint32_t w[4];
+        for (int rb = 0; rb < NB; ++rb) {
+            uint4 (&piece)[3] = pieces[rb];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t g = min(g0 + 8 * g4 + 2 * uint32_t(i), groups - 2);   // (past the end: times a zero bias)
-                const f32x2 pair = {fabsf(sum_s[g * kTileRowsMax + 16 * rb + j]), fabsf(sum_s[(g + 1) * kTileRowsMax + 16 * rb + j])};
-                w[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(pair, bf16x2));
+            for (int w = 0; w < 3; ++w) {
+                piece[w].x = mine < groups ? piece[w].x : 0u; piece[w].y = mine + 2 < groups ? piece[w].y : 0u;
+                piece[w].z = mine + 4 < groups ? piece[w].z : 0u; piece[w].w = mine + 6 < groups ? piece[w].w : 0u;
             }
-            const bf16x8 sum_abs = __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
+            const bf16x8 size = __builtin_bit_cast(bf16x8, make_uint4(piece[0].x & M, piece[0].y & M, piece[0].z & M, piece[0].w & M));
 #pragma unroll
-            for (int q = 0; q < 2; ++q) mag[rb][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sum_abs, bias_abs[q], mag[rb][q], 0, 0, 0);
+            for (int q = 0; q < 2; ++q) {
+#pragma unroll
+                for (int w = 2; w >= 0; --w) total[rb][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, piece[w]), bias[q], total[rb][q], 0, 0, 0);
+                mag[rb][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(size, bias_size[q], mag[rb][q], 0, 0, 0);
+            }
         }
-    }
+    } while ((g0 += 32) < groups);
 #pragma unroll
-    for (int rb = 0; rb < kBlocks; ++rb)
+    for (int rb = 0; rb < NB; ++rb)
 #pragma unroll
         for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int r = 0; r < 4; ++r) mag[rb][q][r] *= 1.0078125f;
-    // two steps per trip, so that the register sets are named at compile time: step g computes from LDS buffer g & 1, requests
-    // step g + 2 into the set that step g's data has just left, and stashes step g + 1 from the other set
-    auto step = [&](uint32_t g, Fetched& mine, Fetched& next) {
-        const uint32_t buf = g & 1u;
-        bf16x8 b[2][2];   // [tile][half of the lane's sixteen codes]
+    // codes -> matrix-core operand, element order 0 4 1 5 2 6 3 7: eight nibbles of a word, or eight bytes of two words
+    auto nibbles = [](uint32_t word) {
+        const uint32_t M = 0x000f000fu;
+        return __builtin_bit_cast(bf16x8, make_uint4(word & M, (word >> 4) & M, (word >> 8) & M, (word >> 12) & M));
+    };
+    auto bytes = [](uint32_t lo, uint32_t hi) {
+        return __builtin_bit_cast(bf16x8, make_uint4(__builtin_amdgcn_perm(hi, lo, 0x0c040c00u), __builtin_amdgcn_perm(hi, lo, 0x0c050c01u),
+                                                     __builtin_amdgcn_perm(hi, lo, 0x0c060c02u), __builtin_amdgcn_perm(hi, lo, 0x0c070c03u)));
+    };
+    // elements of a group that lane (j, g4) multiplies, from this one on: sixteen of them.  Q4: a load brings the four
+    // lanes of a row the four quarters of two groups; a swap between the half waves gives every lane its share of either
+    const uint32_t koff = BITS == 4 ? (g4 & 1u) * 32u + (g4 >> 1) * 16u : g4 * 16u;
+    const uint16_t* a_lane = a_s + j * kPitch + koff;
+    auto work = [&](uint32_t pair, const u32x4 (&slot)[2][kRegs / 4], u32x4 (&last)[2][kRegs / 4], const int odd) {   // odd: pair % 2, known at compile time
+        const uint32_t buf = pair & 1u;
+        // Loads return in the order they were sent, so a wait for token rows is a wait for all weights requested before them:
+        // the rows are requested two pairs before they go to LDS, ahead of the pair's weight request.
+        stash_a(buf ^ 1u, a_next);
+        fetch_a(pair + 2, a_next);
+        // (into the slot of the pair before, which nothing reads any more: loaded behind its own uses, the loop's last slot
+        // got other registers, and the copies at the loop's end waited for every load in flight)
+        fetch_b(pair + kAhead - 1, last);
+        uint32_t codes[2][kRegs];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            if constexpr (BITS == 4) { b[q][0] = expand(mine.b[q][0]); b[q][1] = expand(mine.b[q][1]); }
-            else { b[q][0] = expand_bytes(mine.b[q][0], mine.b[q][1]); b[q][1] = expand_bytes(mine.b[q][2], mine.b[q][3]); }
-        }
-        if (g + 2 < groups) fetch(g + 2, mine);
-        f32x4 dot[kBlocks][2];
+        for (int q = 0; q < 2; ++q)
 #pragma unroll
-        for (int rb = 0; rb < kBlocks; ++rb)
-#pragma unroll
-            for (int q = 0; q < 2; ++q) dot[rb][q] = f32x4{0, 0, 0, 0};
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk) {
-#pragma unroll
-            for (int rb = 0; rb < kBlocks; ++rb) {
-                if (rb >= blocks) break;
-                const bf16x8 a = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&a_s[buf][(16 * rb + j) * kPitch + g4 * 16 + kk * 8]));
-#pragma unroll
-                for (int q = 0; q < 2; ++q) dot[rb][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[q][kk], dot[rb][q], 0, 0, 0);
-            }
-        }
-        float scale[2], bias[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) { scale[q] = b16(scale_s[col_row[q] * pitch + g]); bias[q] = b16(bias_s[col_row[q] * pitch + g]); }
-#pragma unroll
-        for (int rb = 0; rb < kBlocks; ++rb) {
-            if (rb >= blocks) break;
-            const float4 sums4 = *reinterpret_cast<const float4*>(sum_s + g * kTileRowsMax + 16 * rb + 4 * g4);
-            const float sums[4] = {sums4.x, sums4.y, sums4.z, sums4.w};
+            for (int w = 0; w < kRegs; ++w) codes[q][w] = slot[q][w / 4][w % 4];
+        if constexpr (BITS == 4) {
 #pragma unroll
             for (int q = 0; q < 2; ++q)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    total[rb][q][r] = __builtin_fmaf(scale[q], dot[rb][q][r], __builtin_fmaf(bias[q], sums[r], total[rb][q][r]));
-                    mag[rb][q][r] = __builtin_fmaf(fabsf(scale[q]), fabsf(dot[rb][q][r]), mag[rb][q][r]);
+                for (int w = 0; w < 2; ++w) {
+                    const auto both = __builtin_amdgcn_permlane32_swap(codes[q][w], codes[q][w + 2], false, false);
+                    codes[q][w] = both[0]; codes[q][w + 2] = both[1];
                 }
         }
-        if (g + 1 < groups) stash(buf ^ 1u, next);
-        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            bf16x8 b[2][2];   // [tile][half of the lane's sixteen codes]
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int kk = 0; kk < 2; ++kk) {
+                    if constexpr (BITS == 4) b[q][kk] = nibbles(codes[q][2 * h + kk]);
+                    else b[q][kk] = bytes(codes[q][4 * h + 2 * kk], codes[q][4 * h + 2 * kk + 1]);
+                }
+            float scale[2];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) scale[q] = __uint_as_float(h ? scales[q][odd] & 0xffff0000u : scales[q][odd] << 16) * 0x1p33f;
+            bf16x8 a[NB][2];
+#pragma unroll
+            for (int rb = 0; rb < NB; ++rb)
+#pragma unroll
+                for (int kk = 0; kk < 2; ++kk)
+                    a[rb][kk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(a_lane + (buf * kTileRowsMax + 16 * uint32_t(rb)) * kPitch + 64 * h + 8 * kk));
+#pragma unroll
+            for (int rb = 0; rb < NB; ++rb) {
+                f32x4 dot[2];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) dot[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rb][0], b[q][0], f32x4{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+                for (int q = 0; q < 2; ++q) dot[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rb][1], b[q][1], dot[q], 0, 0, 0);
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        total[rb][q][r] = __builtin_fmaf(scale[q], dot[q][r], total[rb][q][r]);
+                        mag[rb][q][r] = __builtin_fmaf(fabsf(scale[q]), fabsf(dot[q][r]), mag[rb][q][r]);
+                    }
+            }
+        }
+        lds_barrier();
     };
-    for (uint32_t g = 0; g < groups; g += 2) {
-        step(g, ahead[0], ahead[1]);
-        if (g + 1 < groups) step(g + 1, ahead[1], ahead[0]);
+    stash_a(0, a_first);
+    lds_barrier();
+    auto next_scales = [&](uint32_t g) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) scales[q][i] = scales_next[q][i];
+        fetch_s(g);
+    };
+    // (An odd pair stands behind the loop: a way round the second half would leave the first half's loads pending at the
+    // loop's head, which then waited for all of them.)
+    uint32_t pair = 0;
+    for (; pair + 1 < pairs; pair += 2) {
+        next_scales(2 * pair + 4);
+        work(pair, ring[0], ring[1], 0);
+        work(pair + 1, ring[1], ring[0], 1);
+    }
+    if (pair < pairs) {
+        next_scales(2 * pair);
+        work(pair, ring[0], ring[1], 0);
     }
     // epilogue: row m of the tile is sorted position first + m.  A sum close to a BF16 rounding boundary could round
-    // the other way under the reference's order of additions: such elements are listed for exact recomputation.
+    // the other way under the reference's order of additions: such elements are listed for exact recomputation.  v rounds to
+    // r; the boundary next to r is half a BF16 step from it, the step that of the smallest magnitude v - e that the sum
+    // could have.  (A magnitude that is not finite, of a row or group that left the operand's range, marks the element.)
     const float margin = p.near_margin;
-    auto near_boundary = [margin](float v, float m) { const float e = m * margin; return __float_as_uint(bf(v - e)) != __float_as_uint(bf(v + e)); };
-    // One bit per output element (sorted position * N + row); every wave owns whole 16-bit pieces of the map: the sixteen
-    // lanes that share a token row hold sixteen neighbouring weight rows.
-    uint16_t* bits = reinterpret_cast<uint16_t*>(p.near_bits);
+    auto near_boundary = [margin](float v, float r, float m) {
+        const float e = m * margin, least = fabsf(v) - e;
+        return !(least > 0.0f) || fabsf(v - r) + e >= __uint_as_float(__float_as_uint(least) & 0x7f800000u) * 0x1p-8f;
+    };
+    // Outputs and marks (one bit per output element, sorted position * N + row) cross through LDS, so that they leave in
+    // whole pieces of a row: two-byte stores straight from the accumulators' lanes took longer than the walk of a short row.
+    constexpr uint32_t kCols = GATED ? 64u : 128u, kOutPitch = kPitch;
+    uint16_t* out_s = a_s;                       // (every wave has passed the walk's last barrier)
 #pragma unroll
-    for (int rb = 0; rb < kBlocks; ++rb) {
-        if (rb >= blocks) break;
+    for (int rb = 0; rb < NB; ++rb)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const uint32_t m = 16 * uint32_t(rb) + 4 * g4 + uint32_t(r);
-            const bool live = m < rows;
-            const uint32_t pos = first + (live ? m : 0u);
-            if constexpr (GATED) {
-                const uint32_t n = n0 + wave * 16 + j;
-                if (live) p.out_b[uint64_t(pos) * N + n] = uint16_t(__float_as_uint(swiglu_bf(total[rb][0][r], total[rb][1][r])) >> 16);
-                const uint64_t marks = __ballot(near_boundary(total[rb][0][r], mag[rb][0][r]) || near_boundary(total[rb][1][r], mag[rb][1][r]));
-                if (live && j == 0) bits[(uint64_t(pos) * N + n) / 16] = uint16_t(marks >> (16 * g4));
-            } else {
-                const uint32_t out_row = p.out_rows ? uint32_t(p.out_rows[pos]) : pos;
 #pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    const uint32_t n = n0 + (2 * wave + uint32_t(q)) * 16 + j;
-                    if (live) {
-                        if (p.out_h) p.out_h[uint64_t(out_row) * N + n] = uint16_t(__float_as_uint(bf(total[rb][q][r])) >> 16);
-                        else p.out_f[uint64_t(out_row) * N + n] = bf(total[rb][q][r]);
-                    }
-                    const uint64_t marks = __ballot(near_boundary(total[rb][q][r], mag[rb][q][r]));
-                    if (live && j == 0) bits[(uint64_t(pos) * N + n) / 16] = uint16_t(marks >> (16 * g4));
+            for (int q = 0; q < (GATED ? 1 : 2); ++q) {
+                const uint32_t col = GATED ? wave * 16 : (2 * wave + uint32_t(q)) * 16;
+                float value = bf(total[rb][q][r]);
+                bool near = near_boundary(total[rb][q][r], value, mag[rb][q][r]);
+                if constexpr (GATED) {
+                    const float up = bf(total[rb][1][r]);
+                    near = near | near_boundary(total[rb][1][r], up, mag[rb][1][r]);
+                    value = swiglu_rounded(value, up);
                 }
+                const uint64_t marks = __ballot(near);
+                out_s[m * kOutPitch + col + j] = uint16_t(__float_as_uint(value) >> 16);
+                if (j == 0) marks_s[m * 8 + col / 16] = uint16_t(marks >> (16 * g4));
             }
         }
+    lds_barrier();
+#pragma unroll
+    for (uint32_t i = 0; i < 16u * NB * (kCols / 8) / 256u + (16u * NB * (kCols / 8) % 256u ? 1u : 0u); ++i) {
+        const uint32_t piece = i * 256 + tid, m = piece / (kCols / 8), c = piece % (kCols / 8);
+        if (m >= rows) continue;
+        const uint32_t pos = first + m;
+        const uint4 v = *reinterpret_cast<const uint4*>(out_s + m * kOutPitch + c * 8);
+        if constexpr (GATED) {
+            *reinterpret_cast<uint4*>(p.out_b + uint64_t(pos) * N + n0 + c * 8) = v;
+            if (c == 0) *reinterpret_cast<uint2*>(p.near_bits + (uint64_t(pos) * N + n0) / 32) = *reinterpret_cast<const uint2*>(marks_s + m * 8);
+        } else {
+            const uint64_t at = uint64_t(p.out_rows ? uint32_t(p.out_rows[pos]) : pos) * N + n0 + c * 8;
+            if (p.out_h) *reinterpret_cast<uint4*>(p.out_h + at) = v;
+            else {
+                *reinterpret_cast<float4*>(p.out_f + at) = make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u));
+                *reinterpret_cast<float4*>(p.out_f + at + 4) = make_float4(__uint_as_float(v.z << 16), __uint_as_float(v.z & 0xffff0000u), __uint_as_float(v.w << 16), __uint_as_float(v.w & 0xffff0000u));
+            }
+            if (c == 0) *reinterpret_cast<uint4*>(p.near_bits + (uint64_t(pos) * N + n0) / 32) = *reinterpret_cast<const uint4*>(marks_s + m * 8);
+        }
     }
+}
+template <bool GATED, int BITS>
+__global__ __launch_bounds__(256, BITS == 4 ? 3 : 2) void prefill_gemm_kernel(PrefillGemm p) {
+    __shared__ __align__(16) uint16_t a_s[2 * kTileRowsMax * kPitch], marks_s[kTileRowsMax * 8];
+    // The workgroups of one tile (neighbours in column block) share its token rows: they go to one of the eight dies, whose
+    // L2 then fetches the rows once.
+    const uint32_t columns = GATED ? p.N / 64u : p.N / 128u, turn = blockIdx.x / 8u;
+    const uint32_t tile = turn / columns * 8u + blockIdx.x % 8u, n0 = turn % columns * (GATED ? 64u : 128u);
+    // (requested together: the lists have room for the grid's last tiles)
+    const uint32_t count = uint32_t(*p.tile_count), expert = uint32_t(p.tile_expert[tile]), first = uint32_t(p.tile_first[tile]), rows = uint32_t(p.tile_rows[tile]);
+    if (tile >= count) return;
+    if (rows <= 16) prefill_tile<GATED, BITS, 1>(p, a_s, marks_s, expert, first, rows, n0);
+    else if (rows <= 32) prefill_tile<GATED, BITS, 2>(p, a_s, marks_s, expert, first, rows, n0);
+    else prefill_tile<GATED, BITS, 3>(p, a_s, marks_s, expert, first, rows, n0);
 }
 
 // Exact recomputation of the listed elements: one group of 32 lanes plays the reference's 32 lanes for one row
@@ -519,8 +591,8 @@ __global__ __launch_bounds__(256) void prefill_patch_kernel(PrefillGemm p, uint3
     const uint32_t expert = p.ids ? uint32_t(p.ids[p.slots[pos]]) : 0u;
     if (p.ids && expert >= p.experts) continue;   // an id the router could not give (reported through the status word)
     const uint8_t* record = p.records + uint64_t(expert) * p.stride;
-    const uint32_t a_row = p.a_rows ? uint32_t(p.a_rows[pos]) / p.a_div : pos;
-    const uint16_t* xr = p.a + uint64_t(a_row) * K;
+    const uint32_t a_row = p.a_rows ? uint32_t(p.a_rows[pos]) : pos;
+    const uint16_t* xr = p.a_plain + uint64_t(a_row) * K;
     static_assert(WIDTH * BITS >= 32 && !(TABLED && BITS == 8), "a block is whole code words; the table holds Q4 chain sums");
     constexpr int DW = WIDTH * BITS / 32, XV = WIDTH >= 8 ? WIDTH / 8 : 1, kAhead = 4;   // a lane's next four blocks are fetched together: one memory latency, not four
     float result[2] = {0, 0};
@@ -644,11 +716,12 @@ __global__ __launch_bounds__(256) void row_norms_kernel(const uint16_t* a, uint3
     // (a row so small that its squares leave the normal range has no usable norm: +inf makes the caller recompute everything)
     if (lane == 0) norms[row] = sum < 0x1p-100f ? __uint_as_float(0x7f800000u) : sqrtf(sum) * 1.0001f;
 }
+constexpr uint32_t kRouterPitch = 72;   // in bf16 elements (144 bytes)
 // approx[t][e] = sum_k a[t][k] b[e][k] (+ offsets[e]): 64 tokens x 64 experts per workgroup, a wave a 32 x 32 block on
 // v_mfma_f32_32x32x16_bf16, K in steps of 64 through LDS (rows padded to 144 bytes), the next step's rows in registers.
 __global__ __launch_bounds__(256) void router_product_kernel(const uint16_t* a, const uint16_t* b, uint32_t T, uint32_t E, uint32_t K,
                                                              const float* offsets, float* approx) {
-    __shared__ __align__(16) uint16_t a_s[2][64 * kPitch], b_s[2][64 * kPitch];
+    __shared__ __align__(16) uint16_t a_s[2][64 * kRouterPitch], b_s[2][64 * kRouterPitch];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, m = lane & 31u, h = lane >> 5;
     const uint32_t t0 = blockIdx.y * 64, e0 = blockIdx.x * 64;
     const uint32_t r = tid >> 3, c8 = tid & 7u;   // a thread moves rows r and r + 32, sixteen bytes each, of both operands
@@ -662,8 +735,8 @@ __global__ __launch_bounds__(256) void router_product_kernel(const uint16_t* a, 
         rb0 = *reinterpret_cast<const uint4*>(b_src0 + g * 64); rb1 = *reinterpret_cast<const uint4*>(b_src1 + g * 64);
     };
     auto stash = [&](uint32_t buf) {
-        *reinterpret_cast<uint4*>(&a_s[buf][r * kPitch + c8 * 8]) = ra0; *reinterpret_cast<uint4*>(&a_s[buf][(r + 32) * kPitch + c8 * 8]) = ra1;
-        *reinterpret_cast<uint4*>(&b_s[buf][r * kPitch + c8 * 8]) = rb0; *reinterpret_cast<uint4*>(&b_s[buf][(r + 32) * kPitch + c8 * 8]) = rb1;
+        *reinterpret_cast<uint4*>(&a_s[buf][r * kRouterPitch + c8 * 8]) = ra0; *reinterpret_cast<uint4*>(&a_s[buf][(r + 32) * kRouterPitch + c8 * 8]) = ra1;
+        *reinterpret_cast<uint4*>(&b_s[buf][r * kRouterPitch + c8 * 8]) = rb0; *reinterpret_cast<uint4*>(&b_s[buf][(r + 32) * kRouterPitch + c8 * 8]) = rb1;
     };
     f32x16 acc;
 #pragma unroll
@@ -676,8 +749,8 @@ __global__ __launch_bounds__(256) void router_product_kernel(const uint16_t* a, 
         if (g + 1 < steps) fetch(g + 1);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const bf16x8 av = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&a_s[buf][row_a * kPitch + q * 16 + h * 8]));
-            const bf16x8 bv = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&b_s[buf][row_b * kPitch + q * 16 + h * 8]));
+            const bf16x8 av = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&a_s[buf][row_a * kRouterPitch + q * 16 + h * 8]));
+            const bf16x8 bv = __builtin_bit_cast(bf16x8, *reinterpret_cast<const uint4*>(&b_s[buf][row_b * kRouterPitch + q * 16 + h * 8]));
             acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
         }
         if (g + 1 < steps) stash(buf ^ 1u);
@@ -822,20 +895,16 @@ void launch_prefill_router(hipStream_t s, const float* x, const uint16_t* xb, co
     hipLaunchKernelGGL(router_refine_kernel, dim3((T + 3) / 4), dim3(256), 4 * K * 2, s, xb, wb, offsets, norms, T, E, K, topk, logits, ids, weights);
 }
 
-void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t K, uint16_t* xb, float* sums, float* sums16, float* plain, int32_t* status) {
-    const uint32_t items = rows * (K / 64);
-    hipLaunchKernelGGL(prefill_rows_kernel, dim3((items + 255) / 256), dim3(256), 0, s, x, rows, K, xb, sums, sums16, plain, status);
+void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain, float* sums16, int32_t* status) {
+    hipLaunchKernelGGL((prefill_rows_kernel<true>), dim3((rows * (K / 4) + 255) / 256), dim3(256), 0, s, x, rows, K, xb, xp, planes, plain, sums16, status);
 }
-void launch_prefill_sums(hipStream_t s, const uint16_t* xb, const int32_t* rows_ptr, uint32_t rows_max, uint32_t K, float* sums, float* sums16, bool plain) {
-    const uint32_t items = rows_max * (K / 64);
-    hipLaunchKernelGGL(prefill_sums_kernel, dim3((items + 255) / 256), dim3(256), 0, s, xb, rows_ptr, rows_max, K, sums, sums16, plain);
+void launch_prefill_acts(hipStream_t s, const uint16_t* xb, uint32_t rows, uint32_t K, uint16_t* xp, uint16_t* planes, uint16_t* plain, float* sums16) {
+    hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3((rows * (K / 4) + 255) / 256), dim3(256), 0, s, xb, rows, K, nullptr, xp, planes, plain, sums16, nullptr);
 }
 void launch_prefill_tiles(hipStream_t s, const int32_t* offsets, uint32_t experts, uint32_t rows, int32_t* tile_expert, int32_t* tile_first,
                           int32_t* tile_rows, int32_t* tile_count) {
     hipLaunchKernelGGL(prefill_tiles_kernel, dim3(1), dim3(1024), 0, s, offsets, experts, rows, tile_expert, tile_first, tile_rows, tile_count);
 }
-// LDS beyond the kernel's fixed arrays: the scales and biases of 128 weight rows and the chain sums of 48 token rows for
-// every step of K.
 void launch_prefill_dispatch(hipStream_t s, const int32_t* ids, uint32_t tokens, uint32_t topk, uint32_t E, int32_t* offsets, int32_t* slots, int32_t* rows,
                              int32_t* status, int32_t* tile_expert, int32_t* tile_first, int32_t* tile_rows, int32_t* tile_count) {
     const uint32_t n = tokens * topk, stretch = ((n + kDispatchParts - 1) / kDispatchParts + 1023) / 1024 * 1024;
@@ -849,16 +918,14 @@ bool prefill_dispatch_fits(const int32_t* ids, uint32_t tokens, uint32_t topk, u
     const uint64_t n = uint64_t(tokens) * topk;
     return reinterpret_cast<uintptr_t>(ids) % 16 == 0 && n > 1024 && n < (1u << 24) && E <= 1024 && n / kDispatchParts + 1024 <= 24 * 1024;
 }
-static uint32_t prefill_gemm_lds(uint32_t K) { const uint32_t groups = K / 64; return 2 * kTileCols * (groups + 2) * 2 + groups * kTileRowsMax * 4; }
 void launch_prefill_gemm(hipStream_t s, const PrefillGemm& p, bool gated, uint32_t max_tiles) {
-    const dim3 grid(gated ? p.N / 64 : p.N / 128, max_tiles);
-    const uint32_t lds = prefill_gemm_lds(p.K);
+    const dim3 grid((max_tiles + 7) / 8 * 8 * (gated ? p.N / 64 : p.N / 128));
     if (p.bits == 8) {
-        if (gated) hipLaunchKernelGGL((prefill_gemm_kernel<true, 8>), grid, dim3(256), lds, s, p);
-        else hipLaunchKernelGGL((prefill_gemm_kernel<false, 8>), grid, dim3(256), lds, s, p);
+        if (gated) hipLaunchKernelGGL((prefill_gemm_kernel<true, 8>), grid, dim3(256), 0, s, p);
+        else hipLaunchKernelGGL((prefill_gemm_kernel<false, 8>), grid, dim3(256), 0, s, p);
     } else {
-        if (gated) hipLaunchKernelGGL((prefill_gemm_kernel<true, 4>), grid, dim3(256), lds, s, p);
-        else hipLaunchKernelGGL((prefill_gemm_kernel<false, 4>), grid, dim3(256), lds, s, p);
+        if (gated) hipLaunchKernelGGL((prefill_gemm_kernel<true, 4>), grid, dim3(256), 0, s, p);
+        else hipLaunchKernelGGL((prefill_gemm_kernel<false, 4>), grid, dim3(256), 0, s, p);
     }
 }
 void launch_prefill_patch(hipStream_t s, const PrefillGemm& p, bool gated) {
@@ -874,7 +941,7 @@ void launch_prefill_patch(hipStream_t s, const PrefillGemm& p, bool gated) {
     else { if (tabled) ZC_PATCH(16, false, true, 4); else if (wide) ZC_PATCH(16, false, false, 4); else ZC_PATCH(8, false, false, 4); }
 #undef ZC_PATCH
 }
-// (hidden and intermediate sizes up to 4096: the product kernel keeps a whole K of scales, biases and chain sums in LDS)
+// (hidden and intermediate sizes up to 4096: the margins of the recomputation are measured up to there)
 bool prefill_shape(uint32_t hidden, uint32_t inter, uint32_t experts) {
     return hidden % 128 == 0 && inter % 128 == 0 && hidden <= 4096 && inter <= 4096 && experts <= 1024;
 }
