@@ -16,8 +16,10 @@
 //
 // Codes as operands.  The matrix cores take subnormal bf16 operands at full precision, and the bit pattern of an integer
 // code 0..255 read as bf16 is the number code * 2^-133: a code needs no conversion, only its place in a 16-bit half, one
-// mask (and shift) per two codes where the conversion to a float and on to bf16 took 3 instructions per two codes, each
-// at half rate.  The token rows carry 2^100 to stay in range, the scales the remaining 2^33: both exact.
+// mask and shift per two codes where the conversion to a float and on to bf16 took 3 instructions per two codes, each
+// at half rate.  The token rows carry 2^100 to stay in range, the scales the rest: both exact.  An instruction drops what
+// lies 24 bits below its largest exponent sum, and a subnormal's exponent counts as that of 2^-126: nibbles stand three bits
+// up (code * 2^-130), so that at most one of those bits is empty.
 // Nibbles i and i + 4 of a word share one mask, so the rows are stored with every eight elements in the order
 // 0 4 1 5 2 6 3 7.  Groups whose values would leave the exact range (|x| >= 2^26, all below 2^-60, inf, NaN) get a NaN
 // chain sum: every output of such a row is then recomputed with the lane arithmetic.
@@ -398,8 +400,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
             for (int r = 0; r < 4; ++r) mag[rb][q][r] *= 1.0078125f;
     // codes -> matrix-core operand, element order 0 4 1 5 2 6 3 7: eight nibbles of a word, or eight bytes of two words
     auto nibbles = [](uint32_t word) {
-        const uint32_t M = 0x000f000fu;
-        return __builtin_bit_cast(bf16x8, make_uint4(word & M, (word >> 4) & M, (word >> 8) & M, (word >> 12) & M));
+        const uint32_t M = 0x00780078u;
+        return __builtin_bit_cast(bf16x8, make_uint4((word << 3) & M, (word >> 1) & M, (word >> 5) & M, (word >> 9) & M));
     };
     auto bytes = [](uint32_t lo, uint32_t hi) {
         return __builtin_bit_cast(bf16x8, make_uint4(__builtin_amdgcn_perm(hi, lo, 0x0c040c00u), __builtin_amdgcn_perm(hi, lo, 0x0c050c01u),
@@ -444,7 +446,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
                 }
             float scale[2];
 #pragma unroll
-            for (int q = 0; q < 2; ++q) scale[q] = __uint_as_float(h ? scales[q][odd] & 0xffff0000u : scales[q][odd] << 16) * 0x1p33f;
+            for (int q = 0; q < 2; ++q) scale[q] = __uint_as_float(h ? scales[q][odd] & 0xffff0000u : scales[q][odd] << 16) * (BITS == 4 ? 0x1p30f : 0x1p33f);
             bf16x8 a[NB][2];
 #pragma unroll
             for (int rb = 0; rb < NB; ++rb)
