@@ -608,43 +608,43 @@ zc_status zc_hip_moe_forward(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
     const uint32_t H = c->hidden, I = c->inter, E = c->experts, k = c->topk;
     // 1-2. router logits, top-k + softmax (model.cpp:434-436)
     zc::launch_router(s, l->router, x, T, H, E, l->router_offsets, w.logits);
-    zc::launch_route(s, w.logits, T, E, k, w.ids, w.weights);
-    // 4. positions / selected, on the device (model.cpp:449-479)
-    zc::launch_dispatch(s, w.ids, T, k, E, w.offsets, w.slots, w.rows, w.selected, w.count, ctx->moe_status);
-    // 5. shared expert and its gate (model.cpp:482-485)
-    zc_linear g, u, d;
-    zc_hip_expert_linear(c, 1, l->shared_record, 0, &g); zc_hip_expert_linear(c, 1, l->shared_record, 1, &u); zc_hip_expert_linear(c, 1, l->shared_record, 2, &d);
-    { zc::AffineDesc a; a.gate = g; a.up = u; a.gated = true; a.x = x; a.out = w.shared_act; a.tokens = T; zc::launch_affine(s, a); }
-    { zc::AffineDesc a; a.gate = d; a.x = w.shared_act; a.out = w.shared; a.tokens = T; zc::launch_affine(s, a); }
+    // 4. positions / selected, on the device (model.cpp:449-479): the expert kernels' job list, at most `chunk` tokens a job
+    const uint32_t chunk = std::min(zc::affine_job_tokens(H, I, c->bits_gate_up), zc::affine_job_tokens(I, H, c->bits_down));
+    uint32_t* jobs = reinterpret_cast<uint32_t*>(w.rows);   // (n words: a job holds at least one slot)
+    zc::launch_route_jobs(s, w.logits, T, E, k, w.ids, w.weights, w.offsets, w.slots, chunk, jobs, w.count, w.selected, ctx->moe_status);
     zc::launch_plain(s, l->shared_gate, 0, x, H, 1, T, w.gate, false);
-    // 6. routed experts (pipeline.cpp:18-29): gate/up on gathered rows, down scattered to its slot
-    zc_linear rg, ru, rd;
-    zc_hip_expert_linear(c, 0, l->expert_records, 0, &rg); zc_hip_expert_linear(c, 0, l->expert_records, 1, &ru); zc_hip_expert_linear(c, 0, l->expert_records, 2, &rd);
-    const auto base = reinterpret_cast<uintptr_t>(l->expert_records);
-    auto off = [&](const void* p) { return uint64_t(reinterpret_cast<uintptr_t>(p) - base); };
-    const uint32_t jobs = uint32_t(std::min<uint64_t>(uint64_t(T) * k, E));
-    {
+    // 5-6. shared expert (model.cpp:482-485) and routed experts (pipeline.cpp:18-29): gate/up on gathered rows, down scattered
+    // to its slot.  One launch per phase where the shared expert's projections have the routed ones' width.
+    auto offsets_of = [&](const void* record, int shared, uint64_t* off, int first, int count) {
+        for (int q = 0; q < count; ++q) {
+            zc_linear lin; zc_hip_expert_linear(c, shared, record, first + q, &lin);
+            const auto base = reinterpret_cast<uintptr_t>(record);
+            off[3 * q] = reinterpret_cast<uintptr_t>(lin.weight) - base; off[3 * q + 1] = reinterpret_cast<uintptr_t>(lin.scales) - base;
+            off[3 * q + 2] = reinterpret_cast<uintptr_t>(lin.biases) - base;
+        }
+    };
+    const uint64_t n = uint64_t(T) * k;
+    for (const bool gated : {true, false}) {
         zc::ExpertPhaseDesc p{};
-        p.records = l->expert_records; p.stride = l->record_stride;
-        p.off[0] = off(rg.weight); p.off[1] = off(rg.scales); p.off[2] = off(rg.biases);
-        p.off[3] = off(ru.weight); p.off[4] = off(ru.scales); p.off[5] = off(ru.biases);
-        p.offsets = w.offsets; p.selected = w.selected; p.count = w.count; p.in_rows = w.rows; p.out_rows = nullptr;
-        p.x = x; p.out = w.act; p.K = H; p.N = I; p.group = c->group; p.bits = c->bits_gate_up; p.x_sorted = 0; p.max_jobs = jobs; p.gated = true;
-        zc::launch_expert_phase(s, p);
-    }
-    {
-        zc::ExpertPhaseDesc p{};
-        p.records = l->expert_records; p.stride = l->record_stride;
-        p.off[0] = off(rd.weight); p.off[1] = off(rd.scales); p.off[2] = off(rd.biases);
-        p.offsets = w.offsets; p.selected = w.selected; p.count = w.count; p.in_rows = nullptr; p.out_rows = w.slots;
-        p.x = w.act; p.out = w.expert_out; p.K = I; p.N = H; p.group = c->group; p.bits = c->bits_down; p.x_sorted = 1; p.max_jobs = jobs; p.gated = false;
+        const int first = gated ? 0 : 2, count = gated ? 2 : 1;
+        p.records = l->expert_records; p.stride = l->record_stride; offsets_of(l->expert_records, 0, p.off, first, count);
+        p.jobs = jobs; p.count = w.count; p.slots = w.slots; p.topk = k; p.tokens = T; p.chunk = chunk;
+        p.max_jobs = uint32_t(std::min(n, std::min<uint64_t>(n, E) + n / chunk));
+        p.K = gated ? H : I; p.N = gated ? I : H; p.group = c->group; p.bits = gated ? c->bits_gate_up : c->bits_down; p.gated = gated;
+        p.x = gated ? x : w.act; p.out = gated ? w.act : w.expert_out; p.shared_x = gated ? x : w.shared_act; p.shared_out = gated ? w.shared_act : w.shared;
+        if ((gated ? c->shared_bits_gate_up : c->shared_bits_down) == p.bits) { p.shared_record = l->shared_record; offsets_of(l->shared_record, 1, p.shared_off, first, count); }
+        else {
+            zc::AffineDesc a; a.gated = gated; a.x = p.shared_x; a.out = p.shared_out; a.tokens = T;
+            zc_hip_expert_linear(c, 1, l->shared_record, first, &a.gate);
+            if (gated) zc_hip_expert_linear(c, 1, l->shared_record, 1, &a.up);
+            zc::launch_affine(s, a);
+        }
         zc::launch_expert_phase(s, p);
     }
     // 7. weighted combine (model.cpp:553-556)
     zc::launch_moe_sum(s, w.expert_out, w.weights, w.shared, w.gate, T, H, k, out);
     ZC_LAUNCHED();
     if (trace) {
-        const uint64_t n = uint64_t(T) * k;
         if (trace->logits) ZC_HIP(hipMemcpyAsync(trace->logits, w.logits, uint64_t(T) * E * 4, hipMemcpyDeviceToDevice, s));
         if (trace->ids) ZC_HIP(hipMemcpyAsync(trace->ids, w.ids, n * 4, hipMemcpyDeviceToDevice, s));
         if (trace->weights) ZC_HIP(hipMemcpyAsync(trace->weights, w.weights, n * 4, hipMemcpyDeviceToDevice, s));

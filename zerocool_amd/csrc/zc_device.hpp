@@ -49,18 +49,6 @@ __device__ __forceinline__ float sigmoid_bf(float x) {
 __device__ __forceinline__ float swiglu_rounded(float g, float u) { return bf(bf(g * sigmoid_bf(g)) * u); }   // g, u: BF16 values
 __device__ __forceinline__ float swiglu_bf(float gate_sum, float up_sum) { return swiglu_rounded(bf(gate_sum), bf(up_sum)); }
 
-// Sum over the 32 reference lanes as an xor butterfly with strides 16,8,4,2,1.
-// A 64-lane wavefront carries two independent 32-lane groups; strides below 32
-// never cross between them.  Every lane of a group ends with the same value.
-__device__ __forceinline__ float lane_sum32(float v) {
-    v = v + __shfl_xor(v, 16);
-    v = v + __shfl_xor(v, 8);
-    v = v + __shfl_xor(v, 4);
-    v = v + __shfl_xor(v, 2);
-    v = v + __shfl_xor(v, 1);
-    return v;
-}
-
 // Read-only data in device memory, addressed in the GLOBAL address space.  A pointer that
 // was itself loaded from memory is generic to the compiler; generic loads share the LDS
 // wait counter, so waiting for an LDS read would also wait for every weight prefetch.
@@ -76,6 +64,12 @@ __device__ __forceinline__ uint2 ldg_u2(const void* p, uint32_t index = 0) {
     const u32x2 v = as_global<u32x2>(p)[index];
     return make_uint2(v.x, v.y);
 }
+// Eight bytes whose address is a multiple of four only.
+__device__ __forceinline__ uint2 ldg_u2_by_words(const void* p) {
+    typedef uint32_t words __attribute__((ext_vector_type(2), aligned(4)));
+    const words v = *as_global<words>(p);
+    return make_uint2(v.x, v.y);
+}
 __device__ __forceinline__ uint16_t ldg_u16(const void* p, uint32_t index = 0) { return as_global<uint16_t>(p)[index]; }
 __device__ __forceinline__ uint32_t ldg_u32(const void* p, uint32_t index = 0) { return as_global<uint32_t>(p)[index]; }
 __device__ __forceinline__ float ldg_f32(const void* p, uint32_t index = 0) { return as_global<float>(p)[index]; }
@@ -87,6 +81,20 @@ __device__ __forceinline__ float dpp_row_shr1(float v) {
 }
 template <int CTRL> __device__ __forceinline__ float dpp_f32(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+// Sum over the 32 reference lanes as an xor butterfly with strides 16,8,4,2,1.
+// A 64-lane wavefront carries two independent 32-lane groups; strides below 32
+// never cross between them.  Every lane of a group ends with the same value.
+// (Moves inside the vector unit: behind stride 8 the values repeat every eight lanes, so a rotation by four is the stride-4
+// exchange; a permute through LDS per stride took five LDS latencies.)
+__device__ __forceinline__ float lane_sum32(float v) {
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
+    v = v + dpp_f32<0x128>(v);   // row_ror:8
+    v = v + dpp_f32<0x124>(v);   // row_ror:4
+    v = v + dpp_f32<0x4e>(v);    // quad_perm [2,3,0,1]
+    v = v + dpp_f32<0xb1>(v);    // quad_perm [1,0,3,2]
+    return v;
 }
 // Maximum over the 64 lanes, returned in every lane: four DPP steps inside each row
 // (quad swaps, half mirror, mirror), then the four row values through scalar lanes.

@@ -4,138 +4,293 @@
 // wavefront carries two output rows.  Results are bit-identical to the CPU statement
 // of the same arithmetic for any input.
 #include "zc_kernels.hpp"
+#include <algorithm>
 #include <type_traits>
 #include "zc_device.hpp"
+#include "zc_decode_common.hpp"   // lds_barrier; route_token: top-k + softmax of one token by one wavefront
 
 namespace zc {
 
 // ---------------------------------------------------------------------------
 // Affine Q4 / Q8 rows (reference: qwen.metal:46-81, 112-144)
+//
+// A half wave plays the 32 reference lanes of one output row: lane l takes the row's blocks l, l + 32, ... of WIDTH elements
+// (Q4 16|8, Q8 8|4: one or two dwords of codes) in order.  It walks two rows at a time (gate and up, or two rows of the one
+// matrix), so that an input block read from LDS serves two rows, and up to four tokens, so that a code is expanded once for
+// four products.  The walk over (row tile, block step) is one flat loop: the codes and scales of its next three steps are in
+// flight, across row tiles too, and the first three are requested before the input rows are staged.
+//
+// The products x * q of a BF16-valued row (magnitudes below 2^100) are exact in fp32, so a fused multiply-add rounds as the
+// reference's multiply and add do: EXACT saves three of eight instructions per four elements.  Rows that hold anything
+// else, infinities and NaN among them, keep the separate operations.
+//
+// What bounds it: with one token per row, the latency of the chain job -> row index -> input row -> LDS -> codes (a launch
+// of a few us); with several, the vector instructions: 1.5 per weight and token, 1.4 per weight for the expansion.
+// One token at a time, codes requested step by step behind the staging, every reduction through LDS permutes and the shared
+// expert in launches of its own took, per layer of hidden 2560 and intermediate 640: 40 tokens 397 us for gate/up and 310 us
+// for down against 172 and 132 us, one token 20.2 and 14.3 us against 12.5 and 9.2 us.
 // ---------------------------------------------------------------------------
-// WIDTH = elements one lane takes per step: Q4 16|8, Q8 8|4; always 1 or 2 dwords.
-template <int BITS, int WIDTH>
-struct Block {
+constexpr uint32_t kAffineTokens = 4;                                            // tokens a workgroup multiplies at once, at most
+constexpr uint32_t kAffineAhead = 3;                                             // steps in flight
+struct AffineMatrix { const uint8_t* w; const uint16_t *s, *b; };
+
+// Input rows in LDS, per token: WIDTH / 4 planes of sixteen-byte pieces, piece (plane, block), then the blocks' bias sums.
+// Lanes read the pieces of neighbouring blocks; the pitch makes the staging's writes, four neighbouring pieces in as many
+// planes, meet different banks.
+template <int WIDTH> __host__ __device__ constexpr uint32_t affine_pitch(uint32_t blocks) { return WIDTH == 4 ? blocks : (blocks + 15) / 16 * 16 + 4; }
+template <int WIDTH> __host__ __device__ constexpr uint32_t affine_token_bytes(uint32_t K) {
+    return WIDTH / 4 * affine_pitch<WIDTH>(K / WIDTH) * 16 + (K / WIDTH + 3) / 4 * 16;
+}
+
+template <int BITS, int WIDTH, bool GATED>
+struct AffineStream {
     static constexpr int DW = WIDTH * BITS / 32;
-    // x-only part of the bias term.
-    __device__ static float xsum(const float* xb) {
-        float sum = 0;
-        if constexpr (BITS == 4) {
+    struct Slot { uint32_t q[2][DW]; uint32_t s[2], b[2]; };
+    static constexpr uint32_t kTileRows = GATED ? 8 : 16;   // rows of a workgroup's tile: eight half waves, one or two each
+    uint32_t K, N, blocks, groups, shift, steps, lane, half, tile, end, step;   // tile, step: the next one to request
+    AffineMatrix m[2];
+    const uint8_t* w[2]; const uint16_t *s[2], *b[2];
+    __device__ __forceinline__ uint32_t row(uint32_t t, int q) const { return GATED ? t * 8 + half : t * 16 + uint32_t(q) * 8 + half; }
+    __device__ __forceinline__ void aim() {
 #pragma unroll
-            for (int i = 0; i < WIDTH; i += 4) sum += bf(bf(bf(xb[i] + xb[i + 1]) + xb[i + 2]) + xb[i + 3]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < WIDTH; ++i) sum += xb[i];
+        for (int q = 0; q < 2; ++q) {
+            const uint64_t r = min(row(tile, q), N - 1);
+            const AffineMatrix& a = m[GATED ? q : 0];
+            w[q] = a.w + r * (K / 8 * BITS); s[q] = a.s + r * groups; b[q] = a.b + r * groups;
         }
-        return sum;
     }
-    __device__ static float dot(const uint32_t* words, const float* xb) {
-        float dot = 0;
-        if constexpr (BITS == 4) {
+    __device__ __forceinline__ void fetch(Slot& slot) {   // past the end: the last tile again, not used
+        const uint32_t at = min(step * 32 + lane, blocks - 1), g = (at * WIDTH) >> shift;
 #pragma unroll
-            for (int i = 0; i < WIDTH; i += 4) {
-                const uint32_t packed = (words[i / 8] >> (4 * (i % 8))) & 0xffffu;
-                dot += xb[i] * float(packed & 15u) + xb[i + 1] * float((packed >> 4) & 15u) +
-                       xb[i + 2] * float((packed >> 8) & 15u) + xb[i + 3] * float((packed >> 12) & 15u);
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < WIDTH; ++i) dot += xb[i] * float((words[i / 4] >> (8 * (i % 4))) & 255u);
+        for (int q = 0; q < 2; ++q) {
+            if constexpr (DW == 2) { const uint2 v = ldg_u2_by_words(w[q] + at * 8); slot.q[q][0] = v.x; slot.q[q][DW - 1] = v.y; }
+            else slot.q[q][0] = ldg_u32(w[q], at);
+            slot.s[q] = ldg_u16(s[q], g); slot.b[q] = ldg_u16(b[q], g);
         }
-        return dot;
+        if (++step == steps) { step = 0; if (tile + 1 < end) { ++tile; aim(); } }
     }
 };
+template <int BITS, int WIDTH>
+__device__ __forceinline__ void affine_codes(const uint32_t* words, float* code) {
+    if constexpr (BITS == 4) {
+#pragma unroll
+        for (int i = 0; i < WIDTH; i += 8) {   // the even and the odd nibbles as bytes: one byte-to-float instruction each
+            const uint32_t even = words[i / 8] & 0x0f0f0f0fu, odd = (words[i / 8] >> 4) & 0x0f0f0f0fu;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) { code[i + 2 * k] = float((even >> (8 * k)) & 0xffu); code[i + 2 * k + 1] = float((odd >> (8 * k)) & 0xffu); }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < WIDTH; ++i) code[i] = float((words[i / 4] >> (8 * (i % 4))) & 255u);
+    }
+}
+template <int BITS, int WIDTH, bool EXACT>
+__device__ __forceinline__ float affine_dot(const float* code, const float* x) {
+    float dot = 0;
+    if constexpr (BITS == 4) {
+#pragma unroll
+        for (int i = 0; i < WIDTH; i += 4) {
+            if constexpr (EXACT) dot += __builtin_fmaf(x[i + 3], code[i + 3], __builtin_fmaf(x[i + 2], code[i + 2], __builtin_fmaf(x[i + 1], code[i + 1], x[i] * code[i])));
+            else dot += x[i] * code[i] + x[i + 1] * code[i + 1] + x[i + 2] * code[i + 2] + x[i + 3] * code[i + 3];
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < WIDTH; ++i) { if constexpr (EXACT) dot = __builtin_fmaf(x[i], code[i], dot); else dot += x[i] * code[i]; }
+    }
+    return dot;
+}
+// The bias half's input sum of one block.
+template <int BITS, int WIDTH>
+__device__ __forceinline__ float affine_sum(const float* x) {
+    float sum = 0;
+    if constexpr (BITS == 4) {
+#pragma unroll
+        for (int i = 0; i < WIDTH; i += 4) sum += bf(bf(bf(x[i] + x[i + 1]) + x[i + 2]) + x[i + 3]);
+    } else {
+#pragma unroll
+        for (int i = 0; i < WIDTH; ++i) sum += x[i];
+    }
+    return sum;
+}
+
+// The walk for nt staged tokens; out_at: lane t < nt (of each half wave) holds where token t's output row begins.
+// (nt and exact are the same in every lane.  As template parameters they made eight walks, whose common first steps the
+// compiler moved in front of the choice between them: 200 registers instead of 144.)
+template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS>
+__device__ __forceinline__ void affine_walk(AffineStream<BITS, WIDTH, GATED>& st, typename AffineStream<BITS, WIDTH, GATED>::Slot (&ring)[kAffineAhead],
+                                            const uint8_t* lds, float* out, uint64_t out_at, uint32_t tile, bool float_output, uint32_t nt, bool exact) {
+    const uint32_t blocks = st.blocks, pitch = affine_pitch<WIDTH>(blocks), token = affine_token_bytes<WIDTH>(st.K), lane = st.lane;
+    const uint32_t total = (st.end - tile) * st.steps;
+    float r[TOKENS][2];
+#pragma unroll
+    for (uint32_t t = 0; t < TOKENS; ++t) r[t][0] = r[t][1] = 0;
+    uint32_t step = 0;
+    for (uint32_t i0 = 0; i0 < total; i0 += kAffineAhead) {
+#pragma unroll
+        for (uint32_t d = 0; d < kAffineAhead; ++d) {
+            if (i0 + d >= total) break;
+            float code[2][WIDTH], scale[2], bias[2];
+            uint32_t words[2][AffineStream<BITS, WIDTH, GATED>::DW];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+#pragma unroll
+                for (uint32_t i = 0; i < AffineStream<BITS, WIDTH, GATED>::DW; ++i) words[q][i] = ring[d].q[q][i];
+                if constexpr (TOKENS > 1) affine_codes<BITS, WIDTH>(words[q], code[q]);
+                scale[q] = b16(uint16_t(ring[d].s[q])); bias[q] = b16(uint16_t(ring[d].b[q]));
+            }
+            st.fetch(ring[d]);
+            const uint32_t b = step * 32 + lane, at = min(b, blocks - 1);
+#pragma unroll
+            for (uint32_t t = 0; t < TOKENS; ++t) {
+                if (t >= nt) break;
+                const uint8_t* row = lds + t * token;
+                float x[WIDTH];
+#pragma unroll
+                for (int i = 0; i < WIDTH; i += 4) {
+                    const float4 v = reinterpret_cast<const float4*>(row)[uint32_t(i / 4) * pitch + at];
+                    x[i] = v.x; x[i + 1] = v.y; x[i + 2] = v.z; x[i + 3] = v.w;
+                }
+                const float sum = reinterpret_cast<const float*>(row + WIDTH / 4 * pitch * 16)[at];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    if constexpr (TOKENS == 1) {   // (one matrix's codes at a time: four waves per SIMD)
+                        __builtin_amdgcn_sched_barrier(0);
+                        affine_codes<BITS, WIDTH>(words[q], code[q]);
+                    }
+                    const float dot = exact ? affine_dot<BITS, WIDTH, true>(code[q], x) : affine_dot<BITS, WIDTH, false>(code[q], x);
+                    const float more = r[t][q] + (scale[q] * dot + sum * bias[q]);
+                    r[t][q] = b < blocks ? more : r[t][q];
+                }
+            }
+            if (++step < st.steps) continue;
+            step = 0;
+#pragma unroll
+            for (uint32_t t = 0; t < TOKENS; ++t) { if (t < nt) { r[t][0] = lane_sum32(r[t][0]); r[t][1] = lane_sum32(r[t][1]); } }
+            // every lane has all the sums: lane t finishes token t
+            float v[2] = {r[0][0], r[0][1]};
+#pragma unroll
+            for (uint32_t t = 1; t < TOKENS; ++t) { if (lane == t) { v[0] = r[t][0]; v[1] = r[t][1]; } }
+            if constexpr (GATED) {
+                const uint32_t row = st.row(tile, 0);
+                const float y = swiglu_bf(v[0], v[1]);
+                if (lane < nt && row < st.N) out[out_at + row] = y;
+            } else {
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const uint32_t row = st.row(tile, q);
+                    if (lane < nt && row < st.N) out[out_at + row] = float_output ? v[q] : bf(v[q]);
+                }
+            }
+#pragma unroll
+            for (uint32_t t = 0; t < TOKENS; ++t) r[t][0] = r[t][1] = 0;
+            ++tile;
+        }
+    }
+}
+
+// Rows tile0 .. end - 1 (tiles) of the matrices for nt <= TOKENS tokens: input row in_row(t), output row out_row(t).
+template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS, class InRow, class OutRow>
+__device__ __forceinline__ void affine_rows(const AffineMatrix (&m)[2], uint32_t K, uint32_t N, uint32_t group, const float* x, float* out, uint32_t nt,
+                                            InRow in_row, OutRow out_row, uint32_t tile0, uint32_t end, bool float_output, uint8_t* lds) {
+    using Stream = AffineStream<BITS, WIDTH, GATED>;
+    __shared__ uint32_t strange_s[4];
+    const uint32_t tid = threadIdx.x;
+    Stream st;
+    st.K = K; st.N = N; st.blocks = K / WIDTH; st.shift = group == 64 ? 6 : 5; st.groups = K >> st.shift; st.steps = (st.blocks + 31) / 32;
+    st.lane = tid & 31u; st.half = tid >> 5; st.tile = tile0; st.end = end; st.step = 0;
+    st.m[0] = m[0]; st.m[1] = m[1];
+    const uint32_t from = st.lane < nt ? in_row(st.lane) : 0u;   // lane t: token t's input row
+    const uint64_t out_at = uint64_t(st.lane < nt ? out_row(st.lane) : 0u) * N;
+    typename Stream::Slot ring[kAffineAhead];
+    st.aim();
+#pragma unroll
+    for (uint32_t d = 0; d < kAffineAhead; ++d) st.fetch(ring[d]);
+    constexpr uint32_t kPlanes = WIDTH / 4;
+    const uint32_t blocks = st.blocks, pitch = affine_pitch<WIDTH>(blocks), token = affine_token_bytes<WIDTH>(K);
+    bool strange = false;
+#pragma unroll 1
+    for (uint32_t t = 0; t < nt; ++t) {
+        const float* src = x + uint64_t(uint32_t(__builtin_amdgcn_readlane(int(from), int(t)))) * K;
+#pragma unroll 2
+        for (uint32_t i = tid; i < K / 4; i += 256) {
+            const uint4 v = ldg_u4(src, i);
+            strange |= ((v.x | v.y | v.z | v.w) & 0xffffu) != 0 ||
+                       max(max(v.x & 0x7fffffffu, v.y & 0x7fffffffu), max(v.z & 0x7fffffffu, v.w & 0x7fffffffu)) >= 0x71800000u;   // 2^100
+            reinterpret_cast<uint4*>(lds + t * token)[i % kPlanes * pitch + i / kPlanes] = v;
+        }
+    }
+    if (__ballot(strange)) strange = true;
+    if ((tid & 63u) == 0) strange_s[tid >> 6] = strange;
+    lds_barrier();
+#pragma unroll 1
+    for (uint32_t t = 0; t < nt; ++t)
+#pragma unroll 1
+        for (uint32_t b = tid; b < blocks; b += 256) {
+            float xb[WIDTH];
+#pragma unroll
+            for (int i = 0; i < WIDTH; i += 4) {
+                const float4 v = reinterpret_cast<const float4*>(lds + t * token)[uint32_t(i / 4) * pitch + b];
+                xb[i] = v.x; xb[i + 1] = v.y; xb[i + 2] = v.z; xb[i + 3] = v.w;
+            }
+            reinterpret_cast<float*>(lds + t * token + kPlanes * pitch * 16)[b] = affine_sum<BITS, WIDTH>(xb);
+        }
+    lds_barrier();
+    const bool exact = __builtin_amdgcn_readfirstlane(int(strange_s[0] | strange_s[1] | strange_s[2] | strange_s[3])) == 0;
+    affine_walk<BITS, WIDTH, GATED, TOKENS>(st, ring, lds, out, out_at, tile0, float_output, nt, exact);
+}
 
 struct AffineJob {
-    const uint8_t *w0, *w1;          // gate (or the only matrix), up
-    const uint16_t *s0, *b0, *s1, *b1;
+    AffineMatrix m[2];               // gate (or the only matrix), up
     const float* x;                  // input rows, K floats each
     const int32_t* in_rows;          // gather of input rows, or null
     const int32_t* out_rows;         // scatter of output rows, or null
     float* out;                      // output rows, N floats each
-    uint32_t K, N, group, tokens;
-    uint32_t float_output;
+    uint32_t K, N, group, tokens, chunk, float_output;   // chunk: tokens of a workgroup
+    uint32_t tiles, share;           // row tiles, and how many of them a workgroup takes
 };
-
-constexpr int kRowsPerBlock = 8;     // 256 threads = 8 groups of 32 reference lanes
-
-template <int BITS, int WIDTH, bool GATED>
-__device__ __forceinline__ void affine_rows(const AffineJob& j, uint32_t tile, float* lds_x, float* lds_sum) {
-    using B = Block<BITS, WIDTH>;
-    const uint32_t tid = threadIdx.x, lane = tid & 31u, row = tile * kRowsPerBlock + (tid >> 5);
-    const uint32_t K = j.K, blocks = K / WIDTH, groups = K / j.group;
-    const uint32_t row_dwords = K * BITS / 32;
-    for (uint32_t t = 0; t < j.tokens; ++t) {
-        const float* xr = j.x + uint64_t(j.in_rows ? uint32_t(j.in_rows[t]) : t) * K;
-        __syncthreads();
-        for (uint32_t i = tid; i < K / 4; i += blockDim.x)
-            reinterpret_cast<float4*>(lds_x)[i] = reinterpret_cast<const float4*>(xr)[i];
-        __syncthreads();
-        for (uint32_t b = tid; b < blocks; b += blockDim.x) lds_sum[b] = B::xsum(lds_x + b * WIDTH);
-        __syncthreads();
-        if (row >= j.N) continue;
-        float r0 = 0, r1 = 0;
-        const uint32_t* w0 = reinterpret_cast<const uint32_t*>(j.w0) + uint64_t(row) * row_dwords;
-        const uint32_t* w1 = GATED ? reinterpret_cast<const uint32_t*>(j.w1) + uint64_t(row) * row_dwords : nullptr;
-        for (uint32_t b = lane; b < blocks; b += 32) {
-            uint32_t q0[B::DW], q1[B::DW];
-#pragma unroll
-            for (int d = 0; d < B::DW; ++d) {
-                q0[d] = w0[b * B::DW + d];
-                if constexpr (GATED) q1[d] = w1[b * B::DW + d];
-            }
-            float xb[WIDTH];
-#pragma unroll
-            for (int i = 0; i < WIDTH; i += 4) {
-                const float4 v = *reinterpret_cast<const float4*>(lds_x + b * WIDTH + i);
-                xb[i] = v.x; xb[i + 1] = v.y; xb[i + 2] = v.z; xb[i + 3] = v.w;
-            }
-            const uint32_t g = row * groups + (b * WIDTH) / j.group;
-            const float sum = lds_sum[b];
-            r0 += b16(j.s0[g]) * B::dot(q0, xb) + sum * b16(j.b0[g]);
-            if constexpr (GATED) r1 += b16(j.s1[g]) * B::dot(q1, xb) + sum * b16(j.b1[g]);
-        }
-        r0 = lane_sum32(r0);
-        if constexpr (GATED) r1 = lane_sum32(r1);
-        if (lane == 0) {
-            float* o = j.out + uint64_t(j.out_rows ? uint32_t(j.out_rows[t]) : t) * j.N + row;
-            if constexpr (GATED) *o = swiglu_bf(r0, r1);
-            else *o = j.float_output ? r0 : bf(r0);
-        }
+template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS>
+__global__ __launch_bounds__(256, 3) void affine_op_kernel(AffineJob j) {
+    extern __shared__ __align__(16) uint8_t affine_lds[];
+    const uint32_t tile0 = blockIdx.x * j.share, end = min(tile0 + j.share, j.tiles);
+    for (uint32_t t0 = blockIdx.y * j.chunk; t0 < j.tokens; t0 += gridDim.y * j.chunk) {
+        affine_rows<BITS, WIDTH, GATED, TOKENS>(j.m, j.K, j.N, j.group, j.x, j.out, min(j.chunk, j.tokens - t0),
+                                        [&](uint32_t t) { return j.in_rows ? uint32_t(j.in_rows[t0 + t]) : t0 + t; },
+                                        [&](uint32_t t) { return j.out_rows ? uint32_t(j.out_rows[t0 + t]) : t0 + t; }, tile0, end, j.float_output != 0, affine_lds);
+        lds_barrier();   // (the next tokens overwrite the rows)
     }
 }
 
-template <int BITS, int WIDTH, bool GATED>
-__global__ __launch_bounds__(256) void affine_op_kernel(AffineJob j) {
-    extern __shared__ float lds[];
-    affine_rows<BITS, WIDTH, GATED>(j, blockIdx.x, lds, lds + j.K);
-}
-
-// Routed experts of one layer: blockIdx.y walks the selected experts that the
-// dispatch kernel listed; jobs past the device-side count exit at once.
+// The routed experts of one layer and, where its formats are theirs, the shared expert: blockIdx.y walks the shared expert's
+// tokens, chunk by chunk, then the list of (expert, sorted positions) that the dispatch left; jobs past the device-side count exit.
 struct ExpertPhase {
-    const uint8_t* records; uint64_t stride;
-    uint64_t w0, s0, b0, w1, s1, b1;     // byte offsets inside a record
-    const int32_t *offsets, *selected, *count;
-    const int32_t *in_rows, *out_rows;   // indexed by sorted slot; either may be null
-    const float* x; float* out;          // x: layer input (gate/up) or sorted activations (down)
-    uint32_t K, N, group, x_sorted;      // x_sorted: x rows follow the sorted slot order
+    const uint8_t* records; uint64_t stride; uint64_t off[6];          // byte offsets inside a record: codes, scales, biases of the (gate | down) projection, of up
+    const uint8_t* shared_record; uint64_t shared_off[6];
+    const uint32_t *jobs; const int32_t *count, *slots;
+    const float *x, *shared_x; float *out, *shared_out;                // x: layer input (gate/up) or sorted activations (down)
+    uint32_t K, N, group, topk, tokens, chunk, shared_jobs, tiles, share;   // chunk: tokens of a job (a shared job too)
 };
-template <int BITS, int WIDTH, bool GATED>
-__global__ __launch_bounds__(256) void expert_phase_kernel(ExpertPhase p) {
-    extern __shared__ float lds[];
-    const uint32_t job = blockIdx.y;
-    if (int32_t(job) >= *p.count) return;
-    const int32_t e = p.selected[job], first = p.offsets[e], n = p.offsets[e + 1] - first;
-    const uint8_t* r = p.records + uint64_t(e) * p.stride;
-    AffineJob j;
-    j.w0 = r + p.w0; j.s0 = reinterpret_cast<const uint16_t*>(r + p.s0); j.b0 = reinterpret_cast<const uint16_t*>(r + p.b0);
-    j.w1 = r + p.w1; j.s1 = reinterpret_cast<const uint16_t*>(r + p.s1); j.b1 = reinterpret_cast<const uint16_t*>(r + p.b1);
-    j.x = p.x_sorted ? p.x + uint64_t(first) * p.K : p.x;
-    j.in_rows = p.in_rows ? p.in_rows + first : nullptr;
-    j.out_rows = p.out_rows ? p.out_rows + first : nullptr;
-    j.out = p.out_rows ? p.out : p.out + uint64_t(first) * p.N;
-    j.K = p.K; j.N = p.N; j.group = p.group; j.tokens = uint32_t(n); j.float_output = 0;
-    affine_rows<BITS, WIDTH, GATED>(j, blockIdx.x, lds, lds + p.K);
+template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS>
+__global__ __launch_bounds__(256, TOKENS == 1 ? 4 : 3) void expert_phase_kernel(ExpertPhase p) {
+    extern __shared__ __align__(16) uint8_t affine_lds[];
+    const uint32_t tile0 = blockIdx.x * p.share, end = min(tile0 + p.share, p.tiles);
+    const uint32_t total = p.shared_jobs + uint32_t(*p.count);
+    for (uint32_t job = blockIdx.y; job < total; job += gridDim.y) {
+        const bool shared = job < p.shared_jobs;
+        uint32_t first, expert = 0, nt;
+        if (shared) { first = job * p.chunk; nt = min(p.chunk, p.tokens - first); }
+        else { const uint32_t packed = p.jobs[job - p.shared_jobs]; first = packed & 0xfffffu; expert = (packed >> 20) & 1023u; nt = (packed >> 30) + 1u; }
+        const uint8_t* r = shared ? p.shared_record : p.records + uint64_t(expert) * p.stride;
+        AffineMatrix m[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            auto at = [&](int i) { return r + (shared ? p.shared_off[3 * q + i] : p.off[3 * q + i]); };
+            m[q] = AffineMatrix{at(0), reinterpret_cast<const uint16_t*>(at(1)), reinterpret_cast<const uint16_t*>(at(2))};
+        }
+        affine_rows<BITS, WIDTH, GATED, TOKENS>(m, p.K, p.N, p.group, shared ? p.shared_x : p.x, shared ? p.shared_out : p.out, nt,
+                                        [&](uint32_t t) { return GATED && !shared ? uint32_t(p.slots[first + t]) / p.topk : first + t; },
+                                        [&](uint32_t t) { return GATED || shared ? first + t : uint32_t(p.slots[first + t]); }, tile0, end, false, affine_lds);
+        lds_barrier();   // (the next job overwrites the rows)
+    }
 }
 
 static bool wide(uint32_t K, uint32_t N) { return K % 512 == 0 && N % 8 == 0; }
@@ -145,17 +300,41 @@ static void by_format(uint32_t bits, bool w, Launch&& launch) {
     if (bits == 4) { if (w) launch.template operator()<4, 16, GATED>(); else launch.template operator()<4, 8, GATED>(); }
     else           { if (w) launch.template operator()<8, 8, GATED>();  else launch.template operator()<8, 4, GATED>(); }
 }
+// Row tiles per workgroup: staging the input rows is paid once per workgroup, so as many as leave the chip a few thousand
+// workgroups (256 compute units, three or four workgroups each).
+static uint32_t affine_share(uint32_t tiles, uint64_t jobs) {
+    uint32_t share = 4;
+    while (share > 1 && uint64_t((tiles + share - 1) / share) * jobs < 2048) share /= 2;
+    return share;
+}
+// Tokens per workgroup: four where their rows leave room for three workgroups in a compute unit's LDS.
+template <int WIDTH> static uint32_t affine_chunk(uint32_t K) {
+    uint32_t chunk = kAffineTokens;
+    while (chunk > 1 && chunk * affine_token_bytes<WIDTH>(K) > 53 * 1024) chunk /= 2;
+    return chunk;
+}
+uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t bits) {
+    uint32_t chunk = 1;
+    by_format<false>(bits, wide(K, N), [&]<int BITS, int WIDTH, bool GATED>() { chunk = affine_chunk<WIDTH>(K); });
+    return chunk;
+}
+constexpr uint32_t kMaxGridY = 32768;   // (the kernels walk what is left)
 
 void launch_affine(hipStream_t s, const AffineDesc& a) {
     AffineJob j{};
-    j.w0 = (const uint8_t*)a.gate.weight; j.s0 = (const uint16_t*)a.gate.scales; j.b0 = (const uint16_t*)a.gate.biases;
-    if (a.gated) { j.w1 = (const uint8_t*)a.up.weight; j.s1 = (const uint16_t*)a.up.scales; j.b1 = (const uint16_t*)a.up.biases; }
+    auto matrix = [](const zc_linear& l) { return AffineMatrix{(const uint8_t*)l.weight, (const uint16_t*)l.scales, (const uint16_t*)l.biases}; };
+    j.m[0] = matrix(a.gate);
+    if (a.gated) j.m[1] = matrix(a.up);
     j.x = a.x; j.in_rows = a.in_rows; j.out_rows = a.out_rows; j.out = a.out;
     j.K = a.gate.input; j.N = a.gate.output; j.group = a.gate.group; j.tokens = a.tokens; j.float_output = a.float_output;
-    const dim3 grid((j.N + kRowsPerBlock - 1) / kRowsPerBlock);
-    const size_t lds = size_t(j.K) * 4 + size_t(j.K / 4) * 4;
     auto go = [&]<int BITS, int WIDTH, bool GATED>() {
-        hipLaunchKernelGGL((affine_op_kernel<BITS, WIDTH, GATED>), grid, dim3(256), lds, s, j);
+        j.chunk = std::min(affine_chunk<WIDTH>(j.K), j.tokens);
+        const uint32_t rows = AffineStream<BITS, WIDTH, GATED>::kTileRows, chunks = (j.tokens + j.chunk - 1) / j.chunk;
+        j.tiles = (j.N + rows - 1) / rows; j.share = affine_share(j.tiles, chunks);
+        const dim3 grid((j.tiles + j.share - 1) / j.share, std::min(chunks, kMaxGridY));
+        const uint32_t lds = j.chunk * affine_token_bytes<WIDTH>(j.K);
+        if (j.chunk == 1) hipLaunchKernelGGL((affine_op_kernel<BITS, WIDTH, GATED, 1>), grid, dim3(256), lds, s, j);
+        else hipLaunchKernelGGL((affine_op_kernel<BITS, WIDTH, GATED, kAffineTokens>), grid, dim3(256), lds, s, j);
     };
     if (a.gated) by_format<true>(a.gate.bits, wide(j.K, j.N), go);
     else by_format<false>(a.gate.bits, wide(j.K, j.N), go);
@@ -163,15 +342,19 @@ void launch_affine(hipStream_t s, const AffineDesc& a) {
 
 void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d) {
     ExpertPhase p{};
-    p.records = (const uint8_t*)d.records; p.stride = d.stride;
-    p.w0 = d.off[0]; p.s0 = d.off[1]; p.b0 = d.off[2]; p.w1 = d.off[3]; p.s1 = d.off[4]; p.b1 = d.off[5];
-    p.offsets = d.offsets; p.selected = d.selected; p.count = d.count;
-    p.in_rows = d.in_rows; p.out_rows = d.out_rows; p.x = d.x; p.out = d.out;
-    p.K = d.K; p.N = d.N; p.group = d.group; p.x_sorted = d.x_sorted;
-    const dim3 grid((d.N + kRowsPerBlock - 1) / kRowsPerBlock, d.max_jobs);
-    const size_t lds = size_t(d.K) * 4 + size_t(d.K / 4) * 4;
+    p.records = (const uint8_t*)d.records; p.stride = d.stride; p.shared_record = (const uint8_t*)d.shared_record;
+    for (int i = 0; i < 6; ++i) { p.off[i] = d.off[i]; p.shared_off[i] = d.shared_off[i]; }
+    p.jobs = d.jobs; p.count = d.count; p.slots = d.slots;
+    p.x = d.x; p.out = d.out; p.shared_x = d.shared_x; p.shared_out = d.shared_out;
+    p.K = d.K; p.N = d.N; p.group = d.group; p.topk = d.topk; p.tokens = d.tokens; p.chunk = d.chunk;
+    p.shared_jobs = d.shared_record ? (d.tokens + d.chunk - 1) / d.chunk : 0;
     auto go = [&]<int BITS, int WIDTH, bool GATED>() {
-        hipLaunchKernelGGL((expert_phase_kernel<BITS, WIDTH, GATED>), grid, dim3(256), lds, s, p);
+        const uint32_t rows = AffineStream<BITS, WIDTH, GATED>::kTileRows;
+        p.tiles = (p.N + rows - 1) / rows; p.share = affine_share(p.tiles, d.max_jobs + p.shared_jobs);
+        const dim3 grid((p.tiles + p.share - 1) / p.share, std::min(d.max_jobs + p.shared_jobs, kMaxGridY));
+        const uint32_t most = std::min(d.chunk, d.tokens), lds = most * affine_token_bytes<WIDTH>(d.K);
+        if (most == 1) hipLaunchKernelGGL((expert_phase_kernel<BITS, WIDTH, GATED, 1>), grid, dim3(256), lds, s, p);
+        else hipLaunchKernelGGL((expert_phase_kernel<BITS, WIDTH, GATED, kAffineTokens>), grid, dim3(256), lds, s, p);
     };
     if (d.gated) by_format<true>(d.bits, wide(d.K, d.N), go);
     else by_format<false>(d.bits, wide(d.K, d.N), go);
@@ -483,16 +666,112 @@ __global__ __launch_bounds__(64) void route_kernel(const float* logits, uint32_t
             if (j < topk) { ids[uint64_t(t) * topk + j] = selected[j]; weights[uint64_t(t) * topk + j] = values[i] * inverse; }
         }
 }
+// The same by route_token (at most 64 picks): candidates by a binary search over the lanes' maxima instead of one reduction
+// through LDS per pick.  512 experts, top-10: 10.4 -> 4.7 us.
+template <int PER>
+__global__ __launch_bounds__(64) void route_fast_kernel(const float* __restrict__ logits, uint32_t E, uint32_t topk, int32_t* __restrict__ ids, float* __restrict__ weights) {
+    __shared__ int32_t ids_s[64];
+    __shared__ float weights_s[64];
+    __shared__ uint32_t pick[128];
+    const uint32_t t = blockIdx.x, lane = threadIdx.x;
+    const float* row = logits + uint64_t(t) * E;
+    route_token<PER>([&](float (&cand)[PER], uint32_t per) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) { const uint32_t e = lane * per + uint32_t(i); cand[i] = (uint32_t(i) < per && e < E) ? row[e] : __uint_as_float(0xff800000u); }
+    }, E, topk, lane, ids_s, weights_s, pick, [] {}, [] {});
+    __syncthreads();
+    if (lane < topk) { ids[uint64_t(t) * topk + lane] = ids_s[lane]; weights[uint64_t(t) * topk + lane] = weights_s[lane]; }
+}
 void launch_route(hipStream_t s, const float* logits, uint32_t T, uint32_t E, uint32_t topk, int32_t* ids, float* weights) {
+    if (topk <= 64) {
+        if (E <= 512) hipLaunchKernelGGL(route_fast_kernel<8>, dim3(T), dim3(64), 0, s, logits, E, topk, ids, weights);
+        else hipLaunchKernelGGL(route_fast_kernel<16>, dim3(T), dim3(64), 0, s, logits, E, topk, ids, weights);
+        return;
+    }
     hipLaunchKernelGGL(route_kernel, dim3(T), dim3(64), 0, s, logits, T, E, topk, ids, weights);
 }
 
 // ---------------------------------------------------------------------------
 // Dispatch: stable counting sort of the flat slots p = t*topk + k by expert id
-// (reference: model.cpp:449-479).  One workgroup; each wavefront owns experts
-// e = wave, wave+16, ... and scans the id array in order, so slots of an expert
-// come out in ascending p without any atomics.
+// (reference: model.cpp:449-479).  Up to 1024 slots and experts: one workgroup, thread p owns slot p and then expert p.  A
+// slot's place among its wave's slots of the same expert comes from ten ballots over the id's bits, the waves' counts of
+// every expert from a table in LDS, without any atomics; two scans over the experts give the rest.  (A wavefront per
+// expert that scanned the whole id array took 14.4 us for 10 slots and 66 us for 400; this takes 5.8 us, the selection
+// included, and 4.8 us.)
+//
+// jobs, optional: the list of (expert, sorted positions) that the expert kernels walk, at most `chunk` <= 4 positions of one
+// expert each: first position | expert << 20 | (positions - 1) << 30 (a call has at most 2^20 slots).  `count` then is its
+// length; else `selected` lists the experts that have slots and `count` is their number.
+//
+// ROUTE: tokens <= 16, and wave t first selects token t's experts (route_token) instead of reading `ids`: one launch less.
 // ---------------------------------------------------------------------------
+struct Dispatch {
+    int32_t *offsets, *slots, *rows, *selected; uint32_t* jobs; int32_t *count, *status;
+    uint32_t topk, E, chunk;
+};
+constexpr uint32_t kDispatchSlots = 1024, kRouteTokens = 16;
+__device__ __forceinline__ uint32_t dispatch_job(uint32_t first, uint32_t expert, uint32_t positions) { return first | expert << 20 | (positions - 1) << 30; }
+template <bool ROUTE, int PER>
+__global__ __launch_bounds__(1024) void dispatch_short_kernel(const float* __restrict__ logits, int32_t* __restrict__ ids, float* __restrict__ weights, uint32_t n, Dispatch d) {
+    __shared__ uint32_t table[16 * 512];           // [wave][expert] counts, two experts a word
+    __shared__ uint32_t start[1024], wave_total[2][16];
+    __shared__ uint16_t held[1024];
+    __shared__ int32_t ids_s[ROUTE ? 1024 : 1];
+    __shared__ float weights_s[ROUTE ? 1024 : 1];
+    __shared__ uint32_t pick[ROUTE ? kRouteTokens * 128 : 1];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, waves = (n + 63) / 64, E = d.E;
+    uint16_t* counts = reinterpret_cast<uint16_t*>(table);
+    for (uint32_t i = tid; i < waves * 512; i += 1024) table[i] = 0;
+    int32_t id = -1;
+    if constexpr (ROUTE) {
+        if (wave < n / d.topk) {
+            const float* row = logits + uint64_t(wave) * E;
+            route_token<PER>([&](float (&cand)[PER], uint32_t per) {
+#pragma unroll
+                for (int i = 0; i < PER; ++i) { const uint32_t e = lane * per + uint32_t(i); cand[i] = (uint32_t(i) < per && e < E) ? row[e] : __uint_as_float(0xff800000u); }
+            }, E, d.topk, lane, ids_s + wave * d.topk, weights_s + wave * d.topk, pick + wave * 128, [] {}, [] {});
+        }
+        __syncthreads();
+        if (tid < n) { id = ids_s[tid]; ids[tid] = id; weights[tid] = weights_s[tid]; }
+    } else {
+        if (tid < n) id = ids[tid];
+        __syncthreads();
+    }
+    if (tid < n && (id < 0 || id >= int32_t(E))) { atomicOr(d.status, 1); id = -1; }
+    // the wave's lanes with this lane's id
+    uint64_t same = __ballot(id >= 0);
+#pragma unroll
+    for (int b = 0; b < 10; ++b) { const uint64_t m = __ballot((id >> b) & 1); same &= ((id >> b) & 1) ? m : ~m; }
+    uint32_t rank = uint32_t(__popcll(same & ((1ull << lane) - 1)));
+    if (id >= 0 && rank == 0) counts[wave * 1024 + uint32_t(id)] = uint16_t(__popcll(same));
+    __syncthreads();
+    // thread e: expert e's slots of earlier waves, their sum, and the scans over the experts (sums of at most 1024 each: two in a word)
+    uint32_t total = 0;
+    if (tid < E)
+        for (uint32_t w = 0; w < waves; ++w) { const uint32_t c = counts[w * 1024 + tid]; counts[w * 1024 + tid] = uint16_t(total); total += c; }
+    const uint32_t mine[2] = {total | (d.jobs ? (total + d.chunk - 1) / d.chunk : 0u) << 16, total ? 1u : 0u};
+    uint32_t incl[2] = {mine[0], mine[1]};
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1)
+#pragma unroll
+        for (int v = 0; v < 2; ++v) { const uint32_t up = __shfl_up(incl[v], o); if (int(lane) >= o) incl[v] += up; }
+    if (lane == 63) { wave_total[0][wave] = incl[0]; wave_total[1][wave] = incl[1]; }
+    __syncthreads();
+    uint32_t before[2] = {incl[0] - mine[0], incl[1] - mine[1]};
+    for (uint32_t w = 0; w < wave; ++w) { before[0] += wave_total[0][w]; before[1] += wave_total[1][w]; }
+    start[tid] = before[0]; held[tid] = uint16_t(total);
+    if (tid < E) d.offsets[tid] = int32_t(before[0] & 0xffffu);
+    if (tid < E && total && d.selected) d.selected[before[1]] = int32_t(tid);
+    if (tid == 1023) { d.offsets[E] = int32_t((before[0] + mine[0]) & 0xffffu); *d.count = int32_t(d.jobs ? (before[0] + mine[0]) >> 16 : before[1] + mine[1]); }
+    __syncthreads();
+    if (id < 0) return;
+    rank += counts[wave * 1024 + uint32_t(id)];
+    const uint32_t first = start[id], at = (first & 0xffffu) + rank;
+    d.slots[at] = int32_t(tid);
+    if (d.rows) d.rows[at] = int32_t(tid / d.topk);
+    if (d.jobs && rank % d.chunk == 0) d.jobs[(first >> 16) + rank / d.chunk] = dispatch_job(at, uint32_t(id), min(d.chunk, uint32_t(held[id]) - rank));
+}
+// More than 1024 experts (up to 8192): each wavefront owns experts e = wave, wave+16, ... and scans the id array in order.
 __global__ __launch_bounds__(1024) void dispatch_kernel(const int32_t* ids, uint32_t n, uint32_t topk, uint32_t E,
                                                         int32_t* offsets, int32_t* slots, int32_t* rows,
                                                         int32_t* selected, int32_t* count, int32_t* status) {
@@ -579,7 +858,8 @@ __global__ __launch_bounds__(256) void dispatch_count_kernel(const int32_t* __re
     for (int o = 32; o; o >>= 1) c += __shfl_xor(c, o);
     if (lane == 0) offsets[1 + e] = c;
 }
-__global__ __launch_bounds__(64) void dispatch_scan_kernel(uint32_t E, int32_t* offsets, int32_t* selected, int32_t* count) {
+// chunk: 0, or the jobs' positions; `selected` then receives every expert's first job, count the number of jobs.
+__global__ __launch_bounds__(64) void dispatch_scan_kernel(uint32_t E, uint32_t chunk, int32_t* offsets, int32_t* selected, int32_t* count) {
     const uint32_t lane = threadIdx.x;
     int32_t running = 0, picked = 0;
     if (lane == 0) offsets[0] = 0;
@@ -590,6 +870,16 @@ __global__ __launch_bounds__(64) void dispatch_scan_kernel(uint32_t E, int32_t* 
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) { const int32_t up = __shfl_up(incl, o); if (int(lane) >= o) incl += up; }
         if (e < E) offsets[e + 1] = running + incl;
+        if (chunk) {
+            const int32_t jobs = (c + int32_t(chunk) - 1) / int32_t(chunk);
+            int32_t before = jobs;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) { const int32_t up = __shfl_up(before, o); if (int(lane) >= o) before += up; }
+            if (e < E) selected[e] = picked + before - jobs;
+            picked += __shfl(before, 63);
+            running += __shfl(incl, 63);
+            continue;
+        }
         const uint64_t mask = __ballot(c > 0);
         if (c > 0) selected[picked + __popcll(mask & ((1ull << lane) - 1))] = int32_t(e);
         picked += __popcll(mask);
@@ -598,11 +888,15 @@ __global__ __launch_bounds__(64) void dispatch_scan_kernel(uint32_t E, int32_t* 
     if (lane == 0) *count = picked;
 }
 __global__ __launch_bounds__(256) void dispatch_place_kernel(const int32_t* __restrict__ ids, uint32_t n, uint32_t topk, uint32_t E, const int32_t* __restrict__ offsets,
-                                                             int32_t* __restrict__ slots, int32_t* __restrict__ rows, bool aligned) {
+                                                             int32_t* __restrict__ slots, int32_t* __restrict__ rows, bool aligned,
+                                                             uint32_t chunk, const int32_t* __restrict__ first_job, uint32_t* __restrict__ jobs) {
     const uint32_t lane = threadIdx.x & 63u, e = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (e >= E) return;
     int32_t pos = offsets[e];
     if (offsets[e + 1] == pos) return;
+    if (jobs)
+        for (uint32_t at = lane * chunk, held = uint32_t(offsets[e + 1] - pos); at < held; at += 64 * chunk)
+            jobs[uint32_t(first_job[e]) + at / chunk] = dispatch_job(uint32_t(pos) + at, e, min(chunk, held - at));
     const uint64_t below = (1ull << lane) - 1;
     // eight steps of 256 slots, in order: four neighbouring slots per lane, slots of lower lanes first, then the lane's own
     auto place = [&](const int4 (&batch)[8], uint32_t q0) {
@@ -651,17 +945,38 @@ __global__ __launch_bounds__(256) void dispatch_place_kernel(const int32_t* __re
         place(ahead, q0);
     }
 }
-void launch_dispatch(hipStream_t s, const int32_t* ids, uint32_t tokens, uint32_t topk, uint32_t E, int32_t* offsets,
-                     int32_t* slots, int32_t* rows, int32_t* selected, int32_t* count, int32_t* status) {
-    const uint32_t n = tokens * topk;
-    if (n <= 1024) {   // decode: one launch
-        hipLaunchKernelGGL(dispatch_kernel, dim3(1), dim3(1024), size_t(E + 1) * 4, s, ids, n, topk, E, offsets, slots, rows, selected, count, status);
+static void launch_dispatch_any(hipStream_t s, const int32_t* ids, uint32_t n, const Dispatch& d) {
+    if (n <= kDispatchSlots && d.E <= 1024) {
+        hipLaunchKernelGGL((dispatch_short_kernel<false, 8>), dim3(1), dim3(1024), 0, s, nullptr, const_cast<int32_t*>(ids), nullptr, n, d);
+        return;
+    }
+    if (n <= kDispatchSlots && !d.jobs) {
+        hipLaunchKernelGGL(dispatch_kernel, dim3(1), dim3(1024), size_t(d.E + 1) * 4, s, ids, n, d.topk, d.E, d.offsets, d.slots, d.rows, d.selected, d.count, d.status);
         return;
     }
     const bool aligned = reinterpret_cast<uintptr_t>(ids) % 16 == 0;
-    hipLaunchKernelGGL(dispatch_count_kernel, dim3((E + 3) / 4), dim3(256), 0, s, ids, n, E, offsets, status, aligned);
-    hipLaunchKernelGGL(dispatch_scan_kernel, dim3(1), dim3(64), 0, s, E, offsets, selected, count);
-    hipLaunchKernelGGL(dispatch_place_kernel, dim3((E + 3) / 4), dim3(256), 0, s, ids, n, topk, E, offsets, slots, rows, aligned);
+    const uint32_t chunk = d.jobs ? d.chunk : 0;
+    hipLaunchKernelGGL(dispatch_count_kernel, dim3((d.E + 3) / 4), dim3(256), 0, s, ids, n, d.E, d.offsets, d.status, aligned);
+    hipLaunchKernelGGL(dispatch_scan_kernel, dim3(1), dim3(64), 0, s, d.E, chunk, d.offsets, d.selected, d.count);
+    hipLaunchKernelGGL(dispatch_place_kernel, dim3((d.E + 3) / 4), dim3(256), 0, s, ids, n, d.topk, d.E, d.offsets, d.slots, d.rows, aligned, chunk, d.selected, d.jobs);
+}
+void launch_dispatch(hipStream_t s, const int32_t* ids, uint32_t tokens, uint32_t topk, uint32_t E, int32_t* offsets,
+                     int32_t* slots, int32_t* rows, int32_t* selected, int32_t* count, int32_t* status) {
+    launch_dispatch_any(s, ids, tokens * topk, Dispatch{offsets, slots, rows, selected, nullptr, count, status, topk, E, 0});
+}
+// Routes, dispatch sort and the expert kernels' job list (E <= 1024; scratch: E words).
+void launch_route_jobs(hipStream_t s, const float* logits, uint32_t tokens, uint32_t E, uint32_t topk, int32_t* ids, float* weights,
+                       int32_t* offsets, int32_t* slots, uint32_t chunk, uint32_t* jobs, int32_t* count, int32_t* scratch, int32_t* status) {
+    const uint32_t n = tokens * topk;
+    Dispatch d{offsets, slots, nullptr, scratch, jobs, count, status, topk, E, chunk};
+    if (n <= kDispatchSlots) d.selected = nullptr;
+    if (tokens <= kRouteTokens && topk <= 64) {   // (n <= 1024)
+        if (E <= 512) hipLaunchKernelGGL((dispatch_short_kernel<true, 8>), dim3(1), dim3(1024), 0, s, logits, ids, weights, n, d);
+        else hipLaunchKernelGGL((dispatch_short_kernel<true, 16>), dim3(1), dim3(1024), 0, s, logits, ids, weights, n, d);
+        return;
+    }
+    launch_route(s, logits, tokens, E, topk, ids, weights);
+    launch_dispatch_any(s, ids, n, d);
 }
 
 // ---------------------------------------------------------------------------

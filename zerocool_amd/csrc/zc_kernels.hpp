@@ -20,12 +20,16 @@ void launch_affine(hipStream_t s, const AffineDesc& a);          // literal lane
 bool xint_supported(const zc_linear& l);                          // wide affine Q4, group 64, 16-byte aligned
 void launch_affine_xint(hipStream_t s, const AffineDesc& a);     // exact-integer matrix-core form
 
+uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t bits);   // tokens one workgroup of these kernels takes at a time: 1, 2 or 4
+
 struct ExpertPhaseDesc {
     const void* records; uint64_t stride;
     uint64_t off[6];             // w,s,b of the first matrix, then of the second (gate/up phase)
-    const int32_t *offsets, *selected, *count, *in_rows, *out_rows;
-    const float* x; float* out;
-    uint32_t K, N, group, bits, x_sorted, max_jobs;
+    const void* shared_record;   // null, or the shared expert joins the launch: its projections have the routed ones' format
+    uint64_t shared_off[6];
+    const uint32_t* jobs; const int32_t *count, *slots;   // launch_route_jobs
+    const float *x, *shared_x; float *out, *shared_out;
+    uint32_t K, N, group, bits, topk, tokens, chunk, max_jobs;
     bool gated;
 };
 void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d);
@@ -37,6 +41,8 @@ void launch_router(hipStream_t s, const void* w, const float* x, uint32_t T, uin
 void launch_route(hipStream_t s, const float* logits, uint32_t T, uint32_t E, uint32_t topk, int32_t* ids, float* weights);
 void launch_dispatch(hipStream_t s, const int32_t* ids, uint32_t tokens, uint32_t topk, uint32_t E, int32_t* offsets,
                      int32_t* slots, int32_t* rows, int32_t* selected, int32_t* count, int32_t* status);
+void launch_route_jobs(hipStream_t s, const float* logits, uint32_t tokens, uint32_t E, uint32_t topk, int32_t* ids, float* weights,
+                       int32_t* offsets, int32_t* slots, uint32_t chunk, uint32_t* jobs, int32_t* count, int32_t* scratch, int32_t* status);
 void launch_scatter(hipStream_t s, const float* x, const int32_t* positions, uint32_t n, uint32_t H, float* out);
 // ---- the callers' glue either side of the layer (zc_glue.hip)
 void launch_unary(hipStream_t s, const float* x, uint64_t n, uint32_t op, float* y);

@@ -44,12 +44,6 @@ typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-// Eight bytes whose address is a multiple of four only.
-__device__ __forceinline__ uint2 ldg_u2_by_words(const void* p) {
-    typedef uint32_t words __attribute__((ext_vector_type(2), aligned(4)));
-    const words v = *as_global<words>(p);
-    return make_uint2(v.x, v.y);
-}
 constexpr uint32_t kTileRows = 32, kTileRowsMax = 48, kPitch = 136;   // LDS row pitch in bf16 elements: 128 elements of a row, sixteen rows on different banks
 
 // What the matrix-core products and the recomputation need of their token rows, from fp32 rows holding BF16 values (F32)
