@@ -70,3 +70,13 @@ def test_dispatch_sort(ctx, tokens, topk, experts):
     n_selected = int(count.numpy(np.int32)[0])
     assert n_selected == len(want_selected) and selected.numpy(np.int32)[:n_selected].tobytes() == want_selected.tobytes()
     assert status.numpy(np.int32)[0] == 0
+
+
+# rows of one weight piece and of several batches, a row too long for LDS (the general kernel), and numbers of tokens and
+# experts that leave a group of either partly empty
+@pytest.mark.parametrize("T,K,E", [(1, 128, 1), (2, 128, 5), (3, 2560, 17), (4, 1152, 512), (63, 640, 33), (1, 16384, 3), (5, 4224, 20)])
+def test_router_logits(ctx, T, K, E):
+    rng = np.random.default_rng(K + T)
+    w, x, off = oracle.bf_bits(rng.standard_normal((E, K))), oracle.bf(rng.standard_normal((T, K))), rng.standard_normal(E).astype(f32)
+    got = ctx.router_logits(ctx.upload(w), ctx.upload(x), T, K, E, ctx.upload(off)).numpy(f32)
+    assert got.tobytes() == oracle.router_logits(w, x, T, K, E, off).tobytes()

@@ -606,13 +606,12 @@ zc_status zc_hip_moe_forward(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
     const Workspace w = carve(c, T, workspace);
     hipStream_t s = ctx->stream;
     const uint32_t H = c->hidden, I = c->inter, E = c->experts, k = c->topk;
-    // 1-2. router logits, top-k + softmax (model.cpp:434-436)
-    zc::launch_router(s, l->router, x, T, H, E, l->router_offsets, w.logits);
+    // 1-2. router logits and the shared expert's gate, top-k + softmax (model.cpp:434-436)
+    zc::launch_router(s, l->router, x, T, H, E, l->router_offsets, w.logits, l->shared_gate, w.gate);
     // 4. positions / selected, on the device (model.cpp:449-479): the expert kernels' job list, at most `chunk` tokens a job
     const uint32_t chunk = std::min(zc::affine_job_tokens(H, I, c->bits_gate_up), zc::affine_job_tokens(I, H, c->bits_down));
     uint32_t* jobs = reinterpret_cast<uint32_t*>(w.rows);   // (n words: a job holds at least one slot)
     zc::launch_route_jobs(s, w.logits, T, E, k, w.ids, w.weights, w.offsets, w.slots, chunk, jobs, w.count, w.selected, ctx->moe_status);
-    zc::launch_plain(s, l->shared_gate, 0, x, H, 1, T, w.gate, false);
     // 5-6. shared expert (model.cpp:482-485) and routed experts (pipeline.cpp:18-29): gate/up on gathered rows, down scattered
     // to its slot.  One launch per phase where the shared expert's projections have the routed ones' width.
     auto offsets_of = [&](const void* record, int shared, uint64_t* off, int first, int count) {

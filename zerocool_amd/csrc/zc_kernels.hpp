@@ -36,8 +36,9 @@ void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d);
 
 void launch_plain(hipStream_t s, const void* w, uint32_t dtype, const float* x, uint32_t K, uint32_t N,
                   uint32_t tokens, float* out, bool float_output);
+// gate_w, optional: a BF16 row whose plain dot with every token goes to gate [T], rounded to BF16 (the shared expert's gate)
 void launch_router(hipStream_t s, const void* w, const float* x, uint32_t T, uint32_t K, uint32_t E,
-                   const float* offsets, float* out);
+                   const float* offsets, float* out, const void* gate_w = nullptr, float* gate = nullptr);
 void launch_route(hipStream_t s, const float* logits, uint32_t T, uint32_t E, uint32_t topk, int32_t* ids, float* weights);
 void launch_dispatch(hipStream_t s, const int32_t* ids, uint32_t tokens, uint32_t topk, uint32_t E, int32_t* offsets,
                      int32_t* slots, int32_t* rows, int32_t* selected, int32_t* count, int32_t* status);
