@@ -1,5 +1,5 @@
 """The exact layer's short-batch kernels at the edges of their ranges, byte for byte against the CPU oracle: the one-workgroup
-selection and dispatch sort with its job list, and the expert kernels' groups of up to four tokens, their two arithmetic
+selection and dispatch sort with its job list, and the expert kernels' groups of tokens, their two arithmetic
 forms (fused products for BF16-valued rows of ordinary magnitude, separate ones for all others) and partial last steps."""
 import numpy as np
 import pytest
@@ -32,7 +32,7 @@ def rows(kind, T, hidden, seed):
 @pytest.mark.parametrize("T,hidden,inter,experts,topk,bits,group,kind", [
     (1, 512, 128, 8, 2, (4, 4, 4, 4), 64, "fp32"),         # one token, both forms
     (1, 544, 96, 8, 8, (8, 8, 8, 8), 32, "large"),         # byte codes, four-element blocks, last step partial
-    (5, 512, 128, 4, 2, (4, 4, 4, 4), 64, "bf16"),         # experts with one to five slots: job groups of four and what is left
+    (5, 512, 128, 4, 2, (4, 4, 4, 4), 64, "bf16"),         # experts with one to five slots: whole groups of tokens and what is left
     (16, 576, 640, 33, 3, (4, 4, 4, 4), 64, "tiny"),       # the most tokens of the joined selection, narrow blocks both ways
     (17, 512, 256, 600, 3, (4, 8, 8, 8), 64, "fp32"),      # one more; sixteen logits a lane; the shared expert in launches of its own
     (9, 512, 160, 96, 70, (8, 4, 8, 4), 32, "bf16"),       # more than 64 picks

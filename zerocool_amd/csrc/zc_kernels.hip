@@ -16,86 +16,143 @@ namespace zc {
 //
 // A half wave plays the 32 reference lanes of one output row: lane l takes the row's blocks l, l + 32, ... of WIDTH elements
 // (Q4 16|8, Q8 8|4: one or two dwords of codes) in order.  It walks two rows at a time (gate and up, or two rows of the one
-// matrix), so that an input block read from LDS serves two rows, and up to four tokens, so that a code is expanded once for
+// matrix), so that an input block read from LDS serves two rows, and up to two tokens, so that a code is unpacked once for
 // four products.  The walk over (row tile, block step) is one flat loop: the codes and scales of its next three steps are in
 // flight, across row tiles too, and the first three are requested before the input rows are staged.
 //
-// The products x * q of a BF16-valued row (magnitudes below 2^100) are exact in fp32, so a fused multiply-add rounds as the
-// reference's multiply and add do: EXACT saves three of eight instructions per four elements.  Rows that hold anything
-// else, infinities and NaN among them, keep the separate operations.
+// The products x * q of a BF16-valued row (zeros and magnitudes from 2^-100 to 2^100) are exact in fp32, so a fused multiply-add
+// rounds as the reference's multiply and add do, also when all of it is scaled by a power of two: such rows multiply codes
+// that were never converted (affine_halves).  Rows that hold anything else, infinities and NaN among them, keep converted codes
+// and separate operations.
 //
 // What bounds it: with one token per row, the latency of the chain job -> row index -> input row -> LDS -> codes (a launch
-// of a few us); with several, the vector instructions: 1.5 per weight and token, 1.4 per weight for the expansion.
-// One token at a time, codes requested step by step behind the staging, every reduction through LDS permutes and the shared
-// expert in launches of its own took, per layer of hidden 2560 and intermediate 640: 40 tokens 397 us for gate/up and 310 us
-// for down against 172 and 132 us, one token 20.2 and 14.3 us against 12.5 and 9.2 us.
+// of a few us); with several, vector instructions, a wave's at four clocks each: 24 per block of sixteen weights and token, 14
+// to unpack the block, and the finish of a row.  Per layer of hidden 2560 and intermediate 640, gate/up and down: 40 tokens 142
+// and 119 us, one token 11.9 and 8.7 us.  With codes converted to floats, addresses formed per lane and four tokens per
+// workgroup it was 172 and 132, 12.5 and 9.2 us.  Four tokens per workgroup take 159 and 112 us: most experts have one or two
+// tokens, and the LDS of four leaves room for three workgroups on a compute unit where two leave six (decoding stacks of
+// hidden 2048 and 3072 at 2 to 64 tokens lost 5 to 25 %).  One token at a time, codes requested step by step behind the staging,
+// sums through LDS permutes and the shared expert in launches of its own took 397 and 310, 20.2 and 14.3 us.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kAffineTokens = 4;                                            // tokens a workgroup multiplies at once, at most
+constexpr uint32_t kAffineTokens = 2;                                            // tokens a workgroup multiplies at once, at most
 constexpr uint32_t kAffineAhead = 3;                                             // steps in flight
 struct AffineMatrix { const uint8_t* w; const uint16_t *s, *b; };
 
-// Input rows in LDS, per token: WIDTH / 4 planes of sixteen-byte pieces, piece (plane, block), then the blocks' bias sums.
-// Lanes read the pieces of neighbouring blocks; the pitch makes the staging's writes, four neighbouring pieces in as many
-// planes, meet different banks.
-template <int WIDTH> __host__ __device__ constexpr uint32_t affine_pitch(uint32_t blocks) { return WIDTH == 4 ? blocks : (blocks + 15) / 16 * 16 + 4; }
-template <int WIDTH> __host__ __device__ constexpr uint32_t affine_token_bytes(uint32_t K) {
-    return WIDTH / 4 * affine_pitch<WIDTH>(K / WIDTH) * 16 + (K / WIDTH + 3) / 4 * 16;
+// Input rows in LDS: a block's WIDTH elements and its bias sum behind them, WIDTH / 4 words further apart than the elements
+// need (20, 10 or 5 words: the blocks of neighbouring lanes meet different banks), so that a lane adds one offset per token.
+template <int WIDTH> __host__ __device__ constexpr uint32_t affine_token_bytes(uint32_t K) { return (K * 5 + 15) / 16 * 16; }
+template <int WIDTH> struct AffineBlock { static constexpr uint32_t kBytes = WIDTH * 5, kPiece = WIDTH == 16 ? 4 : WIDTH == 8 ? 2 : 1; };
+template <int WIDTH>
+__device__ __forceinline__ void affine_inputs(const uint8_t* at, float* x, float& sum) {
+    typedef float piece __attribute__((ext_vector_type(AffineBlock<WIDTH>::kPiece)));
+    constexpr int P = AffineBlock<WIDTH>::kPiece;
+#pragma unroll
+    for (int i = 0; i < WIDTH; i += P) {
+        const piece v = *reinterpret_cast<const piece*>(at + 4 * i);
+#pragma unroll
+        for (int k = 0; k < P; ++k) x[i + k] = v[k];
+    }
+    sum = *reinterpret_cast<const float*>(at + 4 * WIDTH);
 }
 
+// Addresses: the bases are the same in every lane and move with tile and step, the lanes' 32-bit offsets are those of their row
+// and block in the tile.  wide: rows are whole steps (K % 512 == 0), else the last step's idle lanes repeat the last block.
 template <int BITS, int WIDTH, bool GATED>
 struct AffineStream {
     static constexpr int DW = WIDTH * BITS / 32;
+    static constexpr bool kWide = WIDTH * BITS == 64;
     struct Slot { uint32_t q[2][DW]; uint32_t s[2], b[2]; };
     static constexpr uint32_t kTileRows = GATED ? 8 : 16;   // rows of a workgroup's tile: eight half waves, one or two each
     uint32_t K, N, blocks, groups, shift, steps, lane, half, tile, end, step;   // tile, step: the next one to request
     AffineMatrix m[2];
-    const uint8_t* w[2]; const uint16_t *s[2], *b[2];
+    uint32_t w_at[2], g_at[2];
     __device__ __forceinline__ uint32_t row(uint32_t t, int q) const { return GATED ? t * 8 + half : t * 16 + uint32_t(q) * 8 + half; }
     __device__ __forceinline__ void aim() {
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-            const uint64_t r = min(row(tile, q), N - 1);
-            const AffineMatrix& a = m[GATED ? q : 0];
-            w[q] = a.w + r * (K / 8 * BITS); s[q] = a.s + r * groups; b[q] = a.b + r * groups;
+            const uint32_t r = min(row(tile, q), N - 1) - tile * kTileRows;
+            w_at[q] = r * (K / 8 * BITS) + (kWide ? lane * (DW * 4) : 0u);
+            g_at[q] = (r * groups + (kWide ? (lane * WIDTH) >> shift : 0u)) * 2;
         }
     }
     __device__ __forceinline__ void fetch(Slot& slot) {   // past the end: the last tile again, not used
-        const uint32_t at = min(step * 32 + lane, blocks - 1), g = (at * WIDTH) >> shift;
+        const uint64_t first = uint64_t(tile) * kTileRows;
+        const uint32_t at = kWide ? 0u : min(lane, blocks - 1 - step * 32), g = ((step * 32 * WIDTH) >> shift) * 2;
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-            if constexpr (DW == 2) { const uint2 v = ldg_u2_by_words(w[q] + at * 8); slot.q[q][0] = v.x; slot.q[q][DW - 1] = v.y; }
-            else slot.q[q][0] = ldg_u32(w[q], at);
-            slot.s[q] = ldg_u16(s[q], g); slot.b[q] = ldg_u16(b[q], g);
+            const AffineMatrix& a = m[GATED ? q : 0];
+            const uint8_t* w = a.w + (first * (K / 8 * BITS) + step * (32 * DW * 4));
+            const uint32_t w_lane = w_at[q] + (kWide ? 0u : at * (DW * 4)), g_lane = g_at[q] + (kWide ? 0u : ((at * WIDTH) >> shift) * 2);
+            if constexpr (DW == 2) { const uint2 v = ldg_u2_by_words(w + w_lane); slot.q[q][0] = v.x; slot.q[q][DW - 1] = v.y; }
+            else slot.q[q][0] = ldg_u32(w + w_lane);
+            slot.s[q] = ldg_u16(reinterpret_cast<const uint8_t*>(a.s) + (first * groups * 2 + g) + g_lane);
+            slot.b[q] = ldg_u16(reinterpret_cast<const uint8_t*>(a.b) + (first * groups * 2 + g) + g_lane);
         }
         if (++step == steps) { step = 0; if (tile + 1 < end) { ++tile; aim(); } }
     }
 };
+// Codes as f16 bit patterns, two in a word: the pattern of an integer n < 1024 is the number n * 2^-24, which the mixed
+// multiply-add (v_fma_mix_f32) takes as it is, so a code costs its place in a half word and no conversion.  Word k of eight
+// nibbles: nibbles k and k + 4; word k of four bytes: bytes k and k + 2.
 template <int BITS, int WIDTH>
-__device__ __forceinline__ void affine_codes(const uint32_t* words, float* code) {
-    if constexpr (BITS == 4) {
+__device__ __forceinline__ void affine_halves(const uint32_t* words, uint32_t* half) {
+    constexpr int PER = 32 / BITS / 2;   // half-word pairs of a word of codes
 #pragma unroll
-        for (int i = 0; i < WIDTH; i += 8) {   // the even and the odd nibbles as bytes: one byte-to-float instruction each
-            const uint32_t even = words[i / 8] & 0x0f0f0f0fu, odd = (words[i / 8] >> 4) & 0x0f0f0f0fu;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) { code[i + 2 * k] = float((even >> (8 * k)) & 0xffu); code[i + 2 * k + 1] = float((odd >> (8 * k)) & 0xffu); }
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < WIDTH; ++i) code[i] = float((words[i / 4] >> (8 * (i % 4))) & 255u);
-    }
+    for (int i = 0; i < WIDTH / 2; ++i) half[i] = (words[i / PER] >> (BITS * (i % PER))) & (BITS == 4 ? 0x000f000fu : 0x00ff00ffu);
 }
-template <int BITS, int WIDTH, bool EXACT>
-__device__ __forceinline__ float affine_dot(const float* code, const float* x) {
+// x * code i * 2^-24 + c, rounded once.  (In assembly: from the source form the compiler converts the codes once for all tokens
+// instead, one instruction per code and twice the registers.)
+template <int BITS>
+__device__ __forceinline__ float affine_mad(float x, const uint32_t* half, int i, float c) {
+    constexpr int PER = 32 / BITS / 2;
+    const uint32_t h = half[i / (2 * PER) * PER + i % PER];
+    float d;
+    if ((i / PER) % 2) asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(d) : "v"(x), "v"(h), "v"(c));
+    else asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[0,1,0]" : "=v"(d) : "v"(x), "v"(h), "v"(c));
+    return d;
+}
+template <int BITS>
+__device__ __forceinline__ float affine_mul(float x, const uint32_t* half, int i) {
+    constexpr int PER = 32 / BITS / 2;
+    const uint32_t h = half[i / (2 * PER) * PER + i % PER];
+    float d;
+    if ((i / PER) % 2) asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(d) : "v"(x), "v"(h));
+    else asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "=v"(d) : "v"(x), "v"(h));
+    return d;
+}
+// sum of x * code over a block in the reference's order.  (A first quad or product is added to nothing: the reference adds it to
+// +0, which can only turn a -0 into +0, and the row's sum starts from +0.)
+template <int BITS, int WIDTH>
+__device__ __forceinline__ float affine_dot_exact(const uint32_t* half, const float* x) {
     float dot = 0;
     if constexpr (BITS == 4) {
 #pragma unroll
         for (int i = 0; i < WIDTH; i += 4) {
-            if constexpr (EXACT) dot += __builtin_fmaf(x[i + 3], code[i + 3], __builtin_fmaf(x[i + 2], code[i + 2], __builtin_fmaf(x[i + 1], code[i + 1], x[i] * code[i])));
-            else dot += x[i] * code[i] + x[i + 1] * code[i + 1] + x[i + 2] * code[i + 2] + x[i + 3] * code[i + 3];
+            float quad = affine_mul<BITS>(x[i], half, i);
+#pragma unroll
+            for (int k = 1; k < 4; ++k) quad = affine_mad<BITS>(x[i + k], half, i + k, quad);
+            dot = i == 0 ? quad : dot + quad;
         }
     } else {
+        dot = affine_mul<BITS>(x[0], half, 0);
 #pragma unroll
-        for (int i = 0; i < WIDTH; ++i) { if constexpr (EXACT) dot = __builtin_fmaf(x[i], code[i], dot); else dot += x[i] * code[i]; }
+        for (int i = 1; i < WIDTH; ++i) dot = affine_mad<BITS>(x[i], half, i, dot);
+    }
+    return dot * 0x1p24f;
+}
+template <int BITS, int WIDTH>
+__device__ __forceinline__ float affine_dot_any(const uint32_t* codes, const float* x) {
+    uint32_t words[WIDTH * BITS / 32];   // (a copy the compiler cannot see through: it would keep the conversions of both rows for all tokens)
+#pragma unroll
+    for (int i = 0; i < WIDTH * BITS / 32; ++i) asm("" : "=v"(words[i]) : "0"(codes[i]));
+    auto code = [&](int i) { return float((words[i * BITS / 32] >> (i * BITS % 32)) & (BITS == 4 ? 15u : 255u)); };
+    float dot = 0;
+    if constexpr (BITS == 4) {
+#pragma unroll
+        for (int i = 0; i < WIDTH; i += 4) dot += x[i] * code(i) + x[i + 1] * code(i + 1) + x[i + 2] * code(i + 2) + x[i + 3] * code(i + 3);
+    } else {
+#pragma unroll
+        for (int i = 0; i < WIDTH; ++i) dot += x[i] * code(i);
     }
     return dot;
 }
@@ -115,11 +172,12 @@ __device__ __forceinline__ float affine_sum(const float* x) {
 
 // The walk for nt staged tokens; out_at: lane t < nt (of each half wave) holds where token t's output row begins.
 // (nt and exact are the same in every lane.  As template parameters they made eight walks, whose common first steps the
-// compiler moved in front of the choice between them: 200 registers instead of 144.)
+// compiler moved in front of the choice between them: 200 registers.)
 template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS>
 __device__ __forceinline__ void affine_walk(AffineStream<BITS, WIDTH, GATED>& st, typename AffineStream<BITS, WIDTH, GATED>::Slot (&ring)[kAffineAhead],
                                             const uint8_t* lds, float* out, uint64_t out_at, uint32_t tile, bool float_output, uint32_t nt, bool exact) {
-    const uint32_t blocks = st.blocks, pitch = affine_pitch<WIDTH>(blocks), token = affine_token_bytes<WIDTH>(st.K), lane = st.lane;
+    using Stream = AffineStream<BITS, WIDTH, GATED>;
+    const uint32_t blocks = st.blocks, token = affine_token_bytes<WIDTH>(st.K), lane = st.lane;
     const uint32_t total = (st.end - tile) * st.steps;
     float r[TOKENS][2];
 #pragma unroll
@@ -129,39 +187,36 @@ __device__ __forceinline__ void affine_walk(AffineStream<BITS, WIDTH, GATED>& st
 #pragma unroll
         for (uint32_t d = 0; d < kAffineAhead; ++d) {
             if (i0 + d >= total) break;
-            float code[2][WIDTH], scale[2], bias[2];
-            uint32_t words[2][AffineStream<BITS, WIDTH, GATED>::DW];
+            float scale[2], bias[2];
+            uint32_t words[2][Stream::DW];
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
 #pragma unroll
-                for (uint32_t i = 0; i < AffineStream<BITS, WIDTH, GATED>::DW; ++i) words[q][i] = ring[d].q[q][i];
-                if constexpr (TOKENS > 1) affine_codes<BITS, WIDTH>(words[q], code[q]);
+                for (uint32_t i = 0; i < Stream::DW; ++i) words[q][i] = ring[d].q[q][i];
                 scale[q] = b16(uint16_t(ring[d].s[q])); bias[q] = b16(uint16_t(ring[d].b[q]));
             }
             st.fetch(ring[d]);
-            const uint32_t b = step * 32 + lane, at = min(b, blocks - 1);
+            const uint32_t b = step * 32 + lane;
+            const uint8_t* block = lds + (Stream::kWide ? b : min(b, blocks - 1)) * AffineBlock<WIDTH>::kBytes;
+            auto tokens = [&](auto dot_of) {
 #pragma unroll
-            for (uint32_t t = 0; t < TOKENS; ++t) {
-                if (t >= nt) break;
-                const uint8_t* row = lds + t * token;
-                float x[WIDTH];
+                for (uint32_t t = 0; t < TOKENS; ++t) {
+                    if (t >= nt) break;
+                    float x[WIDTH], sum;
+                    affine_inputs<WIDTH>(block + t * token, x, sum);
 #pragma unroll
-                for (int i = 0; i < WIDTH; i += 4) {
-                    const float4 v = reinterpret_cast<const float4*>(row)[uint32_t(i / 4) * pitch + at];
-                    x[i] = v.x; x[i + 1] = v.y; x[i + 2] = v.z; x[i + 3] = v.w;
-                }
-                const float sum = reinterpret_cast<const float*>(row + WIDTH / 4 * pitch * 16)[at];
-#pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    if constexpr (TOKENS == 1) {   // (one matrix's codes at a time: four waves per SIMD)
-                        __builtin_amdgcn_sched_barrier(0);
-                        affine_codes<BITS, WIDTH>(words[q], code[q]);
+                    for (int q = 0; q < 2; ++q) {
+                        const float more = r[t][q] + (scale[q] * dot_of(q, x) + sum * bias[q]);
+                        r[t][q] = Stream::kWide || b < blocks ? more : r[t][q];
                     }
-                    const float dot = exact ? affine_dot<BITS, WIDTH, true>(code[q], x) : affine_dot<BITS, WIDTH, false>(code[q], x);
-                    const float more = r[t][q] + (scale[q] * dot + sum * bias[q]);
-                    r[t][q] = b < blocks ? more : r[t][q];
                 }
-            }
+            };
+            if (exact) {
+                uint32_t half[2][WIDTH / 2];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) affine_halves<BITS, WIDTH>(words[q], half[q]);
+                tokens([&](int q, const float* x) { return affine_dot_exact<BITS, WIDTH>(half[q], x); });
+            } else tokens([&](int q, const float* x) { return affine_dot_any<BITS, WIDTH>(words[q], x); });
             if (++step < st.steps) continue;
             step = 0;
 #pragma unroll
@@ -205,18 +260,29 @@ __device__ __forceinline__ void affine_rows(const AffineMatrix (&m)[2], uint32_t
     st.aim();
 #pragma unroll
     for (uint32_t d = 0; d < kAffineAhead; ++d) st.fetch(ring[d]);
-    constexpr uint32_t kPlanes = WIDTH / 4;
-    const uint32_t blocks = st.blocks, pitch = affine_pitch<WIDTH>(blocks), token = affine_token_bytes<WIDTH>(K);
+    constexpr uint32_t kPieces = WIDTH / 4, P = AffineBlock<WIDTH>::kPiece;
+    const uint32_t blocks = st.blocks, token = affine_token_bytes<WIDTH>(K);
     bool strange = false;
 #pragma unroll 1
     for (uint32_t t = 0; t < nt; ++t) {
         const float* src = x + uint64_t(uint32_t(__builtin_amdgcn_readlane(int(from), int(t)))) * K;
 #pragma unroll 2
         for (uint32_t i = tid; i < K / 4; i += 256) {
-            const uint4 v = ldg_u4(src, i);
-            strange |= ((v.x | v.y | v.z | v.w) & 0xffffu) != 0 ||
-                       max(max(v.x & 0x7fffffffu, v.y & 0x7fffffffu), max(v.z & 0x7fffffffu, v.w & 0x7fffffffu)) >= 0x71800000u;   // 2^100
-            reinterpret_cast<uint4*>(lds + t * token)[i % kPlanes * pitch + i / kPlanes] = v;
+            const uint4 q = ldg_u4(src, i);
+            const uint32_t v[4] = {q.x, q.y, q.z, q.w};
+            uint32_t* to = reinterpret_cast<uint32_t*>(lds + t * token + i / kPieces * AffineBlock<WIDTH>::kBytes + i % kPieces * 16);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {   // (as a magnitude from 2^-100 on: one comparison)
+                const uint32_t a = v[k] & 0x7fffffffu;
+                strange |= (v[k] & 0xffffu) != 0 || (a - 0x0d800000u >= 0x71800000u - 0x0d800000u && a != 0);
+            }
+            typedef uint32_t piece __attribute__((ext_vector_type(P)));
+#pragma unroll
+            for (uint32_t k = 0; k < 4; k += P) {
+                if constexpr (P == 4) *reinterpret_cast<piece*>(to) = piece{v[0], v[1], v[2], v[3]};
+                else if constexpr (P == 2) *reinterpret_cast<piece*>(to + k) = piece{v[k], v[k + 1]};
+                else to[k] = v[k];
+            }
         }
     }
     if (__ballot(strange)) strange = true;
@@ -226,13 +292,10 @@ __device__ __forceinline__ void affine_rows(const AffineMatrix (&m)[2], uint32_t
     for (uint32_t t = 0; t < nt; ++t)
 #pragma unroll 1
         for (uint32_t b = tid; b < blocks; b += 256) {
-            float xb[WIDTH];
-#pragma unroll
-            for (int i = 0; i < WIDTH; i += 4) {
-                const float4 v = reinterpret_cast<const float4*>(lds + t * token)[uint32_t(i / 4) * pitch + b];
-                xb[i] = v.x; xb[i + 1] = v.y; xb[i + 2] = v.z; xb[i + 3] = v.w;
-            }
-            reinterpret_cast<float*>(lds + t * token + kPlanes * pitch * 16)[b] = affine_sum<BITS, WIDTH>(xb);
+            float xb[WIDTH], unset;
+            uint8_t* block = lds + t * token + b * AffineBlock<WIDTH>::kBytes;
+            affine_inputs<WIDTH>(block, xb, unset);
+            *reinterpret_cast<float*>(block + 4 * WIDTH) = affine_sum<BITS, WIDTH>(xb);
         }
     lds_barrier();
     const bool exact = __builtin_amdgcn_readfirstlane(int(strange_s[0] | strange_s[1] | strange_s[2] | strange_s[3])) == 0;
@@ -252,12 +315,11 @@ template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS>
 __global__ __launch_bounds__(256, 3) void affine_op_kernel(AffineJob j) {
     extern __shared__ __align__(16) uint8_t affine_lds[];
     const uint32_t tile0 = blockIdx.x * j.share, end = min(tile0 + j.share, j.tiles);
-    for (uint32_t t0 = blockIdx.y * j.chunk; t0 < j.tokens; t0 += gridDim.y * j.chunk) {
-        affine_rows<BITS, WIDTH, GATED, TOKENS>(j.m, j.K, j.N, j.group, j.x, j.out, min(j.chunk, j.tokens - t0),
-                                        [&](uint32_t t) { return j.in_rows ? uint32_t(j.in_rows[t0 + t]) : t0 + t; },
-                                        [&](uint32_t t) { return j.out_rows ? uint32_t(j.out_rows[t0 + t]) : t0 + t; }, tile0, end, j.float_output != 0, affine_lds);
-        lds_barrier();   // (the next tokens overwrite the rows)
-    }
+    const uint64_t t0 = (uint64_t(blockIdx.z) * gridDim.y + blockIdx.y) * j.chunk;
+    if (t0 >= j.tokens) return;
+    affine_rows<BITS, WIDTH, GATED, TOKENS>(j.m, j.K, j.N, j.group, j.x, j.out, min(j.chunk, j.tokens - uint32_t(t0)),
+                                            [&](uint32_t t) { return j.in_rows ? uint32_t(j.in_rows[t0 + t]) : uint32_t(t0) + t; },
+                                            [&](uint32_t t) { return j.out_rows ? uint32_t(j.out_rows[t0 + t]) : uint32_t(t0) + t; }, tile0, end, j.float_output != 0, affine_lds);
 }
 
 // The routed experts of one layer and, where its formats are theirs, the shared expert: blockIdx.y walks the shared expert's
@@ -267,30 +329,30 @@ struct ExpertPhase {
     const uint8_t* shared_record; uint64_t shared_off[6];
     const uint32_t *jobs; const int32_t *count, *slots;
     const float *x, *shared_x; float *out, *shared_out;                // x: layer input (gate/up) or sorted activations (down)
-    uint32_t K, N, group, topk, tokens, chunk, shared_jobs, tiles, share;   // chunk: tokens of a job (a shared job too)
+    uint32_t K, N, group, topk, tokens, chunk, shared_jobs, max_jobs, tiles, share;   // chunk: tokens of a job (a shared job too)
 };
 template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS>
 __global__ __launch_bounds__(256, TOKENS == 1 ? 4 : 3) void expert_phase_kernel(ExpertPhase p) {
     extern __shared__ __align__(16) uint8_t affine_lds[];
     const uint32_t tile0 = blockIdx.x * p.share, end = min(tile0 + p.share, p.tiles);
-    const uint32_t total = p.shared_jobs + uint32_t(*p.count);
-    for (uint32_t job = blockIdx.y; job < total; job += gridDim.y) {
-        const bool shared = job < p.shared_jobs;
-        uint32_t first, expert = 0, nt;
-        if (shared) { first = job * p.chunk; nt = min(p.chunk, p.tokens - first); }
-        else { const uint32_t packed = p.jobs[job - p.shared_jobs]; first = packed & 0xfffffu; expert = (packed >> 20) & 1023u; nt = (packed >> 30) + 1u; }
-        const uint8_t* r = shared ? p.shared_record : p.records + uint64_t(expert) * p.stride;
-        AffineMatrix m[2];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            auto at = [&](int i) { return r + (shared ? p.shared_off[3 * q + i] : p.off[3 * q + i]); };
-            m[q] = AffineMatrix{at(0), reinterpret_cast<const uint16_t*>(at(1)), reinterpret_cast<const uint16_t*>(at(2))};
-        }
-        affine_rows<BITS, WIDTH, GATED, TOKENS>(m, p.K, p.N, p.group, shared ? p.shared_x : p.x, shared ? p.shared_out : p.out, nt,
-                                        [&](uint32_t t) { return GATED && !shared ? uint32_t(p.slots[first + t]) / p.topk : first + t; },
-                                        [&](uint32_t t) { return GATED || shared ? first + t : uint32_t(p.slots[first + t]); }, tile0, end, false, affine_lds);
-        lds_barrier();   // (the next job overwrites the rows)
+    const uint32_t job = blockIdx.z * gridDim.y + blockIdx.y;
+    const bool shared = job < p.shared_jobs;
+    uint32_t first = job * p.chunk, expert = 0, nt = min(p.chunk, p.tokens - first);
+    if (!shared) {   // (the list has room for every job of the grid; what lies past the count is not used)
+        const uint32_t count = uint32_t(uniform(*p.count)), packed = uint32_t(uniform(int32_t(p.jobs[min(job - p.shared_jobs, p.max_jobs - 1)])));
+        if (job - p.shared_jobs >= count) return;
+        first = packed & 0xfffffu; expert = (packed >> 20) & 1023u; nt = (packed >> 30) + 1u;
     }
+    const uint8_t* r = shared ? p.shared_record : p.records + uint64_t(expert) * p.stride;
+    AffineMatrix m[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        auto at = [&](int i) { return r + (shared ? p.shared_off[3 * q + i] : p.off[3 * q + i]); };
+        m[q] = AffineMatrix{at(0), reinterpret_cast<const uint16_t*>(at(1)), reinterpret_cast<const uint16_t*>(at(2))};
+    }
+    affine_rows<BITS, WIDTH, GATED, TOKENS>(m, p.K, p.N, p.group, shared ? p.shared_x : p.x, shared ? p.shared_out : p.out, nt,
+                                            [&](uint32_t t) { return GATED && !shared ? uint32_t(p.slots[first + t]) / p.topk : first + t; },
+                                            [&](uint32_t t) { return GATED || shared ? first + t : uint32_t(p.slots[first + t]); }, tile0, end, false, affine_lds);
 }
 
 static bool wide(uint32_t K, uint32_t N) { return K % 512 == 0 && N % 8 == 0; }
@@ -307,7 +369,7 @@ static uint32_t affine_share(uint32_t tiles, uint64_t jobs) {
     while (share > 1 && uint64_t((tiles + share - 1) / share) * jobs < 2048) share /= 2;
     return share;
 }
-// Tokens per workgroup: four where their rows leave room for three workgroups in a compute unit's LDS.
+// Tokens per workgroup: two where their rows leave room for three workgroups in a compute unit's LDS.
 template <int WIDTH> static uint32_t affine_chunk(uint32_t K) {
     uint32_t chunk = kAffineTokens;
     while (chunk > 1 && chunk * affine_token_bytes<WIDTH>(K) > 53 * 1024) chunk /= 2;
@@ -318,7 +380,8 @@ uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t bits) {
     by_format<false>(bits, wide(K, N), [&]<int BITS, int WIDTH, bool GATED>() { chunk = affine_chunk<WIDTH>(K); });
     return chunk;
 }
-constexpr uint32_t kMaxGridY = 32768;   // (the kernels walk what is left)
+// (A grid's y holds fewer than 2^16 workgroups: the rest of a longer list goes to z.)
+static dim3 affine_grid(uint32_t x, uint32_t jobs) { const uint32_t y = std::min(jobs, 32768u); return dim3(x, y, (jobs + y - 1) / y); }
 
 void launch_affine(hipStream_t s, const AffineDesc& a) {
     AffineJob j{};
@@ -331,7 +394,7 @@ void launch_affine(hipStream_t s, const AffineDesc& a) {
         j.chunk = std::min(affine_chunk<WIDTH>(j.K), j.tokens);
         const uint32_t rows = AffineStream<BITS, WIDTH, GATED>::kTileRows, chunks = (j.tokens + j.chunk - 1) / j.chunk;
         j.tiles = (j.N + rows - 1) / rows; j.share = affine_share(j.tiles, chunks);
-        const dim3 grid((j.tiles + j.share - 1) / j.share, std::min(chunks, kMaxGridY));
+        const dim3 grid = affine_grid((j.tiles + j.share - 1) / j.share, chunks);
         const uint32_t lds = j.chunk * affine_token_bytes<WIDTH>(j.K);
         if (j.chunk == 1) hipLaunchKernelGGL((affine_op_kernel<BITS, WIDTH, GATED, 1>), grid, dim3(256), lds, s, j);
         else hipLaunchKernelGGL((affine_op_kernel<BITS, WIDTH, GATED, kAffineTokens>), grid, dim3(256), lds, s, j);
@@ -344,14 +407,14 @@ void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d) {
     ExpertPhase p{};
     p.records = (const uint8_t*)d.records; p.stride = d.stride; p.shared_record = (const uint8_t*)d.shared_record;
     for (int i = 0; i < 6; ++i) { p.off[i] = d.off[i]; p.shared_off[i] = d.shared_off[i]; }
-    p.jobs = d.jobs; p.count = d.count; p.slots = d.slots;
+    p.jobs = d.jobs; p.count = d.count; p.slots = d.slots; p.max_jobs = d.max_jobs;
     p.x = d.x; p.out = d.out; p.shared_x = d.shared_x; p.shared_out = d.shared_out;
     p.K = d.K; p.N = d.N; p.group = d.group; p.topk = d.topk; p.tokens = d.tokens; p.chunk = d.chunk;
     p.shared_jobs = d.shared_record ? (d.tokens + d.chunk - 1) / d.chunk : 0;
     auto go = [&]<int BITS, int WIDTH, bool GATED>() {
         const uint32_t rows = AffineStream<BITS, WIDTH, GATED>::kTileRows;
         p.tiles = (p.N + rows - 1) / rows; p.share = affine_share(p.tiles, d.max_jobs + p.shared_jobs);
-        const dim3 grid((p.tiles + p.share - 1) / p.share, std::min(d.max_jobs + p.shared_jobs, kMaxGridY));
+        const dim3 grid = affine_grid((p.tiles + p.share - 1) / p.share, d.max_jobs + p.shared_jobs);
         const uint32_t most = std::min(d.chunk, d.tokens), lds = most * affine_token_bytes<WIDTH>(d.K);
         if (most == 1) hipLaunchKernelGGL((expert_phase_kernel<BITS, WIDTH, GATED, 1>), grid, dim3(256), lds, s, p);
         else hipLaunchKernelGGL((expert_phase_kernel<BITS, WIDTH, GATED, kAffineTokens>), grid, dim3(256), lds, s, p);
@@ -780,7 +843,7 @@ void launch_route(hipStream_t s, const float* logits, uint32_t T, uint32_t E, ui
 // expert that scanned the whole id array took 14.4 us for 10 slots and 66 us for 400; this takes 5.8 us, the selection
 // included, and 4.8 us.)
 //
-// jobs, optional: the list of (expert, sorted positions) that the expert kernels walk, at most `chunk` <= 4 positions of one
+// jobs, optional: the list of (expert, sorted positions) that the expert kernels walk, at most `chunk` (up to four) positions of one
 // expert each: first position | expert << 20 | (positions - 1) << 30 (a call has at most 2^20 slots).  `count` then is its
 // length; else `selected` lists the experts that have slots and `count` is their number.
 //

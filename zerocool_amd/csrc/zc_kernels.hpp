@@ -20,7 +20,7 @@ void launch_affine(hipStream_t s, const AffineDesc& a);          // literal lane
 bool xint_supported(const zc_linear& l);                          // wide affine Q4, group 64, 16-byte aligned
 void launch_affine_xint(hipStream_t s, const AffineDesc& a);     // exact-integer matrix-core form
 
-uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t bits);   // tokens one workgroup of these kernels takes at a time: 1, 2 or 4
+uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t bits);   // tokens one workgroup of these kernels takes at a time: 1 or 2
 
 struct ExpertPhaseDesc {
     const void* records; uint64_t stride;
