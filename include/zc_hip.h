@@ -226,7 +226,9 @@ zc_status zc_hip_stack_create(zc_hip_ctx* ctx, const zc_moe_config* cfg, const z
 zc_status zc_hip_stack_destroy(zc_hip_ctx* ctx, zc_hip_stack* stack);
 zc_status zc_hip_stack_decode(zc_hip_ctx* ctx, zc_hip_stack* stack, const float* x, uint32_t tokens,
                               float* out, const zc_stack_trace* trace, uint32_t flags);
-/* 1 if zc_hip_stack_decode would take the persistent single-launch path for `tokens`. */
+/* 1 if the persistent single-launch kernels take `tokens`.  zc_hip_stack_decode uses them for one token, behind an expert store,
+ * with clocks in the trace, and once zc_hip_stack_set_wait_limit gave the waits a bound; otherwise it may go layer by layer where
+ * that is faster (the same bytes either way). */
 int zc_hip_stack_is_persistent(zc_hip_ctx* ctx, zc_hip_stack* stack, uint32_t tokens);
 /* Bound of every wait of the persistent kernel on another workgroup, in polls (0 restores the default, about four
  * seconds' worth).  A wait that runs out makes the launch give up everywhere and zc_hip_moe_check report it; the stack

@@ -80,3 +80,41 @@ def test_router_logits(ctx, T, K, E):
     w, x, off = oracle.bf_bits(rng.standard_normal((E, K))), oracle.bf(rng.standard_normal((T, K))), rng.standard_normal(E).astype(f32)
     got = ctx.router_logits(ctx.upload(w), ctx.upload(x), T, K, E, ctx.upload(off)).numpy(f32)
     assert got.tobytes() == oracle.router_logits(w, x, T, K, E, off).tobytes()
+
+
+# The single-launch kernels for several tokens, which a stack takes once its waits have a bound of their own, against the layer
+# by layer path that it takes otherwise: the same bytes, and the same reports for inputs that are not BF16-valued or not routable.
+@pytest.mark.parametrize("hidden,bits,tokens", [(1024, (4, 4, 4, 4), (2, 8, 9, 64, 70)), (1024, (4, 8, 8, 8), (2, 9, 64)), (3072, (4, 4, 4, 4), (3, 17))])
+def test_stack_paths_agree(ctx, hidden, bits, tokens):
+    cfg = workload.tiny_config(hidden=hidden, experts=64, topk=10, inter=512, bits=bits)
+    layers = [workload.LayerWeights(ctx, cfg, 800 + l, ("zipf", 1.1)) for l in range(3)]
+    stack = ctx.stack_create(cfg, [l.layer for l in layers], max(tokens))
+    for T in tokens:
+        n = T * cfg.topk
+        x, out = workload.hidden_rows(ctx, T, hidden, 60 + T), ctx.alloc(T * hidden * 4)
+        ids, w, outs = ctx.alloc(3 * n * 4), ctx.alloc(3 * n * 4), ctx.alloc(3 * T * hidden * 4)
+        got = []
+        for polls in (1 << 22, 0):
+            ctx.stack_set_wait_limit(stack, polls)
+            for trace in (z.StackTrace(ids.ptr, w.ptr, outs.ptr, None), None):
+                ctx.fill(out, 0xff)
+                ctx.stack_decode(stack, x, T, out, trace)
+                ctx.moe_check()
+                got.append(out.numpy(np.uint8).tobytes())
+            got[-2:] = [(got[-2], ids.numpy(np.uint8).tobytes(), w.numpy(np.uint8).tobytes(), outs.numpy(np.uint8).tobytes()), got[-1]]
+            assert got[-2][0] == got[-1]
+        assert got[0] == got[2] and got[1] == got[3]
+        for value, text in ((np.float32(1.0000001), "BF16"), (np.float32("nan"), "invalid router output")):
+            bad = x.numpy(f32)
+            bad[-hidden:] = value           # the last token's row
+            dbad = ctx.upload(bad)
+            ctx.stack_decode(stack, dbad, T, out)
+            with pytest.raises(z.ZcError, match=text):
+                ctx.moe_check()
+            ctx.free(dbad)
+        for b in (x, out, ids, w, outs):
+            ctx.free(b)
+    ctx.stack_destroy(stack)
+    for l in layers:
+        for b in (l.router, l.shared_gate, l.shared_record, l.records, l.offsets):
+            ctx.free(b)

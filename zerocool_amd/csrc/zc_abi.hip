@@ -573,41 +573,15 @@ uint64_t zc_hip_moe_workspace_bytes(const zc_moe_config* cfg, uint32_t tokens) {
     if (validate_config(cfg) != ZC_OK || !tokens) return 0;
     return carve(cfg, tokens, nullptr).bytes;
 }
-uint64_t zc_hip_moe_static_scratch_bytes(void) { return kStaticScratchBytes; }
-// zc_hip_moe_forward with its workspace in the static scratch array of the context's device.  Nothing on this path
-// allocates or frees: no hipMalloc / hipFree / hipHostMalloc, no stream or event creation, no host containers --
-// also while a recording is on (zc_hip_profile): this call records no row, and neither do the operators inside it.
-zc_status zc_hip_moe_forward_static(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe_layer* l, const float* x, uint32_t T,
-                                    float* out, const zc_moe_trace* trace) {
-    Untimed untimed(ctx);
-    if (const zc_status s = validate_config(c)) return s;
-    ZC_REQUIRE(ctx && T, "invalid MoE layer buffers");
-    ZC_REQUIRE(ctx->static_scratch, "the static scratch array was not located for this device");
-    const uint64_t need = carve(c, T, nullptr).bytes;
-    if (need > kStaticScratchBytes) {
-        char text[200];
-        snprintf(text, sizeof text, "zc_hip_moe_forward_static: %u tokens of this shape need %llu bytes of scratch, the static array holds %llu; use zc_hip_moe_forward with a workspace",
-                 T, (unsigned long long)need, (unsigned long long)kStaticScratchBytes);
-        return fail(ZC_INVALID_ARGUMENT, text);
-    }
-    return zc_hip_moe_forward(ctx, c, l, x, T, out, ctx->static_scratch, trace);
-}
-zc_status zc_hip_moe_forward(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe_layer* l, const float* x, uint32_t T,
-                             float* out, void* workspace, const zc_moe_trace* trace) {
-    Timed timed(ctx, "moe_forward");
-    if (const zc_status s = validate_config(c)) return s;
-    ZC_REQUIRE(ctx && l && x && out && workspace && T && T <= 8192, "invalid MoE layer buffers");
-    ZC_REQUIRE(l->router && l->shared_gate && l->shared_record && l->expert_records, "missing MoE layer weights");
-    ZC_REQUIRE(l->record_stride >= zc_hip_record_bytes(c, 0) && l->record_stride % 4 == 0, "expert record stride is too small");
-    ZC_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(workspace) % 256 == 0 &&
-               reinterpret_cast<uintptr_t>(l->router) % 16 == 0 && reinterpret_cast<uintptr_t>(l->expert_records) % 4 == 0 &&
-               reinterpret_cast<uintptr_t>(l->shared_record) % 4 == 0, "MoE layer operands are misaligned");
-    ZC_REQUIRE(x != out, "invalid or overlapping linear output");
+// One exact layer on checked operands.  next, optional: the glue's rows for the layer that follows (combine and glue are then one
+// launch where the width allows it, and `out` may be null).  check: report inputs that are not BF16-valued.
+static zc_status moe_layer(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe_layer* l, const float* x, uint32_t T,
+                           float* out, void* workspace, const zc_moe_trace* trace, float* next, bool check) {
     const Workspace w = carve(c, T, workspace);
     hipStream_t s = ctx->stream;
     const uint32_t H = c->hidden, I = c->inter, E = c->experts, k = c->topk;
     // 1-2. router logits and the shared expert's gate, top-k + softmax (model.cpp:434-436)
-    zc::launch_router(s, l->router, x, T, H, E, l->router_offsets, w.logits, l->shared_gate, w.gate);
+    zc::launch_router(s, l->router, x, T, H, E, l->router_offsets, w.logits, l->shared_gate, w.gate, check ? ctx->moe_status : nullptr);
     // 4. positions / selected, on the device (model.cpp:449-479): the expert kernels' job list, at most `chunk` tokens a job
     const uint32_t chunk = std::min(zc::affine_job_tokens(H, I, c->bits_gate_up), zc::affine_job_tokens(I, H, c->bits_down));
     uint32_t* jobs = reinterpret_cast<uint32_t*>(w.rows);   // (n words: a job holds at least one slot)
@@ -641,7 +615,8 @@ zc_status zc_hip_moe_forward(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
         zc::launch_expert_phase(s, p);
     }
     // 7. weighted combine (model.cpp:553-556)
-    zc::launch_moe_sum(s, w.expert_out, w.weights, w.shared, w.gate, T, H, k, out);
+    if (next) zc::launch_moe_sum_glue(s, w.expert_out, w.weights, w.shared, w.gate, T, H, k, out, next);
+    else zc::launch_moe_sum(s, w.expert_out, w.weights, w.shared, w.gate, T, H, k, out);
     ZC_LAUNCHED();
     if (trace) {
         if (trace->logits) ZC_HIP(hipMemcpyAsync(trace->logits, w.logits, uint64_t(T) * E * 4, hipMemcpyDeviceToDevice, s));
@@ -652,6 +627,38 @@ zc_status zc_hip_moe_forward(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
         if (trace->gate) ZC_HIP(hipMemcpyAsync(trace->gate, w.gate, uint64_t(T) * 4, hipMemcpyDeviceToDevice, s));
     }
     return ZC_OK;
+}
+uint64_t zc_hip_moe_static_scratch_bytes(void) { return kStaticScratchBytes; }
+// zc_hip_moe_forward with its workspace in the static scratch array of the context's device.  Nothing on this path
+// allocates or frees: no hipMalloc / hipFree / hipHostMalloc, no stream or event creation, no host containers --
+// also while a recording is on (zc_hip_profile): this call records no row, and neither do the operators inside it.
+zc_status zc_hip_moe_forward_static(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe_layer* l, const float* x, uint32_t T,
+                                    float* out, const zc_moe_trace* trace) {
+    Untimed untimed(ctx);
+    if (const zc_status s = validate_config(c)) return s;
+    ZC_REQUIRE(ctx && T, "invalid MoE layer buffers");
+    ZC_REQUIRE(ctx->static_scratch, "the static scratch array was not located for this device");
+    const uint64_t need = carve(c, T, nullptr).bytes;
+    if (need > kStaticScratchBytes) {
+        char text[200];
+        snprintf(text, sizeof text, "zc_hip_moe_forward_static: %u tokens of this shape need %llu bytes of scratch, the static array holds %llu; use zc_hip_moe_forward with a workspace",
+                 T, (unsigned long long)need, (unsigned long long)kStaticScratchBytes);
+        return fail(ZC_INVALID_ARGUMENT, text);
+    }
+    return zc_hip_moe_forward(ctx, c, l, x, T, out, ctx->static_scratch, trace);
+}
+zc_status zc_hip_moe_forward(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe_layer* l, const float* x, uint32_t T,
+                             float* out, void* workspace, const zc_moe_trace* trace) {
+    Timed timed(ctx, "moe_forward");
+    if (const zc_status s = validate_config(c)) return s;
+    ZC_REQUIRE(ctx && l && x && out && workspace && T && T <= 8192, "invalid MoE layer buffers");
+    ZC_REQUIRE(l->router && l->shared_gate && l->shared_record && l->expert_records, "missing MoE layer weights");
+    ZC_REQUIRE(l->record_stride >= zc_hip_record_bytes(c, 0) && l->record_stride % 4 == 0, "expert record stride is too small");
+    ZC_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(workspace) % 256 == 0 &&
+               reinterpret_cast<uintptr_t>(l->router) % 16 == 0 && reinterpret_cast<uintptr_t>(l->expert_records) % 4 == 0 &&
+               reinterpret_cast<uintptr_t>(l->shared_record) % 4 == 0, "MoE layer operands are misaligned");
+    ZC_REQUIRE(x != out, "invalid or overlapping linear output");
+    return moe_layer(ctx, c, l, x, T, out, workspace, trace, nullptr, false);
 }
 // Prefill: the same layer with the expert products as a sorted-token grouped GEMM on the bf16 matrix cores.
 namespace {
@@ -855,6 +862,7 @@ struct zc_hip_stack {
     uint32_t epoch = 1u << 12;
     uint32_t tag_base = 0;            // tags of the one-token kernel's exchange words: advanced by that kernel's launches only
     uint32_t wait_limit = 1u << 22;   // polls before a wait on another workgroup gives up
+    bool bounded_waits = false;       // the caller set that bound: its launches are the ones that have such waits
     int cus = 0; uint32_t lds_limit = 0;
     bool persistent_ok = false;
     // layered path
@@ -1080,7 +1088,7 @@ static zc_status launch_piece(zc_hip_ctx* ctx, zc_hip_stack* st, const float* x,
 }
 zc_status zc_hip_stack_set_wait_limit(zc_hip_ctx* ctx, zc_hip_stack* st, uint32_t polls) {
     ZC_REQUIRE(ctx && st, "null argument");
-    st->wait_limit = polls ? polls : 1u << 22;
+    st->wait_limit = polls ? polls : 1u << 22; st->bounded_waits = polls != 0;
     return ZC_OK;
 }
 zc_status zc_hip_stack_set_speculation(zc_hip_ctx* ctx, zc_hip_stack* st, int on) {
@@ -1116,6 +1124,19 @@ zc_status zc_hip_stack_settle(zc_hip_ctx* ctx, zc_hip_stack* st) {
     ZC_REQUIRE(ctx && st, "null argument");
     return st->store ? observe_pending(ctx, st) : ZC_OK;
 }
+// Whether a batch that a single launch could take goes layer by layer, five launches each.  us per layer, single launch -> layer by
+// layer, at 2, 8, 32 and 64 tokens, one layer with N(0, 0.5) offsets / four to six layers with Zipf(1.1) offsets, whose tokens
+// agree on nearly all experts behind the first layer:
+//   hidden 2048, Q4        49 -> 38   92 -> 64   195 -> 144   302 -> 232  /  39 -> 36   65 -> 56   147 -> 120   231 -> 202
+//   hidden 2048, mixed     60 -> 45  111 -> 75   272 -> 168   445 -> 260  /  57 -> 46  105 -> 73   236 -> 146   393 -> 235
+//   hidden 3072, Q4        76 -> 62  188 -> 126  494 -> 365   813 -> 625  /  53 -> 55   97 -> 101  256 -> 257   438 -> 480
+// One token stays with its kernel (27 -> 29, 36 -> 39, 35 -> 43): nothing to share, and no launch between the layers.  Large Q4
+// layers whose tokens agree are better off on the matrix cores (a code is unpacked once for eight tokens there) up to eight tokens
+// and beyond thirty-two, so those keep the single launch whatever their tokens do.
+static bool layers_preferred(const zc_moe_config& c, uint32_t tokens) {
+    if (tokens < 2 || tokens > 64) return false;
+    return !all_q4(c) || uint64_t(c.hidden) * c.inter <= 3u << 19 || (tokens > 8 && tokens <= 32);
+}
 zc_status zc_hip_stack_decode(zc_hip_ctx* ctx, zc_hip_stack* st, const float* x, uint32_t tokens, float* out,
                               const zc_stack_trace* trace, uint32_t flags) {
     Timed timed(ctx, "stack_decode");
@@ -1124,11 +1145,14 @@ zc_status zc_hip_stack_decode(zc_hip_ctx* ctx, zc_hip_stack* st, const float* x,
     const zc_moe_config& c = st->cfg;
     const uint32_t L = uint32_t(st->layers.size()), H = c.hidden, k = c.topk;
     LaunchPlan plan;
-    const uint32_t unit = (flags & 1u) ? 0u : launch_unit(ctx, st, tokens);
+    const uint32_t single = (flags & 1u) ? 0u : launch_unit(ctx, st, tokens);
+    const bool preferred = single && !st->store && !st->bounded_waits && !(trace && trace->clocks) && layers_preferred(c, tokens);
+    const uint32_t unit = preferred ? 0u : single;
     if (st->store) {
         ZC_REQUIRE(unit && tokens <= unit, "a stack behind an expert store runs as one launch only");
         if (const zc_status s = zc_hip_store_table_refresh_joining(st->store)) return s;
     }
+    if (preferred && trace && trace->ids) ZC_REQUIRE(trace->weights, "a routing trace needs both ids and weights");
     // More than eight tokens go through the single-launch kernels sixty-four (or eight) at a time, one launch per piece (tokens
     // do not interact inside a layer); every piece stays on the device from the first layer to the last.
     if (unit) {
@@ -1166,9 +1190,11 @@ zc_status zc_hip_stack_decode(zc_hip_ctx* ctx, zc_hip_stack* st, const float* x,
             tr.ids = trace->ids ? trace->ids + uint64_t(l) * tokens * k : nullptr;
             tr.weights = trace->weights ? trace->weights + uint64_t(l) * tokens * k : nullptr;
         }
-        if (const zc_status s = zc_hip_moe_forward(ctx, &c, &st->layers[l], cur, tokens, y, st->workspace, trace ? &tr : nullptr)) return s;
-        if (trace && trace->outputs) ZC_HIP(hipMemcpyAsync(trace->outputs + uint64_t(l) * tokens * H, y, uint64_t(tokens) * H * 4, hipMemcpyDeviceToDevice, ctx->stream));
-        if (l + 1 < L) { zc::launch_stack_glue(ctx->stream, y, tokens, H, st->xb); cur = st->xb; }
+        // the glue's rows go where nothing reads any more: the layer's input is its own, or the previous layer's glue in xb
+        const bool fused = l + 1 < L && zc::moe_sum_glue_fits(H), outputs = trace && trace->outputs;
+        if (const zc_status s = moe_layer(ctx, &c, &st->layers[l], cur, tokens, fused && !outputs ? nullptr : y, st->workspace, trace ? &tr : nullptr, fused ? st->xb : nullptr, l == 0 && preferred)) return s;
+        if (outputs) ZC_HIP(hipMemcpyAsync(trace->outputs + uint64_t(l) * tokens * H, y, uint64_t(tokens) * H * 4, hipMemcpyDeviceToDevice, ctx->stream));
+        if (l + 1 < L) { if (!fused) zc::launch_stack_glue(ctx->stream, y, tokens, H, st->xb); cur = st->xb; }
     }
     ZC_LAUNCHED();
     return ZC_OK;

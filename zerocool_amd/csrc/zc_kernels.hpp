@@ -36,9 +36,10 @@ void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d);
 
 void launch_plain(hipStream_t s, const void* w, uint32_t dtype, const float* x, uint32_t K, uint32_t N,
                   uint32_t tokens, float* out, bool float_output);
-// gate_w, optional: a BF16 row whose plain dot with every token goes to gate [T], rounded to BF16 (the shared expert's gate)
+// gate_w, optional: a BF16 row whose plain dot with every token goes to gate [T], rounded to BF16 (the shared expert's gate);
+// status, optional, for at most 64 tokens and K a multiple of 128 up to 4096: bit 4 is set if an input is not BF16-valued
 void launch_router(hipStream_t s, const void* w, const float* x, uint32_t T, uint32_t K, uint32_t E,
-                   const float* offsets, float* out, const void* gate_w = nullptr, float* gate = nullptr);
+                   const float* offsets, float* out, const void* gate_w = nullptr, float* gate = nullptr, int32_t* status = nullptr);
 void launch_route(hipStream_t s, const float* logits, uint32_t T, uint32_t E, uint32_t topk, int32_t* ids, float* weights);
 void launch_dispatch(hipStream_t s, const int32_t* ids, uint32_t tokens, uint32_t topk, uint32_t E, int32_t* offsets,
                      int32_t* slots, int32_t* rows, int32_t* selected, int32_t* count, int32_t* status);
@@ -55,6 +56,9 @@ void launch_moe_sum(hipStream_t s, const float* experts, const float* weights, c
                     uint32_t T, uint32_t H, uint32_t topk, float* out);
 void launch_moe_sum_half(hipStream_t s, const uint16_t* experts, const float* weights, const float* shared, const float* gate,
                          uint32_t T, uint32_t H, uint32_t topk, float* out);
+void launch_moe_sum_glue(hipStream_t s, const float* experts, const float* weights, const float* shared, const float* gate,
+                         uint32_t T, uint32_t H, uint32_t topk, float* out, float* next);   // out may be null
+bool moe_sum_glue_fits(uint32_t H);
 void launch_stack_glue(hipStream_t s, const float* y, uint32_t T, uint32_t H, float* out);
 void launch_synth_words(hipStream_t s, uint32_t* dst, uint64_t count, uint64_t seed);
 void launch_synth_scales(hipStream_t s, uint16_t* sc, uint16_t* bi, uint64_t count, uint64_t seed, float lo, float span, float factor);
