@@ -58,7 +58,15 @@ struct zc_hip_ctx {
     // The prefill layer runs its shared expert beside the router, the selection and the dispatch sort, which are chains of
     // small kernels: a second stream of default priority, forked from and joined to `stream` by two events per call.
     hipStream_t beside = nullptr; hipEvent_t fork = nullptr, join = nullptr;
-    uint32_t affine_policy = 1;        // 0 literal lane kernels, 1 exact-integer matrix-core kernels where possible
+    // 0 literal lane kernels, 1 exact-integer matrix-core kernels where possible.  The lanes are faster on
+    // every size measured (K and N of 512 to 4096 and 1024 x 8192, 1 to 512 rows) but one, a single gate/up row of 1024 x 8192 (6.1 -> 6.4),
+    // and on rows that are not BF16-valued by two to six times at few rows.  us a call, matrix cores -> lanes, gate/up at 1, 4, 21, 64 and 512 rows / down:
+    //   hidden 2048  7.5 -> 5.2  19.5 -> 6.4  21.4 -> 8.7   22.0 -> 16.3  114 -> 79  /   5.5 -> 4.4   9.7 -> 4.4  10.2 -> 6.8   18.3 -> 10.8   84 -> 52
+    //   hidden 2560  7.2 -> 5.6  19.3 -> 7.2  21.2 -> 11.3  38.6 -> 23.1  175 -> 115 /  (its rows of 640 always went to the lanes)
+    //   hidden 3072  9.0 -> 6.1  25.8 -> 8.1  28.5 -> 16.0  54.7 -> 34.2  320 -> 200 /   7.0 -> 3.9  17.7 -> 5.3  34.4 -> 10.6  51.4 -> 20.6  231 -> 116
+    // A call of the integer form first builds digit planes of its rows in LDS, one workgroup a compute unit, and fills the chip with
+    // tiles of sixteen rows only from a few hundred tokens on.
+    uint32_t affine_policy = 0;
     void* static_scratch = nullptr;    // this device's copy of the static scratch array
     std::mutex mutex;
     // Profiling (KernelConfig::profile + Metal::label, metal.mm:267-270): while on, every operator call made through this
