@@ -116,6 +116,25 @@ def test_single_token_rows(ctx, K, N):  # :1100-1125 shapes plus the benchmark s
         ctx.free(b)
 
 
+@pytest.mark.parametrize("bits,N", [(4, 8), (4, 6), (8, 8), (8, 6)])   # the four block widths
+def test_longest_affine_rows(ctx, bits, N):
+    # 32768 inputs and their block sums are a compute unit's whole LDS.  Besides a BF16-valued row: rows in which the elements
+    # that one wave of the workgroup brings in are not BF16-valued, which the other waves have to learn.
+    K = 32768
+    rng = np.random.default_rng(bits * 100 + N)
+    w = rng.integers(0, 2 ** 32, N * K * bits // 32, dtype=np.uint64).astype(np.uint32)
+    s, b = oracle.bf_bits(0.01 * rng.random(N * K // 64) + 1e-4), oracle.bf_bits(-0.08 * rng.random(N * K // 64))
+    ol, dl = oracle.make_linear(w, s, b, K, N, 64, bits), dev_linear(ctx, w, s, b, K, N, 64, bits)
+    x = np.tile(oracle.bf(rng.standard_normal(K)), (5, 1))
+    for wave in range(4):
+        x[1 + wave].reshape(-1, 4)[64 * wave + 7::256] = rng.standard_normal((K // 1024, 4))
+    dx = ctx.upload(x.astype(f32))
+    assert same_bytes(ctx.linear(dl, dx, 5, float_output=True).numpy(f32), oracle.linear(ol, x.astype(f32), 5, float_output=True))
+    assert same_bytes(ctx.gated_linear(dl, dl, dx, 5, 5).numpy(f32), oracle.gated_linear(ol, ol, x.astype(f32), 5))
+    for buf in dl._keep + (dx,):
+        ctx.free(buf)
+
+
 # the last three: a row of sixteen-load and eight-load batches plus single steps, rows shorter than one batch, and an odd
 # number of weights (their 16-bit words are then read one by one, not through aligned 32-bit words)
 @pytest.mark.parametrize("K,N", [(10240, 4), (2560, 1), (2560, 48), (2048, 1), (3072, 1), (864, 5), (96, 2), (257, 3)])

@@ -256,7 +256,6 @@ template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS, class InRow, class O
 __device__ __forceinline__ void affine_rows(const AffineMatrix (&m)[2], uint32_t K, uint32_t N, uint32_t group, const float* x, float* out, uint32_t nt,
                                             InRow in_row, OutRow out_row, uint32_t tile0, uint32_t end, bool float_output, uint8_t* lds) {
     using Stream = AffineStream<BITS, WIDTH, GATED, TOKENS>;
-    __shared__ uint32_t strange_s[4];
     const uint32_t tid = threadIdx.x;
     Stream st;
     st.K = K; st.N = N; st.blocks = K / WIDTH; st.shift = group == 64 ? 6 : 5; st.groups = K >> st.shift; st.steps = (st.blocks + 31) / 32;
@@ -293,9 +292,20 @@ __device__ __forceinline__ void affine_rows(const AffineMatrix (&m)[2], uint32_t
             }
         }
     }
-    if (__ballot(strange)) strange = true;
-    if ((tid & 63u) == 0) strange_s[tid >> 6] = strange;
+    // Each wave's finding crosses in block w of the first token, wave w's: in the padding behind the bias sum, or, where blocks
+    // have none, in the sum's own place, read before the sums are written.  (An array of its own beside the rows would keep out
+    // the longest rows, of 32768 elements, which fill a compute unit's LDS to the last byte.)
+    constexpr bool kPadded = WIDTH >= 8;
+    auto finding = [&](uint32_t w) { return reinterpret_cast<uint32_t*>(lds + w * AffineBlock<WIDTH>::kBytes + 4 * WIDTH + (kPadded ? 4 : 0)); };
+    const bool any = __ballot(strange) != 0;
+    if ((tid & 63u) == 0) *finding(tid >> 6) = any;
     lds_barrier();
+    uint32_t found = 0;
+    if constexpr (!kPadded) {
+#pragma unroll
+        for (uint32_t w = 0; w < 4; ++w) found |= *finding(w);
+        lds_barrier();
+    }
 #pragma unroll 1
     for (uint32_t t = 0; t < nt; ++t)
 #pragma unroll 1
@@ -306,7 +316,11 @@ __device__ __forceinline__ void affine_rows(const AffineMatrix (&m)[2], uint32_t
             *reinterpret_cast<float*>(block + 4 * WIDTH) = affine_sum<BITS, WIDTH>(xb);
         }
     lds_barrier();
-    const bool exact = __builtin_amdgcn_readfirstlane(int(strange_s[0] | strange_s[1] | strange_s[2] | strange_s[3])) == 0;
+    if constexpr (kPadded) {
+#pragma unroll
+        for (uint32_t w = 0; w < 4; ++w) found |= *finding(w);
+    }
+    const bool exact = __builtin_amdgcn_readfirstlane(int(found)) == 0;
     affine_walk<BITS, WIDTH, GATED, TOKENS>(st, ring, lds, out, out_at, tile0, float_output, nt, exact);
 }
 
