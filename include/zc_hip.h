@@ -88,8 +88,9 @@ zc_status zc_hip_finish(zc_hip_ctx* ctx);
 /* Metal::configure (metal.hpp:87; KernelConfig::policy, metal.hpp:17-26): which kernels
  * serve the affine products.  0 = the literal lane kernels for every shape (the
  * reference's "reference" policy); 1 = the exact-integer matrix-core kernels wherever
- * the shape allows (wide Q4, group 64), literal otherwise.  Default 0, the faster one on
- * nearly every size measured.  Both policies produce identical bytes; only speed differs. */
+ * the shape allows (wide Q4, group 64), literal otherwise; 2 (the default) = the literal
+ * kernels except for sizes where the exact-integer ones are known to be much faster.  All
+ * policies produce identical bytes; only speed differs. */
 zc_status zc_hip_configure(zc_hip_ctx* ctx, uint32_t affine_policy);
 /* HIP-event stopwatch on the context's stream: start enqueues an event, stop enqueues a
  * second one, waits for it and returns the milliseconds between them. */

@@ -103,3 +103,29 @@ def test_xint_32_column_tiles(ctx, kind):
     assert got[2].reshape(T, N)[sample].tobytes() == want[1].tobytes()
     for b in dl._keep + du._keep + (dx, drows):
         ctx.free(b)
+
+
+@pytest.mark.parametrize("K,N,T", [(16384, 12288, 1), (16896, 12288, 1), (16896, 6144, 1), (21504, 6144, 1), (22016, 6144, 1), (16896, 12288, 2)])
+def test_long_rows_by_default(ctx, K, N, T):
+    """Single rows of more than 16384 inputs take the integer form by default when they have many outputs (6144 rows of gate and
+    of up count as 12288): on either side of that line, and of the longest row that it can hold, the bytes of the lane kernels."""
+    rng = np.random.default_rng(K + N + T)
+    bufs = [make(rng, K, N) for _ in range(2)]
+    dl, du = (dev_linear(ctx, *b, K, N) for b in bufs)
+    for kind in ("normal", "special"):
+        x = inputs(rng, K, T, kind); dx = ctx.upload(x)
+        got = {}
+        for policy in (2, 0):
+            ctx.configure(policy)
+            got[policy] = [ctx.linear(dl, dx, T), ctx.linear(dl, dx, T, float_output=True), ctx.gated_linear(dl, du, dx, T, T)]
+        for a, b in zip(got[2], got[0]):
+            assert a.numpy(np.uint8).tobytes() == b.numpy(np.uint8).tobytes(), (K, N, T, kind)
+        sample = np.r_[0:8, N - 8:N]
+        part = lambda v, per: np.ascontiguousarray(v.reshape(N, per)[sample]).ravel()
+        ol = oracle.make_linear(part(bufs[0][0], K // 8), part(bufs[0][1], K // 64), part(bufs[0][2], K // 64), K, 16)
+        assert got[2][0].numpy(f32).reshape(T, N)[:, sample].tobytes() == oracle.linear(ol, x, T).tobytes()
+        for b in got[2] + got[0] + [dx]:
+            ctx.free(b)
+    ctx.configure(2)
+    for b in dl._keep + du._keep:
+        ctx.free(b)

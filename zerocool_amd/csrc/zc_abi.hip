@@ -58,15 +58,8 @@ struct zc_hip_ctx {
     // The prefill layer runs its shared expert beside the router, the selection and the dispatch sort, which are chains of
     // small kernels: a second stream of default priority, forked from and joined to `stream` by two events per call.
     hipStream_t beside = nullptr; hipEvent_t fork = nullptr, join = nullptr;
-    // 0 literal lane kernels, 1 exact-integer matrix-core kernels where possible.  The lanes are faster on
-    // every size measured (K and N of 512 to 4096 and 1024 x 8192, 1 to 512 rows) but one, a single gate/up row of 1024 x 8192 (6.1 -> 6.4),
-    // and on rows that are not BF16-valued by two to six times at few rows.  us a call, matrix cores -> lanes, gate/up at 1, 4, 21, 64 and 512 rows / down:
-    //   hidden 2048  7.5 -> 5.2  19.5 -> 6.4  21.4 -> 8.7   22.0 -> 16.3  114 -> 79  /   5.5 -> 4.4   9.7 -> 4.4  10.2 -> 6.8   18.3 -> 10.8   84 -> 52
-    //   hidden 2560  7.2 -> 5.6  19.3 -> 7.2  21.2 -> 11.3  38.6 -> 23.1  175 -> 115 /  (its rows of 640 always went to the lanes)
-    //   hidden 3072  9.0 -> 6.1  25.8 -> 8.1  28.5 -> 16.0  54.7 -> 34.2  320 -> 200 /   7.0 -> 3.9  17.7 -> 5.3  34.4 -> 10.6  51.4 -> 20.6  231 -> 116
-    // A call of the integer form first builds digit planes of its rows in LDS, one workgroup a compute unit, and fills the chip with
-    // tiles of sixteen rows only from a few hundred tokens on.
-    uint32_t affine_policy = 0;
+    // 0 literal lane kernels, 1 exact-integer matrix-core kernels where possible, 2 the lanes except where prefers_xint() says otherwise.
+    uint32_t affine_policy = 2;
     void* static_scratch = nullptr;    // this device's copy of the static scratch array
     std::mutex mutex;
     // Profiling (KernelConfig::profile + Metal::label, metal.mm:267-270): while on, every operator call made through this
@@ -230,7 +223,7 @@ zc_status zc_hip_copy(zc_hip_ctx* ctx, void* dst, const void* src, uint64_t byte
 }
 zc_status zc_hip_configure(zc_hip_ctx* ctx, uint32_t affine_policy) {
     ZC_REQUIRE(ctx, "null context");
-    ZC_REQUIRE(affine_policy <= 1, "unknown kernel policy");
+    ZC_REQUIRE(affine_policy <= 2, "unknown kernel policy");
     ctx->affine_policy = affine_policy;
     return ZC_OK;
 }
@@ -404,6 +397,21 @@ static uint64_t weight_bytes(const zc_linear* l) {
     return l->quantized ? uint64_t(l->input) * l->output * l->bits / 8 : uint64_t(l->input) * l->output * (l->dtype == 1 ? 4 : 2);
 }
 
+// Which form serves a product of Q4 matrices that both forms take.  us a call, matrix cores -> lanes, gate/up at 1, 4, 21, 64 and 512 rows / down:
+//   hidden 2048  7.5 -> 5.2  19.5 -> 6.4  21.4 -> 8.7   22.0 -> 16.3  114 -> 79  /   5.5 -> 4.4   9.7 -> 4.4  10.2 -> 6.8   18.3 -> 10.8   84 -> 52
+//   hidden 2560  7.2 -> 5.6  19.3 -> 7.2  21.2 -> 11.3  38.6 -> 23.1  175 -> 115 /  (its rows of 640 always went to the lanes)
+//   hidden 3072  9.0 -> 6.1  25.8 -> 8.1  28.5 -> 16.0  54.7 -> 34.2  320 -> 200 /   7.0 -> 3.9  17.7 -> 5.3  34.4 -> 10.6  51.4 -> 20.6  231 -> 116
+// and on rows that are not BF16-valued the lanes are ahead by two to six times.  A call of the integer form first builds digit
+// planes of its rows in LDS, one workgroup a compute unit, and fills the chip with tiles of sixteen rows only from a few
+// hundred tokens on.  It is ahead where its workgroups fill the chip exactly, by up to a tenth on most such sizes (a gate/up row
+// of 1024 x 8192 5.9 -> 6.5, of 2048 x 16384 11.5 -> 13.6; outputs around these sizes lose as much), and by far for one row of
+// more than 16384 inputs: two of those do not fit a compute unit's LDS together, which leaves the lanes four waves on it.
+// 20480 inputs, plain at 8192, 16384 and 32768 outputs 45 -> 51, 49 -> 99, 93 -> 195, gate/up at 6144 and 16384 45 -> 76, 92 -> 203;
+// from 12288 outputs on also rows that are not BF16-valued lose nothing there (84 -> 78, 85 -> 105).
+static bool prefers_xint(const zc_hip_ctx* ctx, const zc_linear& l, uint32_t matrices, uint32_t tokens) {
+    if (ctx->affine_policy != 2) return ctx->affine_policy == 1;
+    return tokens == 1 && l.input > 16384 && l.input <= zc::kXintLongestRow && uint64_t(l.output) * matrices >= 12288;
+}
 zc_status zc_hip_linear_into(zc_hip_ctx* ctx, const zc_linear* l, const float* x, uint32_t tokens, float* out, int float_output) {
     Timed timed(ctx, "linear");
     ZC_REQUIRE(ctx && l, "null argument");
@@ -416,7 +424,7 @@ zc_status zc_hip_linear_into(zc_hip_ctx* ctx, const zc_linear* l, const float* x
                "invalid or overlapping linear output");
     if (l->quantized) {
         zc::AffineDesc a; a.gate = *l; a.x = x; a.out = out; a.tokens = tokens; a.float_output = float_output ? 1 : 0;
-        if (ctx->affine_policy == 1 && zc::xint_supported(*l)) zc::launch_affine_xint(ctx->stream, a);
+        if (prefers_xint(ctx, *l, 1, tokens) && zc::xint_supported(*l)) zc::launch_affine_xint(ctx->stream, a);
         else zc::launch_affine(ctx->stream, a);
     } else {
         ZC_REQUIRE(l->dtype <= 1, "unsupported plain matrix dtype");
@@ -455,7 +463,7 @@ zc_status zc_hip_gated_linear(zc_hip_ctx* ctx, const zc_linear* gate, const zc_l
         for (int32_t r : host) ZC_REQUIRE(r >= 0 && uint32_t(r) < x_rows, "fused gate/up row outside input");
     }
     zc::AffineDesc a; a.gate = *gate; a.up = *up; a.gated = true; a.x = x; a.in_rows = rows; a.out = out; a.tokens = tokens;
-    if (ctx->affine_policy == 1 && zc::xint_supported(*gate) && zc::xint_supported(*up)) zc::launch_affine_xint(ctx->stream, a);
+    if (prefers_xint(ctx, *gate, 2, tokens) && zc::xint_supported(*gate) && zc::xint_supported(*up)) zc::launch_affine_xint(ctx->stream, a);
     else zc::launch_affine(ctx->stream, a);
     ZC_LAUNCHED();
     return ZC_OK;

@@ -19,6 +19,7 @@ struct AffineDesc {
 void launch_affine(hipStream_t s, const AffineDesc& a);          // literal lane arithmetic, any shape
 bool xint_supported(const zc_linear& l);                          // wide affine Q4, group 64, 16-byte aligned
 void launch_affine_xint(hipStream_t s, const AffineDesc& a);     // exact-integer matrix-core form
+constexpr uint32_t kXintLongestRow = 21504;                       // of one token: its digit planes and fp32 copy fill 160 KiB of LDS
 
 uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t bits);   // tokens one workgroup of these kernels takes at a time: 1 or 2
 

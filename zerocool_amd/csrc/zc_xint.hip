@@ -110,6 +110,7 @@ bool xint_supported(const zc_linear& l) {
            reinterpret_cast<uintptr_t>(l.weight) % 16 == 0;
 }
 
+static_assert(XintLayout{kXintLongestRow}.bytes() + 4 * kXintLongestRow <= 160 * 1024 && kXintLongestRow % 512 == 0);
 void launch_affine_xint(hipStream_t s, const AffineDesc& a) {
     XintJob j{};
     j.w0 = (const uint8_t*)a.gate.weight; j.s0 = (const uint16_t*)a.gate.scales; j.b0 = (const uint16_t*)a.gate.biases;

@@ -290,7 +290,8 @@ class Context:
         return ms.value
 
     def configure(self, affine_policy):
-        """0: literal lane kernels everywhere; 1 (default): exact-integer matrix-core kernels where the shape allows."""
+        """0: literal lane kernels everywhere; 1: exact-integer matrix-core kernels where the shape allows; 2 (default): the lanes
+        except for the sizes where the integer form is much faster.  The same bytes in all three."""
         self._call("zc_hip_configure", C.c_uint32(affine_policy))
 
     def finish(self):
