@@ -158,8 +158,9 @@ static void test_heavy_rows() {   // :1500-1533
     auto out = gpu.zeros((uint64_t(T) * TopK + 1) * H), expected = gpu.zeros(uint64_t(T) * TopK * H);
     auto weights = gpu.zeros(uint64_t(T) * TopK), shared = gpu.zeros(uint64_t(T) * H), gate = gpu.zeros(T);
     for (auto& w : weights->floats()) w = 0.125f;
-    for (bool reference_kernels : {false, true}) for (uint32_t count : {127u, 128u, 129u, 257u, 513u}) {
-        KernelConfig config; if (reference_kernels) config.policy = "reference"; gpu.configure(config);
+    CHECK(KernelConfig{}.policy == "automatic");   // configuring an engine for another reason leaves its kernels as they were
+    for (const char* policy : {"automatic", "exact-int", "reference"}) for (uint32_t count : {127u, 128u, 129u, 257u, 513u}) {
+        KernelConfig config; config.policy = policy; gpu.configure(config);
         std::memset(out->data, 0, out->bytes); std::memset(expected->data, 0, expected->bytes);
         std::memset(out->data + expected->bytes, 0xa5, H * 4);
         std::vector<int> positions;

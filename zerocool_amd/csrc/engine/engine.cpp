@@ -61,7 +61,7 @@ std::span<float> Buffer::floats() const {
 }
 
 void KernelConfig::validate() const {
-    if (policy != "reference" && policy != "exact-int") throw std::invalid_argument("unknown kernel policy");
+    if (policy != "automatic" && policy != "reference" && policy != "exact-int") throw std::invalid_argument("unknown kernel policy");
 }
 zc_moe_config MoeShape::abi() const {
     return zc_moe_config{hidden, experts, topk, inter, group, bits_gate_up, bits_down, shared_bits_gate_up, shared_bits_down};
@@ -73,7 +73,7 @@ Metal::~Metal() { if (ctx_) zc_hip_destroy(ctx_); }
 void Metal::budget(uint64_t bytes) { budget_ = bytes; }
 void Metal::configure(KernelConfig config) {
     config.validate();
-    check(zc_hip_configure(ctx_, config.policy == "reference" ? 0u : 1u));
+    check(zc_hip_configure(ctx_, config.policy == "reference" ? 0u : config.policy == "exact-int" ? 1u : 2u));
     check(zc_hip_profile(ctx_, config.profile ? 1 : 0));
 }
 void Metal::label(std::string stage, int layer, uint32_t tokens, uint32_t offset, std::span<const uint32_t>) {

@@ -54,7 +54,7 @@ struct Linear {
 };
 // metal.hpp:17-43, the part that concerns this path
 struct KernelConfig {
-    std::string policy = "exact-int";   // "reference": literal lane kernels everywhere
+    std::string policy = "automatic";   // as an unconfigured engine; "reference": literal lane kernels everywhere, "exact-int": the integer form where it can
     bool profile = false;               // record one timed row per operator call, tagged by Metal::label
     void validate() const;
 };
