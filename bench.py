@@ -117,7 +117,7 @@ def one_launch_layer(ctx, name, tokens, reps, warmup=5, skew=("zipf", 1.1), spec
         ctx.stack_decode(stack, xs[i % INPUTS], tokens, out)
     ms = ctx.timer_stop() / reps
     ctx.moe_check()
-    persistent = tokens == 1 and ctx.stack_is_persistent(stack, tokens)   # (two to 64 tokens of hidden 2048 go layer by layer)
+    persistent = ctx.stack_single_launch(stack, tokens)
     ctx.stack_destroy(stack)
     for b in xs + [out, ws, ref, ids, wts, lw.router, lw.shared_gate, lw.shared_record, lw.records]:
         ctx.free(b)
@@ -125,6 +125,13 @@ def one_launch_layer(ctx, name, tokens, reps, warmup=5, skew=("zipf", 1.1), spec
             "distinct_experts": float(np.mean(unique)), "slots_per_distinct_expert": tokens * c.topk / float(np.mean(unique)),
             "GBps": nbytes / (ms * 1e-3) / 1e9, "frac_of_hbm_peak": nbytes / (ms * 1e-3) / 8e12,
             "guessing": bool(speculate), "path": "persistent single-launch kernel" if persistent else "layer by layer"}
+
+
+def decode_kernel(tokens, single_launch):
+    if not single_launch:
+        return "zc::expert_phase_kernel (five launches a layer)"
+    kernel = "decode_stack_kernel" if tokens == 1 else "decode_multi_kernel" if tokens <= 8 else "decode_wide_kernel"
+    return f"zc::{kernel} (one launch = one step)"
 
 
 def prefill_workload(ctx, args):
@@ -235,7 +242,7 @@ def main():
         ctx.free(a); ctx.free(b)
     r = run(stack, cfg, L, T, args.steps, args.warmup)
     ms, nbytes = r["ms"], r["bytes"]
-    persistent = ctx.stack_is_persistent(stack, T) and not 8 < T <= 32   # (nine to 32 tokens of this shape go layer by layer)
+    persistent = ctx.stack_single_launch(stack, T)
     achieved = nbytes / (ms * 1e-3) / 1e9
     traffic = None
     if (L, T) == (48, 1) and os.path.exists(TRAFFIC_FILE):
@@ -255,8 +262,7 @@ def main():
                    "parity_gate": "output bytes equal the layer-by-layer operator path on this input (checked before timing)"},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": 8000.0, "unit": "GB/s", "frac": achieved / 8000.0,
                      "traffic": traffic, "traffic_source": os.path.relpath(TRAFFIC_FILE, ROOT) if traffic else None,
-                     "kernel": "zc::decode_stack_kernel (one launch = one step)" if T == 1 else "zc::decode_multi_kernel (one launch = one step)" if T <= 8
-                               else "zc::decode_wide_kernel (one launch = one step)" if persistent else "zc::expert_phase_kernel (five launches a layer)",
+                     "kernel": decode_kernel(T, persistent),
                      "algorithmic_bytes_per_launch": int(nbytes), "launch_us": ms * 1e3},
     }
 
@@ -314,12 +320,12 @@ def main():
             r8 = run(stack, cfg, L, 8, quick, 2)
             extra["stack_batch8"] = {"tokens_per_s": 8 / (r8["ms"] * 1e-3), "ms_per_step": r8["ms"], "GBps": r8["bytes"] / (r8["ms"] * 1e-3) / 1e9,
                                      "frac_of_hbm_peak": r8["bytes"] / (r8["ms"] * 1e-3) / 8e12, "distinct_experts_per_layer": r8["unique"],
-                                     "kernel": "zc::decode_multi_kernel"}
-            for tokens in (32, 64):   # layer by layer, and one launch of the kernel for nine to sixty-four tokens
+                                     "kernel": decode_kernel(8, ctx.stack_single_launch(stack, 8))}
+            for tokens in (32, 64):
                 rw = run(stack, cfg, L, tokens, max(4, quick // 4), 1, inputs=2)
                 extra[f"stack_batch{tokens}"] = {"tokens_per_s": tokens / (rw["ms"] * 1e-3), "ms_per_step": rw["ms"], "GBps": rw["bytes"] / (rw["ms"] * 1e-3) / 1e9,
                                                  "distinct_experts_per_layer": rw["unique"],
-                                                 "kernel": "zc::expert_phase_kernel (five launches a layer)" if tokens == 32 else "zc::decode_wide_kernel"}
+                                                 "kernel": decode_kernel(tokens, ctx.stack_single_launch(stack, tokens))}
             # The same records behind routers with a milder popularity skew (Zipf exponent 0.5: the offsets span 3.1 instead
             # of 6.9) and with none at all, so that consecutive tokens share fewer experts and a batch of eight touches
             # several times more records.

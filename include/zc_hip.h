@@ -205,12 +205,14 @@ zc_status zc_hip_moe_check(zc_hip_ctx* ctx);
  * between the reference's MoE layers (attention / GDN / hyper-connections) is outside
  * this path; the stack stands in for it with a glue that keeps activations bounded and
  * BF16-valued: x_next = bf(y * (1 / max|y|)) per token (zc_hip_stack_glue).
- * Up to 64 tokens run as ONE persistent kernel launch for the whole stack (routing,
+ * Up to 64 tokens can run as ONE persistent kernel launch for the whole stack (routing,
  * dispatch and combine stay on the device, no host synchronisation between layers; one
  * kernel each for one token, two to eight, and nine to sixty-four), larger batches as
- * one such launch per 64 tokens; shapes those kernels do not take run layer by layer
- * through zc_hip_moe_forward.  All give identical bytes.
- * out: [tokens][hidden], the last layer's output.  flags bit 0: force the layer-by-layer path. */
+ * one such launch per 64 tokens.  One token does; two to sixty-four go layer by layer (five
+ * launches each) where that is faster, as do shapes those kernels do not take.  All give
+ * identical bytes.
+ * out: [tokens][hidden], the last layer's output.  flags bit 0: force the layer-by-layer path;
+ * bit 1: the single launch where its kernels take the batch, also where layer by layer is faster. */
 typedef struct zc_hip_stack zc_hip_stack;
 typedef struct {       /* optional device buffers, any may be NULL */
     int32_t* ids;      /* [n_layers][tokens][topk] */
@@ -227,12 +229,14 @@ zc_status zc_hip_stack_create(zc_hip_ctx* ctx, const zc_moe_config* cfg, const z
 zc_status zc_hip_stack_destroy(zc_hip_ctx* ctx, zc_hip_stack* stack);
 zc_status zc_hip_stack_decode(zc_hip_ctx* ctx, zc_hip_stack* stack, const float* x, uint32_t tokens,
                               float* out, const zc_stack_trace* trace, uint32_t flags);
-/* 1 if the persistent single-launch kernels take `tokens`.  zc_hip_stack_decode uses them for one token, behind an expert store,
- * with clocks in the trace, and once zc_hip_stack_set_wait_limit gave the waits a bound; otherwise it may go layer by layer where
- * that is faster (the same bytes either way). */
+/* 1 if the persistent single-launch kernels can take `tokens`. */
 int zc_hip_stack_is_persistent(zc_hip_ctx* ctx, zc_hip_stack* stack, uint32_t tokens);
+/* 1 if zc_hip_stack_decode (without flags) takes them for `tokens`: they can, and the stack has a store, a bound of its own for
+ * the waits (below), or they are the faster way.  A trace with clocks takes them wherever they can. */
+int zc_hip_stack_single_launch(zc_hip_ctx* ctx, zc_hip_stack* stack, uint32_t tokens);
 /* Bound of every wait of the persistent kernel on another workgroup, in polls (0 restores the default, about four
- * seconds' worth).  A wait that runs out makes the launch give up everywhere and zc_hip_moe_check report it; the stack
+ * seconds' worth).  While the bound is not the default, batches that would go layer by layer for speed (and wait for nothing)
+ * take the single launch.  A wait that runs out makes the launch give up everywhere and zc_hip_moe_check report it; the stack
  * stays usable.  No counterpart in the reference (its command buffers cannot wait on each other); tests use a bound of
  * one poll to exercise the give-up path without a lost workgroup. */
 zc_status zc_hip_stack_set_wait_limit(zc_hip_ctx* ctx, zc_hip_stack* stack, uint32_t polls);

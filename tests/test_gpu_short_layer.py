@@ -82,8 +82,8 @@ def test_router_logits(ctx, T, K, E):
     assert got.tobytes() == oracle.router_logits(w, x, T, K, E, off).tobytes()
 
 
-# The single-launch kernels for several tokens, which a stack takes once its waits have a bound of their own, against the layer
-# by layer path that it takes otherwise: the same bytes, and the same reports for inputs that are not BF16-valued or not routable.
+# The single-launch kernels for several tokens, which a call can ask for, against the layer by layer path that it takes
+# otherwise: the same bytes, and the same reports for inputs that are not BF16-valued or not routable.
 @pytest.mark.parametrize("hidden,bits,tokens", [(1024, (4, 4, 4, 4), (2, 8, 9, 64, 70)), (1024, (4, 8, 8, 8), (2, 9, 64)), (3072, (4, 4, 4, 4), (3, 17))])
 def test_stack_paths_agree(ctx, hidden, bits, tokens):
     cfg = workload.tiny_config(hidden=hidden, experts=64, topk=10, inter=512, bits=bits)
@@ -94,11 +94,10 @@ def test_stack_paths_agree(ctx, hidden, bits, tokens):
         x, out = workload.hidden_rows(ctx, T, hidden, 60 + T), ctx.alloc(T * hidden * 4)
         ids, w, outs = ctx.alloc(3 * n * 4), ctx.alloc(3 * n * 4), ctx.alloc(3 * T * hidden * 4)
         got = []
-        for polls in (1 << 22, 0):
-            ctx.stack_set_wait_limit(stack, polls)
+        for single in (True, False):
             for trace in (z.StackTrace(ids.ptr, w.ptr, outs.ptr, None), None):
                 ctx.fill(out, 0xff)
-                ctx.stack_decode(stack, x, T, out, trace)
+                ctx.stack_decode(stack, x, T, out, trace, single=single)
                 ctx.moe_check()
                 got.append(out.numpy(np.uint8).tobytes())
             got[-2:] = [(got[-2], ids.numpy(np.uint8).tobytes(), w.numpy(np.uint8).tobytes(), outs.numpy(np.uint8).tobytes()), got[-1]]
@@ -108,9 +107,10 @@ def test_stack_paths_agree(ctx, hidden, bits, tokens):
             bad = x.numpy(f32)
             bad[-hidden:] = value           # the last token's row
             dbad = ctx.upload(bad)
-            ctx.stack_decode(stack, dbad, T, out)
-            with pytest.raises(z.ZcError, match=text):
-                ctx.moe_check()
+            for single in (True, False):
+                ctx.stack_decode(stack, dbad, T, out, single=single)
+                with pytest.raises(z.ZcError, match=text):
+                    ctx.moe_check()
             ctx.free(dbad)
         for b in (x, out, ids, w, outs):
             ctx.free(b)

@@ -41,11 +41,11 @@ def oracle_stack(cfg, layers, x, T):
     return np.stack(ids), np.stack(weights), np.stack(outs)
 
 
-def run_stack(ctx, cfg, stack, x_dev, T, L, layered):
+def run_stack(ctx, cfg, stack, x_dev, T, L, layered, single=False):
     n = T * cfg.topk
     ids, w, outs = ctx.alloc(L * n * 4), ctx.alloc(L * n * 4), ctx.alloc(L * T * cfg.hidden * 4)
     out = ctx.alloc(T * cfg.hidden * 4)
-    ctx.stack_decode(stack, x_dev, T, out, z.StackTrace(ids.ptr, w.ptr, outs.ptr, None), layered=layered)
+    ctx.stack_decode(stack, x_dev, T, out, z.StackTrace(ids.ptr, w.ptr, outs.ptr, None), layered=layered, single=single)
     ctx.moe_check()
     r = (ids.numpy(np.int32).reshape(L, T, cfg.topk), w.numpy(f32).reshape(L, T, cfg.topk),
          outs.numpy(f32).reshape(L, T, cfg.hidden), out.numpy(f32).reshape(T, cfg.hidden))
@@ -66,9 +66,9 @@ def _check_stack(ctx, cfg, L, tokens, seed, skew, persistent, mutate=None):
         x = x_dev.numpy(f32)
         want = oracle_stack(cfg, hosts, x, T)
         assert ctx.stack_is_persistent(stack, T) == (persistent(T) if callable(persistent) else persistent)   # above eight tokens: launches of eight and the rest
-        for layered in (True, False):
-            got = run_stack(ctx, cfg, stack, x_dev, T, L, layered)
-            name = "layered" if layered else "persistent"
+        # layer by layer, by the single-launch kernels where they take the batch, and whichever of the two is the default
+        for name in ("layered", "persistent", "default"):
+            got = run_stack(ctx, cfg, stack, x_dev, T, L, name == "layered", name == "persistent")
             assert got[0].tobytes() == want[0].tobytes(), f"{name}: routing ids differ (T={T})"
             assert got[1].tobytes() == want[1].tobytes(), f"{name}: softmax weights differ (T={T})"
             assert got[2].tobytes() == want[2].tobytes(), f"{name}: layer outputs differ (T={T})"
@@ -161,6 +161,28 @@ def test_stand_in_stack_six_layers(ctx):  # the 48-layer stack's shape and Zipf(
     check_stack(ctx, workload.config("F"), 6, [1, 8], seed=71)
 
 
+def test_which_way_a_batch_goes(ctx):
+    # What the default takes is told by stack_single_launch (decode asks the same rule); a bound of the waits selects the single
+    # launch only where it is not the default's own.
+    cfg = workload.tiny_config(hidden=1024, experts=64, topk=10, inter=512)
+    layers = [workload.LayerWeights(ctx, cfg, 83 + l, None) for l in range(2)]
+    stack = ctx.stack_create(cfg, [l.layer for l in layers], 70)
+    assert all(ctx.stack_is_persistent(stack, T) for T in (1, 2, 64, 70))
+    for polls, single in ((0, [True, False, False, True]), (1 << 22, [True, False, False, True]), (1 << 21, [True] * 4), (0, [True, False, False, True])):
+        ctx.stack_set_wait_limit(stack, polls)
+        assert [ctx.stack_single_launch(stack, T) for T in (1, 2, 64, 70)] == single, polls
+    assert not ctx.stack_single_launch(stack, 71)      # more than the stack was made for
+    ctx.stack_destroy(stack)
+    odd = workload.tiny_config(hidden=768, experts=64, topk=10, inter=512)
+    w = workload.LayerWeights(ctx, odd, 89, None)
+    stack = ctx.stack_create(odd, [w.layer], 4)
+    assert not ctx.stack_is_persistent(stack, 1) and not ctx.stack_single_launch(stack, 1)
+    ctx.stack_destroy(stack)
+    for l in layers + [w]:
+        for b in (l.router, l.shared_gate, l.shared_record, l.records):
+            ctx.free(b)
+
+
 def test_stack_reports_invalid_router_output(ctx):
     cfg = workload.tiny_config(hidden=2048, experts=32, topk=4, inter=512)
     layers = [workload.LayerWeights(ctx, cfg, 77 + l, None) for l in range(2)]
@@ -199,13 +221,13 @@ def test_single_token_launches_across_the_tag_wrap(ctx):
     out1, out2 = ctx.alloc(cfg.hidden * 4), ctx.alloc(2 * cfg.hidden * 4)
     ctx.stack_decode(stack, x1, 1, out1); ctx.moe_check()
     first = out1.numpy(f32).tobytes()
-    ctx.stack_decode(stack, x2, 2, out2); ctx.moe_check()
+    ctx.stack_decode(stack, x2, 2, out2, single=True); ctx.moe_check()
     first2 = out2.numpy(f32).tobytes()
     launches = 65535 // 2 + 300
     for i in range(launches):
         ctx.stack_decode(stack, x1, 1, out1)
         if i % 97 == 0:
-            ctx.stack_decode(stack, x2, 2, out2)
+            ctx.stack_decode(stack, x2, 2, out2, single=True)
         if i % 4000 == 0 or i > launches - 600 and i % 7 == 0:
             ctx.moe_check()
             assert out1.numpy(f32).tobytes() == first, f"launch {i}"
@@ -216,7 +238,7 @@ def test_single_token_launches_across_the_tag_wrap(ctx):
     # that follows must not meet a tag its predecessor left (run lengths around a multiple of the tag period included).
     for run in (1, 409, 1228, 1229, 2979):
         for _ in range(run):
-            ctx.stack_decode(stack, x2, 2, out2)
+            ctx.stack_decode(stack, x2, 2, out2, single=True)
         ctx.stack_decode(stack, x1, 1, out1); ctx.moe_check()
         assert out1.numpy(f32).tobytes() == first, f"after {run} two-token launches"
         assert out2.numpy(f32).tobytes() == first2
@@ -239,7 +261,7 @@ def test_a_wait_that_runs_out_is_reported_and_the_stack_stays_usable(ctx):
     xs = {T: workload.hidden_rows(ctx, T, cfg.hidden, 30 + T) for T in (1, 2, 12)}
     want = {}
     for T in (1, 2, 12):
-        ctx.stack_decode(stack, xs[T], T, out[T]); ctx.moe_check()
+        ctx.stack_decode(stack, xs[T], T, out[T], single=True); ctx.moe_check()
         want[T] = out[T].numpy(f32).tobytes()
     for T in (1, 2, 12):
         ctx.stack_set_wait_limit(stack, 1)
@@ -253,7 +275,7 @@ def test_a_wait_that_runs_out_is_reported_and_the_stack_stays_usable(ctx):
                 reported += 1
         assert reported > 0, "a one-poll bound never ran out"
         ctx.stack_set_wait_limit(stack, 0)
-        ctx.stack_decode(stack, xs[T], T, out[T]); ctx.moe_check()
+        ctx.stack_decode(stack, xs[T], T, out[T], single=True); ctx.moe_check()
         assert out[T].numpy(f32).tobytes() == want[T]
     ctx.stack_destroy(stack)
     for l in layers:
@@ -290,7 +312,7 @@ def test_guessed_experts_never_change_the_result(ctx, skew):
             ctx.stack_decode(stack, xs[i], 1, out); ctx.moe_check()
             assert out.numpy(f32).tobytes() == want[i], f"token {i}, guessing {'on' if on else 'off'}"
             if i == 2:
-                ctx.stack_decode(stack, x2, 2, out2); ctx.moe_check()
+                ctx.stack_decode(stack, x2, 2, out2, single=True); ctx.moe_check()
     ctx.stack_destroy(stack)
     for l in layers:
         for b in (l.router, l.shared_gate, l.shared_record, l.records):

@@ -862,6 +862,7 @@ zc_status zc_hip_stack_glue(zc_hip_ctx* ctx, const float* y, uint32_t tokens, ui
 }
 }  // extern "C"
 
+constexpr uint32_t kWaitPolls = 1u << 22;
 struct zc_hip_stack {
     zc_moe_config cfg{};
     std::vector<zc_moe_layer> layers;
@@ -877,8 +878,7 @@ struct zc_hip_stack {
     uint32_t pred_turn = 0; bool pred_valid = false, speculate = true;
     uint32_t epoch = 1u << 12;
     uint32_t tag_base = 0;            // tags of the one-token kernel's exchange words: advanced by that kernel's launches only
-    uint32_t wait_limit = 1u << 22;   // polls before a wait on another workgroup gives up
-    bool bounded_waits = false;       // the caller set that bound: its launches are the ones that have such waits
+    uint32_t wait_limit = kWaitPolls;   // polls before a wait on another workgroup gives up; another bound than the default selects the launches that have such waits
     int cus = 0; uint32_t lds_limit = 0;
     bool persistent_ok = false;
     // layered path
@@ -1102,9 +1102,27 @@ static zc_status launch_piece(zc_hip_ctx* ctx, zc_hip_stack* st, const float* x,
     }
     return ZC_OK;
 }
+// Whether a batch that a single launch could take goes layer by layer, five launches each.  us per layer, single launch -> layer by
+// layer, at 2, 8, 32 and 64 tokens, one layer with N(0, 0.5) offsets / four to six layers with Zipf(1.1) offsets, whose tokens
+// agree on nearly all experts behind the first layer:
+//   hidden 2048, Q4        49 -> 38   92 -> 64   195 -> 144   302 -> 232  /  39 -> 36   65 -> 56   147 -> 120   231 -> 202
+//   hidden 2048, mixed     60 -> 45  111 -> 75   272 -> 168   445 -> 260  /  57 -> 46  105 -> 73   236 -> 146   393 -> 235
+//   hidden 3072, Q4        76 -> 62  188 -> 126  494 -> 365   813 -> 625  /  53 -> 55   97 -> 101  256 -> 257   438 -> 480
+// One token stays with its kernel (27 -> 29, 36 -> 39, 35 -> 43): nothing to share, and no launch between the layers.  Large Q4
+// layers whose tokens agree are better off on the matrix cores (a code is unpacked once for eight tokens there) up to eight tokens
+// and beyond thirty-two, so those keep the single launch whatever their tokens do.
+// Hidden 512 and 1024 with an intermediate size of 512, 1536 and 2048 with 512 and 1024, 32 to 512 experts, Q4 and mixed, were timed
+// at 2 to 64 tokens both ways too: layer by layer is ahead everywhere, by 2 % (hidden 2048 x 1024, 64 agreeing tokens,
+// which the line below leaves to the single launch with the large ones) to 40 %.
+// (Above sixty-four tokens the rule says nothing: the inputs' check for BF16 values is the short router's, which ends there.)
+static bool layers_preferred(const zc_hip_stack* st, uint32_t tokens) {
+    const zc_moe_config& c = st->cfg;
+    if (tokens < 2 || tokens > 64 || st->store || st->wait_limit != kWaitPolls) return false;
+    return !all_q4(c) || uint64_t(c.hidden) * c.inter <= 3u << 19 || (tokens > 8 && tokens <= 32);
+}
 zc_status zc_hip_stack_set_wait_limit(zc_hip_ctx* ctx, zc_hip_stack* st, uint32_t polls) {
     ZC_REQUIRE(ctx && st, "null argument");
-    st->wait_limit = polls ? polls : 1u << 22; st->bounded_waits = polls != 0;
+    st->wait_limit = polls ? polls : kWaitPolls;
     return ZC_OK;
 }
 zc_status zc_hip_stack_set_speculation(zc_hip_ctx* ctx, zc_hip_stack* st, int on) {
@@ -1116,6 +1134,9 @@ int zc_hip_stack_is_persistent(zc_hip_ctx* ctx, zc_hip_stack* st, uint32_t token
     if (!ctx || !st || !tokens) return 0;
     if (st->store && tokens > 64) return 0;
     return launch_unit(ctx, st, tokens) ? 1 : 0;
+}
+int zc_hip_stack_single_launch(zc_hip_ctx* ctx, zc_hip_stack* st, uint32_t tokens) {
+    return zc_hip_stack_is_persistent(ctx, st, tokens) && !layers_preferred(st, tokens) ? 1 : 0;
 }
 // Waits for the routes of the launch that the store has not seen yet, and shows them to the store.
 static zc_status observe_pending(zc_hip_ctx* ctx, zc_hip_stack* st) {
@@ -1140,19 +1161,6 @@ zc_status zc_hip_stack_settle(zc_hip_ctx* ctx, zc_hip_stack* st) {
     ZC_REQUIRE(ctx && st, "null argument");
     return st->store ? observe_pending(ctx, st) : ZC_OK;
 }
-// Whether a batch that a single launch could take goes layer by layer, five launches each.  us per layer, single launch -> layer by
-// layer, at 2, 8, 32 and 64 tokens, one layer with N(0, 0.5) offsets / four to six layers with Zipf(1.1) offsets, whose tokens
-// agree on nearly all experts behind the first layer:
-//   hidden 2048, Q4        49 -> 38   92 -> 64   195 -> 144   302 -> 232  /  39 -> 36   65 -> 56   147 -> 120   231 -> 202
-//   hidden 2048, mixed     60 -> 45  111 -> 75   272 -> 168   445 -> 260  /  57 -> 46  105 -> 73   236 -> 146   393 -> 235
-//   hidden 3072, Q4        76 -> 62  188 -> 126  494 -> 365   813 -> 625  /  53 -> 55   97 -> 101  256 -> 257   438 -> 480
-// One token stays with its kernel (27 -> 29, 36 -> 39, 35 -> 43): nothing to share, and no launch between the layers.  Large Q4
-// layers whose tokens agree are better off on the matrix cores (a code is unpacked once for eight tokens there) up to eight tokens
-// and beyond thirty-two, so those keep the single launch whatever their tokens do.
-static bool layers_preferred(const zc_moe_config& c, uint32_t tokens) {
-    if (tokens < 2 || tokens > 64) return false;
-    return !all_q4(c) || uint64_t(c.hidden) * c.inter <= 3u << 19 || (tokens > 8 && tokens <= 32);
-}
 zc_status zc_hip_stack_decode(zc_hip_ctx* ctx, zc_hip_stack* st, const float* x, uint32_t tokens, float* out,
                               const zc_stack_trace* trace, uint32_t flags) {
     Timed timed(ctx, "stack_decode");
@@ -1162,7 +1170,7 @@ zc_status zc_hip_stack_decode(zc_hip_ctx* ctx, zc_hip_stack* st, const float* x,
     const uint32_t L = uint32_t(st->layers.size()), H = c.hidden, k = c.topk;
     LaunchPlan plan;
     const uint32_t single = (flags & 1u) ? 0u : launch_unit(ctx, st, tokens);
-    const bool preferred = single && !st->store && !st->bounded_waits && !(trace && trace->clocks) && layers_preferred(c, tokens);
+    const bool preferred = single && !(flags & 2u) && !(trace && trace->clocks) && layers_preferred(st, tokens);
     const uint32_t unit = preferred ? 0u : single;
     if (st->store) {
         ZC_REQUIRE(unit && tokens <= unit, "a stack behind an expert store runs as one launch only");

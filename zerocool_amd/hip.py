@@ -449,9 +449,9 @@ class Context:
     def stack_destroy(self, stack):
         self._call("zc_hip_stack_destroy", stack)
 
-    def stack_decode(self, stack, x, tokens, out, trace=None, layered=False):
+    def stack_decode(self, stack, x, tokens, out, trace=None, layered=False, single=False):
         self._call("zc_hip_stack_decode", stack, _ptr(x), C.c_uint32(tokens), _ptr(out),
-                   C.byref(trace) if trace is not None else None, C.c_uint32(1 if layered else 0))
+                   C.byref(trace) if trace is not None else None, C.c_uint32((1 if layered else 0) | (2 if single else 0)))
 
     def stack_set_speculation(self, stack, on):
         self._call("zc_hip_stack_set_speculation", stack, C.c_int(int(on)))
@@ -464,6 +464,9 @@ class Context:
 
     def stack_is_persistent(self, stack, tokens):
         return bool(self.lib.zc_hip_stack_is_persistent(self.handle, stack, C.c_uint32(tokens)))
+
+    def stack_single_launch(self, stack, tokens):
+        return bool(self.lib.zc_hip_stack_single_launch(self.handle, stack, C.c_uint32(tokens)))
 
     # synthetic tensors ---------------------------------------------------
     def synth_words(self, dst, count, seed):
