@@ -899,10 +899,14 @@ bool all_q4(const zc_moe_config& c) { return c.bits_down == 4 && c.shared_bits_g
 // Routed gate/up is affine Q4 (the exact-integer tiles); the down projection and the shared expert may be affine Q8, which
 // the one-token kernel and the kernel for nine to sixty-four tokens run on literal lanes (two to eight tokens of such an
 // artifact go through the latter as well; the kernel for two to eight tokens takes Q4 only).
+// The widest rows of the single-launch kernels.  Batches that go layer by layer instead owe the same report of inputs that are not
+// BF16-valued, which there is the router's.
+constexpr uint32_t kPersistentHidden = 3072;
+static_assert(kPersistentHidden <= zc::kRouterStatusK);
 bool persistent_shape(const zc_moe_config& c) {
     return c.bits_gate_up == 4 && (c.bits_down == 4 || c.bits_down == 8) && (c.shared_bits_gate_up == 4 || c.shared_bits_gate_up == 8) &&
            (c.shared_bits_down == 4 || c.shared_bits_down == 8) && c.group == 64 &&
-           c.hidden % 512 == 0 && c.inter % 512 == 0 && c.hidden <= 3072 && c.inter <= 1024 && c.experts <= 1024 && c.topk <= 64;
+           c.hidden % 512 == 0 && c.inter % 512 == 0 && c.hidden <= kPersistentHidden && c.inter <= 1024 && c.experts <= 1024 && c.topk <= 64;
 }
 }  // namespace
 

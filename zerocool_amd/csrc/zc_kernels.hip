@@ -762,8 +762,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 void launch_router(hipStream_t s, const void* w, const float* x, uint32_t T, uint32_t K, uint32_t E,
                    const float* offsets, float* out, const void* gate_w, float* gate, int32_t* status) {
     const uint32_t tt = T >= 4 ? 4 : T >= 2 ? 2 : 1;
+    static_assert(4 * (kRouterStatusK + 64) * 4 <= kRouterShortLds && kRouterStatusK % 128 == 0);
     const size_t lds = size_t(tt) * (K + 64) * 4;
-    if (T <= 64 && K % 128 == 0 && lds <= 64 * 1024) {   // (two of its workgroups fit a compute unit's LDS)
+    if (T <= 64 && K % 128 == 0 && lds <= kRouterShortLds) {   // (two of its workgroups fit a compute unit's LDS)
         const uint32_t threads = tt <= 2 ? 64 : 256, experts = threads / 16;
         const dim3 grid((E + experts - 1) / experts + (gate_w ? 1 : 0), (T + tt - 1) / tt);
 #define ZC_ROUTER(TT) hipLaunchKernelGGL(router_short_kernel<TT>, grid, dim3(threads), lds, s, (const uint16_t*)w, x, T, K, E, offsets, out, gate_w, gate, status)

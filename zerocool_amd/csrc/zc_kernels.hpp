@@ -38,7 +38,9 @@ void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d);
 void launch_plain(hipStream_t s, const void* w, uint32_t dtype, const float* x, uint32_t K, uint32_t N,
                   uint32_t tokens, float* out, bool float_output);
 // gate_w, optional: a BF16 row whose plain dot with every token goes to gate [T], rounded to BF16 (the shared expert's gate);
-// status, optional, for at most 64 tokens and K a multiple of 128 up to 4096: bit 4 is set if an input is not BF16-valued
+// status, optional, for at most 64 tokens and K a multiple of 128 up to kRouterStatusK (no other kernel sets it): bit 4 is set if
+// an input is not BF16-valued
+constexpr uint32_t kRouterShortLds = 64 * 1024, kRouterStatusK = 3968;
 void launch_router(hipStream_t s, const void* w, const float* x, uint32_t T, uint32_t K, uint32_t E,
                    const float* offsets, float* out, const void* gate_w = nullptr, float* gate = nullptr, int32_t* status = nullptr);
 void launch_route(hipStream_t s, const float* logits, uint32_t T, uint32_t E, uint32_t topk, int32_t* ids, float* weights);
