@@ -110,6 +110,81 @@ def test_prefill_with_affine_q8_projections(ctx, shape, bits, tokens):
         ctx.free(b)
 
 
+def edit_records(ctx, cfg, weights, edit):
+    """edit(codes, biases) on the gate and up matrices of every routed record and the shared one: codes [N][K] and biases [N][K/64]."""
+    for shared, buf, count in ((False, weights.records, cfg.experts), (True, weights.shared_record, 1)):
+        bits = cfg.shared_bits_gate_up if shared else cfg.bits_gate_up
+        raw = buf.numpy(np.uint8).copy()
+        for e in range(count):
+            for proj in range(2):
+                lin = ctx.expert_linear(cfg, buf, proj, shared=shared)
+                at = e * weights.stride
+                w, b = at + lin.weight - buf.ptr, at + lin.biases - buf.ptr
+                packed = raw[w:w + lin.output * lin.input * bits // 8].reshape(lin.output, -1)
+                codes = packed.copy() if bits == 8 else np.stack([packed & 15, packed >> 4], 2).reshape(lin.output, -1)
+                biases = raw[b:b + lin.output * lin.input // 64 * 2].view(np.uint16).reshape(lin.output, -1)
+                edit(codes, biases)
+                packed[:] = codes if bits == 8 else codes[:, 0::2] | codes[:, 1::2] << 4
+        ctx.upload(raw, into=buf)
+
+
+@pytest.mark.parametrize("bits", [(4, 4, 4, 4), (8, 8, 8, 8), (4, 8, 8, 8)])
+@pytest.mark.parametrize("power", [10, 16])
+def test_prefill_with_outliers_beside_small_codes(ctx, bits, power):
+    # One input of every group is 2^power times the others and meets codes 0 to 3, without biases that would hide what the
+    # product of the others loses beside it: an operand whose exponent the matrix cores read as larger than its value's would
+    # lose up to seven bits of them there, and many values would round to another BF16 number than the exact path's.
+    cfg = workload.tiny_config(2048, 16, 4, 128, bits=bits)
+    weights = workload.LayerWeights(ctx, cfg, 331, ("normal", 0.5))
+    T = 60
+    rng = np.random.default_rng(power)
+    where = rng.integers(0, 64, cfg.hidden // 64) + np.arange(cfg.hidden // 64) * 64
+
+    def edit(codes, biases):
+        codes[:, where] = rng.integers(0, 4, (codes.shape[0], len(where)))
+        biases[:] = 0
+
+    edit_records(ctx, cfg, weights, edit)
+    x = workload.hidden_rows(ctx, T, cfg.hidden, 333).numpy(f32).reshape(T, cfg.hidden).copy()
+    x[:, where] = oracle.bf(x[:, where] * f32(2.0 ** power))
+    dx = ctx.upload(x.ravel())
+    exact, fast = run_both(ctx, cfg, weights, dx, T)
+    assert fast["ids"].tobytes() == exact["ids"].tobytes()
+    for name in ("shared", "expert_out", "out"):
+        assert np.mean(fast[name].view(np.uint32) == exact[name].view(np.uint32)) > 0.9999, name
+        assert rel(fast[name], exact[name]) <= TOLERANCE, name
+    for b in (weights.router, weights.shared_gate, weights.shared_record, weights.records, dx):
+        ctx.free(b)
+
+
+@pytest.mark.parametrize("bits", [(4, 4, 4, 4), (8, 8, 8, 8)])
+def test_prefill_rows_out_of_the_products_range(ctx, bits):
+    # Rows with a group of 2^100 and above or a group all below 2^-60 have every output recomputed on the lanes: the exact
+    # path's values to the bit, zeros and values that are not finite included.  Rows just inside that range, and rows of
+    # ordinary size with single tiny elements or zero groups, take the product.
+    cfg = workload.tiny_config(512, 8, 2, 128, bits=bits)
+    weights = workload.LayerWeights(ctx, cfg, 351, None)
+    T, H = 48, cfg.hidden
+    x = workload.hidden_rows(ctx, T, H, 353).numpy(f32).reshape(T, H).copy()
+    x[3, 64:128] = oracle.bf(x[3, 64:128] * f32(2.0 ** 101)); x[4] = oracle.bf(x[4] * f32(2.0 ** 101))
+    x[5, 64:128] = oracle.bf(x[5, 64:128] * f32(2.0 ** -64)); x[6] = oracle.bf(x[6] * f32(2.0 ** -64)); x[7] = oracle.bf(x[7] * f32(2.0 ** -126))
+    x[8, 200] = f32(2.0 ** 100); x[9, 200] = f32(-3.3895314e38)
+    recomputed = [3, 4, 6, 7, 8, 9]       # row 5: the gate and up products only, its activations are ordinary
+    x[12, 200] = f32(2.0 ** 99); x[13] = oracle.bf(x[13] * f32(2.0 ** 28)); x[14] = oracle.bf(x[14] * f32(2.0 ** -50))
+    x[15, ::7] = f32(2.0 ** -90); x[16, 64:192] = 0.0; x[17] = 0.0
+    dx = ctx.upload(x.ravel())
+    exact, fast = run_both(ctx, cfg, weights, dx, T)
+    assert fast["ids"].tobytes() == exact["ids"].tobytes()
+    per = {"shared": H, "expert_out": 2 * H, "out": H}
+    for name, n in per.items():
+        a, b = fast[name].reshape(T, n), exact[name].reshape(T, n)
+        assert np.array_equal(a[recomputed], b[recomputed], equal_nan=True), name
+        same = (a == b) | (np.isnan(a) & np.isnan(b))
+        assert same.mean() > 0.9999 and same[16].all() and same[17].all(), (name, same.mean())
+    for b in (weights.router, weights.shared_gate, weights.shared_record, weights.records, dx):
+        ctx.free(b)
+
+
 def test_prefill_against_the_cpu_oracle(ctx):
     cfg = workload.tiny_config(512, 32, 4, 128)
     T = 70

@@ -14,15 +14,17 @@
 // specified by a tolerance (max relative error 2e-3 of the layer output), not as bit-exact.  Routing, dispatch and the
 // combine use the exact kernels.
 //
-// Codes as operands.  The matrix cores take subnormal bf16 operands at full precision, and the bit pattern of an integer
-// code 0..255 read as bf16 is the number code * 2^-133: a code needs no conversion, only its place in a 16-bit half, one
-// mask and shift per two codes where the conversion to a float and on to bf16 took 3 instructions per two codes, each
-// at half rate.  The token rows carry 2^100 to stay in range, the scales the rest: both exact.  An instruction drops what
-// lies 24 bits below its largest exponent sum, and a subnormal's exponent counts as that of 2^-126: nibbles stand three bits
-// up (code * 2^-130), so that at most one of those bits is empty.
-// Nibbles i and i + 4 of a word share one mask, so the rows are stored with every eight elements in the order
-// 0 4 1 5 2 6 3 7.  Groups whose values would leave the exact range (|x| >= 2^26, all below 2^-60, inf, NaN) get a NaN
-// chain sum: every output of such a row is then recomputed with the lane arithmetic.
+// Codes as operands.  A nibble, read as an 8-bit float of four exponent and three mantissa bits, is the number code * 2^-9: one
+// conversion instruction makes two bf16 codes of two of them and takes the 2^9 back.  Bytes go over floats, three instructions per
+// two codes.  (The bit pattern of a code is the bf16 number code * 2^-133, which the matrix cores take at full precision without
+// any conversion.  But an instruction drops what lies 24 bits below its largest sum of exponents, and a subnormal operand
+// counts there as 2^-126, up to seven bits above its value: beside a large input that met a small code the other products
+// lost those bits.  Rows with one input of 2^10 per group on codes 1 to 3, 2048 inputs, root mean square error in 2^-24 of the
+// terms' magnitudes: nibbles 1.67, bytes 19.5; converted 0.48 and 0.46.  The layer of 2048 tokens of hidden 2048
+// takes 626 us with either, 1500 tokens of hidden 3072 1195 us with the conversion and 1197 without, 300 of the mixed artifact 389 and 390.)
+// The even nibbles of a word share one mask and the odd ones another, so the rows are stored with every eight elements in the
+// order 0 2 4 6 1 3 5 7.  Groups whose sums could leave the range of exact products (|x| >= 2^100, all below 2^-60, inf, NaN) get a
+// NaN chain sum: every output of such a row is then recomputed with the lane arithmetic.
 //
 // Tiling.  One workgroup (4 waves) owns up to 48 sorted token rows of ONE expert and 128 weight rows (gate/up: 64 gate rows
 // and the 64 up rows of the same indices, so SwiGLU is fused in registers), and walks K in steps of 64 = one scale
@@ -49,7 +51,7 @@ constexpr uint32_t kTileRows = 32, kTileRowsMax = 48, kPitch = 136;   // LDS row
 // What the matrix-core products and the recomputation need of their token rows, from fp32 rows holding BF16 values (F32)
 // or from bf16 rows (the SwiGLU activations): a thread takes four neighbouring elements, so loads and stores are whole runs.
 //   xb      the row as bf16 (F32 only)
-//   xp      the row times 2^100, every eight elements in the order 0 4 1 5 2 6 3 7: the matrix-core operand
+//   xp      the row as bf16, every eight elements in the order 0 2 4 6 1 3 5 7: the matrix-core operand
 //   planes  per (row, group of 64) the group's input sum as three bf16 pieces, [row][piece][prefill_pitch(K)]: the four
 //           blocks' BF16-rounded sum-of-four chains (Q4 lanes), NaN where the group leaves the operand's exact range
 //   plain   the same of the plain fp32 sums (Q8 lanes, qwen.metal:112-125: sum += v, element by element in blocks of eight)
@@ -87,16 +89,12 @@ __global__ __launch_bounds__(256) void prefill_rows_kernel(const void* x, uint32
     for (int k = 0; k < 4; ++k) largest = max(largest, __float_as_uint(v[k]) & 0x7fffffffu);
 #pragma unroll
     for (int o = 1; o < 16; o <<= 1) largest = max(largest, uint32_t(__shfl_xor(int(largest), o)));
-    const bool strange = largest >= 0x4c800000u || (largest != 0 && largest < 0x21800000u);   // 2^26, 2^-60
-    {   // lane 2m of a pair holds elements 0..3, lane 2m + 1 elements 4..7: 0 4 1 5 | 2 6 3 7
-        uint32_t mine[2], other[2];
-#pragma unroll
-        for (int k = 0; k < 2; ++k) mine[k] = (__float_as_uint(v[2 * k] * 0x1p100f) >> 16) | (__float_as_uint(v[2 * k + 1] * 0x1p100f) & 0xffff0000u);
-#pragma unroll
-        for (int k = 0; k < 2; ++k) other[k] = uint32_t(__shfl_xor(int(mine[k]), 1));
+    const bool strange = largest >= 0x71800000u || (largest != 0 && largest < 0x21800000u);   // 2^100, 2^-60
+    {   // lane 2m of a pair holds elements 0..3, lane 2m + 1 elements 4..7: 0 2 4 6 | 1 3 5 7
+        const uint32_t even = (__float_as_uint(v[0]) >> 16) | __float_as_uint(v[2]), uneven = (__float_as_uint(v[1]) >> 16) | __float_as_uint(v[3]);
         const bool odd = lane & 1u;
-        const uint32_t a = odd ? other[1] : mine[0], b = odd ? mine[1] : other[0];   // a: elements (2) 0 and (3) 1; b: elements (6) 4 and (7) 5
-        reinterpret_cast<uint2*>(xp)[i] = make_uint2((a & 0xffffu) | (b << 16), (a >> 16) | (b & 0xffff0000u));
+        const uint32_t other = uint32_t(__shfl_xor(int(odd ? even : uneven), 1));
+        reinterpret_cast<uint2*>(xp)[i] = odd ? make_uint2(other, uneven) : make_uint2(even, other);
     }
     const uint32_t group = r * (3 * pitch) + c / 16, base = lane & ~15u;
     if (planes || sums16) {
@@ -392,14 +390,18 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
         for (int q = 0; q < 2; ++q)
 #pragma unroll
             for (int r = 0; r < 4; ++r) mag[rb][q][r] *= 1.0078125f;
-    // codes -> matrix-core operand, element order 0 4 1 5 2 6 3 7: eight nibbles of a word, or eight bytes of two words
+    // codes -> matrix-core operand, element order 0 2 4 6 1 3 5 7: eight nibbles of a word, or eight bytes of two words
     auto nibbles = [](uint32_t word) {
-        const uint32_t M = 0x00780078u;
-        return __builtin_bit_cast(bf16x8, make_uint4((word << 3) & M, (word >> 1) & M, (word >> 5) & M, (word >> 9) & M));
+        const uint32_t even = word & 0x0f0f0f0fu, odd = (word >> 4) & 0x0f0f0f0fu;
+        auto two = [](bf16x2 v) { return __builtin_bit_cast(uint32_t, v); };
+        return __builtin_bit_cast(bf16x8, make_uint4(two(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, false)), two(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, true)),
+                                                     two(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, false)), two(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, true))));
     };
     auto bytes = [](uint32_t lo, uint32_t hi) {
-        return __builtin_bit_cast(bf16x8, make_uint4(__builtin_amdgcn_perm(hi, lo, 0x0c040c00u), __builtin_amdgcn_perm(hi, lo, 0x0c050c01u),
-                                                     __builtin_amdgcn_perm(hi, lo, 0x0c060c02u), __builtin_amdgcn_perm(hi, lo, 0x0c070c03u)));
+        auto two = [](uint32_t word, int i) {   // bytes i and i + 2: whole numbers up to 255 have all their bits in a float's upper half
+            return __builtin_amdgcn_perm(__float_as_uint(float((word >> (8 * i + 16)) & 0xffu)), __float_as_uint(float((word >> (8 * i)) & 0xffu)), 0x07060302u);
+        };
+        return __builtin_bit_cast(bf16x8, make_uint4(two(lo, 0), two(hi, 0), two(lo, 1), two(hi, 1)));
     };
     // elements of a group that lane (j, g4) multiplies, from this one on: sixteen of them.  Q4: a load brings the four
     // lanes of a row the four quarters of two groups; a swap between the half waves gives every lane its share of either
@@ -440,7 +442,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
                 }
             float scale[2];
 #pragma unroll
-            for (int q = 0; q < 2; ++q) scale[q] = __uint_as_float(h ? scales[q][odd] & 0xffff0000u : scales[q][odd] << 16) * (BITS == 4 ? 0x1p30f : 0x1p33f);
+            for (int q = 0; q < 2; ++q) scale[q] = __uint_as_float(h ? scales[q][odd] & 0xffff0000u : scales[q][odd] << 16);
             bf16x8 a[NB][2];
 #pragma unroll
             for (int rb = 0; rb < NB; ++rb)
