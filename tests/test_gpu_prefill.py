@@ -157,6 +157,25 @@ def test_prefill_with_outliers_beside_small_codes(ctx, bits, power):
         ctx.free(b)
 
 
+# rows per expert around the heights of the product's tiles (16, 32, 48 and, longer, 32 + what is left), with reductions of one
+# to eighteen and of twenty pairs of groups: an odd number of pairs leaves the last one to the code behind the walk's loop
+@pytest.mark.parametrize("rows", [16, 17, 32, 33, 48, 49, 81])
+@pytest.mark.parametrize("hidden,inter,bits", [(2560, 640, (4, 4, 4, 4)), (384, 1152, (4, 4, 4, 4)), (1152, 384, (4, 8, 8, 8)), (640, 128, (8, 8, 8, 8))])
+def test_prefill_tile_heights_and_odd_reductions(ctx, hidden, inter, bits, rows):
+    cfg = workload.tiny_config(hidden, 3, 2, inter, bits=bits)
+    weights = workload.LayerWeights(ctx, cfg, 341 + rows, None)
+    offsets = ctx.upload(np.array([0, 1000, 1000], f32))         # every token goes to the last two experts
+    weights.layer.router_offsets = offsets.ptr
+    x = workload.hidden_rows(ctx, rows, hidden, 343 + rows)
+    exact, fast = run_both(ctx, cfg, weights, x, rows)
+    assert fast["ids"].tobytes() == exact["ids"].tobytes() and (np.sort(exact["ids"].reshape(rows, 2), axis=1) == [1, 2]).all()
+    for name in ("shared", "expert_out", "out"):
+        assert np.mean(fast[name].view(np.uint32) == exact[name].view(np.uint32)) > 0.9999, name
+        assert rel(fast[name], exact[name]) <= TOLERANCE, name
+    for b in (weights.router, weights.shared_gate, weights.shared_record, weights.records, offsets, x):
+        ctx.free(b)
+
+
 @pytest.mark.parametrize("bits", [(4, 4, 4, 4), (8, 8, 8, 8)])
 def test_prefill_rows_out_of_the_products_range(ctx, bits):
     # Rows with a group of 2^100 and above or a group all below 2^-60 have every output recomputed on the lanes: the exact

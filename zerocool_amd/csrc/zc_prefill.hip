@@ -6,11 +6,11 @@
 // BF16-rounded sum-of-four chain (qwen.metal:46-62).  Here the products x * q run on v_mfma_f32_16x16x32_bf16: x is
 // BF16-valued (exact as a bf16 operand), products are exact and accumulate in fp32 over one scale group of 64; per group
 // the accumulator is folded as  total += scale * dot.  The bias half, sum over the groups of bias * chain sum, is a product
-// over the group index and runs on the same instruction before the walk over K, the chain sums cut into three bf16 pieces
-// that add up to them exactly.  Only the order of the fp32 additions
+// over the group index and runs on the matrix cores too, four groups at a time between their dots, the chain sums cut into
+// three bf16 pieces that add up to them exactly.  Only the order of the fp32 additions
 // differs from the reference, so results agree to a few fp32 steps before the BF16 rounding of the outputs.  Every sum
 // that lands within prefill_margin(K) of its term magnitudes of a BF16 rounding boundary is then recomputed with the reference's exact
-// lane arithmetic (about 2-3 % of the elements), which removes the rounding flips in practice; the path is still
+// lane arithmetic (0.2 to 0.5 % of the sums up to 2048 inputs, 1.1 % at 4096; a gate/up element has two), which removes the rounding flips in practice; the path is still
 // specified by a tolerance (max relative error 2e-3 of the layer output), not as bit-exact.  Routing, dispatch and the
 // combine use the exact kernels.
 //
@@ -27,11 +27,11 @@
 // NaN chain sum: every output of such a row is then recomputed with the lane arithmetic.
 //
 // Tiling.  One workgroup (4 waves) owns up to 48 sorted token rows of ONE expert and 128 weight rows (gate/up: 64 gate rows
-// and the 64 up rows of the same indices, so SwiGLU is fused in registers), and walks K in steps of 64 = one scale
-// group.  Each wave multiplies all (two or three) 16-row blocks of the tokens by 2 of the 8 column tiles: the codes
-// of its 32 weight rows go from memory straight into the lanes that feed them to the matrix cores, the token rows are
-// gathered into LDS as bf16, double-buffered, and the
-// scales of all steps are brought into LDS once.  An expert's rows are cut into tiles of 32, except
+// and the 64 up rows of the same indices, so SwiGLU is fused in registers), and walks K in steps of 128 = two scale
+// groups.  Each wave multiplies all (one to three) 16-row blocks of the tokens by 2 of the 8 column tiles: the codes
+// and scales of its 32 weight rows go from memory straight into the lanes that use them, the token rows are
+// gathered into LDS as bf16, double-buffered, and chain sums and biases of all groups are brought into LDS once.  An expert's
+// rows are cut into tiles of 32, except
 // that a run of up to 48 rows (a whole expert with few rows, or the last rows of a longer run) is ONE tile: with about
 // forty rows per expert -- an unskewed router at 2048 tokens -- every expert's codes are then expanded once, not twice.
 #include "zc_kernels.hpp"
@@ -45,6 +45,7 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kTileRows = 32, kTileRowsMax = 48, kPitch = 136;   // LDS row pitch in bf16 elements: 128 elements of a row, sixteen rows on different banks
 
@@ -268,14 +269,15 @@ __global__ __launch_bounds__(256) void prefill_dispatch_kernel(const int32_t* __
 // code: as a run-time bound it cut every step into short blocks that each waited for its own LDS reads.
 //
 // The walk goes two scale groups (128 elements) at a time, weights and token rows one such pair ahead.  What bounds it is
-// the SIMDs' issue: per wave and pair 24 matrix-core instructions (7.7 ns each) and about 165 vector ones (1.0 to 1.5 ns),
+// the SIMDs' issue: per wave and pair, three row blocks, Q4, 27 matrix-core instructions (7.7 ns each) and 171 vector ones (1.0 to
+// 1.5 ns; the listing of the loop: 54 and 342 per two pairs),
 // which overlap only in part -- weights and rows read from a warm cache leave the time of the walk unchanged.  A wave
 // alone issues one vector instruction every five clocks, so the registers are kept to what three waves per SIMD allow
-// (Q4: 166 of 168; with a second set of token rows or four pairs of weights in flight two waves fit, and the layer of
-// hidden 2048 took 680 us at 2048 tokens instead of 621).  At that size the routed gate/up product takes 258 us (369 with
-// converted codes, a run-time number of row blocks and the scales staged through LDS), the down product 174 us (258).
+// (Q4: 165 and 168 of 168; with a second set of token rows or four pairs of weights in flight two waves fit, and the layer of
+// hidden 2048 took 680 us at 2048 tokens instead of 621).  At that size the routed gate/up product takes 237 us, the down product
+// 158 us (369 and 258 with a run-time number of row blocks, codes converted one by one and the scales staged through LDS).
 template <bool GATED, int BITS, int NB>
-__device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s, uint16_t* marks_s, uint32_t expert, uint32_t first, uint32_t rows, uint32_t n0) {
+__device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s, uint16_t* marks_s, uint16_t* bias_s, uint32_t expert, uint32_t first, uint32_t rows, uint32_t n0) {
     constexpr int kAhead = 2, kRegs = BITS;       // pairs of groups in flight; dwords of a column tile's pair per lane
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, j = lane & 15u, g4 = lane >> 4;
     const uint32_t K = p.K, N = p.N, groups = K / 64, pairs = K / 128;
@@ -338,58 +340,79 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
     for (int rb = 0; rb < NB; ++rb)
 #pragma unroll
         for (int q = 0; q < 2; ++q) total[rb][q] = mag[rb][q] = f32x4{0, 0, 0, 0};
-    // The bias half of the totals and of their magnitudes, 32 groups per instruction: three instructions (the pieces of the
-    // chain sums, smallest first) where the fold took a multiply-add per element and group, and one for the magnitudes (the
-    // first piece is the chain sum cut off to bf16, made up for by the factor: the magnitudes only scale a margin).
+    // The bias half of the totals, sum over the groups of bias * chain sum, runs on the matrix cores, four groups per
+    // instruction: quarter g4 of the operand holds piece g4 of the chain sums (the last one zeros).  A group's bias half mostly
+    // cancels its dot, so the four are added in the middle of the same groups' dots: the running totals, which the rounding
+    // errors go with, stay small.  Root mean square error against 64 bits in 2^-24 of the terms' magnitudes, biases of -8 scales,
+    // 512, 2048 and 4096 inputs: 0.19, 0.14, 0.13; a multiply-add per group, the order that errs least, 0.19, 0.15, 0.14; all of the
+    // bias half in front of the walk 0.22, 0.23, 0.24.  (Eight groups at once in front of their dots 0.22, 0.17, 0.15.)  The layer of
+    // 2048 tokens of hidden 2048 takes 628 us, with all of it in front of the walk 620; 1500 tokens of hidden 3072 1166 and 1192.
+    // Chain sums and biases wait in LDS, zeros behind the last group.
     const uint32_t pitch = prefill_pitch(K);
-    const uint16_t* planes_of[NB];
-#pragma unroll
-    for (int rb = 0; rb < NB; ++rb) planes_of[rb] = p.planes + uint64_t(row_of(16 * uint32_t(rb) + j)) * (3 * pitch);
+    uint16_t *planes_s = bias_s + 8, *biases_s = planes_s + kTileRowsMax * 3 * pitch;
+    const uint32_t col[2] = {(GATED ? wave : 2 * wave) * 16 + j, (GATED ? 4 + wave : 2 * wave + 1) * 16 + j};
+    if (tid < 4) reinterpret_cast<uint32_t*>(bias_s)[tid] = 0;
+    const uint16_t* planes_of = p.planes + uint64_t(row_of(16 * min(wave, uint32_t(NB) - 1) + j)) * (3 * pitch);   // wave w: block w
     uint32_t g0 = 0;
     do {   // (at least once: the compiler then knows that no load from before it is pending in the walk)
-        const uint32_t mine = g0 + 8 * g4, M = 0x7fff7fffu;
-        bf16x8 bias[2], bias_size[2];
+        const uint32_t mine = g0 + 8 * g4;
+        uint4 bias[2], piece[3];
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             uint32_t w[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t g = mine + 2 * uint32_t(i), v = ldg_u32(biases_of[q] + (m_at[q] + min(g, groups - 2) * 2));
-                w[i] = g < groups ? v : 0u;
-            }
-            bias[q] = __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
-            bias_size[q] = __builtin_bit_cast(bf16x8, make_uint4(w[0] & M, w[1] & M, w[2] & M, w[3] & M));
-        }
-        uint4 pieces[NB][3];                     // (all requested before the first is used)
-#pragma unroll
-        for (int rb = 0; rb < NB; ++rb) {
-            const uint16_t* src = planes_of[rb] + min(mine, pitch - 8);
-#pragma unroll
-            for (int w = 0; w < 3; ++w) pieces[rb][w] = ldg_u4(src + uint32_t(w) * pitch);
+            for (int i = 0; i < 4; ++i) w[i] = ldg_u32(biases_of[q] + (m_at[q] + min(mine + 2 * uint32_t(i), groups - 2) * 2));
+            bias[q] = make_uint4(w[0], w[1], w[2], w[3]);
         }
 #pragma unroll
-        for (int rb = 0; rb < NB; ++rb) {
-            uint4 (&piece)[3] = pieces[rb];
+        for (int w = 0; w < 3; ++w) piece[w] = ldg_u4(planes_of + min(mine, pitch - 8) + uint32_t(w) * pitch);
+        auto store = [&](uint16_t* at, uint4 v) {
+            *reinterpret_cast<uint4*>(at) = make_uint4(v.x, mine + 2 < groups ? v.y : 0u, mine + 4 < groups ? v.z : 0u, mine + 6 < groups ? v.w : 0u);
+        };
+        if (mine < pitch) {
 #pragma unroll
-            for (int w = 0; w < 3; ++w) {
-                piece[w].x = mine < groups ? piece[w].x : 0u; piece[w].y = mine + 2 < groups ? piece[w].y : 0u;
-                piece[w].z = mine + 4 < groups ? piece[w].z : 0u; piece[w].w = mine + 6 < groups ? piece[w].w : 0u;
-            }
-            const bf16x8 size = __builtin_bit_cast(bf16x8, make_uint4(piece[0].x & M, piece[0].y & M, piece[0].z & M, piece[0].w & M));
+            for (int q = 0; q < 2; ++q) store(biases_s + col[q] * pitch + mine, bias[q]);
+            if (wave < NB) {
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
-#pragma unroll
-                for (int w = 2; w >= 0; --w) total[rb][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, piece[w]), bias[q], total[rb][q], 0, 0, 0);
-                mag[rb][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(size, bias_size[q], mag[rb][q], 0, 0, 0);
+                for (uint32_t w = 0; w < 3; ++w) store(planes_s + ((wave * 16 + j) * 3 + w) * pitch + mine, piece[w]);
             }
         }
     } while ((g0 += 32) < groups);
+    auto from_lds = [](const uint16_t* at) { return *reinterpret_cast<const uint4*>(at); };
+    const uint16_t* sums_at = bias_s + (g4 < 3 ? 8 + (j * 3 + g4) * pitch : 0u);
+    const uint32_t sums_rb = g4 < 3 ? 48 * pitch : 0u;
+    auto add_biases = [&](uint32_t g) {          // of the groups g .. g + 3
+        s16x4 bias[2];
 #pragma unroll
-    for (int rb = 0; rb < NB; ++rb)
+        for (int q = 0; q < 2; ++q) bias[q] = *reinterpret_cast<const s16x4*>(biases_s + col[q] * pitch + g);
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
+        for (uint32_t rb = 0; rb < NB; ++rb) {
+            const s16x4 sums = *reinterpret_cast<const s16x4*>(sums_at + (rb * sums_rb + (g4 < 3 ? g : 0u)));
 #pragma unroll
-            for (int r = 0; r < 4; ++r) mag[rb][q][r] *= 1.0078125f;
+            for (int q = 0; q < 2; ++q) total[rb][q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(sums, bias[q], total[rb][q], 0, 0, 0);
+        }
+    };
+    // Their share of the magnitudes, 32 groups per instruction: the first piece is the chain sum cut off to bf16, made up for
+    // by the factor (the magnitudes only scale a margin).
+    auto add_bias_sizes = [&] {
+        for (uint32_t g = 0; g < groups; g += 32) {
+            const uint32_t at = min(g + 8 * g4, pitch - 8), M = g + 8 * g4 < groups ? 0x7fff7fffu : 0u;
+            auto size = [&](const uint16_t* from) { const uint4 v = from_lds(from + at); return __builtin_bit_cast(bf16x8, make_uint4(v.x & M, v.y & M, v.z & M, v.w & M)); };
+            const bf16x8 bias[2] = {size(biases_s + col[0] * pitch), size(biases_s + col[1] * pitch)};
+#pragma unroll
+            for (uint32_t rb = 0; rb < NB; ++rb) {
+                const bf16x8 sums = size(planes_s + (rb * 16 + j) * 3 * pitch);
+#pragma unroll
+                for (int q = 0; q < 2; ++q) mag[rb][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sums, bias[q], mag[rb][q], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int rb = 0; rb < NB; ++rb)
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) mag[rb][q][r] *= 1.0078125f;
+    };
     // codes -> matrix-core operand, element order 0 2 4 6 1 3 5 7: eight nibbles of a word, or eight bytes of two words
     auto nibbles = [](uint32_t word) {
         const uint32_t even = word & 0x0f0f0f0fu, odd = (word >> 4) & 0x0f0f0f0fu;
@@ -482,12 +505,15 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
     for (; pair + 1 < pairs; pair += 2) {
         next_scales(2 * pair + 4);
         work(pair, ring[0], ring[1], 0);
+        add_biases(2 * pair);
         work(pair + 1, ring[1], ring[0], 1);
     }
     if (pair < pairs) {
         next_scales(2 * pair);
+        add_biases(2 * pair);
         work(pair, ring[0], ring[1], 0);
     }
+    add_bias_sizes();
     // epilogue: row m of the tile is sorted position first + m.  A sum close to a BF16 rounding boundary could round
     // the other way under the reference's order of additions: such elements are listed for exact recomputation.  v rounds to
     // r; the boundary next to r is half a BF16 step from it, the step that of the smallest magnitude v - e that the sum
@@ -545,6 +571,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
 template <bool GATED, int BITS>
 __global__ __launch_bounds__(256, BITS == 4 ? 3 : 2) void prefill_gemm_kernel(PrefillGemm p) {
     __shared__ __align__(16) uint16_t a_s[2 * kTileRowsMax * kPitch], marks_s[kTileRowsMax * 8];
+    extern __shared__ __align__(16) uint16_t bias_s[];   // eight zeros, chain sums [48][3][pitch], biases [128][pitch]
     // The workgroups of one tile (neighbours in column block) share its token rows: they go to one of the eight dies, whose
     // L2 then fetches the rows once.
     const uint32_t columns = GATED ? p.N / 64u : p.N / 128u, turn = blockIdx.x / 8u;
@@ -552,9 +579,9 @@ __global__ __launch_bounds__(256, BITS == 4 ? 3 : 2) void prefill_gemm_kernel(Pr
     // (requested together: the lists have room for the grid's last tiles)
     const uint32_t count = uint32_t(*p.tile_count), expert = uint32_t(p.tile_expert[tile]), first = uint32_t(p.tile_first[tile]), rows = uint32_t(p.tile_rows[tile]);
     if (tile >= count) return;
-    if (rows <= 16) prefill_tile<GATED, BITS, 1>(p, a_s, marks_s, expert, first, rows, n0);
-    else if (rows <= 32) prefill_tile<GATED, BITS, 2>(p, a_s, marks_s, expert, first, rows, n0);
-    else prefill_tile<GATED, BITS, 3>(p, a_s, marks_s, expert, first, rows, n0);
+    if (rows <= 16) prefill_tile<GATED, BITS, 1>(p, a_s, marks_s, bias_s, expert, first, rows, n0);
+    else if (rows <= 32) prefill_tile<GATED, BITS, 2>(p, a_s, marks_s, bias_s, expert, first, rows, n0);
+    else prefill_tile<GATED, BITS, 3>(p, a_s, marks_s, bias_s, expert, first, rows, n0);
 }
 
 // Exact recomputation of the listed elements: one group of 32 lanes plays the reference's 32 lanes for one row
@@ -918,12 +945,13 @@ bool prefill_dispatch_fits(const int32_t* ids, uint32_t tokens, uint32_t topk, u
 }
 void launch_prefill_gemm(hipStream_t s, const PrefillGemm& p, bool gated, uint32_t max_tiles) {
     const dim3 grid((max_tiles + 7) / 8 * 8 * (gated ? p.N / 64 : p.N / 128));
+    const uint32_t lds = (8 + (kTileRowsMax * 3 + 128) * prefill_pitch(p.K)) * 2;
     if (p.bits == 8) {
-        if (gated) hipLaunchKernelGGL((prefill_gemm_kernel<true, 8>), grid, dim3(256), 0, s, p);
-        else hipLaunchKernelGGL((prefill_gemm_kernel<false, 8>), grid, dim3(256), 0, s, p);
+        if (gated) hipLaunchKernelGGL((prefill_gemm_kernel<true, 8>), grid, dim3(256), lds, s, p);
+        else hipLaunchKernelGGL((prefill_gemm_kernel<false, 8>), grid, dim3(256), lds, s, p);
     } else {
-        if (gated) hipLaunchKernelGGL((prefill_gemm_kernel<true, 4>), grid, dim3(256), 0, s, p);
-        else hipLaunchKernelGGL((prefill_gemm_kernel<false, 4>), grid, dim3(256), 0, s, p);
+        if (gated) hipLaunchKernelGGL((prefill_gemm_kernel<true, 4>), grid, dim3(256), lds, s, p);
+        else hipLaunchKernelGGL((prefill_gemm_kernel<false, 4>), grid, dim3(256), lds, s, p);
     }
 }
 void launch_prefill_patch(hipStream_t s, const PrefillGemm& p, bool gated) {
