@@ -75,7 +75,7 @@ def test_dispatch_sort(ctx, tokens, topk, experts):
 # rows of one weight piece and of several batches, a row too long for LDS (the general kernel), and numbers of tokens and
 # experts that leave a group of either partly empty
 @pytest.mark.parametrize("T,K,E", [(1, 128, 1), (2, 128, 5), (3, 2560, 17), (4, 1152, 512), (63, 640, 33), (1, 16384, 3), (5, 4224, 20),
-                                   (64, 3968, 35), (64, 4096, 35), (63, 4096, 17)])   # the longest row of the short kernel, and 64 tokens of a longer one on the tiles
+                                   (64, 3968, 35), (64, 4096, 35), (64, 4096, 272), (63, 4096, 17)])   # the longest row of the short kernel, and 64 tokens of a longer one on the tiles
 def test_router_logits(ctx, T, K, E):
     rng = np.random.default_rng(K + T)
     w, x, off = oracle.bf_bits(rng.standard_normal((E, K))), oracle.bf(rng.standard_normal((T, K))), rng.standard_normal(E).astype(f32)

@@ -777,8 +777,10 @@ void launch_router(hipStream_t s, const void* w, const float* x, uint32_t T, uin
         hipLaunchKernelGGL(router_block_kernel, dim3((E + 15) / 16, (T + 31) / 32), dim3(512), 0, s, (const uint16_t*)w, x, T, K, E, offsets, out);
         return;
     }
-    // (64 tokens of rows too long for the short kernel, from 4096 inputs on, too: 512 experts 51 us, 65 with the general kernel)
-    if (T >= 64 && K % 128 == 0) {
+    // (64 tokens come here with rows too long for the short kernel, from 4096 inputs on.  The general kernel's workgroups hold 16
+    // experts x 4 tokens, one round of them for up to 256 experts: 34 us there, 65 at 320 to 512 and 127 at 1024; the tiled one
+    // takes 50 to 51 us whatever the number.)
+    if ((T > 64 || (T == 64 && E > 256)) && K % 128 == 0) {
         hipLaunchKernelGGL(router_tiled_kernel, dim3((E + 15) / 16, (T + 15) / 16), dim3(256), 0, s, (const uint16_t*)w, x, T, K, E, offsets, out);
         return;
     }
