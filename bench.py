@@ -275,8 +275,8 @@ def main():
             return {"ms_per_step": m["ms"], "tokens_per_s": tokens / (m["ms"] * 1e-3), "GBps": m["bytes"] / (m["ms"] * 1e-3) / 1e9,
                     "frac": m["bytes"] / (m["ms"] * 1e-3) / 8e12, "bound": "hbm", "distinct_experts_per_layer": m["unique"], "kernel": kernel}
         also = {"stack_batch1_without_guessing": line(run(stack, cfg, L, 1, quick, 2, speculate=False), 1, "zc::decode_stack_kernel"),
-                "stack_batch8": line(run(stack, cfg, L, 8, quick, 2), 8, "zc::decode_multi_kernel"),
-                "stack_batch64": line(run(stack, cfg, L, 64, max(4, quick // 4), 1, inputs=2), 64, "zc::decode_wide_kernel")}
+                "stack_batch8": line(run(stack, cfg, L, 8, quick, 2), 8, decode_kernel(8, ctx.stack_single_launch(stack, 8))),
+                "stack_batch64": line(run(stack, cfg, L, 64, max(4, quick // 4), 1, inputs=2), 64, decode_kernel(64, ctx.stack_single_launch(stack, 64)))}
         ctx.stack_set_speculation(stack, True)
         pf = single_layer(ctx, "S", 2048, True, 20, 3, skew=None)
         s_cfg = workload.config("S")

@@ -82,7 +82,7 @@ def test_prefill_matches_the_exact_path(ctx, shape, tokens):
                                                ((1024, 64, 10, 512), (8, 4, 4, 8), 70),
                                                ((2048, 512, 10, 512), (4, 8, 8, 8), 96)])  # BASELINE config 4's shape
 def test_prefill_with_affine_q8_projections(ctx, shape, bits, tokens):
-    # Affine Q8 records through the same grouped product: byte codes are exact in bf16, the fold uses the Q8 lanes' plain
+    # Affine Q8 records through the same grouped product: byte codes are exact in bf16, the bias half uses the Q8 lanes' plain
     # input sums (qwen.metal:112-125), and the sums near a BF16 rounding boundary are recomputed on the Q8 lanes themselves.
     cfg = workload.tiny_config(*shape, bits=bits)
     weights = workload.LayerWeights(ctx, cfg, 161 + tokens, ("normal", 0.5))
@@ -282,7 +282,7 @@ def test_prefill_rejects_what_it_cannot_run(ctx):
     odd = workload.tiny_config(512, 32, 4, 128, group=32)     # only group 64
     assert ctx.moe_prefill_workspace_bytes(odd, 64) == 0
     assert ctx.moe_prefill_workspace_bytes(workload.tiny_config(512, 32, 4, 128, bits=(4, 8, 8, 8)), 64) > 0   # the mixed artifact is taken
-    assert ctx.moe_prefill_workspace_bytes(workload.tiny_config(4224, 32, 4, 128), 64) == 0   # K beyond what the product kernel keeps in LDS
+    assert ctx.moe_prefill_workspace_bytes(workload.tiny_config(4224, 32, 4, 128), 64) == 0   # longer rows than the margins of the recomputation are measured for
     assert ctx.moe_prefill_workspace_bytes(workload.tiny_config(4096, 32, 4, 4096), 64) > 0
     cfg = workload.tiny_config(512, 32, 4, 128)
     weights = workload.LayerWeights(ctx, cfg, 93, None)
