@@ -599,9 +599,13 @@ static zc_status moe_layer(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe
     // 1-2. router logits and the shared expert's gate, top-k + softmax (model.cpp:434-436)
     zc::launch_router(s, l->router, x, T, H, E, l->router_offsets, w.logits, l->shared_gate, w.gate, check ? ctx->moe_status : nullptr);
     // 4. positions / selected, on the device (model.cpp:449-479): the expert kernels' job list, at most `chunk` tokens a job
-    const uint32_t chunk = std::min(zc::affine_job_tokens(H, I, c->bits_gate_up), zc::affine_job_tokens(I, H, c->bits_down));
+    uint32_t chunk = ~0u;
+    for (const uint32_t bits : {c->bits_gate_up, c->shared_bits_gate_up}) chunk = std::min(chunk, zc::affine_job_tokens(H, I, c->group, bits));
+    for (const uint32_t bits : {c->bits_down, c->shared_bits_down}) chunk = std::min(chunk, zc::affine_job_tokens(I, H, c->group, bits));
+    if (T == 1) chunk = 1;
+    float* images = zc::affine_job_images(chunk) ? w.expert_out : nullptr;   // the input rows' images, until the down products write there
     uint32_t* jobs = reinterpret_cast<uint32_t*>(w.rows);   // (n words: a job holds at least one slot)
-    zc::launch_route_jobs(s, w.logits, T, E, k, w.ids, w.weights, w.offsets, w.slots, chunk, jobs, w.count, w.selected, ctx->moe_status);
+    zc::launch_route_jobs(s, w.logits, T, E, k, w.ids, w.weights, w.offsets, w.slots, chunk, jobs, w.count, w.selected, ctx->moe_status, x, H, images);
     // 5-6. shared expert (model.cpp:482-485) and routed experts (pipeline.cpp:18-29): gate/up on gathered rows, down scattered
     // to its slot.  One launch per phase where the shared expert's projections have the routed ones' width.
     auto offsets_of = [&](const void* record, int shared, uint64_t* off, int first, int count) {
@@ -620,13 +624,16 @@ static zc_status moe_layer(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe
         p.jobs = jobs; p.count = w.count; p.slots = w.slots; p.topk = k; p.tokens = T; p.chunk = chunk;
         p.max_jobs = uint32_t(std::min(n, std::min<uint64_t>(n, E) + n / chunk));
         p.K = gated ? H : I; p.N = gated ? I : H; p.group = c->group; p.bits = gated ? c->bits_gate_up : c->bits_down; p.gated = gated;
-        p.x = gated ? x : w.act; p.out = gated ? w.act : w.expert_out; p.shared_x = gated ? x : w.shared_act; p.shared_out = gated ? w.shared_act : w.shared;
-        if ((gated ? c->shared_bits_gate_up : c->shared_bits_down) == p.bits) { p.shared_record = l->shared_record; offsets_of(l->shared_record, 1, p.shared_off, first, count); }
-        else {
-            zc::AffineDesc a; a.gated = gated; a.x = p.shared_x; a.out = p.shared_out; a.tokens = T;
-            zc_hip_expert_linear(c, 1, l->shared_record, first, &a.gate);
-            if (gated) zc_hip_expert_linear(c, 1, l->shared_record, 1, &a.up);
-            zc::launch_affine(s, a);
+        const float* input = images ? images : x;
+        p.x = gated ? input : w.act; p.out = gated ? w.act : w.expert_out; p.shared_x = gated ? input : w.shared_act; p.shared_out = gated ? w.shared_act : w.shared;
+        p.fp32 = gated ? x : nullptr;
+        offsets_of(l->shared_record, 1, p.shared_off, first, count);
+        const uint32_t shared_bits = gated ? c->shared_bits_gate_up : c->shared_bits_down;
+        if (shared_bits == p.bits) p.shared_record = l->shared_record;
+        else {   // a launch of its own, without routed jobs
+            zc::ExpertPhaseDesc own = p;
+            own.shared_record = l->shared_record; own.bits = shared_bits; own.max_jobs = 0;
+            zc::launch_expert_phase(s, own);
         }
         zc::launch_expert_phase(s, p);
     }
@@ -1106,23 +1113,17 @@ static zc_status launch_piece(zc_hip_ctx* ctx, zc_hip_stack* st, const float* x,
     }
     return ZC_OK;
 }
-// Whether a batch that a single launch could take goes layer by layer, five launches each.  us per layer, single launch -> layer by
-// layer, at 2, 8, 32 and 64 tokens, one layer with N(0, 0.5) offsets / four to six layers with Zipf(1.1) offsets, whose tokens
-// agree on nearly all experts behind the first layer:
-//   hidden 2048, Q4        49 -> 38   92 -> 64   195 -> 144   302 -> 232  /  39 -> 36   65 -> 56   147 -> 120   231 -> 202
-//   hidden 2048, mixed     60 -> 45  111 -> 75   272 -> 168   445 -> 260  /  57 -> 46  105 -> 73   236 -> 146   393 -> 235
-//   hidden 3072, Q4        76 -> 62  188 -> 126  494 -> 365   813 -> 625  /  53 -> 55   97 -> 101  256 -> 257   438 -> 480
-// One token stays with its kernel (27 -> 29, 36 -> 39, 35 -> 43): nothing to share, and no launch between the layers.  Large Q4
-// layers whose tokens agree are better off on the matrix cores (a code is unpacked once for eight tokens there) up to eight tokens
-// and beyond thirty-two, so those keep the single launch whatever their tokens do.
-// Hidden 512 and 1024 with an intermediate size of 512, 1536 and 2048 with 512 and 1024, 32 to 512 experts, Q4 and mixed, were timed
-// at 2 to 64 tokens both ways too: layer by layer is ahead everywhere, by 2 % (hidden 2048 x 1024, 64 agreeing tokens,
-// which the line below leaves to the single launch with the large ones) to 40 %.
+// Whether a batch that a single launch could take goes layer by layer, five launches each: from two tokens on.  us per layer, single
+// launch -> layer by layer, at 2, 8, 32 and 64 tokens, one layer with N(0, 0.5) offsets / six layers with Zipf(1.1) offsets, whose
+// tokens agree on nearly all experts behind the first layer:
+//   hidden 2048, Q4        50 -> 39   93 -> 69   194 -> 128   313 -> 185  /  38 -> 36   63 -> 48   144 -> 80    222 -> 120
+//   hidden 2048, mixed     60 -> 50  112 -> 82   272 -> 152   449 -> 216  /  50 -> 45  102 -> 62   212 -> 98    360 -> 146
+//   hidden 3072, Q4        80 -> 65  187 -> 128  456 -> 291   743 -> 461  /  52 -> 53   97 -> 77   259 -> 150   437 -> 245
+// One token stays with its kernel (30 -> 30, 36 -> 36, 39 -> 43 / 22 -> 30, 33 -> 37, 28 -> 45): nothing to share, and no launch
+// between the layers.
 // (Above sixty-four tokens the rule says nothing: the inputs' check for BF16 values is the short router's, which ends there.)
 static bool layers_preferred(const zc_hip_stack* st, uint32_t tokens) {
-    const zc_moe_config& c = st->cfg;
-    if (tokens < 2 || tokens > 64 || st->store || st->wait_limit != kWaitPolls) return false;
-    return !all_q4(c) || uint64_t(c.hidden) * c.inter <= 3u << 19 || (tokens > 8 && tokens <= 32);
+    return tokens >= 2 && tokens <= 64 && !st->store && st->wait_limit == kWaitPolls;
 }
 zc_status zc_hip_stack_set_wait_limit(zc_hip_ctx* ctx, zc_hip_stack* st, uint32_t polls) {
     ZC_REQUIRE(ctx && st, "null argument");

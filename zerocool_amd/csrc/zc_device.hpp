@@ -64,11 +64,16 @@ __device__ __forceinline__ uint2 ldg_u2(const void* p, uint32_t index = 0) {
     const u32x2 v = as_global<u32x2>(p)[index];
     return make_uint2(v.x, v.y);
 }
-// Eight bytes whose address is a multiple of four only.
+// Eight or sixteen bytes whose address is a multiple of four only.
 __device__ __forceinline__ uint2 ldg_u2_by_words(const void* p) {
     typedef uint32_t words __attribute__((ext_vector_type(2), aligned(4)));
     const words v = *as_global<words>(p);
     return make_uint2(v.x, v.y);
+}
+__device__ __forceinline__ uint4 ldg_u4_by_words(const void* p) {
+    typedef uint32_t words __attribute__((ext_vector_type(4), aligned(4)));
+    const words v = *as_global<words>(p);
+    return make_uint4(v.x, v.y, v.z, v.w);
 }
 __device__ __forceinline__ uint16_t ldg_u16(const void* p, uint32_t index = 0) { return as_global<uint16_t>(p)[index]; }
 __device__ __forceinline__ uint32_t ldg_u32(const void* p, uint32_t index = 0) { return as_global<uint32_t>(p)[index]; }

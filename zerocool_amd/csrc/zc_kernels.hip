@@ -7,322 +7,10 @@
 #include <algorithm>
 #include <type_traits>
 #include "zc_device.hpp"
+#include "zc_affine_matrix.hpp"
 #include "zc_decode_common.hpp"   // lds_barrier; route_token: top-k + softmax of one token by one wavefront
 
 namespace zc {
-
-// ---------------------------------------------------------------------------
-// Affine Q4 / Q8 rows (reference: qwen.metal:46-81, 112-144)
-//
-// A half wave plays the 32 reference lanes of one output row: lane l takes the row's blocks l, l + 32, ... of WIDTH elements
-// (Q4 16|8, Q8 8|4: one or two dwords of codes) in order.  It walks two rows at a time (gate and up, or two rows of the one
-// matrix), so that an input block read from LDS serves two rows, and up to two tokens, so that a code is unpacked once for
-// four products.  The walk over (row tile, block step) is one flat loop: the codes and scales of its next three steps are in
-// flight, across row tiles too, and the first three are requested before the input rows are staged.
-//
-// The products x * q of a BF16-valued row (zeros and magnitudes from 2^-100 to 2^100) are exact in fp32, so a fused multiply-add
-// rounds as the reference's multiply and add do, also when all of it is scaled by a power of two: such rows multiply codes
-// that were never converted (affine_halves).  Rows that hold anything else, infinities and NaN among them, keep converted codes
-// and separate operations.
-//
-// What bounds it: with one token per row, the latency of the chain job -> row index -> input row -> LDS -> codes (a launch
-// of a few us); with several, vector instructions, a wave's at four clocks each: 24 per block of sixteen weights and token, 14
-// to unpack the block (the listing's 49 and 28 for the two rows), and the finish of a row.  Per layer of hidden 2560 and intermediate 640, gate/up and down: 40 tokens 142
-// and 119 us, one token 11.9 and 8.7 us.  With codes converted to floats, addresses formed per lane and four tokens per
-// workgroup it was 172 and 132, 12.5 and 9.2 us.  Four tokens per workgroup take 159 and 112 us: most experts have one or two
-// tokens, and the LDS of four leaves room for three workgroups on a compute unit where two leave six (decoding stacks of
-// hidden 2048 and 3072 at 2 to 64 tokens lost 5 to 25 %).  One token at a time, codes requested step by step behind the staging,
-// sums through LDS permutes and the shared expert in launches of its own took 397 and 310, 20.2 and 14.3 us.
-// ---------------------------------------------------------------------------
-constexpr uint32_t kAffineTokens = 2;                                            // tokens a workgroup multiplies at once, at most
-struct AffineMatrix { const uint8_t* w; const uint16_t *s, *b; };
-
-// Input rows in LDS: a block's WIDTH elements and its bias sum behind them, WIDTH / 4 words further apart than the elements
-// need (20, 10 or 5 words: the blocks of neighbouring lanes meet different banks), so that a lane adds one offset per token.
-template <int WIDTH> __host__ __device__ constexpr uint32_t affine_token_bytes(uint32_t K) { return (K * 5 + 15) / 16 * 16; }
-template <int WIDTH> struct AffineBlock { static constexpr uint32_t kBytes = WIDTH * 5, kPiece = WIDTH == 16 ? 4 : WIDTH == 8 ? 2 : 1; };
-template <int WIDTH>
-__device__ __forceinline__ void affine_inputs(const uint8_t* at, float* x, float& sum) {
-    typedef float piece __attribute__((ext_vector_type(AffineBlock<WIDTH>::kPiece)));
-    constexpr int P = AffineBlock<WIDTH>::kPiece;
-#pragma unroll
-    for (int i = 0; i < WIDTH; i += P) {
-        const piece v = *reinterpret_cast<const piece*>(at + 4 * i);
-#pragma unroll
-        for (int k = 0; k < P; ++k) x[i + k] = v[k];
-    }
-    sum = *reinterpret_cast<const float*>(at + 4 * WIDTH);
-}
-
-// Addresses: the bases are the same in every lane and move with tile and step, the lanes' 32-bit offsets are those of their row
-// and block in the tile.  wide: rows are whole steps (K % 512 == 0), else the last step's idle lanes repeat the last block.
-// Streams: the matrix rows a half wave walks at once, gate and up of one row or two rows of the one matrix.  (Four streams, which
-// halve the reads of LDS, took 130 registers: three waves per SIMD.  S-sized layers took 5 % longer, hidden 3072 the same.)
-template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS>
-struct AffineStream {
-    static constexpr int kStreams = 2, kRows = GATED ? kStreams / 2 : kStreams;   // kRows: output rows of a half wave per tile
-    static constexpr uint32_t kAhead = TOKENS == 1 ? 3 : 2;   // steps in flight (three for two tokens: 93 registers, four waves per SIMD instead of five, 5 % longer)
-    static constexpr int DW = WIDTH * BITS / 32;
-    static constexpr bool kWide = WIDTH * BITS == 64;
-    struct Slot { uint32_t q[kStreams][DW]; uint32_t s[kStreams], b[kStreams]; };
-    static constexpr uint32_t kTileRows = 8 * kRows;   // of a workgroup: eight half waves
-    uint32_t K, N, blocks, groups, shift, steps, lane, half, tile, end, step;   // tile, step: the next one to request
-    AffineMatrix m[2];
-    uint32_t w_at[kRows], g_at[kRows];
-    __device__ __forceinline__ uint32_t row(uint32_t t, uint32_t i) const { return t * kTileRows + i * 8 + half; }
-    __device__ __forceinline__ void aim() {
-#pragma unroll
-        for (int i = 0; i < kRows; ++i) {
-            const uint32_t r = min(row(tile, uint32_t(i)), N - 1) - tile * kTileRows;
-            w_at[i] = r * (K / 8 * BITS) + (kWide ? lane * (DW * 4) : 0u);
-            g_at[i] = (r * groups + (kWide ? (lane * WIDTH) >> shift : 0u)) * 2;
-        }
-    }
-    __device__ __forceinline__ void fetch(Slot& slot) {   // past the end: the last tile again, not used
-        const uint64_t first = uint64_t(tile) * kTileRows;
-        const uint32_t at = kWide ? 0u : min(lane, blocks - 1 - step * 32), g = ((step * 32 * WIDTH) >> shift) * 2;
-#pragma unroll
-        for (int q = 0; q < kStreams; ++q) {
-            const AffineMatrix& a = m[GATED ? q % 2 : 0];
-            const int i = GATED ? q / 2 : q;
-            const uint8_t* w = a.w + (first * (K / 8 * BITS) + step * (32 * DW * 4));
-            const uint32_t w_lane = w_at[i] + (kWide ? 0u : at * (DW * 4)), g_lane = g_at[i] + (kWide ? 0u : ((at * WIDTH) >> shift) * 2);
-            if constexpr (DW == 2) { const uint2 v = ldg_u2_by_words(w + w_lane); slot.q[q][0] = v.x; slot.q[q][DW - 1] = v.y; }
-            else slot.q[q][0] = ldg_u32(w + w_lane);
-            slot.s[q] = ldg_u16(reinterpret_cast<const uint8_t*>(a.s) + (first * groups * 2 + g) + g_lane);
-            slot.b[q] = ldg_u16(reinterpret_cast<const uint8_t*>(a.b) + (first * groups * 2 + g) + g_lane);
-        }
-        if (++step == steps) { step = 0; if (tile + 1 < end) { ++tile; aim(); } }
-    }
-};
-// Codes as f16 bit patterns, two in a word: the pattern of an integer n < 1024 is the number n * 2^-24, which the mixed
-// multiply-add (v_fma_mix_f32) takes as it is, so a code costs its place in a half word and no conversion.  Word k of eight
-// nibbles: nibbles k and k + 4; word k of four bytes: bytes k and k + 2.
-template <int BITS, int WIDTH>
-__device__ __forceinline__ void affine_halves(const uint32_t* words, uint32_t* half) {
-    constexpr int PER = 32 / BITS / 2;   // half-word pairs of a word of codes
-#pragma unroll
-    for (int i = 0; i < WIDTH / 2; ++i) half[i] = (words[i / PER] >> (BITS * (i % PER))) & (BITS == 4 ? 0x000f000fu : 0x00ff00ffu);
-}
-// x * code i * 2^-24 + c, rounded once.  (In assembly: from the source form the compiler converts the codes once for all tokens
-// instead, one instruction per code and twice the registers.)
-template <int BITS>
-__device__ __forceinline__ float affine_mad(float x, const uint32_t* half, int i, float c) {
-    constexpr int PER = 32 / BITS / 2;
-    const uint32_t h = half[i / (2 * PER) * PER + i % PER];
-    float d;
-    if ((i / PER) % 2) asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(d) : "v"(x), "v"(h), "v"(c));
-    else asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel_hi:[0,1,0]" : "=v"(d) : "v"(x), "v"(h), "v"(c));
-    return d;
-}
-template <int BITS>
-__device__ __forceinline__ float affine_mul(float x, const uint32_t* half, int i) {
-    constexpr int PER = 32 / BITS / 2;
-    const uint32_t h = half[i / (2 * PER) * PER + i % PER];
-    float d;
-    if ((i / PER) % 2) asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[0,1,0] op_sel_hi:[0,1,0]" : "=v"(d) : "v"(x), "v"(h));
-    else asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[0,1,0]" : "=v"(d) : "v"(x), "v"(h));
-    return d;
-}
-// sum of x * code over a block in the reference's order.  (A first quad or product is added to nothing: the reference adds it to
-// +0, which can only turn a -0 into +0, and the row's sum starts from +0.)
-template <int BITS, int WIDTH>
-__device__ __forceinline__ float affine_dot_exact(const uint32_t* half, const float* x) {
-    float dot = 0;
-    if constexpr (BITS == 4) {
-#pragma unroll
-        for (int i = 0; i < WIDTH; i += 4) {
-            float quad = affine_mul<BITS>(x[i], half, i);
-#pragma unroll
-            for (int k = 1; k < 4; ++k) quad = affine_mad<BITS>(x[i + k], half, i + k, quad);
-            dot = i == 0 ? quad : dot + quad;
-        }
-    } else {
-        dot = affine_mul<BITS>(x[0], half, 0);
-#pragma unroll
-        for (int i = 1; i < WIDTH; ++i) dot = affine_mad<BITS>(x[i], half, i, dot);
-    }
-    return dot * 0x1p24f;
-}
-template <int BITS, int WIDTH>
-__device__ __forceinline__ float affine_dot_any(const uint32_t* codes, const float* x) {
-    uint32_t words[WIDTH * BITS / 32];   // (a copy the compiler cannot see through: it would keep the conversions of both rows for all tokens)
-#pragma unroll
-    for (int i = 0; i < WIDTH * BITS / 32; ++i) asm("" : "=v"(words[i]) : "0"(codes[i]));
-    auto code = [&](int i) { return float((words[i * BITS / 32] >> (i * BITS % 32)) & (BITS == 4 ? 15u : 255u)); };
-    float dot = 0;
-    if constexpr (BITS == 4) {
-#pragma unroll
-        for (int i = 0; i < WIDTH; i += 4) dot += x[i] * code(i) + x[i + 1] * code(i + 1) + x[i + 2] * code(i + 2) + x[i + 3] * code(i + 3);
-    } else {
-#pragma unroll
-        for (int i = 0; i < WIDTH; ++i) dot += x[i] * code(i);
-    }
-    return dot;
-}
-// The bias half's input sum of one block.
-template <int BITS, int WIDTH>
-__device__ __forceinline__ float affine_sum(const float* x) {
-    float sum = 0;
-    if constexpr (BITS == 4) {
-#pragma unroll
-        for (int i = 0; i < WIDTH; i += 4) sum += bf(bf(bf(x[i] + x[i + 1]) + x[i + 2]) + x[i + 3]);
-    } else {
-#pragma unroll
-        for (int i = 0; i < WIDTH; ++i) sum += x[i];
-    }
-    return sum;
-}
-
-// The walk for nt staged tokens; out_at: where the output row of token (lane % TOKENS) begins.
-// (nt and exact are the same in every lane.  As template parameters they made eight walks, whose common first steps the
-// compiler moved in front of the choice between them: 200 registers.)
-template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS>
-__device__ __forceinline__ void affine_walk(AffineStream<BITS, WIDTH, GATED, TOKENS>& st,
-                                            typename AffineStream<BITS, WIDTH, GATED, TOKENS>::Slot (&ring)[AffineStream<BITS, WIDTH, GATED, TOKENS>::kAhead],
-                                            const uint8_t* lds, float* out, uint64_t out_at, uint32_t tile, bool float_output, uint32_t nt, bool exact) {
-    using Stream = AffineStream<BITS, WIDTH, GATED, TOKENS>;
-    constexpr int S = Stream::kStreams;
-    const uint32_t blocks = st.blocks, token = affine_token_bytes<WIDTH>(st.K), lane = st.lane;
-    const uint32_t total = (st.end - tile) * st.steps;
-    float r[TOKENS][S];
-#pragma unroll
-    for (uint32_t t = 0; t < TOKENS; ++t)
-#pragma unroll
-        for (int q = 0; q < S; ++q) r[t][q] = 0;
-    uint32_t step = 0;
-    for (uint32_t i0 = 0; i0 < total; i0 += Stream::kAhead) {
-#pragma unroll
-        for (uint32_t d = 0; d < Stream::kAhead; ++d) {
-            if (i0 + d >= total) break;
-            float scale[S], bias[S];
-            uint32_t words[S][Stream::DW];
-#pragma unroll
-            for (int q = 0; q < S; ++q) {
-#pragma unroll
-                for (uint32_t i = 0; i < Stream::DW; ++i) words[q][i] = ring[d].q[q][i];
-                scale[q] = b16(uint16_t(ring[d].s[q])); bias[q] = b16(uint16_t(ring[d].b[q]));
-            }
-            st.fetch(ring[d]);
-            const uint32_t b = step * 32 + lane;
-            const uint8_t* block = lds + (Stream::kWide ? b : min(b, blocks - 1)) * AffineBlock<WIDTH>::kBytes;
-            auto tokens = [&](auto dot_of) {
-#pragma unroll
-                for (uint32_t t = 0; t < TOKENS; ++t) {
-                    if (t >= nt) break;
-                    asm volatile("");   // (else the compiler moves every token's products in front of the question)
-                    float x[WIDTH], sum;
-                    affine_inputs<WIDTH>(block + t * token, x, sum);
-#pragma unroll
-                    for (int q = 0; q < S; ++q) {
-                        const float more = r[t][q] + (scale[q] * dot_of(q, x) + sum * bias[q]);
-                        r[t][q] = Stream::kWide || b < blocks ? more : r[t][q];
-                    }
-                }
-            };
-            if (exact) {
-                uint32_t half[S][WIDTH / 2];
-#pragma unroll
-                for (int q = 0; q < S; ++q) affine_halves<BITS, WIDTH>(words[q], half[q]);
-                tokens([&](int q, const float* x) { return affine_dot_exact<BITS, WIDTH>(half[q], x); });
-            } else tokens([&](int q, const float* x) { return affine_dot_any<BITS, WIDTH>(words[q], x); });
-            if (++step < st.steps) continue;
-            step = 0;
-            // every lane has all the sums: lane i * TOKENS + t finishes output row i of token t
-            float v[2] = {0, 0};
-#pragma unroll
-            for (uint32_t t = 0; t < TOKENS; ++t) {
-                if (t >= nt) break;
-#pragma unroll
-                for (int i = 0; i < Stream::kRows; ++i) {
-                    const float first = lane_sum32(r[t][GATED ? 2 * i : i]), second = GATED ? lane_sum32(r[t][GATED ? 2 * i + 1 : i]) : 0.0f;
-                    if (lane == uint32_t(i) * TOKENS + t) { v[0] = first; v[1] = second; }
-                }
-            }
-            const uint32_t row = st.row(tile, lane / TOKENS);
-            const float y = GATED ? swiglu_bf(v[0], v[1]) : float_output ? v[0] : bf(v[0]);
-            if (lane < Stream::kRows * TOKENS && lane % TOKENS < nt && row < st.N) out[out_at + row] = y;
-#pragma unroll
-            for (uint32_t t = 0; t < TOKENS; ++t)
-#pragma unroll
-                for (int q = 0; q < S; ++q) r[t][q] = 0;
-            ++tile;
-        }
-    }
-}
-
-// Rows tile0 .. end - 1 (tiles) of the matrices for nt <= TOKENS tokens: input row in_row(t), output row out_row(t).
-template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS, class InRow, class OutRow>
-__device__ __forceinline__ void affine_rows(const AffineMatrix (&m)[2], uint32_t K, uint32_t N, uint32_t group, const float* x, float* out, uint32_t nt,
-                                            InRow in_row, OutRow out_row, uint32_t tile0, uint32_t end, bool float_output, uint8_t* lds) {
-    using Stream = AffineStream<BITS, WIDTH, GATED, TOKENS>;
-    const uint32_t tid = threadIdx.x;
-    Stream st;
-    st.K = K; st.N = N; st.blocks = K / WIDTH; st.shift = group == 64 ? 6 : 5; st.groups = K >> st.shift; st.steps = (st.blocks + 31) / 32;
-    st.lane = tid & 31u; st.half = tid >> 5; st.tile = tile0; st.end = end; st.step = 0;
-    st.m[0] = m[0]; st.m[1] = m[1];
-    const uint32_t from = st.lane < nt ? in_row(st.lane) : 0u;   // lane t: token t's input row
-    const uint64_t out_at = uint64_t(out_row(min(st.lane % TOKENS, nt - 1))) * N;
-    typename Stream::Slot ring[Stream::kAhead];
-    st.aim();
-#pragma unroll
-    for (uint32_t d = 0; d < Stream::kAhead; ++d) st.fetch(ring[d]);
-    constexpr uint32_t kPieces = WIDTH / 4, P = AffineBlock<WIDTH>::kPiece;
-    const uint32_t blocks = st.blocks, token = affine_token_bytes<WIDTH>(K);
-    bool strange = false;
-#pragma unroll 1
-    for (uint32_t t = 0; t < nt; ++t) {
-        const float* src = x + uint64_t(uint32_t(__builtin_amdgcn_readlane(int(from), int(t)))) * K;
-#pragma unroll 2
-        for (uint32_t i = tid; i < K / 4; i += 256) {
-            const uint4 q = ldg_u4(src, i);
-            const uint32_t v[4] = {q.x, q.y, q.z, q.w};
-            uint32_t* to = reinterpret_cast<uint32_t*>(lds + t * token + i / kPieces * AffineBlock<WIDTH>::kBytes + i % kPieces * 16);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {   // (as a magnitude from 2^-100 on: one comparison)
-                const uint32_t a = v[k] & 0x7fffffffu;
-                strange |= (v[k] & 0xffffu) != 0 || (a - 0x0d800000u >= 0x71800000u - 0x0d800000u && a != 0);
-            }
-            typedef uint32_t piece __attribute__((ext_vector_type(P)));
-#pragma unroll
-            for (uint32_t k = 0; k < 4; k += P) {
-                if constexpr (P == 4) *reinterpret_cast<piece*>(to) = piece{v[0], v[1], v[2], v[3]};
-                else if constexpr (P == 2) *reinterpret_cast<piece*>(to + k) = piece{v[k], v[k + 1]};
-                else to[k] = v[k];
-            }
-        }
-    }
-    // Each wave's finding crosses in block w of the first token, wave w's: in the padding behind the bias sum, or, where blocks
-    // have none, in the sum's own place, read before the sums are written.  (An array of its own beside the rows would keep out
-    // the longest rows, of 32768 elements, which fill a compute unit's LDS to the last byte.)
-    constexpr bool kPadded = WIDTH >= 8;
-    auto finding = [&](uint32_t w) { return reinterpret_cast<uint32_t*>(lds + w * AffineBlock<WIDTH>::kBytes + 4 * WIDTH + (kPadded ? 4 : 0)); };
-    const bool any = __ballot(strange) != 0;
-    if ((tid & 63u) == 0) *finding(tid >> 6) = any;
-    lds_barrier();
-    uint32_t found = 0;
-    if constexpr (!kPadded) {
-#pragma unroll
-        for (uint32_t w = 0; w < 4; ++w) found |= *finding(w);
-        lds_barrier();
-    }
-#pragma unroll 1
-    for (uint32_t t = 0; t < nt; ++t)
-#pragma unroll 1
-        for (uint32_t b = tid; b < blocks; b += 256) {
-            float xb[WIDTH], unset;
-            uint8_t* block = lds + t * token + b * AffineBlock<WIDTH>::kBytes;
-            affine_inputs<WIDTH>(block, xb, unset);
-            *reinterpret_cast<float*>(block + 4 * WIDTH) = affine_sum<BITS, WIDTH>(xb);
-        }
-    lds_barrier();
-    if constexpr (kPadded) {
-#pragma unroll
-        for (uint32_t w = 0; w < 4; ++w) found |= *finding(w);
-    }
-    const bool exact = __builtin_amdgcn_readfirstlane(int(found)) == 0;
-    affine_walk<BITS, WIDTH, GATED, TOKENS>(st, ring, lds, out, out_at, tile0, float_output, nt, exact);
-}
 
 struct AffineJob {
     AffineMatrix m[2];               // gate (or the only matrix), up
@@ -344,20 +32,31 @@ __global__ __launch_bounds__(256, TOKENS == 1 ? 4 : 3) void affine_op_kernel(Aff
                                             [&](uint32_t t) { return j.out_rows ? uint32_t(j.out_rows[t0 + t]) : uint32_t(t0) + t; }, tile0, end, j.float_output != 0, affine_lds);
 }
 
+template <int BITS, int WIDTH, bool GATED>
+__global__ __launch_bounds__(kMatrixThreads, 4) void affine_matrix_kernel(AffineJob j) {
+    extern __shared__ __align__(16) uint8_t affine_lds[];
+    matrix_piece_of_work((j.tokens - 1) / kMatrixTokens + 1, (j.tiles + kMatrixWaves - 1) / kMatrixWaves, [&](uint32_t job, uint32_t round, uint32_t rounds) {
+        const uint64_t t0 = uint64_t(job) * j.chunk;
+        matrix_rows<BITS, WIDTH, GATED, false, false>(j.m, j.K, j.N, j.x, nullptr, j.out, min(j.chunk, j.tokens - uint32_t(t0)),
+                                                              [&](uint32_t t) { return j.in_rows ? uint32_t(j.in_rows[t0 + t]) : uint32_t(t0) + t; },
+                                                              [&](uint32_t t) { return j.out_rows ? uint32_t(j.out_rows[t0 + t]) : uint32_t(t0) + t; },
+                                                              round * kMatrixWaves, min(rounds * kMatrixWaves, j.tiles), j.float_output != 0, affine_lds);
+    });
+}
+
 // The routed experts of one layer and, where its formats are theirs, the shared expert: blockIdx.y walks the shared expert's
 // tokens, chunk by chunk, then the list of (expert, sorted positions) that the dispatch left; jobs past the device-side count exit.
 struct ExpertPhase {
     const uint8_t* records; uint64_t stride; uint64_t off[6];          // byte offsets inside a record: codes, scales, biases of the (gate | down) projection, of up
     const uint8_t* shared_record; uint64_t shared_off[6];
     const uint32_t *jobs; const int32_t *count, *slots;
-    const float *x, *shared_x; float *out, *shared_out;                // x: layer input (gate/up) or sorted activations (down)
+    const float *x, *shared_x; float *out, *shared_out;                // x: layer input (gate/up) or sorted activations (down); on the matrix cores both as row images
+    const float* fp32;                                                 // matrix cores: the rows that x and shared_x were made of, null where they were made as images
     uint32_t K, N, group, topk, tokens, chunk, shared_jobs, max_jobs, tiles, share;   // chunk: tokens of a job (a shared job too)
 };
-template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS>
-__global__ __launch_bounds__(256, TOKENS == 1 ? 4 : 3) void expert_phase_kernel(ExpertPhase p) {
-    extern __shared__ __align__(16) uint8_t affine_lds[];
-    const uint32_t tile0 = blockIdx.x * p.share, end = min(tile0 + p.share, p.tiles);
-    const uint32_t job = blockIdx.z * gridDim.y + blockIdx.y;
+// A job, if there is one of that number: its matrices, tokens and rows go to `run`.
+template <bool GATED, class Run>
+__device__ __forceinline__ void expert_job(const ExpertPhase& p, uint32_t job, Run run) {
     const bool shared = job < p.shared_jobs;
     uint32_t first = job * p.chunk, expert = 0, nt = min(p.chunk, p.tokens - first);
     if (!shared) {   // (the list has room for every job of the grid; what lies past the count is not used)
@@ -372,9 +71,28 @@ __global__ __launch_bounds__(256, TOKENS == 1 ? 4 : 3) void expert_phase_kernel(
         auto at = [&](int i) { return r + (shared ? p.shared_off[3 * q + i] : p.off[3 * q + i]); };
         m[q] = AffineMatrix{at(0), reinterpret_cast<const uint16_t*>(at(1)), reinterpret_cast<const uint16_t*>(at(2))};
     }
-    affine_rows<BITS, WIDTH, GATED, TOKENS>(m, p.K, p.N, p.group, shared ? p.shared_x : p.x, shared ? p.shared_out : p.out, nt,
-                                            [&](uint32_t t) { return GATED && !shared ? uint32_t(p.slots[first + t]) / p.topk : first + t; },
-                                            [&](uint32_t t) { return GATED || shared ? first + t : uint32_t(p.slots[first + t]); }, tile0, end, false, affine_lds);
+    run(m, shared ? p.shared_x : p.x, shared ? p.shared_out : p.out, nt,
+        [&, first](uint32_t t) { return GATED && !shared ? uint32_t(p.slots[first + t]) / p.topk : first + t; },
+        [&, first](uint32_t t) { return GATED || shared ? first + t : uint32_t(p.slots[first + t]); });
+}
+template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS>
+__global__ __launch_bounds__(256, TOKENS == 1 ? 4 : 3) void expert_phase_kernel(ExpertPhase p) {
+    extern __shared__ __align__(16) uint8_t affine_lds[];
+    const uint32_t tile0 = blockIdx.x * p.share, end = min(tile0 + p.share, p.tiles);
+    expert_job<GATED>(p, blockIdx.z * gridDim.y + blockIdx.y, [&](const AffineMatrix (&m)[2], const float* x, float* out, uint32_t nt, auto in_row, auto out_row) {
+        affine_rows<BITS, WIDTH, GATED, TOKENS>(m, p.K, p.N, p.group, x, out, nt, in_row, out_row, tile0, end, false, affine_lds);
+    });
+}
+template <int BITS, int WIDTH, bool GATED>
+__global__ __launch_bounds__(kMatrixThreads, 4) void expert_matrix_kernel(ExpertPhase p) {
+    extern __shared__ __align__(16) uint8_t affine_lds[];
+    const uint32_t jobs = p.shared_jobs + (p.max_jobs ? uint32_t(uniform(*p.count)) : 0u);
+    matrix_piece_of_work(jobs, (p.tiles + kMatrixWaves - 1) / kMatrixWaves, [&](uint32_t job, uint32_t round, uint32_t rounds) {
+        expert_job<GATED>(p, job, [&](const AffineMatrix (&m)[2], const float* x, float* out, uint32_t nt, auto in_row, auto out_row) {
+            matrix_rows<BITS, WIDTH, GATED, true, GATED>(m, p.K, p.N, x, p.fp32, out, nt, in_row, out_row, round * kMatrixWaves,
+                                                                 min(rounds * kMatrixWaves, p.tiles), false, affine_lds);
+        });
+    });
 }
 
 static bool wide(uint32_t K, uint32_t N) { return K % 512 == 0 && N % 8 == 0; }
@@ -397,14 +115,30 @@ template <int WIDTH> static uint32_t affine_chunk(uint32_t K) {
     while (chunk > 1 && chunk * affine_token_bytes<WIDTH>(K) > 53 * 1024) chunk /= 2;
     return chunk;
 }
-uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t bits) {
+// Whether the matrix cores take rows of this format: whole half steps, affine groups of 64, Q8 only where its blocks have eight elements, and
+// four tokens' rows that leave room for two workgroups on a compute unit, and offsets in the codes of 32 bits.
+template <int BITS, int WIDTH> static bool matrix_fits(uint32_t K, uint32_t N, uint32_t group) {
+    if constexpr (BITS == 8 && WIDTH == 4) return false;
+    else return group == 64 && uint64_t(K) * N / 8 * BITS < 1ull << 32 && K % (16 * WIDTH) == 0 && MatrixForm<BITS, WIDTH>::steps(K) <= kMatrixSteps && matrix_lds_bytes<BITS, WIDTH>(K) <= 80 * 1024;
+}
+// Workgroups of a launch: as many as fit the chip at once (LDS, and four waves a SIMD by registers), not more than there can be rounds.
+static uint32_t matrix_grid(uint32_t lds, uint32_t tiles, uint64_t jobs) {
+    return uint32_t(std::min<uint64_t>(256 * std::min(160u * 1024 / lds, 4u), (tiles + kMatrixWaves - 1) / kMatrixWaves * jobs));
+}
+uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t group, uint32_t bits) {
     uint32_t chunk = 1;
-    by_format<false>(bits, wide(K, N), [&]<int BITS, int WIDTH, bool GATED>() { chunk = affine_chunk<WIDTH>(K); });
+    by_format<false>(bits, wide(K, N), [&]<int BITS, int WIDTH, bool GATED>() { chunk = matrix_fits<BITS, WIDTH>(K, N, group) ? kMatrixTokens : affine_chunk<WIDTH>(K); });
     return chunk;
 }
+bool affine_job_images(uint32_t chunk) { return chunk > kAffineTokens; }
 // (A grid's y holds fewer than 2^16 workgroups: the rest of a longer list goes to z.)
 static dim3 affine_grid(uint32_t x, uint32_t jobs) { const uint32_t y = std::min(jobs, 32768u); return dim3(x, y, (jobs + y - 1) / y); }
 
+// Tokens from which the operators' products go to the matrix cores: a call of few tokens is a chain of latencies, longer there by the images' making
+// and a barrier.  us a call, lanes -> matrix cores: gate/up at 16, 32, 48 and 128 rows, hidden 2048 7.5 -> 9.1, 9.9 -> 9.2, 13.2 -> 11.2, 24 -> 17;
+// 2560 9.7 -> 10.4, 12.5 -> 13.2, 18 -> 13, 34 -> 27; 3072 12.7 -> 12.1, 21 -> 15, 28 -> 20, 57 -> 31.  Down at 32, 48, 96 and 128: 8.6 -> 6.7, 11.1 -> 7.6,
+// 14.4 -> 12.1, 15.5 -> 12.0; 10.9 -> 10.4, 14.9 -> 12.4, 22 -> 18, 27 -> 22; 13.7 -> 11.9, 15.7 -> 20.2, 25.2 -> 26.2, 32 -> 26.
+constexpr uint32_t kMatrixFrom[2] = {128, 48};   // plain, gate/up
 void launch_affine(hipStream_t s, const AffineDesc& a) {
     AffineJob j{};
     auto matrix = [](const zc_linear& l) { return AffineMatrix{(const uint8_t*)l.weight, (const uint16_t*)l.scales, (const uint16_t*)l.biases}; };
@@ -413,6 +147,15 @@ void launch_affine(hipStream_t s, const AffineDesc& a) {
     j.x = a.x; j.in_rows = a.in_rows; j.out_rows = a.out_rows; j.out = a.out;
     j.K = a.gate.input; j.N = a.gate.output; j.group = a.gate.group; j.tokens = a.tokens; j.float_output = a.float_output;
     auto go = [&]<int BITS, int WIDTH, bool GATED>() {
+        if constexpr (BITS == 4 || WIDTH == 8) {
+            if (j.tokens >= kMatrixFrom[GATED] && matrix_fits<BITS, WIDTH>(j.K, j.N, j.group)) {
+                using Stream = MatrixStream<BITS, WIDTH, GATED>;
+                j.chunk = kMatrixTokens; j.tiles = (j.N + Stream::kTileRows - 1) / Stream::kTileRows;
+                const uint32_t lds = matrix_lds_bytes<BITS, WIDTH>(j.K), grid = matrix_grid(lds, j.tiles, (uint64_t(j.tokens) + kMatrixTokens - 1) / kMatrixTokens);
+                hipLaunchKernelGGL((affine_matrix_kernel<BITS, WIDTH, GATED>), dim3(grid), dim3(kMatrixThreads), lds, s, j);
+                return;
+            }
+        }
         j.chunk = std::min(affine_chunk<WIDTH>(j.K), j.tokens);
         const uint32_t rows = j.chunk == 1 ? AffineStream<BITS, WIDTH, GATED, 1>::kTileRows : AffineStream<BITS, WIDTH, GATED, kAffineTokens>::kTileRows;
         const uint32_t chunks = (j.tokens + j.chunk - 1) / j.chunk;
@@ -431,10 +174,19 @@ void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d) {
     p.records = (const uint8_t*)d.records; p.stride = d.stride; p.shared_record = (const uint8_t*)d.shared_record;
     for (int i = 0; i < 6; ++i) { p.off[i] = d.off[i]; p.shared_off[i] = d.shared_off[i]; }
     p.jobs = d.jobs; p.count = d.count; p.slots = d.slots; p.max_jobs = d.max_jobs;
-    p.x = d.x; p.out = d.out; p.shared_x = d.shared_x; p.shared_out = d.shared_out;
+    p.x = d.x; p.out = d.out; p.shared_x = d.shared_x; p.shared_out = d.shared_out; p.fp32 = d.fp32;
     p.K = d.K; p.N = d.N; p.group = d.group; p.topk = d.topk; p.tokens = d.tokens; p.chunk = d.chunk;
     p.shared_jobs = d.shared_record ? (d.tokens + d.chunk - 1) / d.chunk : 0;
     auto go = [&]<int BITS, int WIDTH, bool GATED>() {
+        if constexpr (BITS == 4 || WIDTH == 8) {
+            if (d.chunk > kAffineTokens) {
+                using Stream = MatrixStream<BITS, WIDTH, GATED>;
+                p.tiles = (p.N + Stream::kTileRows - 1) / Stream::kTileRows;
+                const uint32_t lds = matrix_lds_bytes<BITS, WIDTH>(d.K), grid = matrix_grid(lds, p.tiles, d.max_jobs + p.shared_jobs);
+                hipLaunchKernelGGL((expert_matrix_kernel<BITS, WIDTH, GATED>), dim3(grid), dim3(kMatrixThreads), lds, s, p);
+                return;
+            }
+        }
         const uint32_t most = std::min(d.chunk, d.tokens), lds = most * affine_token_bytes<WIDTH>(d.K);
         const uint32_t rows = most == 1 ? AffineStream<BITS, WIDTH, GATED, 1>::kTileRows : AffineStream<BITS, WIDTH, GATED, kAffineTokens>::kTileRows;
         p.tiles = (p.N + rows - 1) / rows; p.share = affine_share(p.tiles, d.max_jobs + p.shared_jobs);
@@ -887,10 +639,14 @@ struct Dispatch {
     int32_t *offsets, *slots, *rows, *selected; uint32_t* jobs; int32_t *count, *status;
     uint32_t topk, E, chunk;
 };
-constexpr uint32_t kDispatchSlots = 1024, kRouteTokens = 16;
 __device__ __forceinline__ uint32_t dispatch_job(uint32_t first, uint32_t expert, uint32_t positions) { return first | expert << 20 | (positions - 1) << 30; }
+// The rows whose images the same launch leaves for the matrix cores, a workgroup a row (rows: 0 if none are wanted).
+struct RowImages { const float* x; float* out; uint32_t rows, K; };
+__global__ __launch_bounds__(256) void row_images_kernel(RowImages images) { matrix_image_row(images.x, images.out, blockIdx.x, images.K); }
+constexpr uint32_t kDispatchSlots = 1024, kRouteTokens = 16;
 template <bool ROUTE, int PER>
-__global__ __launch_bounds__(1024) void dispatch_short_kernel(const float* __restrict__ logits, int32_t* __restrict__ ids, float* __restrict__ weights, uint32_t n, Dispatch d) {
+__global__ __launch_bounds__(1024) void dispatch_short_kernel(const float* __restrict__ logits, int32_t* __restrict__ ids, float* __restrict__ weights, uint32_t n, Dispatch d, RowImages images) {
+    if (blockIdx.x) { matrix_image_row(images.x, images.out, blockIdx.x - 1, images.K); return; }
     __shared__ uint32_t table[16 * 512];           // [wave][expert] counts, two experts a word
     __shared__ uint32_t start[1024], wave_total[2][16];
     __shared__ uint16_t held[1024];
@@ -1123,11 +879,12 @@ __global__ __launch_bounds__(256) void dispatch_place_kernel(const int32_t* __re
         place(ahead, q0);
     }
 }
-static void launch_dispatch_any(hipStream_t s, const int32_t* ids, uint32_t n, const Dispatch& d) {
+static void launch_dispatch_any(hipStream_t s, const int32_t* ids, uint32_t n, const Dispatch& d, const RowImages& images) {
     if (n <= kDispatchSlots && d.E <= 1024) {
-        hipLaunchKernelGGL((dispatch_short_kernel<false, 8>), dim3(1), dim3(1024), 0, s, nullptr, const_cast<int32_t*>(ids), nullptr, n, d);
+        hipLaunchKernelGGL((dispatch_short_kernel<false, 8>), dim3(1 + images.rows), dim3(1024), 0, s, nullptr, const_cast<int32_t*>(ids), nullptr, n, d, images);
         return;
     }
+    if (images.rows) hipLaunchKernelGGL(row_images_kernel, dim3(images.rows), dim3(256), 0, s, images);
     if (n <= kDispatchSlots && !d.jobs) {
         hipLaunchKernelGGL(dispatch_kernel, dim3(1), dim3(1024), size_t(d.E + 1) * 4, s, ids, n, d.topk, d.E, d.offsets, d.slots, d.rows, d.selected, d.count, d.status);
         return;
@@ -1140,21 +897,23 @@ static void launch_dispatch_any(hipStream_t s, const int32_t* ids, uint32_t n, c
 }
 void launch_dispatch(hipStream_t s, const int32_t* ids, uint32_t tokens, uint32_t topk, uint32_t E, int32_t* offsets,
                      int32_t* slots, int32_t* rows, int32_t* selected, int32_t* count, int32_t* status) {
-    launch_dispatch_any(s, ids, tokens * topk, Dispatch{offsets, slots, rows, selected, nullptr, count, status, topk, E, 0});
+    launch_dispatch_any(s, ids, tokens * topk, Dispatch{offsets, slots, rows, selected, nullptr, count, status, topk, E, 0}, RowImages{});
 }
 // Routes, dispatch sort and the expert kernels' job list (E <= 1024; scratch: E words).
 void launch_route_jobs(hipStream_t s, const float* logits, uint32_t tokens, uint32_t E, uint32_t topk, int32_t* ids, float* weights,
-                       int32_t* offsets, int32_t* slots, uint32_t chunk, uint32_t* jobs, int32_t* count, int32_t* scratch, int32_t* status) {
+                       int32_t* offsets, int32_t* slots, uint32_t chunk, uint32_t* jobs, int32_t* count, int32_t* scratch, int32_t* status,
+                       const float* x, uint32_t K, float* row_images) {
     const uint32_t n = tokens * topk;
+    const RowImages images{x, row_images, row_images ? tokens : 0, K};
     Dispatch d{offsets, slots, nullptr, scratch, jobs, count, status, topk, E, chunk};
     if (n <= kDispatchSlots) d.selected = nullptr;
     if (tokens <= kRouteTokens && topk <= 64) {   // (n <= 1024)
-        if (E <= 512) hipLaunchKernelGGL((dispatch_short_kernel<true, 8>), dim3(1), dim3(1024), 0, s, logits, ids, weights, n, d);
-        else hipLaunchKernelGGL((dispatch_short_kernel<true, 16>), dim3(1), dim3(1024), 0, s, logits, ids, weights, n, d);
+        if (E <= 512) hipLaunchKernelGGL((dispatch_short_kernel<true, 8>), dim3(1 + images.rows), dim3(1024), 0, s, logits, ids, weights, n, d, images);
+        else hipLaunchKernelGGL((dispatch_short_kernel<true, 16>), dim3(1 + images.rows), dim3(1024), 0, s, logits, ids, weights, n, d, images);
         return;
     }
     launch_route(s, logits, tokens, E, topk, ids, weights);
-    launch_dispatch_any(s, ids, n, d);
+    launch_dispatch_any(s, ids, n, d, images);
 }
 
 // ---------------------------------------------------------------------------

@@ -21,7 +21,10 @@ bool xint_supported(const zc_linear& l);                          // wide affine
 void launch_affine_xint(hipStream_t s, const AffineDesc& a);     // exact-integer matrix-core form
 constexpr uint32_t kXintLongestRow = 21504;                       // of one token: its digit planes and fp32 copy fill 160 KiB of LDS
 
-uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t bits);   // tokens one workgroup of these kernels takes at a time: 1 or 2
+// Tokens one workgroup of the expert kernels takes at a time: 1 or 2 (lanes), 4 (matrix cores: they read rows as images, which take
+// the rows' place)
+uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t group, uint32_t bits);
+bool affine_job_images(uint32_t chunk);
 
 struct ExpertPhaseDesc {
     const void* records; uint64_t stride;
@@ -29,7 +32,8 @@ struct ExpertPhaseDesc {
     const void* shared_record;   // null, or the shared expert joins the launch: its projections have the routed ones' format
     uint64_t shared_off[6];
     const uint32_t* jobs; const int32_t *count, *slots;   // launch_route_jobs
-    const float *x, *shared_x; float *out, *shared_out;
+    const float *x, *shared_x; float *out, *shared_out;   // chunk > 2: x, shared_x and gate/up's out are images; fp32: what x's were made of, or null
+    const float* fp32;
     uint32_t K, N, group, bits, topk, tokens, chunk, max_jobs;
     bool gated;
 };
@@ -47,7 +51,8 @@ void launch_route(hipStream_t s, const float* logits, uint32_t T, uint32_t E, ui
 void launch_dispatch(hipStream_t s, const int32_t* ids, uint32_t tokens, uint32_t topk, uint32_t E, int32_t* offsets,
                      int32_t* slots, int32_t* rows, int32_t* selected, int32_t* count, int32_t* status);
 void launch_route_jobs(hipStream_t s, const float* logits, uint32_t tokens, uint32_t E, uint32_t topk, int32_t* ids, float* weights,
-                       int32_t* offsets, int32_t* slots, uint32_t chunk, uint32_t* jobs, int32_t* count, int32_t* scratch, int32_t* status);
+                       int32_t* offsets, int32_t* slots, uint32_t chunk, uint32_t* jobs, int32_t* count, int32_t* scratch, int32_t* status,
+                       const float* x, uint32_t K, float* row_images);   // row_images, optional: the images of x's rows, tokens * K floats
 void launch_scatter(hipStream_t s, const float* x, const int32_t* positions, uint32_t n, uint32_t H, float* out);
 // ---- the callers' glue either side of the layer (zc_glue.hip)
 void launch_unary(hipStream_t s, const float* x, uint64_t n, uint32_t op, float* y);
