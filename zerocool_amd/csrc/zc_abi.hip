@@ -602,10 +602,13 @@ static zc_status moe_layer(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe
     uint32_t chunk = ~0u;
     for (const uint32_t bits : {c->bits_gate_up, c->shared_bits_gate_up}) chunk = std::min(chunk, zc::affine_job_tokens(H, I, c->group, bits));
     for (const uint32_t bits : {c->bits_down, c->shared_bits_down}) chunk = std::min(chunk, zc::affine_job_tokens(I, H, c->group, bits));
-    if (T == 1) chunk = 1;
-    float* images = zc::affine_job_images(chunk) ? w.expert_out : nullptr;   // the input rows' images, until the down products write there
+    float* images = T > 1 && zc::affine_job_images(chunk) ? w.expert_out : nullptr;   // the input rows' images, until the down products write there
     uint32_t* jobs = reinterpret_cast<uint32_t*>(w.rows);   // (n words: a job holds at least one slot)
-    zc::launch_route_jobs(s, w.logits, T, E, k, w.ids, w.weights, w.offsets, w.slots, chunk, jobs, w.count, w.selected, ctx->moe_status, x, H, images);
+    if (T > 1) zc::launch_route_jobs(s, w.logits, T, E, k, w.ids, w.weights, w.offsets, w.slots, chunk, jobs, w.count, w.selected, ctx->moe_status, x, H, images);
+    else {   // its picks are the job list
+        chunk = 1;
+        if (!zc::expert_phase_routes(H, k)) zc::launch_route(s, w.logits, 1, E, k, w.ids, w.weights);
+    }
     // 5-6. shared expert (model.cpp:482-485) and routed experts (pipeline.cpp:18-29): gate/up on gathered rows, down scattered
     // to its slot.  One launch per phase where the shared expert's projections have the routed ones' width.
     auto offsets_of = [&](const void* record, int shared, uint64_t* off, int first, int count) {
@@ -621,6 +624,7 @@ static zc_status moe_layer(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe
         zc::ExpertPhaseDesc p{};
         const int first = gated ? 0 : 2, count = gated ? 2 : 1;
         p.records = l->expert_records; p.stride = l->record_stride; offsets_of(l->expert_records, 0, p.off, first, count);
+        if (T == 1) { p.logits = w.logits; p.ids = w.ids; p.weights = w.weights; p.status = ctx->moe_status; p.E = E; }
         p.jobs = jobs; p.count = w.count; p.slots = w.slots; p.topk = k; p.tokens = T; p.chunk = chunk;
         p.max_jobs = uint32_t(std::min(n, std::min<uint64_t>(n, E) + n / chunk));
         p.K = gated ? H : I; p.N = gated ? I : H; p.group = c->group; p.bits = gated ? c->bits_gate_up : c->bits_down; p.gated = gated;

@@ -52,8 +52,17 @@ struct ExpertPhase {
     const uint32_t *jobs; const int32_t *count, *slots;
     const float *x, *shared_x; float *out, *shared_out;                // x: layer input (gate/up) or sorted activations (down); on the matrix cores both as row images
     const float* fp32;                                                 // matrix cores: the rows that x and shared_x were made of, null where they were made as images
+    const float* logits; int32_t *ids, *status; float* weights; uint32_t E;   // of one token alone: job j of the routed ones is its pick j
     uint32_t K, N, group, topk, tokens, chunk, shared_jobs, max_jobs, tiles, share;   // chunk: tokens of a job (a shared job too)
 };
+__device__ __forceinline__ void expert_matrices(const ExpertPhase& p, bool shared, uint32_t expert, AffineMatrix (&m)[2]) {
+    const uint8_t* r = shared ? p.shared_record : p.records + uint64_t(expert) * p.stride;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        auto at = [&](int i) { return r + (shared ? p.shared_off[3 * q + i] : p.off[3 * q + i]); };
+        m[q] = AffineMatrix{at(0), reinterpret_cast<const uint16_t*>(at(1)), reinterpret_cast<const uint16_t*>(at(2))};
+    }
+}
 // A job, if there is one of that number: its matrices, tokens and rows go to `run`.
 template <bool GATED, class Run>
 __device__ __forceinline__ void expert_job(const ExpertPhase& p, uint32_t job, Run run) {
@@ -64,13 +73,8 @@ __device__ __forceinline__ void expert_job(const ExpertPhase& p, uint32_t job, R
         if (job - p.shared_jobs >= count) return;
         first = packed & 0xfffffu; expert = (packed >> 20) & 1023u; nt = (packed >> 30) + 1u;
     }
-    const uint8_t* r = shared ? p.shared_record : p.records + uint64_t(expert) * p.stride;
     AffineMatrix m[2];
-#pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        auto at = [&](int i) { return r + (shared ? p.shared_off[3 * q + i] : p.off[3 * q + i]); };
-        m[q] = AffineMatrix{at(0), reinterpret_cast<const uint16_t*>(at(1)), reinterpret_cast<const uint16_t*>(at(2))};
-    }
+    expert_matrices(p, shared, expert, m);
     run(m, shared ? p.shared_x : p.x, shared ? p.shared_out : p.out, nt,
         [&, first](uint32_t t) { return GATED && !shared ? uint32_t(p.slots[first + t]) / p.topk : first + t; },
         [&, first](uint32_t t) { return GATED || shared ? first + t : uint32_t(p.slots[first + t]); });
@@ -82,6 +86,61 @@ __global__ __launch_bounds__(256, TOKENS == 1 ? 4 : 3) void expert_phase_kernel(
     expert_job<GATED>(p, blockIdx.z * gridDim.y + blockIdx.y, [&](const AffineMatrix (&m)[2], const float* x, float* out, uint32_t nt, auto in_row, auto out_row) {
         affine_rows<BITS, WIDTH, GATED, TOKENS>(m, p.K, p.N, p.group, x, out, nt, in_row, out_row, tile0, end, false, affine_lds);
     });
+}
+// One token alone: there is nothing to sort, pick j's rows are row j.  The gate/up kernel makes the picks too (PER: candidates a lane, 0
+// where `ids` holds the picks): the first wave of every workgroup selects them from the logits, all of them, while the others
+// stage the input row.  Bound by the chain of latencies: logits -> picks -> codes, 2 to 2.5 us longer than a list's job -> codes, in
+// place of a launch of 6 us and the gap behind it.  Hidden 2048, intermediate 512: picks, gate/up, down 5.9 + 9.0 + 5.6 -> 11.4 + 5.8 us, a
+// layer 28.8 -> 23.6; hidden 2560, intermediate 640: 5.8 + 12.0 + 8.2 -> 13.0 + 7.0, a layer of a stack 37.7 -> 31.7.
+template <int BITS, int WIDTH, bool GATED, int PER>
+__global__ __launch_bounds__(256, 4) void expert_token_kernel(ExpertPhase p) {
+    extern __shared__ __align__(16) uint8_t affine_lds[];
+    const uint32_t tile0 = blockIdx.x * p.share, end = min(tile0 + p.share, p.tiles), tid = threadIdx.x;
+    const bool shared = blockIdx.y < p.shared_jobs;
+    const uint32_t row = shared ? 0u : blockIdx.y - p.shared_jobs;
+    auto valid = [&](int32_t id) {
+        if (uint32_t(id) < p.E) return true;
+        if (tid == 0) atomicOr(p.status, 1);
+        return false;
+    };
+    const float* x = shared ? p.shared_x : p.x;
+    float* out = shared ? p.shared_out : p.out;
+    auto in_row = [&](uint32_t) { return GATED ? 0u : row; };
+    auto out_row = [&](uint32_t) { return row; };
+    AffineMatrix m[2];
+    if constexpr (PER == 0) {
+        const int32_t id = shared ? 0 : uniform(p.ids[row]);
+        if (!shared && !valid(id)) return;
+        expert_matrices(p, shared, uint32_t(id), m);
+        affine_rows<BITS, WIDTH, GATED, 1>(m, p.K, p.N, p.group, x, out, 1, in_row, out_row, tile0, end, false, affine_lds);
+    } else {
+        __shared__ int32_t ids_s[64];
+        __shared__ float weights_s[64];
+        __shared__ uint32_t pick[128];
+        struct Picks {
+            const ExpertPhase& p; const bool shared; const uint32_t row, tid; decltype(valid)& check;
+            int32_t* ids; float* weights; uint32_t* pick;
+            __device__ __forceinline__ void find() const {
+                if (shared || tid >= 64) return;
+                route_token<PER>([&](float (&cand)[PER], uint32_t per) {
+#pragma unroll
+                    for (int i = 0; i < PER; ++i) { const uint32_t e = tid * per + uint32_t(i); cand[i] = (uint32_t(i) < per && e < p.E) ? p.logits[e] : __uint_as_float(0xff800000u); }
+                }, p.E, p.topk, tid, ids, weights, pick, [] {}, [] {});
+            }
+            __device__ __forceinline__ bool take(AffineMatrix (&m)[2]) const {
+                int32_t id = 0;
+                if (!shared) {
+                    if (row == 0 && blockIdx.x == 0 && tid < p.topk) { p.ids[tid] = ids[tid]; p.weights[tid] = weights[tid]; }
+                    id = uniform(ids[row]);
+                    if (!check(id)) return false;
+                }
+                expert_matrices(p, shared, uint32_t(id), m);
+                return true;
+            }
+        };
+        affine_rows<BITS, WIDTH, GATED, 1>(m, p.K, p.N, p.group, x, out, 1, in_row, out_row, tile0, end, false, affine_lds,
+                                           Picks{p, shared, row, tid, valid, ids_s, weights_s, pick});
+    }
 }
 template <int BITS, int WIDTH, bool GATED>
 __global__ __launch_bounds__(kMatrixThreads, 4) void expert_matrix_kernel(ExpertPhase p) {
@@ -169,8 +228,11 @@ void launch_affine(hipStream_t s, const AffineDesc& a) {
     else by_format<false>(a.gate.bits, wide(j.K, j.N), go);
 }
 
+// (the selection's words beside the longest rows, which fill a compute unit's LDS)
+bool expert_phase_routes(uint32_t K, uint32_t topk) { return topk <= 64 && affine_token_bytes<16>(K) + 1024 <= 160 * 1024; }
 void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d) {
     ExpertPhase p{};
+    p.logits = d.logits; p.ids = d.ids; p.weights = d.weights; p.status = d.status; p.E = d.E;
     p.records = (const uint8_t*)d.records; p.stride = d.stride; p.shared_record = (const uint8_t*)d.shared_record;
     for (int i = 0; i < 6; ++i) { p.off[i] = d.off[i]; p.shared_off[i] = d.shared_off[i]; }
     p.jobs = d.jobs; p.count = d.count; p.slots = d.slots; p.max_jobs = d.max_jobs;
@@ -186,6 +248,21 @@ void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d) {
                 hipLaunchKernelGGL((expert_matrix_kernel<BITS, WIDTH, GATED>), dim3(grid), dim3(kMatrixThreads), lds, s, p);
                 return;
             }
+        }
+        if (d.ids) {
+            constexpr uint32_t rows = AffineStream<BITS, WIDTH, GATED, 1>::kTileRows;
+            p.tiles = (p.N + rows - 1) / rows; p.share = affine_share(p.tiles, d.max_jobs + p.shared_jobs);
+            const dim3 grid((p.tiles + p.share - 1) / p.share, d.max_jobs + p.shared_jobs);
+            const uint32_t lds = affine_token_bytes<WIDTH>(d.K);
+            if constexpr (GATED) {
+                if (d.max_jobs && expert_phase_routes(d.K, d.topk)) {
+                    if (d.E <= 512) hipLaunchKernelGGL((expert_token_kernel<BITS, WIDTH, true, 8>), grid, dim3(256), lds, s, p);
+                    else hipLaunchKernelGGL((expert_token_kernel<BITS, WIDTH, true, 16>), grid, dim3(256), lds, s, p);
+                    return;
+                }
+            }
+            hipLaunchKernelGGL((expert_token_kernel<BITS, WIDTH, GATED, 0>), grid, dim3(256), lds, s, p);
+            return;
         }
         const uint32_t most = std::min(d.chunk, d.tokens), lds = most * affine_token_bytes<WIDTH>(d.K);
         const uint32_t rows = most == 1 ? AffineStream<BITS, WIDTH, GATED, 1>::kTileRows : AffineStream<BITS, WIDTH, GATED, kAffineTokens>::kTileRows;

@@ -34,9 +34,12 @@ struct ExpertPhaseDesc {
     const uint32_t* jobs; const int32_t *count, *slots;   // launch_route_jobs
     const float *x, *shared_x; float *out, *shared_out;   // chunk > 2: x, shared_x and gate/up's out are images; fp32: what x's were made of, or null
     const float* fp32;
+    // one token alone: its picks instead of a job list; the gate/up phase makes them from the logits where expert_phase_routes
+    const float* logits; int32_t *ids, *status; float* weights; uint32_t E;
     uint32_t K, N, group, bits, topk, tokens, chunk, max_jobs;
     bool gated;
 };
+bool expert_phase_routes(uint32_t K, uint32_t topk);
 void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d);
 
 void launch_plain(hipStream_t s, const void* w, uint32_t dtype, const float* x, uint32_t K, uint32_t N,
