@@ -610,7 +610,7 @@ static zc_status moe_layer(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe
         if (!zc::expert_phase_routes(H, k)) zc::launch_route(s, w.logits, 1, E, k, w.ids, w.weights);
     }
     // 5-6. shared expert (model.cpp:482-485) and routed experts (pipeline.cpp:18-29): gate/up on gathered rows, down scattered
-    // to its slot.  One launch per phase where the shared expert's projections have the routed ones' width.
+    // to its slot.  One launch per phase (two where the lanes' kernels walk a list and the shared expert has another format).
     auto offsets_of = [&](const void* record, int shared, uint64_t* off, int first, int count) {
         for (int q = 0; q < count; ++q) {
             zc_linear lin; zc_hip_expert_linear(c, shared, record, first + q, &lin);
@@ -632,13 +632,7 @@ static zc_status moe_layer(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe
         p.x = gated ? input : w.act; p.out = gated ? w.act : w.expert_out; p.shared_x = gated ? input : w.shared_act; p.shared_out = gated ? w.shared_act : w.shared;
         p.fp32 = gated ? x : nullptr;
         offsets_of(l->shared_record, 1, p.shared_off, first, count);
-        const uint32_t shared_bits = gated ? c->shared_bits_gate_up : c->shared_bits_down;
-        if (shared_bits == p.bits) p.shared_record = l->shared_record;
-        else {   // a launch of its own, without routed jobs
-            zc::ExpertPhaseDesc own = p;
-            own.shared_record = l->shared_record; own.bits = shared_bits; own.max_jobs = 0;
-            zc::launch_expert_phase(s, own);
-        }
+        p.shared_record = l->shared_record; p.shared_bits = gated ? c->shared_bits_gate_up : c->shared_bits_down;
         zc::launch_expert_phase(s, p);
     }
     // 7. weighted combine (model.cpp:553-556)

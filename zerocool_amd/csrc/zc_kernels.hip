@@ -44,7 +44,7 @@ __global__ __launch_bounds__(kMatrixThreads, 4) void affine_matrix_kernel(Affine
     });
 }
 
-// The routed experts of one layer and, where its formats are theirs, the shared expert: blockIdx.y walks the shared expert's
+// The routed experts of one layer and the shared expert (the lanes' lists: where its format is theirs): blockIdx.y walks the shared expert's
 // tokens, chunk by chunk, then the list of (expert, sorted positions) that the dispatch left; jobs past the device-side count exit.
 struct ExpertPhase {
     const uint8_t* records; uint64_t stride; uint64_t off[6];          // byte offsets inside a record: codes, scales, biases of the (gate | down) projection, of up
@@ -55,6 +55,8 @@ struct ExpertPhase {
     const float* logits; int32_t *ids, *status; float* weights; uint32_t E;   // of one token alone: job j of the routed ones is its pick j
     uint32_t K, N, group, topk, tokens, chunk, shared_jobs, max_jobs, tiles, share;   // chunk: tokens of a job (a shared job too)
 };
+// Elements of a block of the shared expert's rows, of SHARED bits, where the routed experts have BITS and WIDTH: the row lengths are the same.
+constexpr int shared_width(int BITS, int WIDTH, int SHARED) { return SHARED == BITS ? WIDTH : SHARED == 4 ? 2 * WIDTH : WIDTH / 2; }
 __device__ __forceinline__ void expert_matrices(const ExpertPhase& p, bool shared, uint32_t expert, AffineMatrix (&m)[2]) {
     const uint8_t* r = shared ? p.shared_record : p.records + uint64_t(expert) * p.stride;
 #pragma unroll
@@ -92,7 +94,7 @@ __global__ __launch_bounds__(256, TOKENS == 1 ? 4 : 3) void expert_phase_kernel(
 // stage the input row.  Bound by the chain of latencies: logits -> picks -> codes, 2 to 2.5 us longer than a list's job -> codes, in
 // place of a launch of 6 us and the gap behind it.  Hidden 2048, intermediate 512: picks, gate/up, down 5.9 + 9.0 + 5.6 -> 11.4 + 5.8 us, a
 // layer 28.8 -> 23.6; hidden 2560, intermediate 640: 5.8 + 12.0 + 8.2 -> 13.0 + 7.0, a layer of a stack 37.7 -> 31.7.
-template <int BITS, int WIDTH, bool GATED, int PER>
+template <int BITS, int WIDTH, bool GATED, int PER, int SHARED>
 __global__ __launch_bounds__(256, 4) void expert_token_kernel(ExpertPhase p) {
     extern __shared__ __align__(16) uint8_t affine_lds[];
     const uint32_t tile0 = blockIdx.x * p.share, end = min(tile0 + p.share, p.tiles), tid = threadIdx.x;
@@ -108,6 +110,13 @@ __global__ __launch_bounds__(256, 4) void expert_token_kernel(ExpertPhase p) {
     auto in_row = [&](uint32_t) { return GATED ? 0u : row; };
     auto out_row = [&](uint32_t) { return row; };
     AffineMatrix m[2];
+    if constexpr (SHARED != BITS) {
+        if (shared) {
+            expert_matrices(p, true, 0, m);
+            affine_rows<SHARED, shared_width(BITS, WIDTH, SHARED), GATED, 1>(m, p.K, p.N, p.group, x, out, 1, in_row, out_row, tile0, end, false, affine_lds);
+            return;
+        }
+    }
     if constexpr (PER == 0) {
         const int32_t id = shared ? 0 : uniform(p.ids[row]);
         if (!shared && !valid(id)) return;
@@ -142,12 +151,21 @@ __global__ __launch_bounds__(256, 4) void expert_token_kernel(ExpertPhase p) {
                                            Picks{p, shared, row, tid, valid, ids_s, weights_s, pick});
     }
 }
-template <int BITS, int WIDTH, bool GATED>
+// SHARED: the bits of the shared expert's rows.  Where they are not BITS its jobs could have a launch of their own, 9.7 us for the Q8 gate/up of
+// five tokens (hidden 2048, intermediate 512) in front of the routed Q4 jobs' 20 us; in one launch they take 26 us, a layer 63 -> 56.
+template <int BITS, int WIDTH, bool GATED, int SHARED>
 __global__ __launch_bounds__(kMatrixThreads, 4) void expert_matrix_kernel(ExpertPhase p) {
     extern __shared__ __align__(16) uint8_t affine_lds[];
-    const uint32_t jobs = p.shared_jobs + (p.max_jobs ? uint32_t(uniform(*p.count)) : 0u);
+    const uint32_t jobs = p.shared_jobs + uint32_t(uniform(*p.count));
     matrix_piece_of_work(jobs, (p.tiles + kMatrixWaves - 1) / kMatrixWaves, [&](uint32_t job, uint32_t round, uint32_t rounds) {
         expert_job<GATED>(p, job, [&](const AffineMatrix (&m)[2], const float* x, float* out, uint32_t nt, auto in_row, auto out_row) {
+            if constexpr (SHARED != BITS) {
+                if (job < p.shared_jobs) {
+                    matrix_rows<SHARED, shared_width(BITS, WIDTH, SHARED), GATED, true, GATED>(m, p.K, p.N, x, p.fp32, out, nt, in_row, out_row, round * kMatrixWaves,
+                                                                                               min(rounds * kMatrixWaves, p.tiles), false, affine_lds);
+                    return;
+                }
+            }
             matrix_rows<BITS, WIDTH, GATED, true, GATED>(m, p.K, p.N, x, p.fp32, out, nt, in_row, out_row, round * kMatrixWaves,
                                                                  min(rounds * kMatrixWaves, p.tiles), false, affine_lds);
         });
@@ -238,41 +256,65 @@ void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d) {
     p.jobs = d.jobs; p.count = d.count; p.slots = d.slots; p.max_jobs = d.max_jobs;
     p.x = d.x; p.out = d.out; p.shared_x = d.shared_x; p.shared_out = d.shared_out; p.fp32 = d.fp32;
     p.K = d.K; p.N = d.N; p.group = d.group; p.topk = d.topk; p.tokens = d.tokens; p.chunk = d.chunk;
-    p.shared_jobs = d.shared_record ? (d.tokens + d.chunk - 1) / d.chunk : 0;
+    p.shared_jobs = (d.tokens + d.chunk - 1) / d.chunk;
+    auto with_shared = [&](auto bits, auto launch) {   // the shared expert's bits as a constant
+        if (d.shared_bits == d.bits) launch(bits);
+        else launch(std::integral_constant<int, 12 - decltype(bits)::value>{});
+    };
     auto go = [&]<int BITS, int WIDTH, bool GATED>() {
+        const std::integral_constant<int, BITS> bits;
         if constexpr (BITS == 4 || WIDTH == 8) {
             if (d.chunk > kAffineTokens) {
-                using Stream = MatrixStream<BITS, WIDTH, GATED>;
-                p.tiles = (p.N + Stream::kTileRows - 1) / Stream::kTileRows;
-                const uint32_t lds = matrix_lds_bytes<BITS, WIDTH>(d.K), grid = matrix_grid(lds, p.tiles, d.max_jobs + p.shared_jobs);
-                hipLaunchKernelGGL((expert_matrix_kernel<BITS, WIDTH, GATED>), dim3(grid), dim3(kMatrixThreads), lds, s, p);
+                with_shared(bits, [&](auto other) {
+                    constexpr int SHARED = decltype(other)::value, OTHER = shared_width(BITS, WIDTH, SHARED);
+                    if constexpr (SHARED == 4 || OTHER == 8) {   // (the other formats have jobs of fewer tokens)
+                        using Stream = MatrixStream<BITS, WIDTH, GATED>;
+                        static_assert(Stream::kTileRows == MatrixStream<SHARED, OTHER, GATED>::kTileRows);
+                        p.tiles = (p.N + Stream::kTileRows - 1) / Stream::kTileRows;
+                        const uint32_t lds = std::max(matrix_lds_bytes<BITS, WIDTH>(d.K), matrix_lds_bytes<SHARED, OTHER>(d.K)), grid = matrix_grid(lds, p.tiles, d.max_jobs + p.shared_jobs);
+                        hipLaunchKernelGGL((expert_matrix_kernel<BITS, WIDTH, GATED, SHARED>), dim3(grid), dim3(kMatrixThreads), lds, s, p);
+                    }
+                });
                 return;
             }
         }
         if (d.ids) {
-            constexpr uint32_t rows = AffineStream<BITS, WIDTH, GATED, 1>::kTileRows;
-            p.tiles = (p.N + rows - 1) / rows; p.share = affine_share(p.tiles, d.max_jobs + p.shared_jobs);
-            const dim3 grid((p.tiles + p.share - 1) / p.share, d.max_jobs + p.shared_jobs);
-            const uint32_t lds = affine_token_bytes<WIDTH>(d.K);
-            if constexpr (GATED) {
-                if (d.max_jobs && expert_phase_routes(d.K, d.topk)) {
-                    if (d.E <= 512) hipLaunchKernelGGL((expert_token_kernel<BITS, WIDTH, true, 8>), grid, dim3(256), lds, s, p);
-                    else hipLaunchKernelGGL((expert_token_kernel<BITS, WIDTH, true, 16>), grid, dim3(256), lds, s, p);
-                    return;
+            with_shared(bits, [&](auto other) {
+                constexpr int SHARED = decltype(other)::value, OTHER = shared_width(BITS, WIDTH, SHARED);
+                constexpr uint32_t rows = AffineStream<BITS, WIDTH, GATED, 1>::kTileRows;
+                static_assert(rows == AffineStream<SHARED, OTHER, GATED, 1>::kTileRows);
+                p.tiles = (p.N + rows - 1) / rows; p.share = affine_share(p.tiles, d.max_jobs + p.shared_jobs);
+                const dim3 grid((p.tiles + p.share - 1) / p.share, d.max_jobs + p.shared_jobs);
+                const uint32_t lds = affine_token_bytes<WIDTH>(d.K);
+                if constexpr (GATED) {
+                    if (expert_phase_routes(d.K, d.topk)) {
+                        if (d.E <= 512) hipLaunchKernelGGL((expert_token_kernel<BITS, WIDTH, true, 8, SHARED>), grid, dim3(256), lds, s, p);
+                        else hipLaunchKernelGGL((expert_token_kernel<BITS, WIDTH, true, 16, SHARED>), grid, dim3(256), lds, s, p);
+                        return;
+                    }
                 }
-            }
-            hipLaunchKernelGGL((expert_token_kernel<BITS, WIDTH, GATED, 0>), grid, dim3(256), lds, s, p);
+                hipLaunchKernelGGL((expert_token_kernel<BITS, WIDTH, GATED, 0, SHARED>), grid, dim3(256), lds, s, p);
+            });
             return;
         }
         const uint32_t most = std::min(d.chunk, d.tokens), lds = most * affine_token_bytes<WIDTH>(d.K);
         const uint32_t rows = most == 1 ? AffineStream<BITS, WIDTH, GATED, 1>::kTileRows : AffineStream<BITS, WIDTH, GATED, kAffineTokens>::kTileRows;
-        p.tiles = (p.N + rows - 1) / rows; p.share = affine_share(p.tiles, d.max_jobs + p.shared_jobs);
-        const dim3 grid = affine_grid((p.tiles + p.share - 1) / p.share, d.max_jobs + p.shared_jobs);
+        p.tiles = (p.N + rows - 1) / rows; p.share = affine_share(p.tiles, p.max_jobs + p.shared_jobs);
+        const dim3 grid = affine_grid((p.tiles + p.share - 1) / p.share, p.max_jobs + p.shared_jobs);
         if (most == 1) hipLaunchKernelGGL((expert_phase_kernel<BITS, WIDTH, GATED, 1>), grid, dim3(256), lds, s, p);
         else hipLaunchKernelGGL((expert_phase_kernel<BITS, WIDTH, GATED, kAffineTokens>), grid, dim3(256), lds, s, p);
     };
-    if (d.gated) by_format<true>(d.bits, wide(d.K, d.N), go);
-    else by_format<false>(d.bits, wide(d.K, d.N), go);
+    auto launch = [&](uint32_t bits) {
+        if (d.gated) by_format<true>(bits, wide(d.K, d.N), go);
+        else by_format<false>(bits, wide(d.K, d.N), go);
+    };
+    // The lists of the lanes' kernels: a shared expert of the other format has a launch of its own, without routed jobs.
+    if (d.shared_bits != d.bits && !d.ids && d.chunk <= kAffineTokens) {
+        p.max_jobs = 0;
+        launch(d.shared_bits);
+        p.max_jobs = d.max_jobs; p.shared_jobs = 0;
+    }
+    launch(d.bits);
 }
 
 // ---------------------------------------------------------------------------
