@@ -426,26 +426,30 @@ __global__ __launch_bounds__(256) void router_kernel(const uint16_t* w, const fl
 }
 // The same chains for short batches of rows that are a multiple of 128 long.  A chain is P = K / 16 dependent multiply-adds
 // and the rest is latency: a lane's next 64 weights are requested before the current ones are used, the first before the input
-// rows are staged in LDS (one padded piece per partition, so that the sixteen partitions' reads meet different banks).  A
-// workgroup has four experts per wave and TT tokens; one or two tokens take workgroups of one wave, which spreads 512 experts over
-// 128 compute units instead of 32.  The workgroups behind the last expert's, if gate_w is not null, form the shared gate's plain
-// dots of their tokens: a launch less, and its latency beside the logits'.
-// 512 experts, hidden 2560: one token 8.9 -> 6.7 us, 40 tokens 42 -> 15 us (and the shared gate's launch, 14 and 19 us, gone).
-template <int TT>
+// rows are staged in LDS, twelve loads a thread in flight (one padded piece per partition, so that the partitions' reads meet different
+// banks).  A workgroup has four experts per wave and up to four tokens.  The workgroups behind the last expert's, if gate_w is not null, form
+// the shared gate's plain dots of their tokens: a launch less, and its latency beside the logits'.
+// Several tokens go to the matrix cores: a v_mfma_f32_4x4x1_16b_f32 is one fused multiply-add for each of sixteen partitions, four
+// tokens and four experts, rounded as the chains' own.  Lane (partition, j) brings one input of token j and one weight of
+// expert j, a quarter of the reads of LDS that a lane with four tokens' chains needs, and half the time on the vector unit.
+// 512 experts: one token of 2048 inputs 5.0 us, of 2560 6.5; on the vector unit, with the staging's loads waited for one by one, -> here:
+// 5 tokens of 2048 8.4 -> 5.8, 8 of 3072 11.4 -> 7.4, 40 of 2560 15.3 -> 12.3, 64 of 3072 19.2 -> 15.9.
+template <uint32_t TOKENS>
 __global__ __launch_bounds__(256) void router_short_kernel(const uint16_t* __restrict__ w, const float* __restrict__ x, uint32_t T, uint32_t K, uint32_t E,
-                                                           const float* __restrict__ offsets, float* __restrict__ out, const void* __restrict__ gate_w, float* __restrict__ gate,
-                                                           int32_t* status) {
-    extern __shared__ __align__(16) float router_x[];   // [TT][16][P + 4]
-    const uint32_t tid = threadIdx.x, split = tid % 16, experts = blockDim.x / 16, t0 = blockIdx.y * TT, P = K / 16, pitch = P + 4;
+                                                            const float* __restrict__ offsets, float* __restrict__ out, const void* __restrict__ gate_w, float* __restrict__ gate,
+                                                            int32_t* status, uint32_t rows) {   // rows: tokens of a workgroup, at most TOKENS
+    extern __shared__ __align__(16) float router_x[];   // [rows][16][P + 4], then the waves' partial sums: [4 * TOKENS][17]
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, j = lane & 3u, split = lane >> 2, experts = blockDim.x / 16, t0 = blockIdx.y * rows, P = K / 16, pitch = P + 4;
+    const uint32_t nt = min(T - t0, rows);
     if (blockIdx.x * experts >= E) {
-        for (uint32_t t = tid >> 5; t < TT && t0 + t < T; t += blockDim.x >> 5) {
+        for (uint32_t t = tid >> 5; t < nt; t += blockDim.x >> 5) {
             const float sum = plain_dot(gate_w, 0, x + uint64_t(t0 + t) * K, K, 1, 0, tid & 31u);
             if ((tid & 31u) == 0) gate[t0 + t] = bf(sum);
         }
         return;
     }
-    const uint32_t e = blockIdx.x * experts + tid / 16;
-    const uint16_t* wr = w + uint64_t(min(e, E - 1)) * K + split * P;
+    const uint32_t e0 = blockIdx.x * experts + wave * 4;
+    const uint16_t* wr = w + uint64_t(min(e0 + j, E - 1)) * K + split * P;
     uint4 ahead[8];
     auto request = [&](uint32_t i0) {
 #pragma unroll
@@ -453,20 +457,27 @@ __global__ __launch_bounds__(256) void router_short_kernel(const uint16_t* __res
     };
     request(0);
     uint32_t low = 0;
-    for (uint32_t i = tid; i < K / 4; i += blockDim.x) {
-        const uint32_t part = i / (P / 4), at = part * pitch + (i - part * (P / 4)) * 4;
+    constexpr uint32_t kBatch = 12 / TOKENS;
+    for (uint32_t i0 = tid; i0 < K / 4; i0 += kBatch * blockDim.x) {   // (past the end: the last piece again, not used)
+        uint4 v[TOKENS][kBatch];
 #pragma unroll
-        for (int t = 0; t < TT; ++t) {
-            const uint4 v = ldg_u4(x + uint64_t(min(t0 + t, T - 1)) * K, i);
-            low |= v.x | v.y | v.z | v.w;
-            *reinterpret_cast<uint4*>(router_x + t * 16 * pitch + at) = v;
+        for (uint32_t t = 0; t < TOKENS; ++t)
+#pragma unroll
+            for (uint32_t u = 0; u < kBatch; ++u) v[t][u] = ldg_u4(x + uint64_t(t0 + min(t, nt - 1)) * K, min(i0 + u * blockDim.x, K / 4 - 1));
+#pragma unroll
+        for (uint32_t u = 0; u < kBatch; ++u) {
+            const uint32_t i = i0 + u * blockDim.x, part = i / (P / 4), at = part * pitch + (i - part * (P / 4)) * 4;
+#pragma unroll
+            for (uint32_t t = 0; t < TOKENS; ++t) {
+                low |= v[t][u].x | v[t][u].y | v[t][u].z | v[t][u].w;
+                if (t < nt && i < K / 4) *reinterpret_cast<uint4*>(router_x + t * 16 * pitch + at) = v[t][u];
+            }
         }
     }
     if (status && blockIdx.x == 0 && (low & 0xffffu)) atomicOr(status, 4);
     lds_barrier();
-    float c[TT];
-#pragma unroll
-    for (int t = 0; t < TT; ++t) c[t] = 0;
+    const float* xr = router_x + (min(j, nt - 1) * 16 + split) * pitch;   // (tokens that are not there: the last one again, not used)
+    f32x4 c = {0, 0, 0, 0};
     for (uint32_t i0 = 0; i0 < P; i0 += 64) {
         uint4 piece[8];
 #pragma unroll
@@ -476,26 +487,28 @@ __global__ __launch_bounds__(256) void router_short_kernel(const uint16_t* __res
         for (int q = 0; q < 8; ++q) {
             if (i0 + 8 * uint32_t(q) >= P) break;
             const uint32_t ww[4] = {piece[q].x, piece[q].y, piece[q].z, piece[q].w};
+            const float4 a = *reinterpret_cast<const float4*>(xr + i0 + 8 * q), b = *reinterpret_cast<const float4*>(xr + i0 + 8 * q + 4);
+            const float xv[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
 #pragma unroll
-            for (int t = 0; t < TT; ++t) {
-                const float* xr = router_x + (t * 16 + split) * pitch + i0 + 8 * q;
-                const float4 a = *reinterpret_cast<const float4*>(xr), b = *reinterpret_cast<const float4*>(xr + 4);
-                const float xv[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-                for (int k = 0; k < 8; ++k) c[t] = __builtin_fmaf(xv[k], __uint_as_float((k & 1) ? (ww[k / 2] & 0xffff0000u) : (ww[k / 2] << 16)), c[t]);
+            for (int k = 0; k < 8; ++k) {
+                const float weight = (k & 1) ? high_bf16(ww[k / 2]) : low_bf16(ww[k / 2]);
+                if constexpr (TOKENS == 1) c[0] = __builtin_fmaf(xv[k], weight, c[0]);
+                else c = matrix_chain_step(xv[k], weight, c);
             }
         }
     }
+    // the partials added 0..15, by lane 4 t + j for token t and expert j
+    float* partial = router_x + rows * 16 * pitch + wave * (4 * TOKENS * 17);
 #pragma unroll
-    for (int t = 0; t < TT; ++t) {
-        // the partials added 0..15, each handed round its row of sixteen lanes (row_newbcast)
-        float sum = 0;
-        sum += dpp_f32<0x150>(c[t]); sum += dpp_f32<0x151>(c[t]); sum += dpp_f32<0x152>(c[t]); sum += dpp_f32<0x153>(c[t]);
-        sum += dpp_f32<0x154>(c[t]); sum += dpp_f32<0x155>(c[t]); sum += dpp_f32<0x156>(c[t]); sum += dpp_f32<0x157>(c[t]);
-        sum += dpp_f32<0x158>(c[t]); sum += dpp_f32<0x159>(c[t]); sum += dpp_f32<0x15a>(c[t]); sum += dpp_f32<0x15b>(c[t]);
-        sum += dpp_f32<0x15c>(c[t]); sum += dpp_f32<0x15d>(c[t]); sum += dpp_f32<0x15e>(c[t]); sum += dpp_f32<0x15f>(c[t]);
-        if (split == 0 && e < E && t0 + t < T) out[uint64_t(t0 + t) * E + e] = offsets ? sum + offsets[e] : sum;
-    }
+    for (uint32_t t = 0; t < TOKENS; ++t) partial[(t * 4 + j) * 17 + split] = c[t];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    float sum = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 16; ++i) sum += partial[min(lane, 4 * TOKENS - 1) * 17 + i];
+    const uint32_t e = e0 + j;
+    if (split < nt && e < E) out[uint64_t(t0 + split) * E + e] = offsets ? sum + offsets[e] : sum;
 }
 // The same chains for long batches, register-tiled: a lane owns one K partition for 4 tokens x 4 experts, so every
 // sixteen-byte weight piece and every eight inputs feed sixteen multiply-accumulate chains.  A workgroup covers
@@ -632,14 +645,21 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 }
 void launch_router(hipStream_t s, const void* w, const float* x, uint32_t T, uint32_t K, uint32_t E,
                    const float* offsets, float* out, const void* gate_w, float* gate, int32_t* status) {
-    const uint32_t tt = T >= 4 ? 4 : T >= 2 ? 2 : 1;
+    const auto row_bytes = [&](uint32_t rows) { return size_t(rows) * (K + 64) * 4; };
+    const uint32_t rows = T >= 4 ? 4 : T == 3 && row_bytes(3) > kRouterShortLds ? 2 : T;
     static_assert(4 * (kRouterStatusK + 64) * 4 <= kRouterShortLds && kRouterStatusK % 128 == 0);
-    const size_t lds = size_t(tt) * (K + 64) * 4;
-    if (T <= 64 && K % 128 == 0 && lds <= kRouterShortLds) {   // (two of its workgroups fit a compute unit's LDS)
-        const uint32_t threads = tt <= 2 ? 64 : 256, experts = threads / 16;
-        const dim3 grid((E + experts - 1) / experts + (gate_w ? 1 : 0), (T + tt - 1) / tt);
-#define ZC_ROUTER(TT) hipLaunchKernelGGL(router_short_kernel<TT>, grid, dim3(threads), lds, s, (const uint16_t*)w, x, T, K, E, offsets, out, gate_w, gate, status)
-        if (tt == 4) ZC_ROUTER(4); else if (tt == 2) ZC_ROUTER(2); else ZC_ROUTER(1);
+    if (T <= 64 && K % 128 == 0 && row_bytes(rows) <= kRouterShortLds) {   // (two of its workgroups fit a compute unit's LDS)
+        auto grid_of = [&](uint32_t waves) { return dim3((E + 4 * waves - 1) / (4 * waves) + (gate_w ? 1 : 0), (T + rows - 1) / rows); };
+        auto lds_of = [&](uint32_t waves) { return row_bytes(rows) + waves * 4 * (T == 1 ? 1 : 4) * 17 * 4; };
+        // Two waves spread the experts over more compute units, and stage the tokens' rows twice as often as four: while all workgroups
+        // are on the chip at once (512 experts, us with one, two and four waves: 8 tokens of 3072 inputs 9.3, 7.4, 9.0, 32 of 2048
+        // 12.7, 8.8, 10.6, 40 of 2560 21.4, 12.3, 13.7; 64 of 3072 24.7, 18.2, 15.9).
+        const dim3 two = grid_of(2);
+        const uint32_t waves = T == 1 ? 1 : two.x * two.y <= 256 * (160 * 1024 / lds_of(2)) ? 2 : 4;
+        const dim3 grid = grid_of(waves);
+        const size_t lds = lds_of(waves);
+#define ZC_ROUTER(TOKENS) hipLaunchKernelGGL(router_short_kernel<TOKENS>, grid, dim3(64 * waves), lds, s, (const uint16_t*)w, x, T, K, E, offsets, out, gate_w, gate, status, rows)
+        if (T == 1) ZC_ROUTER(1); else ZC_ROUTER(4);
 #undef ZC_ROUTER
         return;
     }
