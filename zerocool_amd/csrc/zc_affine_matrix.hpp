@@ -183,18 +183,25 @@ struct MatrixStream {
     uint32_t K, N, steps, lane, tile, end, step;             // tile, step: the next one to request
     AffineMatrix m[2];
     const uint8_t* meta[GATED ? 2 : 1];                      // this lane's array: scales or biases
-    uint32_t w_at[kRows], g_at[kRows];                       // byte offsets of this lane's blocks in the next step (a matrix has less than 4 GiB): one addition a step, no scalar work
-    __device__ __forceinline__ uint32_t block() const {      // this lane's first block in the next step (past the row's end: its last pair)
-        const uint32_t b = step * 32 + (lane >> 2) * 2;
-        return Form::kWhole ? b : min(b, K / WIDTH - 2);
+    // Byte offsets of this lane's blocks in the next step (a matrix has less than 4 GiB).  They move by one addition a step, the same in every lane.
+    // Rows of half a step more stop at the matrix's last load: past it are rows behind the last one, which are not stored, and the missing half
+    // of its last step; the missing halves of other rows read the row behind.  (Whole rows come eight at a time and never end inside a tile.)
+    uint32_t w_at[kRows], g_at[kRows];
+    __device__ __forceinline__ void move(uint32_t w, uint32_t g) {
+#pragma unroll
+        for (uint32_t i = 0; i < kRows; ++i) {
+            w_at[i] += w; g_at[i] += g;
+            if constexpr (!Form::kWhole) { w_at[i] = min(w_at[i], N * (K / 8 * BITS) - DW * 8); g_at[i] = min(g_at[i], N * (K / 64) * 2 - 2); }
+        }
     }
     __device__ __forceinline__ void aim() {
 #pragma unroll
         for (uint32_t i = 0; i < kRows; ++i) {
             const uint32_t r = min(tile * kTileRows + i * 4 + (lane & 3u), N - 1);
-            w_at[i] = r * (K / 8 * BITS) + block() * (DW * 4);
-            g_at[i] = (r * (K / 64) + block() * WIDTH / 64) * 2;
+            w_at[i] = r * (K / 8 * BITS) + (lane >> 2) * (DW * 8);
+            g_at[i] = (r * (K / 64) + (lane >> 2) * 2 * WIDTH / 64) * 2;
         }
+        move(0, 0);
     }
     __device__ __forceinline__ void fetch(Slot& slot) {      // past the end: the last tile again, not used
 #pragma unroll
@@ -207,12 +214,12 @@ struct MatrixStream {
             } else { const uint2 v = ldg_u2_by_words(a.w + w_at[i]); slot.q[q][0] = v.x; slot.q[q][1] = v.y; }
             slot.g[q] = ldg_u16(meta[GATED ? q : 0] + g_at[i]);
         }
-        if (++step == steps) { step = 0; tile = tile + kMatrixWaves < end ? tile + kMatrixWaves : tile; aim(); }
-        else if constexpr (!Form::kWhole) aim();
-        else {
-#pragma unroll
-            for (uint32_t i = 0; i < kRows; ++i) { w_at[i] += 32 * DW * 4; g_at[i] += Form::kStep / 64 * 2; }
-        }
+        constexpr uint32_t kW = 32 * DW * 4, kG = Form::kStep / 64 * 2;
+        if (++step < steps) { move(kW, kG); return; }
+        step = 0;
+        if (tile + kMatrixWaves >= end) return;
+        tile += kMatrixWaves;
+        move(kMatrixWaves * kTileRows * (K / 8 * BITS) - (steps - 1) * kW, kMatrixWaves * kTileRows * (K / 64) * 2 - (steps - 1) * kG);
     }
 };
 
@@ -222,11 +229,15 @@ __device__ __forceinline__ float high_bf16(uint32_t pair) { return __uint_as_flo
 
 // Four tokens' partial sums (register r: token r) over the lanes of equal (lane % 4), strides 16, 8, 4, 2 of the reference's lanes: every lane
 // ends with the sum of row lane % 4 for token {0, 2, 1, 3}[lane / 16].
+__device__ __forceinline__ float matrix_add_rows(float a, float b) {   // rows of sixteen lanes 0 and 2: a's rows 0 + 1, 2 + 3; rows 1 and 3: b's
+    const auto rows = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(rows[0]) + __uint_as_float(rows[1]);
+}
 __device__ __forceinline__ float matrix_reduce(f32x4 v) {
     auto swap_sum = [](auto rows) { return __uint_as_float(rows[0]) + __uint_as_float(rows[1]); };
     const float a = swap_sum(__builtin_amdgcn_permlane32_swap(__float_as_uint(v[0]), __float_as_uint(v[1]), false, false));
     const float b = swap_sum(__builtin_amdgcn_permlane32_swap(__float_as_uint(v[2]), __float_as_uint(v[3]), false, false));
-    float s = swap_sum(__builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false));
+    float s = matrix_add_rows(a, b);
     s = s + dpp_f32<0x128>(s);   // row_ror:8
     return s + dpp_f32<0x124>(s);   // row_ror:4
 }
@@ -337,20 +348,37 @@ __device__ __forceinline__ void matrix_walk(MatrixStream<BITS, WIDTH, GATED>& st
         }
         if (++step < st.steps) continue;
         step = 0;
-        // lane 4 b + j: row j, the second stream's if b is odd (plain); b / 4 the token
         float v[2];
+        uint32_t in_tile;                                  // lane 4 b + j: row j of the tile, or of its second four
+        bool mine = token < nt;                            // (one lane of each result)
+        if constexpr (TOKENS <= 2) {                       // halves and streams take the places of four tokens in the sums (rows of a step or two are mostly their end: with
+                                                           // this and offsets that move by an addition 40 tokens' down of 640 inputs 111 -> 104 us, 32 tokens' of 512 47 -> 45)
+            float s[TOKENS];
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            f32x4 first = zero, second = zero;
+            for (uint32_t t = 0; t < TOKENS; ++t) s[t] = matrix_reduce(f32x4{acc[0][0][t], acc[1][0][t], acc[0][1][t], acc[1][1][t]});
+            v[0] = v[1] = matrix_add_rows(s[0], s[TOKENS - 1]);   // lanes from 32 on: the second stream's; odd rows of lanes: token 1's
+            in_tile = (lane & 3u) + (GATED ? 0u : lane >> 5 << 2);
+            mine = mine && !(lane & (GATED ? 44u : 12u));
+            if constexpr (GATED) {
+                const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[0]), __float_as_uint(v[0]), false, false);
+                v[0] = __uint_as_float(both[0]); v[1] = __uint_as_float(both[1]);
+            }
+        } else {                                           // the second four where b is odd; b / 4 the token
 #pragma unroll
-            for (uint32_t r = 0; r < TOKENS; ++r) { first[r] = acc[q][0][r]; second[r] = acc[q][1][r]; }
-            v[q] = matrix_reduce(first) + matrix_reduce(second);
+            for (int q = 0; q < 2; ++q) {
+                f32x4 first, second;
+#pragma unroll
+                for (uint32_t r = 0; r < TOKENS; ++r) { first[r] = acc[q][0][r]; second[r] = acc[q][1][r]; }
+                v[q] = matrix_reduce(first) + matrix_reduce(second);
+            }
+            in_tile = lane & (GATED ? 3u : 7u);
+            mine = mine && !(lane & (GATED ? 12u : 8u));
+            if (!GATED && (lane & 4u)) v[0] = v[1];
         }
         clear();
-        if (!GATED && (lane & 4u)) v[0] = v[1];
         const float y = GATED ? swiglu_bf(v[0], v[1]) : float_output ? v[0] : bf(v[0]);
-        const uint32_t row = tile * Stream::kTileRows + (GATED ? lane & 3u : lane & 7u);
-        const bool mine = !(lane & (GATED ? 12u : 8u)) && token < nt && row < st.N;
+        const uint32_t row = tile * Stream::kTileRows + in_tile;
+        mine = mine && row < st.N;
         if constexpr (IMAGE) {   // the wave's four outputs of a token are a quad
             const uint32_t quad[4] = {__float_as_uint(dpp_f32<0x00>(y)), __float_as_uint(dpp_f32<0x55>(y)), __float_as_uint(dpp_f32<0xaa>(y)), __float_as_uint(dpp_f32<0xff>(y))};
             const MatrixQuad put = matrix_quad(quad);
@@ -421,7 +449,7 @@ __device__ __forceinline__ void matrix_rows(const AffineMatrix (&m)[2], uint32_t
     typename Stream::Slot next;
     st.aim();
     st.fetch(next);
-    const uint32_t row16 = st.lane >> 4, token = row16 == 1 ? 2u : row16 == 2 ? 1u : row16;   // as matrix_reduce leaves them
+    const uint32_t row16 = st.lane >> 4, token = nt <= 2 ? row16 & 1u : row16 == 1 ? 2u : row16 == 2 ? 1u : row16;   // as the sums are left
     const uint64_t out_at = uint64_t(out_row(min(token, nt - 1))) * N;
     uint32_t* found = reinterpret_cast<uint32_t*>(lds + Form::found_at(K));
     const bool any = __ballot(matrix_stage<BITS, WIDTH, IN>(x, K, nt, from, lds)) != 0;
