@@ -57,3 +57,24 @@ def test_a_token_without_picks_is_reported(ctx, topk):
     assert (bufs["ids"].numpy(np.int32) == -1).all()
     run(ctx, cfg, w, oracle.bf(np.ones((1, 512), f32)))
     ctx.moe_check()                              # reported once
+
+
+# One token: by the one-token kernel, except where a stack has a single layer or Q8 parts; the same bytes and the same reports either way.
+@pytest.mark.parametrize("layers,bits,single", [(1, (4, 4, 4, 4), False), (2, (4, 4, 4, 4), True), (2, (4, 8, 8, 8), False), (2, (4, 4, 8, 4), False)])
+def test_which_way_a_stack_goes(ctx, layers, bits, single):
+    cfg = workload.tiny_config(hidden=1024, experts=64, topk=10, inter=512, bits=bits)
+    ws = [workload.LayerWeights(ctx, cfg, 300 + l, ("zipf", 1.1)) for l in range(layers)]
+    stack = ctx.stack_create(cfg, [w.layer for w in ws], 1)
+    assert ctx.stack_is_persistent(stack, 1) and ctx.stack_single_launch(stack, 1) == single
+    x, outs = workload.hidden_rows(ctx, 1, cfg.hidden, 5), []
+    for how in ({}, {"single": True}, {"layered": True}):
+        out = ctx.alloc(cfg.hidden * 4)
+        ctx.stack_decode(stack, x, 1, out, **how)
+        ctx.moe_check()
+        outs.append(out.numpy(f32).tobytes())
+    assert outs[0] == outs[1] == outs[2]
+    bad = np.full(cfg.hidden, 0.5, f32); bad[7] = f32(1 + 2.0 ** -20)
+    ctx.stack_decode(stack, ctx.upload(bad), 1, ctx.alloc(cfg.hidden * 4))
+    with pytest.raises(z.ZcError, match="not BF16-valued"):
+        ctx.moe_check()
+    ctx.stack_destroy(stack)

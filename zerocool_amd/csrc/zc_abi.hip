@@ -1111,17 +1111,21 @@ static zc_status launch_piece(zc_hip_ctx* ctx, zc_hip_stack* st, const float* x,
     }
     return ZC_OK;
 }
-// Whether a batch that a single launch could take goes layer by layer, five launches each: from two tokens on.  us per layer, single
+// Whether a batch that a single launch could take goes layer by layer, four to six launches each: from two tokens on.  us per layer, single
 // launch -> layer by layer, at 2, 8, 32 and 64 tokens, one layer with N(0, 0.5) offsets / six layers with Zipf(1.1) offsets, whose
 // tokens agree on nearly all experts behind the first layer:
-//   hidden 2048, Q4        50 -> 39   93 -> 69   194 -> 128   313 -> 185  /  38 -> 36   63 -> 48   144 -> 80    222 -> 120
-//   hidden 2048, mixed     60 -> 50  112 -> 82   272 -> 152   449 -> 216  /  50 -> 45  102 -> 62   212 -> 98    360 -> 146
-//   hidden 3072, Q4        80 -> 65  187 -> 128  456 -> 291   743 -> 461  /  52 -> 53   97 -> 77   259 -> 150   437 -> 245
-// One token stays with its kernel (30 -> 30, 36 -> 36, 39 -> 43 / 22 -> 30, 33 -> 37, 28 -> 45): nothing to share, and no launch
-// between the layers.
+//   hidden 2048, Q4        51 -> 37   94 -> 65   194 -> 124   312 -> 182  /  38 -> 34   62 -> 46   144 -> 77    222 -> 117
+//   hidden 2048, mixed     60 -> 39  110 -> 74   277 -> 156   447 -> 235  /  50 -> 37  101 -> 52   212 -> 96    360 -> 158
+//   hidden 3072, Q4        76 -> 59  186 -> 125  462 -> 299   746 -> 464  /  53 -> 51   97 -> 73   259 -> 146   436 -> 243
+// One token of all-Q4 layers stays with its kernel, which has no launch between the layers and starts on the previous step's experts: two
+// layers 28 -> 24 and 33 -> 36, six layers 23 -> 24 and 29 -> 38, sixteen 22.5 -> 25.7.  A stack of one layer has nothing between layers to
+// gain from: 31 -> 24 and 38 -> 34.  That kernel's Q8 rows are walked a row at a time: one, two, six and sixteen mixed layers of hidden 2048
+// 37 -> 24, 35 -> 25, 33 -> 25, 37 -> 27, Q8 only in the shared expert 33 -> 24, 30 -> 24, 29 -> 24; of hidden 3072 69 -> 40, 61 -> 37, 68 -> 41,
+// 66 -> 41, and 48 -> 37, 43 -> 35, 42 -> 38.
 // (Above sixty-four tokens the rule says nothing: the inputs' check for BF16 values is the short router's, which ends there.)
 static bool layers_preferred(const zc_hip_stack* st, uint32_t tokens) {
-    return tokens >= 2 && tokens <= 64 && !st->store && st->wait_limit == kWaitPolls;
+    if (tokens > 64 || st->store || st->wait_limit != kWaitPolls) return false;
+    return tokens > 1 || st->layers.size() == 1 || !all_q4(st->cfg);
 }
 zc_status zc_hip_stack_set_wait_limit(zc_hip_ctx* ctx, zc_hip_stack* st, uint32_t polls) {
     ZC_REQUIRE(ctx && st, "null argument");
