@@ -208,9 +208,9 @@ zc_status zc_hip_moe_check(zc_hip_ctx* ctx);
  * Up to 64 tokens can run as ONE persistent kernel launch for the whole stack (routing,
  * dispatch and combine stay on the device, no host synchronisation between layers; one
  * kernel each for one token, two to eight, and nine to sixty-four), larger batches as
- * one such launch per 64 tokens.  One token does; two to sixty-four go layer by layer (five
- * launches each) where that is faster, as do shapes those kernels do not take.  All give
- * identical bytes.
+ * one such launch per 64 tokens.  One token of all-Q4 stacks of two layers and more does; other
+ * stacks and two to sixty-four tokens go layer by layer (four to six launches each), which is
+ * faster, as do shapes those kernels do not take.  All give identical bytes.
  * out: [tokens][hidden], the last layer's output.  flags bit 0: force the layer-by-layer path;
  * bit 1: the single launch where its kernels take the batch, also where layer by layer is faster. */
 typedef struct zc_hip_stack zc_hip_stack;
