@@ -21,8 +21,8 @@
 // eight, scale and bias in one load (lanes of b and b + 1 share a group: one takes the scale, the other the bias); 32 tokens of
 // hidden 2048, 512 experts: gate/up 96 -> 62 us, down 53 -> 47.  Workgroups that take a contiguous share of the work list instead of a grid over
 // all jobs there could be: 64 tokens of hidden 3072 that agree on eleven experts 157 -> 125 us.
-// Two tokens a workgroup on the lanes of zc_affine.hpp -> this, gate/up and down, us: hidden 2560, 40 tokens 154 and 124 -> 104 and 109; hidden 2048, 32 tokens
-// 80 and 51 -> 62 and 47; hidden 3072, 64 tokens that agree 290 and 140 -> 136 and 74.  Eight tokens a workgroup (half the conversions, twice the accumulators: two
+// Two tokens a workgroup on the lanes of zc_affine.hpp -> this, gate/up and down, us: hidden 2560, 40 tokens 154 and 124 -> 104 and 105; hidden 2048, 32 tokens
+// 80 and 51 -> 62 and 46; hidden 3072, 64 tokens that agree 290 and 140 -> 136 and 74.  Eight tokens a workgroup (half the conversions, twice the accumulators: two
 // waves a SIMD) took 121 and 75 for the last, but 83 and 78 for 32 tokens of hidden 2048, most of whose experts have one token or two.
 #pragma once
 #include "zc_affine.hpp"
