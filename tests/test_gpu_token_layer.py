@@ -31,7 +31,8 @@ def run(ctx, cfg, w, x):
 # rows of either width, groups of 32, Q8, a shared expert of another format (a launch without routed jobs)
 @pytest.mark.parametrize("hidden,inter,experts,topk,bits,group", [
     (128, 128, 1, 1, (4, 4, 4, 4), 64), (512, 640, 3, 3, (4, 4, 4, 4), 64), (512, 512, 64, 63, (4, 4, 4, 4), 64), (512, 128, 66, 64, (4, 8, 8, 8), 64),
-    (512, 128, 66, 65, (4, 8, 8, 8), 64), (640, 128, 512, 10, (8, 8, 4, 4), 64), (256, 128, 513, 10, (8, 4, 4, 8), 32), (128, 64, 1024, 64, (4, 4, 4, 4), 64)])
+    (512, 128, 66, 65, (4, 8, 8, 8), 64), (640, 128, 512, 10, (8, 8, 4, 4), 64), (256, 128, 513, 10, (8, 4, 4, 8), 32), (128, 64, 1024, 64, (4, 4, 4, 4), 64),
+    (32512, 64, 3, 2, (4, 4, 4, 4), 64), (32576, 64, 3, 2, (4, 4, 4, 4), 64)])   # the longest row beside which the selection has room in LDS, and one more
 def test_layer(ctx, hidden, inter, experts, topk, bits, group):
     cfg = workload.tiny_config(hidden=hidden, experts=experts, topk=topk, inter=inter, bits=bits, group=group)
     w = workload.LayerWeights(ctx, cfg, 500 + topk, ("normal", 0.5))
