@@ -41,7 +41,13 @@ def rows(kind, T, K, seed):
 @pytest.mark.parametrize("bits,K,N,T,kind", [
     (4, 512, 8, 133, "normal"), (4, 1024, 24, 131, "spread"), (4, 512, 40, 130, "edge"), (4, 1536, 8, 129, "powers"), (4, 512, 16, 132, "far"),
     (4, 512, 8, 130, "strange"), (4, 640, 24, 133, "normal"), (4, 128, 8, 131, "spread"), (4, 384, 12, 130, "edge"), (4, 512, 7, 129, "powers"),
-    (4, 640, 8, 130, "strange"), (8, 512, 8, 133, "normal"), (8, 1024, 24, 131, "spread"), (8, 512, 40, 130, "powers"), (8, 512, 16, 129, "strange")])
+    (4, 640, 8, 130, "strange"), (8, 512, 8, 133, "normal"), (8, 1024, 24, 131, "spread"), (8, 512, 40, 130, "powers"), (8, 512, 16, 129, "strange"),
+    # either side of the numbers of rows from which the two products go to the matrix cores
+    (4, 512, 24, 47, "strange"), (4, 512, 24, 48, "strange"), (4, 640, 24, 127, "edge"), (4, 640, 24, 128, "edge"), (8, 512, 24, 47, "spread"), (8, 512, 24, 48, "spread"),
+    # the longest rows of each format whose four tokens leave room for two workgroups, and one step more; rows that are not BF16
+    # one at a time (5632 and 8704 inputs) and two
+    (4, 8704, 8, 129, "strange"), (4, 8704, 8, 50, "edge"), (4, 9216, 8, 129, "strange"), (4, 7936, 8, 129, "strange"), (4, 7936, 8, 51, "edge"), (4, 8064, 8, 129, "strange"),
+    (8, 7680, 8, 129, "strange"), (8, 8192, 8, 129, "strange"), (4, 4096, 8, 129, "strange"), (4, 4224, 8, 129, "strange"), (4, 5120, 8, 129, "strange"), (4, 5632, 8, 129, "strange")])
 def test_operators(ctx, bits, K, N, T, kind):
     rng = np.random.default_rng(K + N + T)
     mats = []
@@ -64,7 +70,10 @@ def test_operators(ctx, bits, K, N, T, kind):
 @pytest.mark.parametrize("T,hidden,inter,experts,topk,bits,kind", [
     (2, 512, 512, 8, 4, (4, 4, 4, 4), "normal"), (3, 1024, 128, 3, 3, (4, 4, 4, 4), "spread"), (7, 640, 640, 4, 2, (4, 4, 4, 4), "edge"),
     (11, 512, 512, 5, 3, (4, 8, 8, 8), "normal"), (6, 512, 512, 6, 6, (8, 4, 4, 8), "powers"), (9, 512, 640, 3, 1, (4, 4, 4, 4), "strange"),
-    (66, 512, 512, 6, 2, (4, 4, 4, 4), "spread"), (520, 512, 128, 3, 2, (4, 4, 4, 4), "normal")])
+    (66, 512, 512, 6, 2, (4, 4, 4, 4), "spread"), (520, 512, 128, 3, 2, (4, 4, 4, 4), "normal"),
+    # the longest rows and one step more (then both phases are the lanes'), rows of either form's own width, and lists of jobs with one to four tokens
+    (7, 8704, 512, 3, 2, (4, 4, 4, 4), "strange"), (7, 9216, 512, 3, 2, (4, 4, 4, 4), "strange"), (9, 512, 8704, 3, 2, (4, 4, 4, 4), "normal"),
+    (33, 1024, 640, 24, 3, (4, 4, 4, 4), "strange"), (37, 1536, 512, 40, 4, (4, 8, 8, 8), "strange"), (70, 512, 512, 64, 4, (8, 8, 8, 8), "strange")])
 def test_layer(ctx, T, hidden, inter, experts, topk, bits, kind):
     cfg = workload.tiny_config(hidden=hidden, experts=experts, topk=topk, inter=inter, bits=bits)
     w = workload.LayerWeights(ctx, cfg, 900 + T, ("normal", 0.5))

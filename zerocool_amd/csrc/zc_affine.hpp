@@ -170,13 +170,13 @@ __device__ __forceinline__ float affine_sum(const float* x) {
     return sum;
 }
 
-// The walk for nt staged tokens; out_at: where the output row of token (lane % TOKENS) begins in `out`.
+// The walk for nt staged tokens; out_at: where the output row of token (lane % TOKENS) begins; put(out_at, row, y) stores.
 // (nt and exact are the same in every lane.  As template parameters they made eight walks, whose common first steps the
 // compiler moved in front of the choice between them: 200 registers.)
-template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS>
+template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS, class Put>
 __device__ __forceinline__ void affine_walk(AffineStream<BITS, WIDTH, GATED, TOKENS>& st,
                                             typename AffineStream<BITS, WIDTH, GATED, TOKENS>::Slot (&ring)[AffineStream<BITS, WIDTH, GATED, TOKENS>::kAhead],
-                                            const uint8_t* lds, uint64_t out_at, uint32_t tile, bool float_output, uint32_t nt, bool exact, float* out) {
+                                            const uint8_t* lds, uint64_t out_at, uint32_t tile, bool float_output, uint32_t nt, bool exact, Put put) {
     using Stream = AffineStream<BITS, WIDTH, GATED, TOKENS>;
     constexpr int S = Stream::kStreams;
     const uint32_t blocks = st.blocks, token = affine_token_bytes<WIDTH>(st.K), lane = st.lane;
@@ -237,7 +237,7 @@ __device__ __forceinline__ void affine_walk(AffineStream<BITS, WIDTH, GATED, TOK
             }
             const uint32_t row = st.row(tile, lane / TOKENS);
             const float y = GATED ? swiglu_bf(v[0], v[1]) : float_output ? v[0] : bf(v[0]);
-            if (lane < Stream::kRows * TOKENS && lane % TOKENS < nt && row < st.N) out[out_at + row] = y;
+            if (lane < Stream::kRows * TOKENS && lane % TOKENS < nt && row < st.N) put(out_at, row, y);
 #pragma unroll
             for (uint32_t t = 0; t < TOKENS; ++t)
 #pragma unroll
@@ -248,14 +248,14 @@ __device__ __forceinline__ void affine_walk(AffineStream<BITS, WIDTH, GATED, TOK
 }
 
 // Rows tile0 .. end - 1 (tiles) of the matrices for nt <= TOKENS tokens, by 256 threads: input row in_row(t), output row out_row(t).
+// load(row, i): the four elements from 4 i on of an input row; put(at, row, y): stores y as element `row` of the output row that begins at `at`.
 // choice, optional: what the matrices depend on is found while the input rows are staged.  choice.find() runs in front of the staging
 // and choice.take(matrices) behind the workgroup's barrier; false: there is nothing to do.
 struct AffineKnown {};
-template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS, class InRow, class OutRow, class Choice = AffineKnown>
-__device__ __forceinline__ void affine_rows(const AffineMatrix (&m)[2], uint32_t K, uint32_t N, uint32_t group, const float* x, float* out, uint32_t nt,
-                                            InRow in_row, OutRow out_row, uint32_t tile0, uint32_t end, bool float_output, uint8_t* lds, Choice choice = {}) {
+template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS, class Load, class Put, class InRow, class OutRow, class Choice = AffineKnown>
+__device__ __forceinline__ void affine_rows_by(const AffineMatrix (&m)[2], uint32_t K, uint32_t N, uint32_t group, Load load, Put put, uint32_t nt,
+                                               InRow in_row, OutRow out_row, uint32_t tile0, uint32_t end, bool float_output, uint8_t* lds, uint32_t tid, Choice choice = {}) {
     constexpr bool kKnown = std::is_same_v<Choice, AffineKnown>;
-    const uint32_t tid = threadIdx.x;
     using Stream = AffineStream<BITS, WIDTH, GATED, TOKENS>;
     Stream st;
     st.K = K; st.N = N; st.blocks = K / WIDTH; st.shift = group == 64 ? 6 : 5; st.groups = K >> st.shift; st.steps = (st.blocks + 31) / 32;
@@ -279,7 +279,7 @@ __device__ __forceinline__ void affine_rows(const AffineMatrix (&m)[2], uint32_t
         const uint32_t src = uint32_t(__builtin_amdgcn_readlane(int(from), int(t)));
 #pragma unroll 2
         for (uint32_t i = tid; i < K / 4; i += 256) {
-            const uint4 q = ldg_u4(x + uint64_t(src) * K, i);
+            const uint4 q = load(src, i);
             const uint32_t v[4] = {q.x, q.y, q.z, q.w};
             uint32_t* to = reinterpret_cast<uint32_t*>(lds + t * token + i / kPieces * AffineBlock<WIDTH>::kBytes + i % kPieces * 16);
 #pragma unroll
@@ -329,6 +329,13 @@ __device__ __forceinline__ void affine_rows(const AffineMatrix (&m)[2], uint32_t
         for (uint32_t w = 0; w < 4; ++w) found |= *finding(w);
     }
     const bool exact = __builtin_amdgcn_readfirstlane(int(found)) == 0;
-    affine_walk<BITS, WIDTH, GATED, TOKENS>(st, ring, lds, out_at, tile0, float_output, nt, exact, out);
+    affine_walk<BITS, WIDTH, GATED, TOKENS>(st, ring, lds, out_at, tile0, float_output, nt, exact, put);
+}
+// The same for fp32 rows of x and out.
+template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS, class InRow, class OutRow, class Choice = AffineKnown>
+__device__ __forceinline__ void affine_rows(const AffineMatrix (&m)[2], uint32_t K, uint32_t N, uint32_t group, const float* x, float* out, uint32_t nt,
+                                            InRow in_row, OutRow out_row, uint32_t tile0, uint32_t end, bool float_output, uint8_t* lds, Choice choice = {}) {
+    affine_rows_by<BITS, WIDTH, GATED, TOKENS>(m, K, N, group, [=](uint32_t row, uint32_t i) { return ldg_u4(x + uint64_t(row) * K, i); },
+                                               [=](uint64_t at, uint32_t row, float y) { out[at + row] = y; }, nt, in_row, out_row, tile0, end, float_output, lds, threadIdx.x, choice);
 }
 }  // namespace zc

@@ -47,10 +47,15 @@ struct MatrixForm {
     __host__ __device__ static constexpr uint32_t bits_at(uint32_t K) { return steps(K) * 2 * (kHalfBytes + 256); }
     __host__ __device__ static constexpr uint32_t found_at(uint32_t K) { return bits_at(K) + kMatrixTokens * kMatrixSteps; }
 };
+template <int BITS, int WIDTH> __host__ __device__ constexpr uint32_t matrix_staged_bytes(uint32_t K) { return MatrixForm<BITS, WIDTH>::found_at(K) + 4 * kMatrixWaves; }
+// Workgroups of a compute unit: by LDS, and four waves a SIMD by registers.
+__host__ __device__ constexpr uint32_t matrix_per_cu(uint32_t lds) { return 160 * 1024 / lds < 4 ? 160 * 1024 / lds : 4; }
+// The rows whose products may round take turns in the same memory as the lanes stage them: two tokens at a time where room for them (a ninth
+// more) costs no workgroup of a compute unit, else one.
 template <int BITS, int WIDTH>
-constexpr uint32_t matrix_lds_bytes(uint32_t K) {   // (the way of strange rows needs one row as the lanes stage it)
-    const uint32_t staged = MatrixForm<BITS, WIDTH>::found_at(K) + 4 * kMatrixWaves, lanes = affine_token_bytes<WIDTH>(K);
-    return staged > lanes ? staged : lanes;
+__host__ __device__ constexpr uint32_t matrix_lds_bytes(uint32_t K) {
+    const uint32_t staged = matrix_staged_bytes<BITS, WIDTH>(K), two = 2 * affine_token_bytes<WIDTH>(K);
+    return two > staged && two <= 160 * 1024 && matrix_per_cu(two) == matrix_per_cu(staged) ? two : staged;
 }
 
 // Where token i's piece of block b stands among a half step's 64 sixteen-byte pieces: reads take blocks of all four tokens side by side, writes
@@ -388,51 +393,27 @@ __device__ __forceinline__ void matrix_walk(MatrixStream<BITS, WIDTH, GATED>& st
     }
 }
 
-// Output rows first .. last - 1 for rows whose products may round: a half wave plays the reference's lanes of one row, a token at a time.
-// (Inputs are BF16 by contract; this is the way of all others, and short on registers, which the kernel's waves have in common.)
-template <int BITS, int WIDTH, bool GATED, class InRow, class OutRow, class Load, class Put>
-__device__ __forceinline__ void matrix_strange_rows(const AffineMatrix (&m)[2], uint32_t K, uint32_t N, uint32_t nt, InRow in_row, OutRow out_row,
-                                                    uint32_t first, uint32_t last, bool float_output, uint8_t* lds, Load load, Put put) {
-    constexpr uint32_t DW = WIDTH * BITS / 32, kBytes = AffineBlock<WIDTH>::kBytes;
-    const uint32_t tid = matrix_thread(), lane = tid & 31u, blocks = K / WIDTH;
+// Output rows first .. last - 1 of a job where a token's products may round: on the lanes (zc_affine.hpp), two tokens at a time.  Inputs are BF16 by
+// contract; rows that are not cost more here than by the lanes' own kernels, since the work list is cut as if all jobs took the same time, and a job
+// of four tokens is two turns.  us, a row at a time with nothing requested ahead -> this (the lanes' kernels): layers whose rows are all fp32, 8 tokens of
+// hidden 2048 145 -> 95 (70), 64 of 2048 659 -> 382 (276), 64 of 3072 2087 -> 1026 (684); gate/up 3072 x 1024 at 128 and 512 rows 163 -> 107 (82) and
+// 602 -> 343 (292), with one such row among them 97 -> 48 (58) and 357 -> 149 (202).
+template <int BITS, int WIDTH, bool GATED, class Load, class Put, class InRow, class OutRow>
+__device__ __forceinline__ void matrix_strange_rows(const AffineMatrix (&m)[2], uint32_t K, uint32_t N, Load load, Put put, uint32_t nt, InRow in_row, OutRow out_row,
+                                                    uint32_t first, uint32_t last, bool float_output, uint8_t* lds) {
+    constexpr uint32_t kRows = AffineStream<BITS, WIDTH, GATED, kAffineTokens>::kTileRows;
+    static_assert(kMatrixWaves * MatrixStream<BITS, WIDTH, GATED>::kTileRows % kRows == 0);   // a workgroup's range is whole tiles of either form
+    const uint32_t most = kAffineTokens * affine_token_bytes<WIDTH>(K) <= matrix_lds_bytes<BITS, WIDTH>(K) ? kAffineTokens : 1u;
 #pragma unroll 1
-    for (uint32_t t = 0; t < nt; ++t) {
+    for (uint32_t t0 = 0; t0 < nt; t0 += most) {
         lds_barrier();   // what was staged before has been read
-        const uint32_t from = uint32_t(uniform(int32_t(in_row(t))));
-#pragma unroll 1
-        for (uint32_t i = tid; i < K / 4; i += kMatrixThreads) {
-            const uint4 v = load(from, i);
-            uint32_t* to = reinterpret_cast<uint32_t*>(lds + i / (WIDTH / 4) * kBytes + i % (WIDTH / 4) * 16);
-            to[0] = v.x; to[1] = v.y; to[2] = v.z; to[3] = v.w;
-        }
-        lds_barrier();
-        const uint64_t out_at = uint64_t(out_row(t)) * N;
-#pragma unroll 1
-        for (uint32_t row = first + tid / 32; row < last; row += kMatrixThreads / 32) {
-            float r[2] = {0, 0};
-#pragma unroll 1
-            for (uint32_t b = lane; b < blocks; b += 32) {
-                float x[WIDTH];
-#pragma unroll
-                for (int i = 0; i < WIDTH; ++i) x[i] = *reinterpret_cast<const float*>(lds + b * kBytes + 4 * i);
-                const float sum = affine_sum<BITS, WIDTH>(x);
-#pragma unroll
-                for (int q = 0; q < (GATED ? 2 : 1); ++q) {
-                    uint32_t words[DW];
-#pragma unroll
-                    for (uint32_t i = 0; i < DW; ++i) words[i] = ldg_u32(m[q].w + (uint64_t(row) * blocks + b) * (DW * 4), i);
-                    const uint64_t g = uint64_t(row) * (K / 64) + b * WIDTH / 64;
-                    r[q] = r[q] + (b16(ldg_u16(m[q].s + g)) * affine_dot_any<BITS, WIDTH>(words, x) + sum * b16(ldg_u16(m[q].b + g)));
-                }
-            }
-            const float v = lane_sum32(r[0]), u = GATED ? lane_sum32(r[1]) : 0.0f, y = GATED ? swiglu_bf(v, u) : float_output ? v : bf(v);
-            if (lane == 0) put(out_at, row, y);
-        }
+        affine_rows_by<BITS, WIDTH, GATED, kAffineTokens>(m, K, N, 64, load, put, min(most, nt - t0), [&](uint32_t t) { return in_row(t0 + t); },
+                                                          [&](uint32_t t) { return out_row(t0 + t); }, first / kRows, (last + kRows - 1) / kRows, float_output, lds, matrix_thread());
     }
 }
 
 // Tiles tile0 .. end - 1 (of MatrixStream) for nt <= 4 tokens: input row in_row(t), output row out_row(t).
-// IN: input rows are images (fp32, if not null: the rows they were made of); OUT: output rows are to be.
+// IN: input rows are images (gate/up: made of the rows `fp32`; else written as images); OUT: output rows are to be.
 // (A workgroup that runs several of them waits in front of each: what the one before staged has then been read.)
 template <int BITS, int WIDTH, bool GATED, bool IN, bool OUT, class InRow, class OutRow>
 __device__ __forceinline__ void matrix_rows(const AffineMatrix (&m)[2], uint32_t K, uint32_t N, const float* x, const float* fp32, float* out, uint32_t nt,
@@ -467,16 +448,17 @@ __device__ __forceinline__ void matrix_rows(const AffineMatrix (&m)[2], uint32_t
         else walk.template operator()<4>();
         return;
     }
-    matrix_strange_rows<BITS, WIDTH, GATED>(m, K, N, nt, in_row, out_row, tile0 * Stream::kTileRows, min(end * Stream::kTileRows, N), float_output, lds,
-                                            [&](uint32_t row, uint32_t i) {
+    matrix_strange_rows<BITS, WIDTH, GATED>(m, K, N, [&](uint32_t row, uint32_t i) {
         if constexpr (!IN) return ldg_u4(x + uint64_t(row) * K, i);
-        else if (fp32) return ldg_u4(fp32 + uint64_t(row) * K, i);
-        const uint2 pairs = ldg_u2(x + uint64_t(row) * K, i);   // (rows that were made as images are BF16)
-        return make_uint4(pairs.x << 16, pairs.y << 16, pairs.x & 0xffff0000u, pairs.y & 0xffff0000u);
+        else if constexpr (GATED) return ldg_u4(fp32 + uint64_t(row) * K, i);
+        else {   // (rows that were made as images are BF16)
+            const uint2 pairs = ldg_u2(x + uint64_t(row) * K, i);
+            return make_uint4(pairs.x << 16, pairs.y << 16, pairs.x & 0xffff0000u, pairs.y & 0xffff0000u);
+        }
     }, [&](uint64_t at, uint32_t row, float y) {
         if constexpr (OUT) reinterpret_cast<uint16_t*>(out + at)[row / 4 * 4 + (row & 1u) * 2 + (row >> 1 & 1u)] = uint16_t(__float_as_uint(y) >> 16);
         else out[at + row] = y;
-    });
+    }, nt, in_row, out_row, tile0 * Stream::kTileRows, min(end * Stream::kTileRows, N), float_output, lds);
     if constexpr (OUT) {   // the information words, from the pairs that the workgroup has just stored
         __syncthreads();
         const uint32_t first = tile0 * Stream::kTileRows / 4, quads = min(end * Stream::kTileRows, N) / 4 - first;

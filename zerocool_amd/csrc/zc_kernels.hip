@@ -51,7 +51,7 @@ struct ExpertPhase {
     const uint8_t* shared_record; uint64_t shared_off[6];
     const uint32_t *jobs; const int32_t *count, *slots;
     const float *x, *shared_x; float *out, *shared_out;                // x: layer input (gate/up) or sorted activations (down); on the matrix cores both as row images
-    const float* fp32;                                                 // matrix cores: the rows that x and shared_x were made of, null where they were made as images
+    const float* fp32;                                                 // matrix cores, gate/up: the rows that the images x and shared_x were made of
     const float* logits; int32_t *ids, *status; float* weights; uint32_t E;   // of one token alone: job j of the routed ones is its pick j
     uint32_t K, N, group, topk, tokens, chunk, shared_jobs, max_jobs, tiles, share;   // chunk: tokens of a job (a shared job too)
 };
@@ -196,11 +196,11 @@ template <int WIDTH> static uint32_t affine_chunk(uint32_t K) {
 // four tokens' rows that leave room for two workgroups on a compute unit, and offsets in the codes of 32 bits.
 template <int BITS, int WIDTH> static bool matrix_fits(uint32_t K, uint32_t N, uint32_t group) {
     if constexpr (BITS == 8 && WIDTH == 4) return false;
-    else return group == 64 && uint64_t(K) * N / 8 * BITS < 1ull << 32 && K % (16 * WIDTH) == 0 && MatrixForm<BITS, WIDTH>::steps(K) <= kMatrixSteps && matrix_lds_bytes<BITS, WIDTH>(K) <= 80 * 1024;
+    else return group == 64 && uint64_t(K) * N / 8 * BITS < 1ull << 32 && K % (16 * WIDTH) == 0 && MatrixForm<BITS, WIDTH>::steps(K) <= kMatrixSteps && matrix_staged_bytes<BITS, WIDTH>(K) <= 80 * 1024;
 }
 // Workgroups of a launch: as many as fit the chip at once (LDS, and four waves a SIMD by registers), not more than there can be rounds.
 static uint32_t matrix_grid(uint32_t lds, uint32_t tiles, uint64_t jobs) {
-    return uint32_t(std::min<uint64_t>(256 * std::min(160u * 1024 / lds, 4u), (tiles + kMatrixWaves - 1) / kMatrixWaves * jobs));
+    return uint32_t(std::min<uint64_t>(256 * matrix_per_cu(lds), (tiles + kMatrixWaves - 1) / kMatrixWaves * jobs));
 }
 uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t group, uint32_t bits) {
     uint32_t chunk = 1;

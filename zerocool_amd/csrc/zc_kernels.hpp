@@ -31,7 +31,7 @@ struct ExpertPhaseDesc {
     uint64_t off[6];             // w,s,b of the first matrix, then of the second (gate/up phase)
     const void* shared_record; uint64_t shared_off[6];
     const uint32_t* jobs; const int32_t *count, *slots;   // launch_route_jobs
-    const float *x, *shared_x; float *out, *shared_out;   // chunk > 2: x, shared_x and gate/up's out are images; fp32: what x's were made of, or null
+    const float *x, *shared_x; float *out, *shared_out;   // chunk > 2: x, shared_x and gate/up's out are images; fp32 (gate/up): what x's were made of
     const float* fp32;
     // one token alone: its picks instead of a job list; the gate/up phase makes them from the logits where expert_phase_routes
     const float* logits; int32_t *ids, *status; float* weights; uint32_t E;
