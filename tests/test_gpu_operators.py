@@ -169,6 +169,19 @@ def test_router_random_with_offsets(ctx, H, E, T):
     assert same_bytes(got, oracle.router_logits(w, x, T, H, E, off))
 
 
+# rows whose every logit, or every lane's first one, is the same number, whatever the number
+@pytest.mark.parametrize("E", [505, 512, 1024])
+def test_route_equal_logits(ctx, E):
+    v = np.stack([np.full(E, c, f32) for c in (12345.678, -12345.678, 0.0, 3e38)])
+    first = np.linspace(-1, 1, E).astype(f32)
+    first[::8 if E <= 512 else E // 64] = f32(12345.678)
+    v = np.concatenate([v, first[None]])
+    for k in (1, 10, 64, 65):
+        ids, w = ctx.route(ctx.upload(v), len(v), E, k)
+        oi, ow = oracle.route(v, len(v), E, k)
+        assert same_bytes(ids.numpy(np.int32), oi) and same_bytes(w.numpy(f32), ow), k
+
+
 def test_route_stress_rows(ctx):  # :744-797
     v = route_stress_values()
     T = v.shape[0]

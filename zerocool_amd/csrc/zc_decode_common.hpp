@@ -223,7 +223,8 @@ __device__ __forceinline__ void route_token(Fetch fetch, uint32_t E, uint32_t to
 #pragma unroll
     for (int i = 0; i < PER; ++i) cand[i] = cand[i] > ninf ? cand[i] : ninf;   // NaN and -inf never win
     float score = ninf, top = ninf;   // lane j keeps score j
-    if (__ballot(cand[0] == 12345.678f) == ~0ull) return;   // (forces the loads to complete before the stamp)
+#pragma unroll
+    for (int i = 0; i < PER; ++i) asm volatile("" : "+v"(cand[i]));   // (the loads complete before the stamp)
     clock();
     bool done = false;
     if constexpr (PER == 8) {
