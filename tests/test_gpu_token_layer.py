@@ -27,11 +27,14 @@ def run(ctx, cfg, w, x):
     return bufs, out
 
 
-# 64 picks by the first wave, 65 by the launch of their own; up to 512 experts by the candidates' search, from 513 on one by one;
-# rows of either width, groups of 32, Q8, a shared expert of another format (a launch without routed jobs)
+# Up to twenty picks inside the gate/up launch where they are found together (up to 512 experts, as many lanes as picks), up to twelve where they
+# are found one by one, and one more by the launch of their own, up to 64 by its first wave's lanes; rows of either width, groups of 32, Q8, a
+# shared expert of another format
 @pytest.mark.parametrize("hidden,inter,experts,topk,bits,group", [
     (128, 128, 1, 1, (4, 4, 4, 4), 64), (512, 640, 3, 3, (4, 4, 4, 4), 64), (512, 512, 64, 63, (4, 4, 4, 4), 64), (512, 128, 66, 64, (4, 8, 8, 8), 64),
-    (512, 128, 66, 65, (4, 8, 8, 8), 64), (640, 128, 512, 10, (8, 8, 4, 4), 64), (256, 128, 513, 10, (8, 4, 4, 8), 32), (128, 64, 1024, 64, (4, 4, 4, 4), 64),
+    (512, 128, 66, 65, (4, 8, 8, 8), 64), (512, 128, 512, 20, (4, 4, 4, 4), 64), (512, 128, 153, 20, (4, 4, 4, 4), 64), (512, 128, 152, 20, (4, 8, 8, 8), 64),
+    (512, 128, 512, 21, (4, 4, 4, 4), 64), (512, 128, 96, 12, (4, 4, 4, 4), 64), (512, 128, 70, 12, (4, 4, 4, 4), 64), (512, 128, 70, 13, (4, 4, 4, 4), 64),
+    (512, 128, 1024, 12, (4, 4, 4, 4), 64), (512, 128, 1024, 13, (4, 4, 4, 4), 64), (640, 128, 512, 10, (8, 8, 4, 4), 64), (256, 128, 513, 10, (8, 4, 4, 8), 32), (128, 64, 1024, 64, (4, 4, 4, 4), 64),
     (32512, 64, 3, 2, (4, 4, 4, 4), 64), (32576, 64, 3, 2, (4, 4, 4, 4), 64)])   # the longest row beside which the selection has room in LDS, and one more
 def test_layer(ctx, hidden, inter, experts, topk, bits, group):
     cfg = workload.tiny_config(hidden=hidden, experts=experts, topk=topk, inter=inter, bits=bits, group=group)

@@ -607,7 +607,7 @@ static zc_status moe_layer(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe
     if (T > 1) zc::launch_route_jobs(s, w.logits, T, E, k, w.ids, w.weights, w.offsets, w.slots, chunk, jobs, w.count, w.selected, ctx->moe_status, x, H, images);
     else {   // its picks are the job list
         chunk = 1;
-        if (!zc::expert_phase_routes(H, k)) zc::launch_route(s, w.logits, 1, E, k, w.ids, w.weights);
+        if (!zc::expert_phase_routes(H, E, k)) zc::launch_route(s, w.logits, 1, E, k, w.ids, w.weights);
     }
     // 5-6. shared expert (model.cpp:482-485) and routed experts (pipeline.cpp:18-29): gate/up on gathered rows, down scattered
     // to its slot.  One launch per phase (two where the lanes' kernels walk a list and the shared expert has another format).

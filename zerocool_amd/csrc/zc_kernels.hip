@@ -246,8 +246,18 @@ void launch_affine(hipStream_t s, const AffineDesc& a) {
     else by_format<false>(a.gate.bits, wide(j.K, j.N), go);
 }
 
-// (the selection's words beside the longest rows, which fill a compute unit's LDS)
-bool expert_phase_routes(uint32_t K, uint32_t topk) { return topk <= 64 && affine_token_bytes<16>(K) + 1024 <= 160 * 1024; }
+// Whether one token's gate/up launch makes the picks: every workgroup waits for them, so only while they take less than the launch they replace and
+// the gap behind it.  Where there are as many lanes with candidates (eight a lane, up to 512 experts) as picks, they are found together, else
+// one by one.  us a layer, a launch of their own -> inside, hidden 2048 and 3072:
+//   together: 512 experts, 10, 20, 28 and 48 picks 24 -> 22, 37 -> 36, 45 -> 47, 73 -> 95 and 35 -> 34, 56 -> 56, 68 -> 70, 105 -> 124;
+//             256 experts, 16, 20 and 24 picks 33 -> 31, 36 -> 36, 42 -> 42 and 49 -> 49, 56 -> 56, 61 -> 63
+//   one by one: 64 experts, 10, 12, 16 and 28 picks 25 -> 24, 31 -> 30, 36 -> 34, 51 -> 58 and 35 -> 34, 42 -> 42, 49 -> 53, 70 -> 86; 1024 experts, 10, 12,
+//             16, 28 and 63 picks 28 -> 27, 35 -> 34, 40 -> 40, 60 -> 79, 102 -> 143 and 40 -> 41, 49 -> 50, 57 -> 69, 81 -> 118, 144 -> 180
+// (And the selection's words have to fit beside the longest rows, which fill a compute unit's LDS.)
+bool expert_phase_routes(uint32_t K, uint32_t E, uint32_t topk) {
+    const bool together = E <= 512 && topk <= (E + 7) / 8;
+    return topk <= (together ? 20 : 12) && affine_token_bytes<16>(K) + 1024 <= 160 * 1024;
+}
 void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d) {
     ExpertPhase p{};
     p.logits = d.logits; p.ids = d.ids; p.weights = d.weights; p.status = d.status; p.E = d.E;
@@ -287,7 +297,7 @@ void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d) {
                 const dim3 grid((p.tiles + p.share - 1) / p.share, d.max_jobs + p.shared_jobs);
                 const uint32_t lds = affine_token_bytes<WIDTH>(d.K);
                 if constexpr (GATED) {
-                    if (expert_phase_routes(d.K, d.topk)) {
+                    if (expert_phase_routes(d.K, d.E, d.topk)) {
                         if (d.E <= 512) hipLaunchKernelGGL((expert_token_kernel<BITS, WIDTH, true, 8, SHARED>), grid, dim3(256), lds, s, p);
                         else hipLaunchKernelGGL((expert_token_kernel<BITS, WIDTH, true, 16, SHARED>), grid, dim3(256), lds, s, p);
                         return;

@@ -38,7 +38,7 @@ struct ExpertPhaseDesc {
     uint32_t K, N, group, bits, shared_bits, topk, tokens, chunk, max_jobs;
     bool gated;
 };
-bool expert_phase_routes(uint32_t K, uint32_t topk);
+bool expert_phase_routes(uint32_t K, uint32_t E, uint32_t topk);
 void launch_expert_phase(hipStream_t s, const ExpertPhaseDesc& d);
 
 void launch_plain(hipStream_t s, const void* w, uint32_t dtype, const float* x, uint32_t K, uint32_t N,
