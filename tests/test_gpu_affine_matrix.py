@@ -73,7 +73,11 @@ def test_operators(ctx, bits, K, N, T, kind):
     (66, 512, 512, 6, 2, (4, 4, 4, 4), "spread"), (520, 512, 128, 3, 2, (4, 4, 4, 4), "normal"),
     # the longest rows and one step more (then both phases are the lanes'), rows of either form's own width, and lists of jobs with one to four tokens
     (7, 8704, 512, 3, 2, (4, 4, 4, 4), "strange"), (7, 9216, 512, 3, 2, (4, 4, 4, 4), "strange"), (9, 512, 8704, 3, 2, (4, 4, 4, 4), "normal"),
-    (33, 1024, 640, 24, 3, (4, 4, 4, 4), "strange"), (37, 1536, 512, 40, 4, (4, 8, 8, 8), "strange"), (70, 512, 512, 64, 4, (8, 8, 8, 8), "strange")])
+    (33, 1024, 640, 24, 3, (4, 4, 4, 4), "strange"), (37, 1536, 512, 40, 4, (4, 8, 8, 8), "strange"), (70, 512, 512, 64, 4, (8, 8, 8, 8), "strange"),
+    # either side of the numbers of tokens from which a batch goes to the matrix cores
+    (2, 2048, 1024, 6, 3, (4, 4, 4, 4), "edge"), (3, 2048, 1024, 6, 3, (4, 4, 4, 4), "edge"), (8, 512, 512, 9, 4, (4, 4, 4, 4), "normal"), (9, 512, 512, 9, 4, (4, 4, 4, 4), "normal"),
+    (2, 512, 512, 6, 4, (4, 8, 8, 8), "edge"), (2, 512, 512, 6, 4, (4, 4, 8, 4), "spread"), (11, 512, 512, 9, 4, (8, 8, 8, 8), "normal"), (12, 512, 512, 9, 4, (8, 8, 8, 8), "normal"),
+    (12, 512, 512, 97, 4, (8, 4, 8, 4), "normal"), (12, 512, 512, 96, 4, (8, 4, 8, 4), "normal"), (3, 4096, 2048, 4, 3, (8, 8, 8, 8), "normal"), (4, 4096, 2048, 4, 3, (8, 8, 8, 8), "normal")])
 def test_layer(ctx, T, hidden, inter, experts, topk, bits, kind):
     cfg = workload.tiny_config(hidden=hidden, experts=experts, topk=topk, inter=inter, bits=bits)
     w = workload.LayerWeights(ctx, cfg, 900 + T, ("normal", 0.5))

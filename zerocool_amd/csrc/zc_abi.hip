@@ -589,6 +589,24 @@ uint64_t zc_hip_moe_workspace_bytes(const zc_moe_config* cfg, uint32_t tokens) {
     if (validate_config(cfg) != ZC_OK || !tokens) return 0;
     return carve(cfg, tokens, nullptr).bytes;
 }
+// Whether a batch's expert products go to the matrix cores, where those take its rows.  A job there costs about the same with one token as with
+// four, on the lanes it goes by tokens; but how many tokens share an expert is not known here.  us a layer, lanes -> matrix cores, tokens that share few
+// experts / tokens that agree on most of them:
+//   Q4, 512 x 512, 16 experts, 2, 6, 12 tokens  23.6 -> 24.9, 26.8 -> 27.9, 31.6 -> 29.3 / 26.7 -> 28.2, 29.0 -> 30.6, 33.6 -> 32.6
+//   1024 x 512, 64 experts, 2, 4, 8 tokens      27.7 -> 29.7, 35.2 -> 33.1, 41.1 -> 42.3 / 28.7 -> 31.2, 32.7 -> 35.5, 38.0 -> 36.4
+//   2048 x 512, 512 experts, 2, 4, 8 tokens     36.3 -> 35.9, 46.8 -> 50.0, 62.6 -> 64.4 / 34.5 -> 33.5, 41.6 -> 39.6, 53.8 -> 46.8
+//   4096 x 2048, 128 experts, 2, 4, 8 tokens    86 -> 96, 161 -> 170, 245 -> 258 / 76 -> 77, 141 -> 121, 195 -> 148
+// A shared expert of another format costs the lanes two launches more; 2048 x 512 with Q8 down and shared, 2 and 8 tokens 43.3 -> 39.4, 75 -> 73 / 41.9 ->
+// 36.7, 62 -> 52.  Q8 gate/up has its chains on the fp32 instruction, which a job of one token fills to a quarter:
+//   1024 x 512, 64 experts, 2, 6, 12, 16 tokens 28.6 -> 32.4, 40.3 -> 49.2, 49.0 -> 51.6, 54.6 -> 53.4 / 29.5 -> 33.7, 37.7 -> 39.1, 46.5 -> 43.5, 52 -> 54
+//   2048 x 512, 512 experts, 4, 12, 24 tokens   56 -> 67, 108 -> 114, 178 -> 175 / 43 -> 47, 73 -> 72, 109 -> 95
+//   4096 x 2048, 128 experts, 2, 4, 8 tokens    128 -> 129, 233 -> 229, 360 -> 357 / 103 -> 103, 181 -> 150, 245 -> 202
+static bool matrix_preferred(const zc_moe_config& c, uint32_t T) {
+    const uint64_t weights = uint64_t(c.hidden) * c.inter;
+    if (c.bits_gate_up == 8) return weights >= 1u << 23 ? T >= 4 : T >= 12 && 2ull * T * c.topk >= c.experts;
+    if (c.shared_bits_gate_up != c.bits_gate_up || c.shared_bits_down != c.bits_down) return true;
+    return T > 2 && T * weights > 1u << 21;
+}
 // One exact layer on checked operands.  next, optional: the glue's rows for the layer that follows (combine and glue are then one
 // launch where the width allows it, and `out` may be null).  check: report inputs that are not BF16-valued.
 static zc_status moe_layer(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe_layer* l, const float* x, uint32_t T,
@@ -600,8 +618,9 @@ static zc_status moe_layer(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_moe
     zc::launch_router(s, l->router, x, T, H, E, l->router_offsets, w.logits, l->shared_gate, w.gate, check ? ctx->moe_status : nullptr);
     // 4. positions / selected, on the device (model.cpp:449-479): the expert kernels' job list, at most `chunk` tokens a job
     uint32_t chunk = ~0u;
-    for (const uint32_t bits : {c->bits_gate_up, c->shared_bits_gate_up}) chunk = std::min(chunk, zc::affine_job_tokens(H, I, c->group, bits));
-    for (const uint32_t bits : {c->bits_down, c->shared_bits_down}) chunk = std::min(chunk, zc::affine_job_tokens(I, H, c->group, bits));
+    const bool matrix = matrix_preferred(*c, T);
+    for (const uint32_t bits : {c->bits_gate_up, c->shared_bits_gate_up}) chunk = std::min(chunk, zc::affine_job_tokens(H, I, c->group, bits, matrix));
+    for (const uint32_t bits : {c->bits_down, c->shared_bits_down}) chunk = std::min(chunk, zc::affine_job_tokens(I, H, c->group, bits, matrix));
     float* images = T > 1 && zc::affine_job_images(chunk) ? w.expert_out : nullptr;   // the input rows' images, until the down products write there
     uint32_t* jobs = reinterpret_cast<uint32_t*>(w.rows);   // (n words: a job holds at least one slot)
     if (T > 1) zc::launch_route_jobs(s, w.logits, T, E, k, w.ids, w.weights, w.offsets, w.slots, chunk, jobs, w.count, w.selected, ctx->moe_status, x, H, images);

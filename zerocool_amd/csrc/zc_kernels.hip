@@ -202,9 +202,9 @@ template <int BITS, int WIDTH> static bool matrix_fits(uint32_t K, uint32_t N, u
 static uint32_t matrix_grid(uint32_t lds, uint32_t tiles, uint64_t jobs) {
     return uint32_t(std::min<uint64_t>(256 * matrix_per_cu(lds), (tiles + kMatrixWaves - 1) / kMatrixWaves * jobs));
 }
-uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t group, uint32_t bits) {
+uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t group, uint32_t bits, bool matrix) {
     uint32_t chunk = 1;
-    by_format<false>(bits, wide(K, N), [&]<int BITS, int WIDTH, bool GATED>() { chunk = matrix_fits<BITS, WIDTH>(K, N, group) ? kMatrixTokens : affine_chunk<WIDTH>(K); });
+    by_format<false>(bits, wide(K, N), [&]<int BITS, int WIDTH, bool GATED>() { chunk = matrix && matrix_fits<BITS, WIDTH>(K, N, group) ? kMatrixTokens : affine_chunk<WIDTH>(K); });
     return chunk;
 }
 bool affine_job_images(uint32_t chunk) { return chunk > kAffineTokens; }

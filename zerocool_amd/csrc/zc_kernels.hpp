@@ -21,9 +21,9 @@ bool xint_supported(const zc_linear& l);                          // wide affine
 void launch_affine_xint(hipStream_t s, const AffineDesc& a);     // exact-integer matrix-core form
 constexpr uint32_t kXintLongestRow = 21504;                       // of one token: its digit planes and fp32 copy fill 160 KiB of LDS
 
-// Tokens one workgroup of the expert kernels takes at a time: 1 or 2 (lanes), 4 (matrix cores: they read rows as images, which take
-// the rows' place)
-uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t group, uint32_t bits);
+// Tokens one workgroup of the expert kernels takes at a time: 1 or 2 (lanes), 4 (matrix cores, if allowed: they read rows as images, which
+// take the rows' place)
+uint32_t affine_job_tokens(uint32_t K, uint32_t N, uint32_t group, uint32_t bits, bool matrix);
 bool affine_job_images(uint32_t chunk);
 
 struct ExpertPhaseDesc {
