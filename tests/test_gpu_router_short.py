@@ -1,5 +1,5 @@
 """Router logits of two to 64 tokens, whose chains run on the matrix cores, byte for byte against the CPU oracle: the longest rows of
-two, three and four tokens a workgroup and one piece more, workgroups of two waves and of four, partly filled either way; sums
+two, three and four tokens a workgroup and one piece more, workgroups of two waves and of four, partly filled either way, and short rows; sums
 that stay subnormal, that overflow, and that are not numbers."""
 import numpy as np
 import pytest
@@ -19,7 +19,9 @@ def ctx():
 
 @pytest.mark.parametrize("T,K,E,kind", [
     (2, 8064, 9, "normal"), (2, 8192, 9, "normal"), (3, 5376, 4, "normal"), (3, 5504, 7, "normal"), (4, 3968, 8, "normal"), (7, 2048, 11, "normal"),
-    (64, 3968, 247, "normal"), (62, 3968, 273, "normal"), (5, 256, 40, "tiny"), (6, 384, 40, "huge"), (2, 1152, 5, "nan")])
+    (64, 3968, 247, "normal"), (62, 3968, 273, "normal"), (5, 256, 40, "tiny"), (6, 384, 40, "huge"), (2, 1152, 5, "nan"),
+    # one piece of a row a thread and more, in workgroups of two waves and of four (more than the chip holds of two)
+    (5, 128, 40, "normal"), (3, 512, 40, "nan"), (5, 640, 40, "normal"), (64, 128, 1024, "tiny"), (64, 1024, 1021, "normal"), (63, 1152, 1024, "huge")])
 def test_router_logits(ctx, T, K, E, kind):
     rng = np.random.default_rng(K + T)
     w, x = rng.standard_normal((E, K)), rng.standard_normal((T, K))

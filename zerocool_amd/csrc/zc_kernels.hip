@@ -444,7 +444,7 @@ __global__ __launch_bounds__(256) void router_kernel(const uint16_t* w, const fl
 // expert j, a quarter of the reads of LDS that a lane with four tokens' chains needs, and half the time on the vector unit.
 // 512 experts: one token of 2048 inputs 5.0 us, of 2560 6.5; on the vector unit, with the staging's loads waited for one by one, -> here:
 // 5 tokens of 2048 8.4 -> 5.8, 8 of 3072 11.4 -> 7.4, 40 of 2560 15.3 -> 12.3, 64 of 3072 19.2 -> 15.9.
-template <uint32_t TOKENS>
+template <uint32_t TOKENS, uint32_t BATCH>   // BATCH: sixteen-byte pieces of a row that a thread requests at once
 __global__ __launch_bounds__(256) void router_short_kernel(const uint16_t* __restrict__ w, const float* __restrict__ x, uint32_t T, uint32_t K, uint32_t E,
                                                             const float* __restrict__ offsets, float* __restrict__ out, const void* __restrict__ gate_w, float* __restrict__ gate,
                                                             int32_t* status, uint32_t rows) {   // rows: tokens of a workgroup, at most TOKENS
@@ -467,15 +467,14 @@ __global__ __launch_bounds__(256) void router_short_kernel(const uint16_t* __res
     };
     request(0);
     uint32_t low = 0;
-    constexpr uint32_t kBatch = 12 / TOKENS;
-    for (uint32_t i0 = tid; i0 < K / 4; i0 += kBatch * blockDim.x) {   // (past the end: the last piece again, not used)
-        uint4 v[TOKENS][kBatch];
+    for (uint32_t i0 = tid; i0 < K / 4; i0 += BATCH * blockDim.x) {   // (past the end: the last piece again, not used)
+        uint4 v[TOKENS][BATCH];
 #pragma unroll
         for (uint32_t t = 0; t < TOKENS; ++t)
 #pragma unroll
-            for (uint32_t u = 0; u < kBatch; ++u) v[t][u] = ldg_u4(x + uint64_t(t0 + min(t, nt - 1)) * K, min(i0 + u * blockDim.x, K / 4 - 1));
+            for (uint32_t u = 0; u < BATCH; ++u) v[t][u] = ldg_u4(x + uint64_t(t0 + min(t, nt - 1)) * K, min(i0 + u * blockDim.x, K / 4 - 1));
 #pragma unroll
-        for (uint32_t u = 0; u < kBatch; ++u) {
+        for (uint32_t u = 0; u < BATCH; ++u) {
             const uint32_t i = i0 + u * blockDim.x, part = i / (P / 4), at = part * pitch + (i - part * (P / 4)) * 4;
 #pragma unroll
             for (uint32_t t = 0; t < TOKENS; ++t) {
@@ -662,14 +661,17 @@ void launch_router(hipStream_t s, const void* w, const float* x, uint32_t T, uin
         auto grid_of = [&](uint32_t waves) { return dim3((E + 4 * waves - 1) / (4 * waves) + (gate_w ? 1 : 0), (T + rows - 1) / rows); };
         auto lds_of = [&](uint32_t waves) { return row_bytes(rows) + waves * 4 * (T == 1 ? 1 : 4) * 17 * 4; };
         // Two waves spread the experts over more compute units, and stage the tokens' rows twice as often as four: while all workgroups
-        // are on the chip at once (512 experts, us with one, two and four waves: 8 tokens of 3072 inputs 9.3, 7.4, 9.0, 32 of 2048
+        // are on the chip at once, by LDS and, at three waves a SIMD, by registers (512 experts, us with one, two and four waves: 8 tokens of 3072 inputs 9.3, 7.4, 9.0, 32 of 2048
         // 12.7, 8.8, 10.6, 40 of 2560 21.4, 12.3, 13.7; 64 of 3072 24.7, 18.2, 15.9).
         const dim3 two = grid_of(2);
-        const uint32_t waves = T == 1 ? 1 : two.x * two.y <= 256 * (160 * 1024 / lds_of(2)) ? 2 : 4;
+        const uint32_t waves = T == 1 ? 1 : two.x * two.y <= 256 * std::min<size_t>(160 * 1024 / lds_of(2), 6) ? 2 : 4;
         const dim3 grid = grid_of(waves);
         const size_t lds = lds_of(waves);
-#define ZC_ROUTER(TOKENS) hipLaunchKernelGGL(router_short_kernel<TOKENS>, grid, dim3(64 * waves), lds, s, (const uint16_t*)w, x, T, K, E, offsets, out, gate_w, gate, status, rows)
-        if (T == 1) ZC_ROUTER(1); else ZC_ROUTER(4);
+        // (Rows of one piece a thread request no more.  Both: 1024 experts, 64 tokens of 256 and 1024 inputs 8.1 -> 6.3 and 10.2 -> 7.7 us.)
+#define ZC_ROUTER(...) hipLaunchKernelGGL((router_short_kernel<__VA_ARGS__>), grid, dim3(64 * waves), lds, s, (const uint16_t*)w, x, T, K, E, offsets, out, gate_w, gate, status, rows)
+        if (T == 1) ZC_ROUTER(1, 12);
+        else if (K <= 256 * waves) ZC_ROUTER(4, 1);
+        else ZC_ROUTER(4, 3);
 #undef ZC_ROUTER
         return;
     }
