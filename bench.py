@@ -85,9 +85,31 @@ def write_traffic_file(fetch_dir, write_dir):
     print(json.dumps(record))
 
 
+def other_way(ctx, stack, tokens):
+    """How to ask stack_decode for the way a batch does not go by itself: layer by layer, or as a single launch."""
+    if ctx.stack_single_launch(stack, tokens):
+        return {"layered": True}
+    if not ctx.stack_is_persistent(stack, tokens):
+        raise SystemExit("bench.py: no single-launch kernel takes this stack; nothing to check the layers against")
+    return {"single": True}
+
+
+def check_ways(ctx, stack, x, tokens, out, trace):
+    """The parity gate of a stack: one step the way the batch goes by itself, traced, and one the other way, the same bytes."""
+    import numpy as np
+    steps = []
+    for how in ({"trace": trace}, other_way(ctx, stack, tokens)):
+        ctx.stack_decode(stack, x, tokens, out, **how)
+        ctx.moe_check()
+        steps.append(out.numpy(np.float32).tobytes())
+    if steps[0] != steps[1]:
+        raise SystemExit("bench.py: the single launch and the layer-by-layer path disagree; refusing to time")
+
+
 def one_launch_layer(ctx, name, tokens, reps, warmup=5, skew=("zipf", 1.1), speculate=True):
-    """The same single-layer configuration through the persistent decode kernels as a stack of one layer: one launch per
-    step up to sixty-four tokens (pieces of sixty-four above that); over 8 distinct inputs in rotation."""
+    """The same single-layer configuration through the persistent decode kernels as a stack of one layer, one launch per
+    step, which has to be asked for (by itself a stack of one layer goes the way of `single_layer`); up to sixty-four tokens,
+    over 8 distinct inputs in rotation."""
     import numpy as np
     import zerocool_amd as z
     from zerocool_amd import workload
@@ -102,7 +124,7 @@ def one_launch_layer(ctx, name, tokens, reps, warmup=5, skew=("zipf", 1.1), spec
     ids, wts = ctx.alloc(tokens * c.topk * 4), ctx.alloc(tokens * c.topk * 4)
     unique = []
     for x in xs:   # parity gate: the operator path's bytes (glue of layer 0 is the identity on the input)
-        ctx.stack_decode(stack, x, tokens, out, z.StackTrace(ids.ptr, wts.ptr, None, None))
+        ctx.stack_decode(stack, x, tokens, out, z.StackTrace(ids.ptr, wts.ptr, None, None), single=True)
         ctx.moe_forward(c, lw.layer, x, tokens, ref, ws)
         ctx.moe_check()
         if out.numpy(np.float32).tobytes() != ref.numpy(np.float32).tobytes():
@@ -110,21 +132,20 @@ def one_launch_layer(ctx, name, tokens, reps, warmup=5, skew=("zipf", 1.1), spec
         unique.append(len(np.unique(ids.numpy(np.int32))))
     nbytes = float(np.mean([workload.layer_bytes(c, u, tokens, ctx) for u in unique]))
     for i in range(warmup):
-        ctx.stack_decode(stack, xs[i % INPUTS], tokens, out)
+        ctx.stack_decode(stack, xs[i % INPUTS], tokens, out, single=True)
     ctx.finish()
     ctx.timer_start()
     for i in range(reps):
-        ctx.stack_decode(stack, xs[i % INPUTS], tokens, out)
+        ctx.stack_decode(stack, xs[i % INPUTS], tokens, out, single=True)
     ms = ctx.timer_stop() / reps
     ctx.moe_check()
-    persistent = ctx.stack_single_launch(stack, tokens)
     ctx.stack_destroy(stack)
     for b in xs + [out, ws, ref, ids, wts, lw.router, lw.shared_gate, lw.shared_record, lw.records]:
         ctx.free(b)
     return {"tokens": tokens, "us_per_layer": ms * 1e3, "tokens_per_s": tokens / (ms * 1e-3), "router_skew": list(skew) if skew else None,
             "distinct_experts": float(np.mean(unique)), "slots_per_distinct_expert": tokens * c.topk / float(np.mean(unique)),
             "GBps": nbytes / (ms * 1e-3) / 1e9, "frac_of_hbm_peak": nbytes / (ms * 1e-3) / 8e12,
-            "guessing": bool(speculate), "path": "persistent single-launch kernel" if persistent else "layer by layer"}
+            "guessing": bool(speculate), "path": "persistent single-launch kernel"}
 
 
 def decode_kernel(tokens, single_launch):
@@ -199,8 +220,8 @@ def main():
     def run(stack, cfg, n_layers, tokens, steps, warmup, speculate=True, inputs=INPUTS, seed=workload.BASE_SEED + 4 * 7):
         """Times `steps` launches that cycle through `inputs` distinct token batches (a decode loop never sees the same
         hidden rows twice; the one-token kernel guesses each layer's experts from the step before, so a replayed input
-        would make every guess a hit).  Every input is first checked against the layer-by-layer operator path, byte for
-        byte, and its route ids are kept: they give the distinct records (the algorithmic bytes) of each launch and the
+        would make every guess a hit).  Every input first goes both ways, as a single launch and layer by layer, byte for
+        byte the same, and its route ids are kept: they give the distinct records (the algorithmic bytes) of each launch and the
         share of a step's experts that the step before had also chosen (what the guessing can hit)."""
         xs = [workload.hidden_rows(ctx, tokens, cfg.hidden, seed + tokens + 97 * i) for i in range(inputs)]
         out = ctx.alloc(tokens * cfg.hidden * 4)
@@ -209,13 +230,7 @@ def main():
         ctx.stack_set_speculation(stack, speculate)
         chosen, nbytes, unique = [], [], []
         for x in xs:
-            ctx.stack_decode(stack, x, tokens, out, z.StackTrace(ids.ptr, w.ptr, None, None))
-            ctx.moe_check()
-            fused = out.numpy(np.float32).tobytes()
-            ctx.stack_decode(stack, x, tokens, out, layered=True)
-            ctx.moe_check()
-            if out.numpy(np.float32).tobytes() != fused:
-                raise SystemExit("bench.py: persistent kernel and layer-by-layer path disagree; refusing to time")
+            check_ways(ctx, stack, x, tokens, out, z.StackTrace(ids.ptr, w.ptr, None, None))
             rows = ids.numpy(np.int32).reshape(n_layers, n).copy()
             chosen.append(rows)
             u = [len(np.unique(r)) for r in rows]
@@ -261,7 +276,7 @@ def main():
                    "inputs": f"{INPUTS} distinct token batches in rotation", "distinct_experts_per_layer": r["unique"],
                    "experts_repeated_from_previous_step": r["repeat_share"],
                    "path": "persistent single-launch kernel" if persistent else "layer by layer",
-                   "parity_gate": "output bytes equal the layer-by-layer operator path on this input (checked before timing)"},
+                   "parity_gate": "output bytes of the single launch and of the layer-by-layer operator path are equal on these inputs (checked before timing)"},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": 8000.0, "unit": "GB/s", "frac": achieved / 8000.0,
                      "traffic": traffic, "traffic_source": os.path.relpath(TRAFFIC_FILE, ROOT) if traffic else None,
                      "kernel": decode_kernel(T, persistent),
