@@ -223,8 +223,7 @@ __device__ __forceinline__ void route_token(Fetch fetch, uint32_t E, uint32_t to
 #pragma unroll
     for (int i = 0; i < PER; ++i) cand[i] = cand[i] > ninf ? cand[i] : ninf;   // NaN and -inf never win
     float score = ninf, top = ninf;   // lane j keeps score j
-#pragma unroll
-    for (int i = 0; i < PER; ++i) asm volatile("" : "+v"(cand[i]));   // (the loads complete before the stamp)
+    if (__ballot(__float_as_uint(cand[0]) == 0x7fc00001u) == ~0ull) return;   // (never: no candidate is a NaN here; forces the loads to complete before the stamp)
     clock();
     bool done = false;
     if constexpr (PER == 8) {
