@@ -152,7 +152,7 @@ def decode_kernel(tokens, single_launch):
     if not single_launch:   # the shapes measured here: wide affine rows in groups of 64
         if tokens == 1:
             return "zc::expert_token_kernel (four launches a layer)"
-        return f"zc::expert_matrix_kernel ({'five' if tokens <= 16 else 'six'} launches a layer)"
+        return f"zc::expert_{'phase' if tokens == 2 else 'matrix'}_kernel ({'five' if tokens <= 16 else 'six'} launches a layer)"
     kernel = "decode_stack_kernel" if tokens == 1 else "decode_multi_kernel" if tokens <= 8 else "decode_wide_kernel"
     return f"zc::{kernel} (one launch = one step)"
 

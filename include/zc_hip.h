@@ -209,8 +209,8 @@ zc_status zc_hip_moe_check(zc_hip_ctx* ctx);
  * dispatch and combine stay on the device, no host synchronisation between layers; one
  * kernel each for one token, two to eight, and nine to sixty-four), larger batches as
  * one such launch per 64 tokens.  One token of all-Q4 stacks of two layers and more does; other
- * stacks and two to sixty-four tokens go layer by layer (four to six launches each), which is
- * faster, as do shapes those kernels do not take.  All give identical bytes.
+ * stacks and two to sixty-four tokens go layer by layer, which is faster, as do shapes those
+ * kernels do not take.  All give identical bytes.
  * out: [tokens][hidden], the last layer's output.  flags bit 0: force the layer-by-layer path;
  * bit 1: the single launch where its kernels take the batch, also where layer by layer is faster. */
 typedef struct zc_hip_stack zc_hip_stack;

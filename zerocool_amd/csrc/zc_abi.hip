@@ -397,11 +397,12 @@ static uint64_t weight_bytes(const zc_linear* l) {
     return l->quantized ? uint64_t(l->input) * l->output * l->bits / 8 : uint64_t(l->input) * l->output * (l->dtype == 1 ? 4 : 2);
 }
 
-// Which form serves a product of Q4 matrices that both forms take.  us a call, matrix cores -> lanes, gate/up at 1, 4, 21, 64 and 512 rows / down:
-//   hidden 2048  7.5 -> 5.2  19.5 -> 6.4  21.4 -> 8.7   22.0 -> 16.3  114 -> 79  /   5.5 -> 4.4   9.7 -> 4.4  10.2 -> 6.8   18.3 -> 10.8   84 -> 52
-//   hidden 2560  7.2 -> 5.6  19.3 -> 7.2  21.2 -> 11.3  38.6 -> 23.1  175 -> 115 /  (its rows of 640 always went to the lanes)
-//   hidden 3072  9.0 -> 6.1  25.8 -> 8.1  28.5 -> 16.0  54.7 -> 34.2  320 -> 200 /   7.0 -> 3.9  17.7 -> 5.3  34.4 -> 10.6  51.4 -> 20.6  231 -> 116
-// and on rows that are not BF16-valued the lanes are ahead by two to six times.  A call of the integer form first builds digit
+// Which form serves a product of Q4 matrices that both forms take.  us a call, integer form -> the other (the lanes; from 48 rows of gate/up and 128 of
+// down on the matrix cores quad by quad), gate/up at 1, 4, 21, 64 and 512 rows / down:
+//   hidden 2048  7.5 -> 5.1  19.2 -> 6.3  20.0 -> 8.8   21.3 -> 12.3  114 -> 43  /   4.2 -> 4.1   7.1 -> 4.3   8.1 -> 6.9   14.3 -> 11.1   71 -> 25
+//   hidden 2560  8.0 -> 5.6  21.0 -> 7.1  21.2 -> 11.5  40.6 -> 18.4  177 -> 60  /  (the integer form does not take its rows of 640)
+//   hidden 3072  9.1 -> 6.0  26.8 -> 7.9  27.4 -> 16.1  53.8 -> 25.5  323 -> 101 /   4.9 -> 3.9  10.9 -> 5.3  20.5 -> 10.7  33.1 -> 21.2  169 -> 58
+// and on rows that are not BF16-valued, at 21, 64 and 512 rows, hidden 3072 51 -> 21, 101 -> 66, 576 -> 341 / 37 -> 13, 57 -> 28, 296 -> 190.  A call of the integer form first builds digit
 // planes of its rows in LDS, one workgroup a compute unit, and fills the chip with tiles of sixteen rows only from a few
 // hundred tokens on.  It is ahead where its workgroups fill the chip exactly, by up to a tenth on most such sizes (a gate/up row
 // of 1024 x 8192 5.9 -> 6.5, of 2048 x 16384 11.5 -> 13.6; outputs around these sizes lose as much), and by far for one row of
@@ -1130,14 +1131,15 @@ static zc_status launch_piece(zc_hip_ctx* ctx, zc_hip_stack* st, const float* x,
     }
     return ZC_OK;
 }
-// Whether a batch that a single launch could take goes layer by layer, four to six launches each: from two tokens on.  us per layer, single
+// Whether a batch that a single launch could take goes layer by layer: from two tokens on.  us per layer, single
 // launch -> layer by layer, at 2, 8, 32 and 64 tokens, one layer with N(0, 0.5) offsets / six layers with Zipf(1.1) offsets, whose
 // tokens agree on nearly all experts behind the first layer:
 //   hidden 2048, Q4        51 -> 37   94 -> 65   194 -> 124   312 -> 182  /  38 -> 34   62 -> 46   144 -> 77    222 -> 117
 //   hidden 2048, mixed     60 -> 39  110 -> 74   277 -> 156   447 -> 235  /  50 -> 37  101 -> 52   212 -> 96    360 -> 158
 //   hidden 3072, Q4        76 -> 59  186 -> 125  462 -> 299   746 -> 464  /  53 -> 51   97 -> 73   259 -> 146   436 -> 243
 // One token of all-Q4 layers stays with its kernel, which has no launch between the layers and starts on the previous step's experts: two
-// layers 28 -> 24 and 33 -> 36, six layers 23 -> 24 and 29 -> 38, sixteen 22.5 -> 25.7.  A stack of one layer has nothing between layers to
+// layers of hidden 2048 and 3072 28 -> 24 and 33 -> 36 (so two layers of the narrower ones would gain from the other way; the line is drawn by depth alone), six
+// layers 23 -> 24 and 29 -> 38, sixteen of hidden 2048 22.5 -> 25.7.  A stack of one layer has nothing between layers to
 // gain from: 31 -> 24 and 38 -> 34.  That kernel's Q8 rows are walked a row at a time: one, two, six and sixteen mixed layers of hidden 2048
 // 37 -> 24, 35 -> 25, 33 -> 25, 37 -> 27, Q8 only in the shared expert 33 -> 24, 30 -> 24, 29 -> 24; of hidden 3072 69 -> 40, 61 -> 37, 68 -> 41,
 // 66 -> 41, and 48 -> 37, 43 -> 35, 42 -> 38.

@@ -22,10 +22,10 @@ namespace zc {
 //
 // What bounds it: with one token per row, the latency of the chain job -> row index -> input row -> LDS -> codes (a launch
 // of a few us); with several, vector instructions, a wave's at four clocks each: 24 per block of sixteen weights and token, 14
-// to unpack the block (the listing's 49 and 28 for the two rows), and the finish of a row.  Per layer of hidden 2560 and intermediate 640, gate/up and down: 40 tokens 142
-// and 119 us, one token 11.9 and 8.7 us.  With codes converted to floats, addresses formed per lane and four tokens per
+// to unpack the block (the listing's 49 and 28 for the two rows), and the finish of a row.  Per layer of hidden 2560 and intermediate 640, gate/up and down: 40 tokens 144
+// and 116 us, one token 11.9 and 8.7 us.  With codes converted to floats, addresses formed per lane and four tokens per
 // workgroup it was 172 and 132, 12.5 and 9.2 us.  (One token's gate/up that makes its picks takes 13.2 us, down 7.0; 40 tokens now go to the
-// matrix cores, 104 and 105 us: zc_affine_matrix.hpp.)  Four tokens per workgroup take 159 and 112 us: most experts have one or two
+// matrix cores, 105 and 105 us: zc_affine_matrix.hpp.)  Four tokens per workgroup take 159 and 112 us: most experts have one or two
 // tokens, and the LDS of four leaves room for three workgroups on a compute unit where two leave six (decoding stacks of
 // hidden 2048 and 3072 at 2 to 64 tokens lost 5 to 25 %).  One token at a time, codes requested step by step behind the staging,
 // sums through LDS permutes and the shared expert in launches of its own took 397 and 310, 20.2 and 14.3 us.

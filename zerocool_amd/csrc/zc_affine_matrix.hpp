@@ -21,9 +21,10 @@
 // eight, scale and bias in one load (lanes of b and b + 1 share a group: one takes the scale, the other the bias); 32 tokens of
 // hidden 2048, 512 experts: gate/up 96 -> 62 us, down 53 -> 47.  Workgroups that take a contiguous share of the work list instead of a grid over
 // all jobs there could be: 64 tokens of hidden 3072 that agree on eleven experts 157 -> 125 us.
-// Two tokens a workgroup on the lanes of zc_affine.hpp -> this, gate/up and down, us: hidden 2560, 40 tokens 154 and 124 -> 104 and 105; hidden 2048, 32 tokens
-// 80 and 51 -> 62 and 46; hidden 3072, 64 tokens that agree 290 and 140 -> 136 and 74.  Eight tokens a workgroup (half the conversions, twice the accumulators: two
-// waves a SIMD) took 121 and 75 for the last, but 83 and 78 for 32 tokens of hidden 2048, most of whose experts have one token or two.
+// Two tokens a workgroup on the lanes of zc_affine.hpp -> this, gate/up and down, us: hidden 2560, 40 tokens 144 and 116 -> 105 and 105; hidden 2048, 32 tokens
+// 81 and 52 -> 67 and 47; hidden 3072, average of six layers, 64 tokens 291 and 162 -> 138 and 87.  Eight tokens a workgroup (half the conversions, twice the
+// accumulators: two waves a SIMD) took 121 and 75 where four took 136 and 74 (64 tokens of hidden 3072 that agree), but 83 and 78 where four took 62 and
+// 46 (32 tokens of hidden 2048, most of whose experts have one token or two).
 #pragma once
 #include "zc_affine.hpp"
 
@@ -33,7 +34,7 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
-constexpr uint32_t kMatrixTokens = 4, kMatrixSteps = 64;                  // of a workgroup, at most: tokens and steps of a row
+constexpr uint32_t kMatrixTokens = 4, kMatrixSteps = 64;                  // of a workgroup, at most: tokens and steps of a row (a lane each; the LDS rule ends at 31)
 constexpr uint32_t kMatrixWaves = 4, kMatrixThreads = 64 * kMatrixWaves;
 
 template <int BITS, int WIDTH>

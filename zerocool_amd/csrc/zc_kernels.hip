@@ -1,8 +1,9 @@
-// Operator kernels of the MoE path with the reference's arithmetic kept literally:
+// Operator kernels of the MoE path with the reference's arithmetic kept to the bit:
 // the 32-lane partition of every affine dot, the scalar order inside a lane, every
-// BF16 rounding boundary.  One GPU lane plays one reference lane, so a 64-lane
-// wavefront carries two output rows.  Results are bit-identical to the CPU statement
-// of the same arithmetic for any input.
+// BF16 rounding boundary.  On the lanes (zc_affine.hpp) one GPU lane plays one reference
+// lane; on the matrix cores (zc_affine_matrix.hpp) sums that are exact in any order are
+// formed together.  Results are bit-identical to the CPU statement of the same
+// arithmetic for any input.
 #include "zc_kernels.hpp"
 #include <algorithm>
 #include <type_traits>
@@ -215,6 +216,9 @@ static dim3 affine_grid(uint32_t x, uint32_t jobs) { const uint32_t y = std::min
 // and a barrier.  us a call, lanes -> matrix cores: gate/up at 16, 32, 48 and 128 rows, hidden 2048 7.5 -> 9.1, 9.9 -> 9.2, 13.2 -> 11.2, 24 -> 17;
 // 2560 9.7 -> 10.4, 12.5 -> 13.2, 18 -> 13, 34 -> 27; 3072 12.7 -> 12.1, 21 -> 15, 28 -> 20, 57 -> 31.  Down at 32, 48, 96 and 128: 8.6 -> 6.7, 11.1 -> 7.6,
 // 14.4 -> 12.1, 15.5 -> 12.0; 10.9 -> 10.4, 14.9 -> 12.4, 22 -> 18, 27 -> 22; 13.7 -> 11.9, 15.7 -> 20.2, 25.2 -> 26.2, 32 -> 26.
+// Q8: gate/up at 48, 64 and 128, 2048 x 512 14.7 -> 13.9, 18.9 -> 14.2, 30 -> 23; 3072 x 1024 at 48 and 128 33 -> 24, 71 -> 53; down at 128
+// and 192, 512 x 2048 16.8 -> 12.4, 22.6 -> 18.3; 1024 x 3072 37 -> 26, 52 -> 39.  Q4 rows of half steps: gate/up at 48 and 128, 640 x 2560 25.6 -> 15.2, 56 -> 27;
+// 1920 x 640 18.4 -> 12.6, 36 -> 28; down at 128, 640 x 2560 26.8 -> 17.5, 1920 x 2560 59 -> 37.
 constexpr uint32_t kMatrixFrom[2] = {128, 48};   // plain, gate/up
 void launch_affine(hipStream_t s, const AffineDesc& a) {
     AffineJob j{};
