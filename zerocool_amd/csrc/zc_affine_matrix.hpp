@@ -397,13 +397,14 @@ __device__ __forceinline__ void matrix_walk(MatrixStream<BITS, WIDTH, GATED>& st
 // Output rows first .. last - 1 of a job where a token's products may round: on the lanes (zc_affine.hpp), two tokens at a time.  Inputs are BF16 by
 // contract; rows that are not cost more here than by the lanes' own kernels, since the work list is cut as if all jobs took the same time, and a job
 // of four tokens is two turns.  us, a row at a time with nothing requested ahead -> this (the lanes' kernels): layers whose rows are all fp32, 8 tokens of
-// hidden 2048 145 -> 95 (70), 64 of 2048 659 -> 382 (276), 64 of 3072 2087 -> 1026 (684); gate/up 3072 x 1024 at 128 and 512 rows 163 -> 107 (82) and
-// 602 -> 343 (292), with one such row among them 97 -> 48 (58) and 357 -> 149 (202).
+// hidden 2048 145 -> 93 (69), 64 of 2048 656 -> 361 (273), 64 of 3072 2089 -> 965 (668); gate/up 3072 x 1024 at 128 and 512 rows 163 -> 104 (82) and
+// 599 -> 328 (291), with one such row among them 97 -> 46 (58) and 356 -> 146 (201).
 template <int BITS, int WIDTH, bool GATED, class Load, class Put, class InRow, class OutRow>
 __device__ __forceinline__ void matrix_strange_rows(const AffineMatrix (&m)[2], uint32_t K, uint32_t N, Load load, Put put, uint32_t nt, InRow in_row, OutRow out_row,
                                                     uint32_t first, uint32_t last, bool float_output, uint8_t* lds) {
     constexpr uint32_t kRows = AffineStream<BITS, WIDTH, GATED, kAffineTokens>::kTileRows;
     static_assert(kMatrixWaves * MatrixStream<BITS, WIDTH, GATED>::kTileRows % kRows == 0);   // a workgroup's range is whole tiles of either form
+    asm volatile("" : "+s"(K), "+s"(N), "+s"(first), "+s"(last));   // (else what is formed from them is formed in front of the loop over jobs, for every job)
     const uint32_t most = kAffineTokens * affine_token_bytes<WIDTH>(K) <= matrix_lds_bytes<BITS, WIDTH>(K) ? kAffineTokens : 1u;
 #pragma unroll 1
     for (uint32_t t0 = 0; t0 < nt; t0 += most) {
