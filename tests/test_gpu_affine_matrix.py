@@ -42,12 +42,17 @@ def rows(kind, T, K, seed):
     (4, 512, 8, 133, "normal"), (4, 1024, 24, 131, "spread"), (4, 512, 40, 130, "edge"), (4, 1536, 8, 129, "powers"), (4, 512, 16, 132, "far"),
     (4, 512, 8, 130, "strange"), (4, 640, 24, 133, "normal"), (4, 128, 8, 131, "spread"), (4, 384, 12, 130, "edge"), (4, 512, 7, 129, "powers"),
     (4, 640, 8, 130, "strange"), (8, 512, 8, 133, "normal"), (8, 1024, 24, 131, "spread"), (8, 512, 40, 130, "powers"), (8, 512, 16, 129, "strange"),
-    # either side of the numbers of rows from which the two products go to the matrix cores
-    (4, 512, 24, 47, "strange"), (4, 512, 24, 48, "strange"), (4, 640, 24, 127, "edge"), (4, 640, 24, 128, "edge"), (8, 512, 24, 47, "spread"), (8, 512, 24, 48, "spread"),
+    # products of fewer outputs and rows than fill the chip's SIMDs stay with the lanes, as those above; from here on not
+    (4, 512, 256, 133, "normal"), (4, 1024, 264, 131, "spread"), (4, 512, 296, 130, "edge"), (4, 1536, 256, 129, "powers"), (4, 512, 272, 132, "far"), (4, 512, 256, 130, "strange"),
+    (4, 640, 280, 133, "normal"), (4, 128, 264, 131, "spread"), (4, 384, 268, 130, "edge"), (4, 512, 263, 129, "powers"), (4, 640, 264, 130, "strange"), (8, 512, 256, 133, "normal"),
+    (8, 1024, 280, 131, "spread"), (8, 512, 296, 130, "powers"), (8, 512, 272, 129, "strange"),
+    # either side of the numbers of rows, and of waves, from which the two products go to the matrix cores
+    (4, 512, 352, 47, "strange"), (4, 512, 352, 48, "strange"), (4, 640, 264, 127, "edge"), (4, 640, 264, 128, "edge"), (8, 512, 352, 47, "spread"), (8, 512, 352, 48, "spread"),
+    (4, 512, 124, 128, "edge"), (4, 512, 128, 128, "edge"), (4, 512, 248, 128, "edge"), (4, 512, 12, 2724, "edge"), (4, 512, 12, 2732, "edge"), (4, 384, 12, 2732, "strange"),
     # the longest rows of each format whose four tokens leave room for two workgroups, and one step more; rows that are not BF16
     # one at a time (5632 and 8704 inputs) and two
-    (4, 8704, 8, 129, "strange"), (4, 8704, 8, 50, "edge"), (4, 9216, 8, 129, "strange"), (4, 7936, 8, 129, "strange"), (4, 7936, 8, 51, "edge"), (4, 8064, 8, 129, "strange"),
-    (8, 7680, 8, 129, "strange"), (8, 8192, 8, 129, "strange"), (4, 4096, 8, 129, "strange"), (4, 4224, 8, 129, "strange"), (4, 5120, 8, 129, "strange"), (4, 5632, 8, 129, "strange")])
+    (4, 8704, 256, 129, "strange"), (4, 8704, 320, 50, "edge"), (4, 9216, 256, 129, "strange"), (4, 7936, 256, 129, "strange"), (4, 7936, 320, 51, "edge"), (4, 8064, 256, 129, "strange"),
+    (8, 7680, 256, 129, "strange"), (8, 8192, 256, 129, "strange"), (4, 4096, 256, 129, "strange"), (4, 4224, 256, 129, "strange"), (4, 5120, 256, 129, "strange"), (4, 5632, 256, 129, "strange")])
 def test_operators(ctx, bits, K, N, T, kind):
     rng = np.random.default_rng(K + N + T)
     mats = []

@@ -220,6 +220,10 @@ static dim3 affine_grid(uint32_t x, uint32_t jobs) { const uint32_t y = std::min
 // and 192, 512 x 2048 16.8 -> 12.4, 22.6 -> 18.3; 1024 x 3072 37 -> 26, 52 -> 39.  Q4 rows of half steps: gate/up at 48 and 128, 640 x 2560 25.6 -> 15.2, 56 -> 27;
 // 1920 x 640 18.4 -> 12.6, 36 -> 28; down at 128, 640 x 2560 26.8 -> 17.5, 1920 x 2560 59 -> 37.
 constexpr uint32_t kMatrixFrom[2] = {128, 48};   // plain, gate/up
+// And from a wave a SIMD on (two where a matrix has less than a workgroup's tiles), since with fewer the call lasts as long as one workgroup's chain,
+// which is longer there.  Gate/up with 512, 768, 1024 and 2048 waves: 2048 x 64 7.6 -> 10.0, 9.0 -> 9.9, 10.4 -> 10.1, 17.4 -> 12.8; down 2048 x 128 7.2 -> 9.6, 8.5 ->
+// 9.6, 9.7 -> 9.8, 16.4 -> 12.3; gate/up 4096 x 8 11.2 -> 15.7 at 512 and 16.4 -> 20.6 at 1024.
+constexpr uint64_t kMatrixWavesFrom = 1024;
 void launch_affine(hipStream_t s, const AffineDesc& a) {
     AffineJob j{};
     auto matrix = [](const zc_linear& l) { return AffineMatrix{(const uint8_t*)l.weight, (const uint16_t*)l.scales, (const uint16_t*)l.biases}; };
@@ -229,10 +233,12 @@ void launch_affine(hipStream_t s, const AffineDesc& a) {
     j.K = a.gate.input; j.N = a.gate.output; j.group = a.gate.group; j.tokens = a.tokens; j.float_output = a.float_output;
     auto go = [&]<int BITS, int WIDTH, bool GATED>() {
         if constexpr (BITS == 4 || WIDTH == 8) {
-            if (j.tokens >= kMatrixFrom[GATED] && matrix_fits<BITS, WIDTH>(j.K, j.N, j.group)) {
-                using Stream = MatrixStream<BITS, WIDTH, GATED>;
-                j.chunk = kMatrixTokens; j.tiles = (j.N + Stream::kTileRows - 1) / Stream::kTileRows;
-                const uint32_t lds = matrix_lds_bytes<BITS, WIDTH>(j.K), grid = matrix_grid(lds, j.tiles, (uint64_t(j.tokens) + kMatrixTokens - 1) / kMatrixTokens);
+            using Stream = MatrixStream<BITS, WIDTH, GATED>;
+            j.tiles = (j.N + Stream::kTileRows - 1) / Stream::kTileRows;
+            const uint64_t jobs = (uint64_t(j.tokens) + kMatrixTokens - 1) / kMatrixTokens;
+            if (j.tokens >= kMatrixFrom[GATED] && jobs * j.tiles >= kMatrixWavesFrom * (j.tiles < kMatrixWaves ? 2 : 1) && matrix_fits<BITS, WIDTH>(j.K, j.N, j.group)) {
+                j.chunk = kMatrixTokens;
+                const uint32_t lds = matrix_lds_bytes<BITS, WIDTH>(j.K), grid = matrix_grid(lds, j.tiles, jobs);
                 hipLaunchKernelGGL((affine_matrix_kernel<BITS, WIDTH, GATED>), dim3(grid), dim3(kMatrixThreads), lds, s, j);
                 return;
             }
