@@ -1,0 +1,33 @@
+"""The gather's row check of the fused gate/up operator: a refused call leaves the output alone, an accepted one is the oracle's.
+Lists up to 256 rows are looked at by the product's own kernel (lanes, and from 48 rows on matrix cores), longer ones in front of it."""
+import numpy as np
+import pytest
+import oracle
+import zerocool_amd as z
+from test_gpu_operators import ctx, dev_linear, same_bytes   # noqa: F401  (ctx: the fixture)
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+
+
+@pytest.mark.parametrize("n", [1, 2, 47, 64, 65, 255, 256, 257, 1030])
+@pytest.mark.parametrize("K,N", [(320, 7), (512, 64)])
+def test_gathered_rows_are_checked_whichever_kernel_looks(ctx, n, K, N):
+    T, rng = 9, np.random.RandomState(n)
+    w = rng.randint(0, 2 ** 32, N * K // 8, dtype=np.uint32)
+    s, b = np.full(N * K // 64, 0x3c00, np.uint16), np.full(N * K // 64, 0xbd80, np.uint16)
+    x = oracle.bf(rng.standard_normal(T * K).astype(f32))
+    lin, dx = dev_linear(ctx, w, s, b, K, N), ctx.upload(x)
+    rows = rng.randint(0, T, n).astype(np.int32)
+    out = ctx.upload(np.full(n * N, 7, f32))
+    for at in sorted({0, n // 2, n - 1}):
+        for wrong in (T, -1, 2 ** 31 - 1):
+            bad = rows.copy(); bad[at] = wrong
+            with pytest.raises(z.ZcError, match="row outside input"):
+                ctx.gated_linear(lin, lin, dx, T, n, ctx.upload(bad), out=out)
+    ctx.finish()
+    assert (out.numpy(f32) == 7).all()
+    for _ in range(70):   # (more calls than there are words for the answers)
+        ctx.gated_linear(lin, lin, dx, T, n, ctx.upload(rows), out=out)
+    host = oracle.make_linear(w, s, b, K, N)
+    assert same_bytes(out.numpy(f32), oracle.gated_linear(host, host, x, n, rows))

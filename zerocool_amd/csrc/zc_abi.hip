@@ -5,6 +5,7 @@
 #include "../../include/zc_hip.h"
 #include "zc_kernels.hpp"
 #include <algorithm>
+#include <atomic>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -42,6 +43,7 @@ bool overlaps(const void* a, uint64_t an, const void* b, uint64_t bn) {
     const auto x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
     return a && b && x < y + bn && y < x + an;
 }
+constexpr uint32_t kAnswers = 64;
 uint64_t align_up(uint64_t v, uint64_t a) { return (v + a - 1) / a * a; }
 }  // namespace
 
@@ -54,6 +56,8 @@ struct zc_hip_ctx {
     std::vector<hipEvent_t> tickets;   // live tickets: ticket t -> tickets[t - retired - 1]
     uint64_t retired = 0;              // tickets known complete and destroyed
     int32_t* moe_status = nullptr;     // device flag: an id outside [0,E) was seen
+    uint32_t* answers = nullptr;       // pinned words in which kernels answer gather checks, one per call in turn (calls of several threads may wait at once)
+    std::atomic<uint32_t> asked{0};
     hipEvent_t timer[2] = {nullptr, nullptr};
     // The prefill layer runs its shared expert beside the router, the selection and the dispatch sort, which are chains of
     // small kernels: a second stream of default priority, forked from and joined to `stream` by two events per call.
@@ -136,6 +140,10 @@ zc_status zc_hip_create(int device, uint64_t budget_bytes, zc_hip_ctx** out) {
     if (hipMalloc(&ctx->moe_status, 256) != hipSuccess || hipMemsetAsync(ctx->moe_status, 0, 256, ctx->stream) != hipSuccess) {
         hipStreamDestroy(ctx->stream); delete ctx; return fail(ZC_RUNTIME_ERROR, "HIP execution: cannot allocate status word");
     }
+    if (hipHostMalloc(reinterpret_cast<void**>(&ctx->answers), kAnswers * 4, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+        hipFree(ctx->moe_status); hipStreamDestroy(ctx->stream); delete ctx; return fail(ZC_RUNTIME_ERROR, "HIP execution: cannot allocate answer words");
+    }
+    std::memset(ctx->answers, 0, kAnswers * 4);
     *out = ctx;
     return ZC_OK;
 }
@@ -149,6 +157,7 @@ zc_status zc_hip_destroy(zc_hip_ctx* ctx) {
     for (auto& b : ctx->blocks) hipFree(b.first);
     for (auto& b : ctx->host_blocks) hipHostFree(b.first);
     hipFree(ctx->moe_status);
+    hipHostFree(ctx->answers);
     if (ctx->beside) { hipStreamSynchronize(ctx->beside); hipStreamDestroy(ctx->beside); }
     if (ctx->fork) hipEventDestroy(ctx->fork);
     if (ctx->join) hipEventDestroy(ctx->join);
@@ -446,6 +455,22 @@ zc_status zc_hip_router_logits(zc_hip_ctx* ctx, const void* w, const float* x, u
     ZC_LAUNCHED();
     return ZC_OK;
 }
+// Waits for the answer of a kernel that is on the stream.  The word is polled: waiting for the kernel's end would take the product's time too.
+static zc_status await_answer(zc_hip_ctx* ctx, const zc::GatherCheck& check) {
+    for (uint32_t polls = 1;; ++polls) {
+        const uint32_t word = __atomic_load_n(check.slot, __ATOMIC_ACQUIRE);
+        if ((word & ~1u) == check.answer) {
+            ZC_REQUIRE(!(word & 1u), "fused gate/up row outside input");
+            return ZC_OK;
+        }
+        __builtin_ia32_pause();
+        if (polls % 4096) continue;
+        const hipError_t state = hipStreamQuery(ctx->stream);   // (an error on the stream ends the wait; a stream that is done has stored the word)
+        if (state == hipErrorNotReady) { (void)hipGetLastError(); continue; }
+        ZC_HIP(state);
+        if ((__atomic_load_n(check.slot, __ATOMIC_ACQUIRE) & ~1u) != check.answer) return fail(ZC_RUNTIME_ERROR, "HIP execution: a gather's rows were not checked");
+    }
+}
 zc_status zc_hip_gated_linear(zc_hip_ctx* ctx, const zc_linear* gate, const zc_linear* up, const float* x, uint32_t x_rows,
                               uint32_t tokens, const int32_t* rows, float* out) {
     Timed timed(ctx, "gated_linear");
@@ -457,14 +482,25 @@ zc_status zc_hip_gated_linear(zc_hip_ctx* ctx, const zc_linear* gate, const zc_l
     ZC_REQUIRE(tokens && x && x_rows && (rows || x_rows >= tokens), "fused gate/up input shape");
     ZC_REQUIRE(out && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
                !overlaps(out, uint64_t(tokens) * gate->output * 4, x, uint64_t(x_rows) * gate->input * 4), "invalid or overlapping linear output");
-    if (rows) {   // metal.mm:852-856: every gathered row must lie inside x
-        std::vector<int32_t> host(tokens);
-        ZC_HIP(hipMemcpyAsync(host.data(), rows, uint64_t(tokens) * 4, hipMemcpyDeviceToHost, ctx->stream));
-        ZC_HIP(hipStreamSynchronize(ctx->stream));
-        for (int32_t r : host) ZC_REQUIRE(r >= 0 && uint32_t(r) < x_rows, "fused gate/up row outside input");
-    }
     zc::AffineDesc a; a.gate = *gate; a.up = *up; a.gated = true; a.x = x; a.in_rows = rows; a.out = out; a.tokens = tokens;
-    if (prefers_xint(ctx, *gate, 2, tokens) && zc::xint_supported(*gate) && zc::xint_supported(*up)) zc::launch_affine_xint(ctx->stream, a);
+    const bool xint = prefers_xint(ctx, *gate, 2, tokens) && zc::xint_supported(*gate) && zc::xint_supported(*up);
+    // metal.mm:852-856: every gathered row must lie inside x.  The GPU looks, since what is in front on the stream may write the list: the product's
+    // kernel itself if the list is short, so that the host waits while the product runs, else a kernel in front of it (a list as long as all
+    // input rows there can be, read by every workgroup, would cost more than the wait).
+    if (rows) {
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        ZC_HIP(hipStreamIsCapturing(ctx->stream, &capturing));
+        if (capturing != hipStreamCaptureStatusNone) return fail(ZC_RUNTIME_ERROR, "HIP execution: a gather's rows cannot be checked while the stream is captured");
+        const uint32_t turn = ctx->asked.fetch_add(1, std::memory_order_relaxed);
+        zc::GatherCheck check; check.slot = ctx->answers + turn % kAnswers; check.answer = (turn << 1) | 1u << 31; check.x_rows = x_rows;
+        const bool together = !xint && tokens <= zc::kGatherInKernel;
+        if (together) { a.check = check; zc::launch_affine(ctx->stream, a); }
+        else zc::launch_gather_check(ctx->stream, rows, tokens, check);
+        ZC_LAUNCHED();
+        if (const zc_status s = await_answer(ctx, check)) return s;
+        if (together) return ZC_OK;
+    }
+    if (xint) zc::launch_affine_xint(ctx->stream, a);
     else zc::launch_affine(ctx->stream, a);
     ZC_LAUNCHED();
     return ZC_OK;

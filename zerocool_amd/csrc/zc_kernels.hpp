@@ -6,6 +6,11 @@
 
 namespace zc {
 
+// Where a kernel tells the host whether the row list of a gather lies inside the input: *slot (pinned host memory) becomes
+// `answer`, plus one if a row does not.  A kernel that is handed one (slot not null) looks at the whole list first and does nothing else then.
+struct GatherCheck { uint32_t* slot = nullptr; uint32_t answer = 0, x_rows = 0; };
+constexpr uint32_t kGatherInKernel = 256;                        // rows that the product kernels look at themselves
+void launch_gather_check(hipStream_t s, const int32_t* rows, uint32_t n, const GatherCheck& check);   // any number of rows, a launch of its own
 struct AffineDesc {
     zc_linear gate, up;          // up used only when gated
     bool gated = false;
@@ -15,6 +20,7 @@ struct AffineDesc {
     float* out = nullptr;
     uint32_t tokens = 0;
     uint32_t float_output = 0;
+    GatherCheck check;           // literal lane arithmetic, at most kGatherInKernel rows
 };
 void launch_affine(hipStream_t s, const AffineDesc& a);          // literal lane arithmetic, any shape
 bool xint_supported(const zc_linear& l);                          // wide affine Q4, group 64, 16-byte aligned
