@@ -185,7 +185,7 @@ template <int BITS, int WIDTH, bool GATED>
 struct MatrixStream {
     using Form = MatrixForm<BITS, WIDTH>;
     static constexpr uint32_t kTileRows = GATED ? 4 : 8, kRows = GATED ? 1 : 2, DW = Form::DW;   // output rows of a tile, rows of a lane
-    struct Slot { uint32_t q[2][2 * DW]; uint32_t g[2]; };   // of each stream: two neighbouring blocks' codes, and their group's scale (even b) or bias (odd b)
+    struct Slot { uint32_t q[2][2 * DW]; uint16_t g[2]; };   // of each stream: two neighbouring blocks' codes, and their group's scale (even b) or bias (odd b)
     uint32_t K, N, steps, lane, tile, end, step;             // tile, step: the next one to request
     AffineMatrix m[2];
     const uint8_t* meta[GATED ? 2 : 1];                      // this lane's array: scales or biases
@@ -209,7 +209,9 @@ struct MatrixStream {
         }
         move(0, 0);
     }
-    __device__ __forceinline__ void fetch(Slot& slot) {      // past the end: the last tile again, not used
+    __device__ __forceinline__ void fetch(Slot& slot) {      // past the end: the matrix's first row, the same bytes in every lane, not used
+#pragma unroll
+        for (uint32_t i = 0; i < kRows; ++i) asm volatile("" : "+v"(w_at[i]), "+v"(g_at[i]));   // (else a step that is requested again is copied, which waits for it)
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const AffineMatrix& a = m[GATED ? q : 0];
@@ -223,9 +225,13 @@ struct MatrixStream {
         constexpr uint32_t kW = 32 * DW * 4, kG = Form::kStep / 64 * 2;
         if (++step < steps) { move(kW, kG); return; }
         step = 0;
-        if (tile + kMatrixWaves >= end) return;
-        tile += kMatrixWaves;
-        move(kMatrixWaves * kTileRows * (K / 8 * BITS) - (steps - 1) * kW, kMatrixWaves * kTileRows * (K / 64) * 2 - (steps - 1) * kG);
+        if (tile + kMatrixWaves < end) {
+            tile += kMatrixWaves;
+            move(kMatrixWaves * kTileRows * (K / 8 * BITS) - (steps - 1) * kW, kMatrixWaves * kTileRows * (K / 64) * 2 - (steps - 1) * kG);
+            return;
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < kRows; ++i) w_at[i] = g_at[i] = 0;
     }
 };
 
@@ -248,11 +254,27 @@ __device__ __forceinline__ float matrix_reduce(f32x4 v) {
     return s + dpp_f32<0x124>(s);   // row_ror:4
 }
 
+// The priority of a wave among those of its SIMD, by what is left of its workgroup's share (in steps): the top one at first, one less at
+// a half, a quarter and an eighth.  A SIMD issues its oldest wave first among equals, so that of four workgroups on a compute unit, with shares
+// alike, the first ended at 55 us and the last at 130, the end of it alone (64 tokens of hidden 3072 that agree, gate/up); this way those ahead
+// give way to those behind.
+struct MatrixPace {
+    uint32_t next, level;
+    __device__ __forceinline__ explicit MatrixPace(uint32_t all) : next(all / 2), level(3) { __builtin_amdgcn_s_setprio(3); }
+    __device__ __forceinline__ void left(uint32_t steps) {
+        if (steps > next || level == 0) return;
+        next /= 2; --level;
+        if (level == 2) __builtin_amdgcn_s_setprio(2);
+        else if (level == 1) __builtin_amdgcn_s_setprio(1);
+        else __builtin_amdgcn_s_setprio(0);
+    }
+};
+
 // The walk over tiles for nt <= TOKENS staged tokens (1, 2 or 4); out_at: where the output row of this lane's token begins; chains: lane s holds
 // step s's quad bits.  IMAGE (gate/up): output rows are images of the activations.
 template <int BITS, int WIDTH, bool GATED, uint32_t TOKENS, bool IMAGE>
-__device__ __forceinline__ void matrix_walk(MatrixStream<BITS, WIDTH, GATED>& st, typename MatrixStream<BITS, WIDTH, GATED>::Slot& next, const uint8_t* lds, uint32_t chains,
-                                            float* out, uint64_t out_at, uint32_t tile, bool float_output, uint32_t nt, uint32_t token) {
+__device__ __forceinline__ void matrix_walk(MatrixStream<BITS, WIDTH, GATED>& st, const typename MatrixStream<BITS, WIDTH, GATED>::Slot& next, const uint8_t* lds, uint32_t chains,
+                                            float* out, uint64_t out_at, uint32_t tile, bool float_output, uint32_t nt, uint32_t token, MatrixPace& pace, uint32_t after) {
     using Stream = MatrixStream<BITS, WIDTH, GATED>;
     using Slot = typename Stream::Slot;
     using Form = MatrixForm<BITS, WIDTH>;
@@ -265,16 +287,16 @@ __device__ __forceinline__ void matrix_walk(MatrixStream<BITS, WIDTH, GATED>& st
         for (uint32_t i = 0; i < 4 * TOKENS; ++i) (&acc[0][0][0])[i] = 0;
     };
     clear();
+    Slot ring[2] = {next, {}};
+    st.fetch(ring[1]);
     uint32_t step = 0;
-    for (uint32_t i = 0; i < total; ++i) {
+    auto one = [&](const Slot& now) {
         asm volatile("; %0 tokens" : : "n"(TOKENS));   // (else the walks' first steps move in front of the choice between the walks)
-        const Slot now = next;
-        st.fetch(next);
         const uint32_t chained = BITS == 4 ? uint32_t(__builtin_amdgcn_readlane(int(chains), int(step))) : 0u;
         float scale[2], bias[2];
 #pragma unroll
         for (int q = 0; q < 2; ++q) {   // (a bank of four lanes is one b: odd banks take the scale from the bank before, even ones the bias from the one behind)
-            const int mine = int(now.g[q] << 16);
+            const int mine = int(uint32_t(now.g[q]) << 16);
             scale[q] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(mine, mine, 0x114, 0xf, 0xa, false));
             bias[q] = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(mine, mine, 0x104, 0xf, 0x5, false));
         }
@@ -352,7 +374,7 @@ __device__ __forceinline__ void matrix_walk(MatrixStream<BITS, WIDTH, GATED>& st
                 else { multiply.template operator()<true>(bits); asm volatile("; chains run"); }   // (an end of its own: else the last sums of both ways are joined behind them)
             } else multiply.template operator()<false>(0);
         }
-        if (++step < st.steps) continue;
+        if (++step < st.steps) return;
         step = 0;
         float v[2];
         uint32_t in_tile;                                  // lane 4 b + j: row j of the tile, or of its second four
@@ -391,6 +413,19 @@ __device__ __forceinline__ void matrix_walk(MatrixStream<BITS, WIDTH, GATED>& st
             if (mine && (lane & 3u) == 0) matrix_image_put(out + out_at, st.N, row / 4, put);
         } else if (mine) out[out_at + row] = y;
         tile += kMatrixWaves;
+    };
+    // A slot is requested again, in place, as soon as its step is done.  (With a copy of the slot in use the compiler waited at the loop's end for all
+    // loads in flight; so it did where the loop could be left in its middle, hence the question in front of a step past the end.  Three slots: 3 to 8 % longer.)
+#pragma unroll 1
+    for (uint32_t i = 0; i < total; i += 2) {
+        pace.left(after + total - i);
+#pragma unroll
+        for (uint32_t k = 0; k < 2; ++k) {
+            if (i + k < total) one(ring[k]);
+            __builtin_amdgcn_sched_barrier(0);
+            st.fetch(ring[k]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
 }
 
@@ -414,12 +449,12 @@ __device__ __forceinline__ void matrix_strange_rows(const AffineMatrix (&m)[2], 
     }
 }
 
-// Tiles tile0 .. end - 1 (of MatrixStream) for nt <= 4 tokens: input row in_row(t), output row out_row(t).
+// Tiles tile0 .. end - 1 (of MatrixStream) for nt <= 4 tokens: input row in_row(t), output row out_row(t); after: rounds that the workgroup has left then.
 // IN: input rows are images (gate/up: made of the rows `fp32`; else written as images); OUT: output rows are to be.
 // (A workgroup that runs several of them waits in front of each: what the one before staged has then been read.)
 template <int BITS, int WIDTH, bool GATED, bool IN, bool OUT, class InRow, class OutRow>
 __device__ __forceinline__ void matrix_rows(const AffineMatrix (&m)[2], uint32_t K, uint32_t N, const float* x, const float* fp32, float* out, uint32_t nt,
-                                            InRow in_row, OutRow out_row, uint32_t tile0, uint32_t end, bool float_output, uint8_t* lds) {
+                                            InRow in_row, OutRow out_row, uint32_t tile0, uint32_t end, bool float_output, uint8_t* lds, MatrixPace& pace, uint32_t after) {
     using Stream = MatrixStream<BITS, WIDTH, GATED>;
     using Form = MatrixForm<BITS, WIDTH>;
     Stream st;
@@ -444,7 +479,7 @@ __device__ __forceinline__ void matrix_rows(const AffineMatrix (&m)[2], uint32_t
         if constexpr (BITS == 4) {
             for (uint32_t t = 0; t < nt; ++t) chains |= lds[Form::bits_at(K) + t * kMatrixSteps + min(st.lane, st.steps - 1)];
         }
-        auto walk = [&]<uint32_t TOKENS>() { matrix_walk<BITS, WIDTH, GATED, TOKENS, OUT>(st, next, lds, chains, out, out_at, first_tile, float_output, nt, token); };
+        auto walk = [&]<uint32_t TOKENS>() { matrix_walk<BITS, WIDTH, GATED, TOKENS, OUT>(st, next, lds, chains, out, out_at, first_tile, float_output, nt, token, pace, after * st.steps); };
         if (nt == 1) walk.template operator()<1>();
         else if (nt == 2) walk.template operator()<2>();
         else walk.template operator()<4>();
@@ -476,18 +511,19 @@ __device__ __forceinline__ void matrix_rows(const AffineMatrix (&m)[2], uint32_t
 
 // How the work of a launch, `jobs` jobs of `rounds` rounds (a tile per wave), is cut: workgroup w of n takes a contiguous piece, so that it stages a
 // job's rows once and all pieces are alike to a round; workgroups of one XCD (every eighth) take neighbouring pieces, so that the jobs of
-// one expert read its weights through one L2.  run(job, first round, end round).
+// one expert read its weights through one L2.  run(job, first round, end round, pace, rounds left then).
 template <class Run>
-__device__ __forceinline__ void matrix_piece_of_work(uint32_t jobs, uint32_t rounds, Run run) {
+__device__ __forceinline__ void matrix_piece_of_work(uint32_t jobs, uint32_t rounds, uint32_t steps, Run run) {
     const uint32_t n = gridDim.x, w = n % 8 == 0 ? blockIdx.x % 8 * (n / 8) + blockIdx.x / 8 : blockIdx.x;
     const uint64_t work = uint64_t(jobs) * rounds;
     const uint64_t first = work * w / n, end = work * (w + 1) / n;
     uint32_t job = uint32_t(first / rounds), round = uint32_t(first - uint64_t(job) * rounds);
     uint64_t left = end - first;
+    MatrixPace pace(uint32_t(left) * steps);
 #pragma unroll 1
     while (left) {
         const uint32_t take = uint32_t(min(left, uint64_t(rounds - round)));
-        run(job, round, round + take);
+        run(job, round, round + take, pace, uint32_t(left - take));
         left -= take; round = 0; ++job;
         if (left) lds_barrier();
     }

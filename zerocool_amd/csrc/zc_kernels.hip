@@ -67,12 +67,12 @@ template <int BITS, int WIDTH, bool GATED>
 __global__ __launch_bounds__(kMatrixThreads, 4) void affine_matrix_kernel(AffineJob j) {
     extern __shared__ __align__(16) uint8_t affine_lds[];
     if constexpr (GATED) { if (gather_refused(j)) return; }
-    matrix_piece_of_work((j.tokens - 1) / kMatrixTokens + 1, (j.tiles + kMatrixWaves - 1) / kMatrixWaves, [&](uint32_t job, uint32_t round, uint32_t rounds) {
+    matrix_piece_of_work((j.tokens - 1) / kMatrixTokens + 1, (j.tiles + kMatrixWaves - 1) / kMatrixWaves, MatrixForm<BITS, WIDTH>::steps(j.K), [&](uint32_t job, uint32_t round, uint32_t rounds, MatrixPace& pace, uint32_t after) {
         const uint64_t t0 = uint64_t(job) * j.chunk;
         matrix_rows<BITS, WIDTH, GATED, false, false>(j.m, j.K, j.N, j.x, nullptr, j.out, min(j.chunk, j.tokens - uint32_t(t0)),
                                                               [&](uint32_t t) { return j.in_rows ? uint32_t(j.in_rows[t0 + t]) : uint32_t(t0) + t; },
                                                               [&](uint32_t t) { return j.out_rows ? uint32_t(j.out_rows[t0 + t]) : uint32_t(t0) + t; },
-                                                              round * kMatrixWaves, min(rounds * kMatrixWaves, j.tiles), j.float_output != 0, affine_lds);
+                                                              round * kMatrixWaves, min(rounds * kMatrixWaves, j.tiles), j.float_output != 0, affine_lds, pace, after);
     });
 }
 
@@ -189,17 +189,17 @@ template <int BITS, int WIDTH, bool GATED, int SHARED>
 __global__ __launch_bounds__(kMatrixThreads, 4) void expert_matrix_kernel(ExpertPhase p) {
     extern __shared__ __align__(16) uint8_t affine_lds[];
     const uint32_t jobs = p.shared_jobs + uint32_t(uniform(*p.count));
-    matrix_piece_of_work(jobs, (p.tiles + kMatrixWaves - 1) / kMatrixWaves, [&](uint32_t job, uint32_t round, uint32_t rounds) {
+    matrix_piece_of_work(jobs, (p.tiles + kMatrixWaves - 1) / kMatrixWaves, MatrixForm<BITS, WIDTH>::steps(p.K), [&](uint32_t job, uint32_t round, uint32_t rounds, MatrixPace& pace, uint32_t after) {
         expert_job<GATED>(p, job, [&](const AffineMatrix (&m)[2], const float* x, float* out, uint32_t nt, auto in_row, auto out_row) {
             if constexpr (SHARED != BITS) {
                 if (job < p.shared_jobs) {
                     matrix_rows<SHARED, shared_width(BITS, WIDTH, SHARED), GATED, true, GATED>(m, p.K, p.N, x, p.fp32, out, nt, in_row, out_row, round * kMatrixWaves,
-                                                                                               min(rounds * kMatrixWaves, p.tiles), false, affine_lds);
+                                                                                               min(rounds * kMatrixWaves, p.tiles), false, affine_lds, pace, after);
                     return;
                 }
             }
             matrix_rows<BITS, WIDTH, GATED, true, GATED>(m, p.K, p.N, x, p.fp32, out, nt, in_row, out_row, round * kMatrixWaves,
-                                                                 min(rounds * kMatrixWaves, p.tiles), false, affine_lds);
+                                                                 min(rounds * kMatrixWaves, p.tiles), false, affine_lds, pace, after);
         });
     });
 }
