@@ -61,7 +61,7 @@ struct zc_hip_ctx {
     hipEvent_t timer[2] = {nullptr, nullptr};
     // The prefill layer runs its shared expert beside the router, the selection and the dispatch sort, which are chains of
     // small kernels: a second stream of default priority, forked from and joined to `stream` by two events per call.
-    hipStream_t beside = nullptr; hipEvent_t fork = nullptr, join = nullptr;
+    hipStream_t beside = nullptr; hipEvent_t fork = nullptr, rows_ready = nullptr, join = nullptr;
     // 0 literal lane kernels, 1 exact-integer matrix-core kernels where possible, 2 the lanes except where prefers_xint() says otherwise.
     uint32_t affine_policy = 2;
     void* static_scratch = nullptr;    // this device's copy of the static scratch array
@@ -159,8 +159,7 @@ zc_status zc_hip_destroy(zc_hip_ctx* ctx) {
     hipFree(ctx->moe_status);
     hipHostFree(ctx->answers);
     if (ctx->beside) { hipStreamSynchronize(ctx->beside); hipStreamDestroy(ctx->beside); }
-    if (ctx->fork) hipEventDestroy(ctx->fork);
-    if (ctx->join) hipEventDestroy(ctx->join);
+    for (hipEvent_t e : {ctx->fork, ctx->rows_ready, ctx->join}) if (e) hipEventDestroy(e);
     hipStreamDestroy(ctx->stream);
     delete ctx;
     return ZC_OK;
@@ -747,7 +746,7 @@ struct PrefillSpace {
     uint32_t max_tiles, max_shared_tiles;
     uint32_t* near_bits;      // one bit per product element: recompute exactly
     uint32_t* shared_near_bits;   // the same for the shared expert's products, which run beside the routed ones
-    float* norms;             // |row| of the inputs and of the router's rows (the fast router's bound)
+    float* norms;             // |row| of the inputs and of the router's rows (the router on bounds)
     uint64_t bytes;
 };
 PrefillSpace carve_prefill(const zc_moe_config* c, uint32_t T, void* base) {
@@ -774,6 +773,10 @@ PrefillSpace carve_prefill(const zc_moe_config* c, uint32_t T, void* base) {
     w.bytes = at;
     return w;
 }
+// From here on the router on bounds is ahead: the exact one's chains fill the chip, where the other's short kernels leave room for the
+// shared expert beside them.  us a layer, exact logits / bounds: hidden 2048 without router skew, 200 tokens 318 / 350, 400 352 / 365, 700 393 / 406, 2048
+// 637 / 626; hidden 3072 with Zipf(1.1) offsets, 128 tokens 259 / 304, 300 392 / 420, 700 669 / 672, 1500 1187 / 1169.
+constexpr uint32_t kPrefillBoundsTokens = 768;
 bool prefill_config(const zc_moe_config* c) {
     // every projection affine Q4 or affine Q8 (the mixed 4/8-bit artifact: Q4 routed gate/up, Q8 down and shared expert)
     auto q = [](uint32_t bits) { return bits == 4 || bits == 8; };
@@ -803,22 +806,27 @@ zc_status zc_hip_moe_prefill(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
     const uint32_t H = c->hidden, I = c->inter, E = c->experts, k = c->topk;
     const uint64_t n = uint64_t(T) * k;
     const bool half_out = !(trace && trace->expert_out) && reinterpret_cast<uintptr_t>(out) % 16 == 0;
-    // router logits, top-k + softmax, dispatch (model.cpp:434-479), shared gate: the exact kernels, except that a long batch
-    // whose logits nobody asks for gets exact logits only where the selection can see the difference (launch_prefill_router)
-    const bool x_q4 = c->bits_gate_up == 4 || c->shared_bits_gate_up == 4, x_q8 = c->bits_gate_up == 8 || c->shared_bits_gate_up == 8;
-    zc::launch_prefill_rows(s, x, T, H, w.xb, w.xp, x_q4 ? w.xplanes : nullptr, x_q8 ? w.xplain : nullptr, x_q4 ? w.xsum16 : nullptr, ctx->moe_status);
-    // the shared expert needs the bf16 rows and nothing of the routing: it runs on a stream of its own from here to the combine
-    if (!ctx->beside) {
-        ZC_HIP(hipStreamCreateWithFlags(&ctx->beside, hipStreamNonBlocking));
-        ZC_HIP(hipEventCreateWithFlags(&ctx->fork, hipEventDisableTiming)); ZC_HIP(hipEventCreateWithFlags(&ctx->join, hipEventDisableTiming));
-    }
+    // router logits, top-k + softmax, dispatch (model.cpp:434-479): the exact kernels, except that a long batch whose logits nobody asks
+    // for gets exact logits only where the selection can see the difference (launch_prefill_router).  The shared expert needs the matrix
+    // cores' rows and nothing of the routing: it runs on a stream of its own from there to the combine.  The exact router needs the inputs
+    // only, so that the rows are made beside it.
+    for (hipEvent_t* e : {&ctx->fork, &ctx->rows_ready, &ctx->join}) if (!*e) ZC_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming));
+    if (!ctx->beside) ZC_HIP(hipStreamCreateWithFlags(&ctx->beside, hipStreamNonBlocking));
     hipStream_t s2 = ctx->beside;
+    const bool bounds = T >= kPrefillBoundsTokens && !(trace && trace->logits);
+    const bool x_q4 = c->bits_gate_up == 4 || c->shared_bits_gate_up == 4, x_q8 = c->bits_gate_up == 8 || c->shared_bits_gate_up == 8;
+    auto rows_on = [&](hipStream_t t) {
+        zc::launch_prefill_rows(t, x, T, H, w.xb, w.xp, x_q4 ? w.xplanes : nullptr, x_q8 ? w.xplain : nullptr, x_q4 ? w.xsum16 : nullptr, ctx->moe_status);
+    };
+    if (bounds) rows_on(s);
     ZC_HIP(hipEventRecord(ctx->fork, s)); ZC_HIP(hipStreamWaitEvent(s2, ctx->fork, 0));
-    if (T >= 128 && !(trace && trace->logits)) {
+    if (bounds) {
         const bool select = k <= 64;   // the refinement's wavefront selects its token's experts too
         zc::launch_prefill_router(s, x, w.xb, l->router, l->router_offsets, T, H, E, k, w.norms, w.base.logits, select ? w.base.ids : nullptr, select ? w.base.weights : nullptr);
         if (!select) zc::launch_route(s, w.base.logits, T, E, k, w.base.ids, w.base.weights);
     } else {
+        rows_on(s2);
+        ZC_HIP(hipEventRecord(ctx->rows_ready, s2));
         zc::launch_router(s, l->router, x, T, H, E, l->router_offsets, w.base.logits);
         zc::launch_route(s, w.base.logits, T, E, k, w.base.ids, w.base.weights);
     }
@@ -839,6 +847,7 @@ zc_status zc_hip_moe_prefill(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
             off[3 * q + 2] = reinterpret_cast<uintptr_t>(lin.biases) - base;
         }
     };
+    if (!bounds) ZC_HIP(hipStreamWaitEvent(s, ctx->rows_ready, 0));
     {   // routed gate/up + SwiGLU on gathered rows (pipeline.cpp:18-24), then down scattered to the slots (pipeline.cpp:25-29)
         zc::PrefillGemm g{};
         g.bits = c->bits_gate_up;

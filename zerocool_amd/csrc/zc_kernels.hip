@@ -560,139 +560,6 @@ __global__ __launch_bounds__(256) void router_short_kernel(const uint16_t* __res
     const uint32_t e = e0 + j;
     if (split < nt && e < E) out[uint64_t(t0 + split) * E + e] = offsets ? sum + offsets[e] : sum;
 }
-// The same chains for long batches, register-tiled: a lane owns one K partition for 4 tokens x 4 experts, so every
-// sixteen-byte weight piece and every eight inputs feed sixteen multiply-accumulate chains.  A workgroup covers
-// 16 tokens x 16 experts; lane = (partition, token group, expert group).
-__global__ __launch_bounds__(256) void router_tiled_kernel(const uint16_t* w, const float* x, uint32_t T, uint32_t K,
-                                                           uint32_t E, const float* offsets, float* out) {
-    const uint32_t split = threadIdx.x % 16, pair = threadIdx.x / 16, tg = pair % 4, eg = pair / 4;
-    const uint32_t t0 = blockIdx.y * 16 + tg * 4, e0 = blockIdx.x * 16 + eg * 4, P = K / 16;
-    float c[4][4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) c[t][e] = 0;
-    const float* xr[4]; const uint16_t* wr[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) xr[t] = x + uint64_t(min(t0 + t, T - 1)) * K + split * P;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) wr[e] = w + uint64_t(min(e0 + e, E - 1)) * K + split * P;
-    for (uint32_t i = 0; i < P; i += 8) {
-        float xv[4][8], wv[4][8];
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const float4 a = *reinterpret_cast<const float4*>(xr[t] + i), b = *reinterpret_cast<const float4*>(xr[t] + i + 4);
-            xv[t][0] = a.x; xv[t][1] = a.y; xv[t][2] = a.z; xv[t][3] = a.w; xv[t][4] = b.x; xv[t][5] = b.y; xv[t][6] = b.z; xv[t][7] = b.w;
-        }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const uint4 v = *reinterpret_cast<const uint4*>(wr[e] + i);
-            const uint32_t ww[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-            for (int k = 0; k < 8; ++k) wv[e][k] = __uint_as_float((k & 1) ? (ww[k / 2] & 0xffff0000u) : (ww[k / 2] << 16));
-        }
-#pragma unroll
-        for (int t = 0; t < 4; ++t)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int k = 0; k < 8; ++k) c[t][e] = __builtin_fmaf(xv[t][k], wv[e][k], c[t][e]);
-    }
-    const uint32_t base = (threadIdx.x & 63u) & ~15u;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            float sum = 0;
-            for (uint32_t sidx = 0; sidx < 16; ++sidx) sum += __shfl(c[t][e], base + sidx);
-            if (split == 0 && e0 + e < E && t0 + t < T) out[uint64_t(t0 + t) * E + e0 + e] = offsets ? sum + offsets[e0 + e] : sum;
-        }
-}
-// Long batches with K a multiple of 256: a workgroup of 512 threads covers 32 tokens x 16 experts and stages 16 elements
-// of every K partition through LDS at a time (whole 64-byte pieces of the inputs, read once per workgroup), so a token
-// row is fetched from the L2 by 32 workgroups instead of 128.  Lane = (partition, token group, expert group) with a
-// 4 x 4 register tile as above; the chains still run k-ascending inside each partition.  The chunk is small on purpose:
-// 52 KB of LDS and few registers let two or three workgroups share a compute unit and hide each other's load latency.
-constexpr uint32_t kRouterChunk = 16;
-constexpr uint32_t kRouterXPitch = 20, kRouterWPitch = 12;   // words per (row, partition) piece: 16 fp32 + 4, 16 bf16 + 4 (conflict-free 16-/8-byte reads)
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void router_block_kernel(const uint16_t* w, const float* x, uint32_t T, uint32_t K,
-                                                              uint32_t E, const float* offsets, float* out) {
-    __shared__ __align__(16) uint32_t xs[32 * 16 * kRouterXPitch];   // [token][partition][16 fp32]
-    __shared__ __align__(16) uint32_t ws[16 * 16 * kRouterWPitch];   // [expert][partition][16 bf16]
-    const uint32_t tid = threadIdx.x, split = tid % 16, pair = tid / 16, tg = pair % 8, eg = pair / 8;
-    const uint32_t t0 = blockIdx.y * 32, e0 = blockIdx.x * 16, P = K / 16;
-    float c[4][4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) c[t][e] = 0;
-    // staging duty per chunk: 32 rows x 16 partitions x 4 sixteen-byte parts of x (4 per thread), 16 x 16 x 2 of w (1 per thread)
-    // staging registers as plain 32-bit words (arrays of the vector type end up in scratch memory here)
-    uint32_t xr[16], wr[4];
-    auto fetch = [&](uint32_t chunk) {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t piece = tid + q * 512, part = piece % 4, sp = (piece / 4) % 16, row = piece / 64;
-            const uint4 v = *reinterpret_cast<const uint4*>(x + uint64_t(min(t0 + row, T - 1)) * K + sp * P + chunk * kRouterChunk + part * 4);
-            xr[4 * q] = v.x; xr[4 * q + 1] = v.y; xr[4 * q + 2] = v.z; xr[4 * q + 3] = v.w;
-        }
-        {
-            const uint32_t part = tid % 2, sp = (tid / 2) % 16, row = tid / 32;
-            const uint4 v = ldg_u4(w + uint64_t(min(e0 + row, E - 1)) * K + sp * P + chunk * kRouterChunk + part * 8);
-            wr[0] = v.x; wr[1] = v.y; wr[2] = v.z; wr[3] = v.w;
-        }
-    };
-    auto stash = [&]() {
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t piece = tid + q * 512, part = piece % 4, sp = (piece / 4) % 16, row = piece / 64;
-            *reinterpret_cast<uint4*>(&xs[(row * 16 + sp) * kRouterXPitch + part * 4]) = make_uint4(xr[4 * q], xr[4 * q + 1], xr[4 * q + 2], xr[4 * q + 3]);
-        }
-        {
-            const uint32_t part = tid % 2, sp = (tid / 2) % 16, row = tid / 32;
-            *reinterpret_cast<uint4*>(&ws[(row * 16 + sp) * kRouterWPitch + part * 4]) = make_uint4(wr[0], wr[1], wr[2], wr[3]);
-        }
-    };
-    const uint32_t chunks = P / kRouterChunk;
-    fetch(0);
-    for (uint32_t chunk = 0; chunk < chunks; ++chunk) {
-        __syncthreads();            // the previous chunk has been consumed
-        stash();
-        __syncthreads();
-        if (chunk + 1 < chunks) fetch(chunk + 1);
-#pragma unroll
-        for (int k = 0; k < int(kRouterChunk); k += 4) {
-            float xv[4][4], wv[4][4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const uint4 v = *reinterpret_cast<const uint4*>(&xs[((tg * 4 + t) * 16 + split) * kRouterXPitch + k]);
-                xv[t][0] = __uint_as_float(v.x); xv[t][1] = __uint_as_float(v.y); xv[t][2] = __uint_as_float(v.z); xv[t][3] = __uint_as_float(v.w);
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint2 v = *reinterpret_cast<const uint2*>(&ws[((eg * 4 + e) * 16 + split) * kRouterWPitch + k / 2]);
-                wv[e][0] = __uint_as_float(v.x << 16); wv[e][1] = __uint_as_float(v.x & 0xffff0000u);
-                wv[e][2] = __uint_as_float(v.y << 16); wv[e][3] = __uint_as_float(v.y & 0xffff0000u);
-            }
-#pragma unroll
-            for (int t = 0; t < 4; ++t)
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) c[t][e] = __builtin_fmaf(xv[t][i], wv[e][i], c[t][e]);
-        }
-    }
-    const uint32_t base = (tid & 63u) & ~15u;
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            float sum = 0;
-            for (uint32_t sidx = 0; sidx < 16; ++sidx) sum += __shfl(c[t][e], base + sidx);
-            const uint32_t tt = t0 + tg * 4 + t, ee = e0 + eg * 4 + e;
-            if (split == 0 && ee < E && tt < T) out[uint64_t(tt) * E + ee] = offsets ? sum + offsets[ee] : sum;
-        }
-}
 void launch_router(hipStream_t s, const void* w, const float* x, uint32_t T, uint32_t K, uint32_t E,
                    const float* offsets, float* out, const void* gate_w, float* gate, int32_t* status) {
     const auto row_bytes = [&](uint32_t rows) { return size_t(rows) * (K + 64) * 4; };
@@ -717,15 +584,8 @@ void launch_router(hipStream_t s, const void* w, const float* x, uint32_t T, uin
         return;
     }
     if (gate_w) launch_plain(s, gate_w, 0, x, K, 1, T, gate, false);
-    if (T >= 256 && K % 256 == 0) {
-        hipLaunchKernelGGL(router_block_kernel, dim3((E + 15) / 16, (T + 31) / 32), dim3(512), 0, s, (const uint16_t*)w, x, T, K, E, offsets, out);
-        return;
-    }
-    // (64 tokens come here with rows too long for the short kernel, from 4096 inputs on.  The general kernel's workgroups hold 16
-    // experts x 4 tokens, one round of them for up to 256 experts: 34 us there, 65 at 320 to 512 and 127 at 1024; the tiled one
-    // takes 50 to 51 us whatever the number.)
-    if ((T > 64 || (T == 64 && E > 256)) && K % 128 == 0) {
-        hipLaunchKernelGGL(router_tiled_kernel, dim3((E + 15) / 16, (T + 15) / 16), dim3(256), 0, s, (const uint16_t*)w, x, T, K, E, offsets, out);
+    if (T >= 64 && K % 128 == 0) {
+        launch_router_batch(s, w, x, T, K, E, offsets, out);
         return;
     }
     const uint32_t gx = (E + 15) / 16;

@@ -55,6 +55,8 @@ void launch_plain(hipStream_t s, const void* w, uint32_t dtype, const float* x, 
 constexpr uint32_t kRouterShortLds = 64 * 1024, kRouterStatusK = 3968;
 void launch_router(hipStream_t s, const void* w, const float* x, uint32_t T, uint32_t K, uint32_t E,
                    const float* offsets, float* out, const void* gate_w = nullptr, float* gate = nullptr, int32_t* status = nullptr);
+// the same of long batches, K a multiple of 128 (zc_router.hip)
+void launch_router_batch(hipStream_t s, const void* w, const float* x, uint32_t T, uint32_t K, uint32_t E, const float* offsets, float* out);
 void launch_route(hipStream_t s, const float* logits, uint32_t T, uint32_t E, uint32_t topk, int32_t* ids, float* weights);
 void launch_dispatch(hipStream_t s, const int32_t* ids, uint32_t tokens, uint32_t topk, uint32_t E, int32_t* offsets,
                      int32_t* slots, int32_t* rows, int32_t* selected, int32_t* count, int32_t* status);

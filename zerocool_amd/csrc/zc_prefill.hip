@@ -36,7 +36,7 @@
 // forty rows per expert -- an unskewed router at 2048 tokens -- every expert's codes are then expanded once, not twice.
 #include "zc_kernels.hpp"
 #include "zc_device.hpp"
-#include "zc_decode_common.hpp"   // route_token: top-k + softmax of one token by one wavefront
+#include "zc_decode_common.hpp"   // lds_barrier; route_token: top-k + softmax of one token by one wavefront
 
 namespace zc {
 
