@@ -1,0 +1,36 @@
+"""The prefill products' first requests: rows of 33 to 64 scale groups, whole and broken pieces of eight groups, tiles of one row to three
+blocks, against the exact layer (its outputs byte for byte but for sums on a rounding boundary)."""
+import numpy as np
+import pytest
+import zerocool_amd as z
+from zerocool_amd import workload
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = z.Context(0)
+    yield c
+    c.close()
+
+
+# groups of hidden and intermediate rows: 34 and 36, 40 and 42, 62 and 64, 2 and 6
+@pytest.mark.parametrize("hidden,inter,bits", [(2176, 2304, (4, 4, 4, 4)), (2560, 2688, (4, 8, 8, 8)), (3968, 4096, (4, 4, 4, 4)), (128, 384, (8, 4, 4, 8))])
+@pytest.mark.parametrize("T", [1, 15, 33, 47])
+def test_prefill_matches_the_exact_layer(ctx, hidden, inter, bits, T):
+    cfg = workload.tiny_config(hidden, 3, 2, inter, bits=bits)
+    weights = workload.LayerWeights(ctx, cfg, 17 + T, ("normal", 0.5))
+    x, outs = workload.hidden_rows(ctx, T, hidden, 18), []
+    for call, size in ((ctx.moe_forward, ctx.moe_workspace_bytes), (ctx.moe_prefill, ctx.moe_prefill_workspace_bytes)):
+        out, ws = ctx.alloc(T * hidden * 4), ctx.alloc(size(cfg, T))
+        call(cfg, weights.layer, x, T, out, ws)
+        ctx.moe_check()
+        outs.append(out.numpy(f32).copy())
+        ctx.free(out); ctx.free(ws)
+    exact, fast = outs
+    assert np.max(np.abs(fast - exact)) <= 2e-3 * np.max(np.abs(exact))
+    assert np.mean(fast.view(np.uint32) == exact.view(np.uint32)) > 0.9999
+    for b in (weights.router, weights.shared_gate, weights.shared_record, weights.records, x):
+        ctx.free(b)

@@ -148,7 +148,7 @@ struct PrefillGemm {
     const uint16_t* a_plain;  // the same rows as bf16 in their own order (read by the recomputation)
     const uint16_t* planes;   // per (row, group of 64): the input sum in three bf16 pieces
     const float* asum16;      // per (row, block of 16): that block's chain sum (read by the recomputation; null: formed there)
-    const int32_t* a_rows;    // row of `a` for sorted position pos: a_rows ? a_rows[pos] : pos
+    const int32_t* a_rows;    // row of `a` for sorted position pos: a_rows ? a_rows[pos] : pos   (gate/up; down: null)
     const int32_t* out_rows;  // output row for sorted position pos: out_rows ? out_rows[pos] : pos   (down projection)
     const uint8_t* records; uint64_t stride;   // expert e's record at records + e * stride
     uint64_t off[6];          // byte offsets in a record: codes, scales, biases of the (gate | down) projection, then of up

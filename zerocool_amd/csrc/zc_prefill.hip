@@ -282,6 +282,23 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, j = lane & 15u, g4 = lane >> 4;
     const uint32_t K = p.K, N = p.N, groups = K / 64, pairs = K / 128;
     const uint8_t* record = p.records + uint64_t(expert) * p.stride;
+    // What a workgroup needs before its walk is requested in one go, the indices of its rows first: loads return in the order they were
+    // sent, and only the rows have to wait for an answer.  (Indices, rows, biases and chain sums one after the other were four more
+    // latencies of a workgroup that lives about ten.  us a layer: 2048 tokens of hidden 2048 642 -> 618, 700 397 -> 377, 300 of the mixed artifact 365 ->
+    // 342, 1500 of hidden 3072 1190 -> 1143.  With that the bytes in flight are enough: tiles of sixteen rows in a kernel with four pairs
+    // of weights in flight and four waves a SIMD took 304 us for 200 tokens where this takes 302, and 433 where this takes 369, 300 tokens of
+    // hidden 3072 behind Zipf(1.1) offsets.)
+    // Row of `a` for row m of the tile; rows past the end repeat the last one (never stored).  Thread: sixteen bytes of one row of every block.
+    uint32_t a_row[NB];
+#pragma unroll
+    for (int rb = 0; rb < NB; ++rb) {
+        const uint32_t pos = first + min(16 * uint32_t(rb) + (tid >> 4), rows - 1);
+        a_row[rb] = pos;
+        if constexpr (GATED) {   // (without a list of rows: a word that is there, not used)
+            const uint32_t listed = *as_global<uint32_t>(p.a_rows ? p.a_rows + pos : p.tile_count);
+            a_row[rb] = p.a_rows ? listed : pos;
+        }
+    }
     // The wave's two column tiles (rows of the workgroup's 128 weight rows) for every block of sixteen token rows; gate/up:
     // a gate tile and the up tile of the same rows.  The codes go from memory straight into the lanes that feed them to
     // the matrix cores, whole 64-byte pieces of a row per load.
@@ -304,25 +321,6 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
     };
 #pragma unroll
     for (int d = 0; d + 1 < kAhead; ++d) fetch_b(uint32_t(d), ring[d]);
-    auto row_of = [&](uint32_t m) {              // row of `a` for row m of the tile; rows past the end repeat the last one (never stored)
-        const uint32_t pos = first + min(m, rows - 1);
-        return p.a_rows ? uint32_t(p.a_rows[pos]) : pos;
-    };
-    const uint16_t* a_src[NB];                   // thread: sixteen bytes of one row of every block
-    const uint32_t a_at = (tid >> 4) * kPitch + (tid & 15u) * 8;
-#pragma unroll
-    for (int rb = 0; rb < NB; ++rb) a_src[rb] = p.a + uint64_t(row_of(16 * uint32_t(rb) + (tid >> 4))) * K + (tid & 15u) * 8;
-    u32x4 a_next[NB];
-    auto fetch_a = [&](uint32_t pair, u32x4 (&to)[NB]) {
-#pragma unroll
-        for (int rb = 0; rb < NB; ++rb) to[rb] = *as_global<u32x4>(a_src[rb] + min(pair, pairs - 1) * 128);
-    };
-    auto stash_a = [&](uint32_t buf, const u32x4 (&from)[NB]) {
-#pragma unroll
-        for (int rb = 0; rb < NB; ++rb) *reinterpret_cast<u32x4*>(a_s + (buf * kTileRowsMax + 16 * uint32_t(rb)) * kPitch + a_at) = from[rb];
-    };
-    u32x4 a_first[NB];
-    fetch_a(0, a_first); fetch_a(1, a_next);
     // The scales of the lane's two weight rows, four groups per load (the four lanes of a row fetch the same bytes), one load
     // ahead.  (In LDS, filled by a loop of dependent loads and stores before the walk, they cost 11 us of a workgroup's
     // 29: nearly as much as the walk.)  A row's last load may run into the rows behind it, which the biases always follow.
@@ -335,6 +333,48 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
         }
     };
     fetch_s(0);
+    // biases of eight groups of the lane's two weight rows, for up to 64 groups (past the end: not used)
+    const uint32_t pitch = prefill_pitch(K);
+    uint4 bias_first[2][2];
+    auto fetch_biases = [&](int part) {
+        const uint32_t mine = 32 * uint32_t(part) + 8 * g4;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            if (groups % 8 == 0) bias_first[part][q] = ldg_u4_by_words(biases_of[q] + (m_at[q] + min(mine, groups - 8) * 2));
+            else {
+                uint32_t w[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[i] = ldg_u32(biases_of[q] + (m_at[q] + min(mine + 2 * uint32_t(i), groups - 2) * 2));
+                bias_first[part][q] = make_uint4(w[0], w[1], w[2], w[3]);
+            }
+        }
+    };
+    fetch_biases(0);
+    if (groups > 32) fetch_biases(1);
+    const uint16_t* a_src[NB];
+    const uint32_t a_at = (tid >> 4) * kPitch + (tid & 15u) * 8;
+#pragma unroll
+    for (int rb = 0; rb < NB; ++rb) a_src[rb] = p.a + uint64_t(a_row[rb]) * K + (tid & 15u) * 8;
+    u32x4 a_next[NB];
+    auto fetch_a = [&](uint32_t pair, u32x4 (&to)[NB]) {
+#pragma unroll
+        for (int rb = 0; rb < NB; ++rb) to[rb] = *as_global<u32x4>(a_src[rb] + min(pair, pairs - 1) * 128);
+    };
+    auto stash_a = [&](uint32_t buf, const u32x4 (&from)[NB]) {
+#pragma unroll
+        for (int rb = 0; rb < NB; ++rb) *reinterpret_cast<u32x4*>(a_s + (buf * kTileRowsMax + 16 * uint32_t(rb)) * kPitch + a_at) = from[rb];
+    };
+    u32x4 a_first[NB];
+    fetch_a(0, a_first); fetch_a(1, a_next);
+    // chain sums: the rows' pieces as they lie in memory, sixteen threads a row
+    const uint32_t octets = pitch / 8, row_octets = 3 * octets;
+    uint4 sums_first[2][NB];
+    auto fetch_sums = [&](int part) {
+#pragma unroll
+        for (int rb = 0; rb < NB; ++rb) sums_first[part][rb] = ldg_u4(p.planes + uint64_t(a_row[rb]) * (3 * pitch) + min(16 * uint32_t(part) + (tid & 15u), row_octets - 1) * 8);
+    };
+    fetch_sums(0);
+    if (groups > 32) fetch_sums(1);
     f32x4 total[NB][2], mag[NB][2];   // mag: sum of the magnitudes of the folded terms, the scale of the rounding error
 #pragma unroll
     for (int rb = 0; rb < NB; ++rb)
@@ -348,36 +388,25 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
     // bias half in front of the walk 0.22, 0.23, 0.24.  (Eight groups at once in front of their dots 0.22, 0.17, 0.15.)  The layer of
     // 2048 tokens of hidden 2048 takes 628 us, with all of it in front of the walk 620; 1500 tokens of hidden 3072 1166 and 1192.
     // Chain sums and biases wait in LDS, zeros behind the last group.
-    const uint32_t pitch = prefill_pitch(K);
     uint16_t *planes_s = bias_s + 8, *biases_s = planes_s + kTileRowsMax * 3 * pitch;
     const uint32_t col[2] = {(GATED ? wave : 2 * wave) * 16 + j, (GATED ? 4 + wave : 2 * wave + 1) * 16 + j};
     if (tid < 4) reinterpret_cast<uint32_t*>(bias_s)[tid] = 0;
-    const uint16_t* planes_of = p.planes + uint64_t(row_of(16 * min(wave, uint32_t(NB) - 1) + j)) * (3 * pitch);   // wave w: block w
-    uint32_t g0 = 0;
-    do {   // (at least once: the compiler then knows that no load from before it is pending in the walk)
-        const uint32_t mine = g0 + 8 * g4;
-        uint4 bias[2], piece[3];
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            uint32_t w[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) w[i] = ldg_u32(biases_of[q] + (m_at[q] + min(mine + 2 * uint32_t(i), groups - 2) * 2));
-            bias[q] = make_uint4(w[0], w[1], w[2], w[3]);
-        }
-#pragma unroll
-        for (int w = 0; w < 3; ++w) piece[w] = ldg_u4(planes_of + min(mine, pitch - 8) + uint32_t(w) * pitch);
-        auto store = [&](uint16_t* at, uint4 v) {
-            *reinterpret_cast<uint4*>(at) = make_uint4(v.x, mine + 2 < groups ? v.y : 0u, mine + 4 < groups ? v.z : 0u, mine + 6 < groups ? v.w : 0u);
-        };
+    auto store = [&](uint16_t* at, uint4 v, uint32_t g) {   // of the groups g .. g + 7
+        *reinterpret_cast<uint4*>(at) = make_uint4(v.x, g + 2 < groups ? v.y : 0u, g + 4 < groups ? v.z : 0u, g + 6 < groups ? v.w : 0u);
+    };
+    auto store_first = [&](int part) {
+        const uint32_t mine = 32 * uint32_t(part) + 8 * g4, i = 16 * uint32_t(part) + (tid & 15u), piece = (i >= octets ? 1u : 0u) + (i >= 2 * octets ? 1u : 0u);
         if (mine < pitch) {
 #pragma unroll
-            for (int q = 0; q < 2; ++q) store(biases_s + col[q] * pitch + mine, bias[q]);
-            if (wave < NB) {
-#pragma unroll
-                for (uint32_t w = 0; w < 3; ++w) store(planes_s + ((wave * 16 + j) * 3 + w) * pitch + mine, piece[w]);
-            }
+            for (int q = 0; q < 2; ++q) store(biases_s + col[q] * pitch + mine, bias_first[part][q], mine);
         }
-    } while ((g0 += 32) < groups);
+        if (i < row_octets) {
+#pragma unroll
+            for (int rb = 0; rb < NB; ++rb) store(planes_s + (16 * uint32_t(rb) + (tid >> 4)) * (3 * pitch) + i * 8, sums_first[part][rb], (i - piece * octets) * 8);
+        }
+    };
+    store_first(0);
+    if (groups > 32) store_first(1);
     auto from_lds = [](const uint16_t* at) { return *reinterpret_cast<const uint4*>(at); };
     const uint16_t* sums_at = bias_s + (g4 < 3 ? 8 + (j * 3 + g4) * pitch : 0u);
     const uint32_t sums_rb = g4 < 3 ? 48 * pitch : 0u;
@@ -513,6 +542,13 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
         add_biases(2 * pair);
         work(pair, ring[0], ring[1], 0);
     }
+    uint32_t out_row[NB];                        // (asked for here, the answer is back when the outputs are)
+#pragma unroll
+    for (int rb = 0; rb < NB; ++rb) {
+        const uint32_t pos = first + min(16 * uint32_t(rb) + (tid >> 4), rows - 1);
+        out_row[rb] = pos;
+        if constexpr (!GATED) { if (p.out_rows) out_row[rb] = ldg_u32(p.out_rows, pos); }
+    }
     add_bias_sizes();
     // epilogue: row m of the tile is sorted position first + m.  A sum close to a BF16 rounding boundary could round
     // the other way under the reference's order of additions: such elements are listed for exact recomputation.  v rounds to
@@ -558,7 +594,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
             *reinterpret_cast<uint4*>(p.out_b + uint64_t(pos) * N + n0 + c * 8) = v;
             if (c == 0) *reinterpret_cast<uint2*>(p.near_bits + (uint64_t(pos) * N + n0) / 32) = *reinterpret_cast<const uint2*>(marks_s + m * 8);
         } else {
-            const uint64_t at = uint64_t(p.out_rows ? uint32_t(p.out_rows[pos]) : pos) * N + n0 + c * 8;
+            const uint64_t at = uint64_t(out_row[i]) * N + n0 + c * 8;   // (a piece's row is the thread's row of block i)
             if (p.out_h) *reinterpret_cast<uint4*>(p.out_h + at) = v;
             else {
                 *reinterpret_cast<float4*>(p.out_f + at) = make_float4(__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u));
