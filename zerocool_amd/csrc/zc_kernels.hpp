@@ -147,7 +147,6 @@ struct PrefillGemm {
     const uint16_t* a;        // rows [.][K] as the product kernel reads them (prefill_rows_kernel's xp)
     const uint16_t* a_plain;  // the same rows as bf16 in their own order (read by the recomputation)
     const uint16_t* planes;   // per (row, group of 64): the input sum in three bf16 pieces
-    const float* asum16;      // per (row, block of 16): that block's chain sum (read by the recomputation; null: formed there)
     const int32_t* a_rows;    // row of `a` for sorted position pos: a_rows ? a_rows[pos] : pos   (gate/up; down: null)
     const int32_t* out_rows;  // output row for sorted position pos: out_rows ? out_rows[pos] : pos   (down projection)
     const uint8_t* records; uint64_t stride;   // expert e's record at records + e * stride
@@ -159,8 +158,8 @@ struct PrefillGemm {
     float* out_f;             // down: BF16-rounded fp32 [output row][N]
     uint16_t* out_h;          // down, instead of out_f when not null: the same values as bf16 (what the combine reads is half as long)
     // Sums that land within near_margin * (sum of term magnitudes) of a BF16 rounding boundary are marked in a bit map
-    // (bit sorted position * N + row; near_words 32-bit words, all written by the product kernel)
-    // and recomputed afterwards with the reference's exact lane arithmetic (launch_prefill_patch).
+    // ([sorted position][gate, up][N / 32] words for gate/up, else [sorted position][N / 32]; near_words of them, all written by the product
+    // kernel) and formed again afterwards with the reference's exact lane arithmetic (launch_prefill_patch).
     uint32_t* near_bits; uint32_t near_words; float near_margin;
     const int32_t* ids;       // expert of sorted position pos: ids ? ids[slots[pos]] : 0 (used by the recomputation)
     const int32_t* slots;
@@ -181,8 +180,8 @@ struct PrefillGemm {
 // magnitude, so that one element in some millions may differ there by a step, which the path's tolerance allows.
 constexpr float prefill_margin(uint32_t K) { return K / 64 < 8 ? 0x1p-22f : (K / 64 <= 32 ? 0x1p-23f : float(K / 64) * 0x1p-28f); }
 constexpr uint32_t prefill_pitch(uint32_t K) { return (K / 64 + 7) / 8 * 8; }   // of a piece's row: sixteen-byte loads
-void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain, float* sums16, int32_t* status);
-void launch_prefill_acts(hipStream_t s, const uint16_t* xb, uint32_t rows, uint32_t K, uint16_t* xp, uint16_t* planes, uint16_t* plain, float* sums16);
+void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain, int32_t* status);
+void launch_prefill_acts(hipStream_t s, const uint16_t* xb, uint32_t rows, uint32_t K, uint16_t* xp, uint16_t* planes, uint16_t* plain);
 // ids / weights not null (topk <= 64): the selection runs in the same launch and the logits are not written
 void launch_prefill_router(hipStream_t s, const float* x, const uint16_t* xb, const void* w, const float* offsets, uint32_t T, uint32_t K,
                            uint32_t E, uint32_t topk, float* norms, float* logits, int32_t* ids, float* weights);

@@ -34,6 +34,8 @@
 // rows are cut into tiles of 32, except
 // that a run of up to 48 rows (a whole expert with few rows, or the last rows of a longer run) is ONE tile: with about
 // forty rows per expert -- an unskewed router at 2048 tokens -- every expert's codes are then expanded once, not twice.
+#include <algorithm>
+#include <type_traits>
 #include "zc_kernels.hpp"
 #include "zc_device.hpp"
 #include "zc_decode_common.hpp"   // lds_barrier; route_token: top-k + softmax of one token by one wavefront
@@ -56,7 +58,6 @@ constexpr uint32_t kTileRows = 32, kTileRowsMax = 48, kPitch = 136;   // LDS row
 //   planes  per (row, group of 64) the group's input sum as three bf16 pieces, [row][piece][prefill_pitch(K)]: the four
 //           blocks' BF16-rounded sum-of-four chains (Q4 lanes), NaN where the group leaves the operand's exact range
 //   plain   the same of the plain fp32 sums (Q8 lanes, qwen.metal:112-125: sum += v, element by element in blocks of eight)
-//   sums16  per (row, block of 16) the chain sum itself (read by the recomputation)
 // status bit 4: a value was not BF16-valued.
 __device__ __forceinline__ void store_pieces(uint16_t* at, uint32_t pitch, float v) {
     const uint32_t hi = __float_as_uint(v) & 0xffff0000u;
@@ -66,7 +67,7 @@ __device__ __forceinline__ void store_pieces(uint16_t* at, uint32_t pitch, float
 }
 template <bool F32>
 __global__ __launch_bounds__(256) void prefill_rows_kernel(const void* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain,
-                                                           float* sums16, int32_t* status) {
+                                                           int32_t* status) {
     const uint32_t quads = K / 4, i = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63u;
     if (i >= rows * quads) return;               // (whole groups of sixteen lanes: K is a multiple of 128)
     const uint32_t r = i / quads, c = i % quads, pitch = prefill_pitch(K);
@@ -98,18 +99,15 @@ __global__ __launch_bounds__(256) void prefill_rows_kernel(const void* x, uint32
         reinterpret_cast<uint2*>(xp)[i] = odd ? make_uint2(other, uneven) : make_uint2(even, other);
     }
     const uint32_t group = r * (3 * pitch) + c / 16, base = lane & ~15u;
-    if (planes || sums16) {
+    if (planes) {
         const float quad = bf(bf(bf(v[0] + v[1]) + v[2]) + v[3]);
         float sum = 0;
 #pragma unroll
         for (int k = 0; k < 4; ++k) sum += __shfl(quad, int((lane & ~3u) + uint32_t(k)));
-        if (sums16 && (lane & 3u) == 0) sums16[i / 4] = sum;
-        if (planes) {
-            float total = 0;
+        float total = 0;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) total += __shfl(sum, int(base + 4u * uint32_t(k)));
-            if ((lane & 15u) == 0) store_pieces(planes + group, pitch, strange ? __uint_as_float(0x7fc00000u) : total);
-        }
+        for (int k = 0; k < 4; ++k) total += __shfl(sum, int(base + 4u * uint32_t(k)));
+        if ((lane & 15u) == 0) store_pieces(planes + group, pitch, strange ? __uint_as_float(0x7fc00000u) : total);
     }
     if (plain) {
         const float head = (((0.0f + v[0]) + v[1]) + v[2]) + v[3], before = __shfl_xor(head, 1);
@@ -559,7 +557,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
         const float e = m * margin, least = fabsf(v) - e;
         return !(least > 0.0f) || fabsf(v - r) + e >= __uint_as_float(__float_as_uint(least) & 0x7f800000u) * 0x1p-8f;
     };
-    // Outputs and marks (one bit per output element, sorted position * N + row) cross through LDS, so that they leave in
+    // Outputs and marks (one bit per sum: [sorted position][gate, up][N / 32] words, or [sorted position][N / 32]) cross through LDS, so that they leave in
     // whole pieces of a row: two-byte stores straight from the accumulators' lanes took longer than the walk of a short row.
     constexpr uint32_t kCols = GATED ? 64u : 128u, kOutPitch = kPitch;
     uint16_t* out_s = a_s;                       // (every wave has passed the walk's last barrier)
@@ -572,15 +570,17 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
             for (int q = 0; q < (GATED ? 1 : 2); ++q) {
                 const uint32_t col = GATED ? wave * 16 : (2 * wave + uint32_t(q)) * 16;
                 float value = bf(total[rb][q][r]);
-                bool near = near_boundary(total[rb][q][r], value, mag[rb][q][r]);
-                if constexpr (GATED) {
-                    const float up = bf(total[rb][1][r]);
-                    near = near | near_boundary(total[rb][1][r], up, mag[rb][1][r]);
-                    value = swiglu_rounded(value, up);
-                }
+                const bool near = near_boundary(total[rb][q][r], value, mag[rb][q][r]);
                 const uint64_t marks = __ballot(near);
-                out_s[m * kOutPitch + col + j] = uint16_t(__float_as_uint(value) >> 16);
                 if (j == 0) marks_s[m * 8 + col / 16] = uint16_t(marks >> (16 * g4));
+                if constexpr (GATED) {   // where one of the two is marked the other waits in the output's place
+                    const float up = bf(total[rb][1][r]);
+                    const bool up_near = near_boundary(total[rb][1][r], up, mag[rb][1][r]);
+                    const uint64_t up_marks = __ballot(up_near);
+                    if (j == 0) marks_s[m * 8 + 4 + col / 16] = uint16_t(up_marks >> (16 * g4));
+                    value = near ? up : up_near ? value : swiglu_rounded(value, up);
+                }
+                out_s[m * kOutPitch + col + j] = uint16_t(__float_as_uint(value) >> 16);
             }
         }
     lds_barrier();
@@ -592,7 +592,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
         const uint4 v = *reinterpret_cast<const uint4*>(out_s + m * kOutPitch + c * 8);
         if constexpr (GATED) {
             *reinterpret_cast<uint4*>(p.out_b + uint64_t(pos) * N + n0 + c * 8) = v;
-            if (c == 0) *reinterpret_cast<uint2*>(p.near_bits + (uint64_t(pos) * N + n0) / 32) = *reinterpret_cast<const uint2*>(marks_s + m * 8);
+            if (c < 2) *reinterpret_cast<uint2*>(p.near_bits + (uint64_t(pos) * 2 * N + c * N + n0) / 32) = *reinterpret_cast<const uint2*>(marks_s + m * 8 + c * 4);
         } else {
             const uint64_t at = uint64_t(out_row[i]) * N + n0 + c * 8;   // (a piece's row is the thread's row of block i)
             if (p.out_h) *reinterpret_cast<uint4*>(p.out_h + at) = v;
@@ -620,124 +620,170 @@ __global__ __launch_bounds__(256, BITS == 4 ? 3 : 2) void prefill_gemm_kernel(Pr
     else prefill_tile<GATED, BITS, 3>(p, a_s, marks_s, bias_s, expert, first, rows, n0);
 }
 
-// Exact recomputation of the listed elements: one group of 32 lanes plays the reference's 32 lanes for one row
+// Exact recomputation of the marked elements: one group of 32 lanes plays the reference's 32 lanes for one element
 // (qwen.metal:46-62: lane width 16 when K % 512 == 0 and N % 8 == 0, else 8; xor-butterfly lane sum).
 // BITS 8: the affine Q8 lanes (qwen.metal:112-125: lane width 8 when K % 512 == 0 and N % 8 == 0, else 4; the input sum is the
 // plain fp32 sum, the dot a multiply-add chain element by element).
-constexpr uint32_t kPatchWordsMax = 256;
-template <int WIDTH, bool GATED, bool TABLED, int BITS>
-__global__ __launch_bounds__(256) void prefill_patch_kernel(PrefillGemm p, uint32_t words_per_group) {
-    // each workgroup scans words_per_group words of the map (few for a small map, so that it still spreads over the chip),
-    // gathers the marked elements in LDS, then its eight 32-lane groups take them in turn
-    __shared__ uint16_t found[kPatchWordsMax * 32];
+// A workgroup has the elements of a few positions: it fetches those rows of inputs and forms their blocks' input sums in LDS once, beside
+// the look at the marks; its eight groups of lanes then take the marked elements in turn.  Of a gate/up element only the marked sum is formed
+// again (both are marked in one element of some hundreds): the product kernel left the other one in the output's place.
+// AHEAD: blocks of a lane that are fetched together: one memory latency, not several; no more than a lane has (a row of 512 has one).
+// What bounds it is the vector unit, about 70 instructions a block of sixteen, with the latencies of a workgroup's few turns.  Gate/up and
+// down, us, with every element's rows fetched by its own lanes, both sums of a gate/up element and four blocks at a time whatever the row -> here: 2048 tokens
+// of hidden 2048 92 + 38 -> 72 + 36, 1500 of hidden 3072 247 + 67 -> 168 + 55, 300 of the mixed artifact 26 + 12 -> 20 + 12.
+constexpr uint32_t kPatchRows = 16, kPatchLds = 24 * 1024;
+template <int WIDTH, bool GATED, int BITS, int AHEAD>
+__global__ __launch_bounds__(256) void prefill_patch_kernel(PrefillGemm p, uint32_t rows_per) {
+    extern __shared__ __align__(16) uint4 patch_x[];   // [rows][K / 8] inputs, [rows][K / WIDTH] input sums, then the marked elements: n | row << 12 (| sums << 16)
     __shared__ uint32_t found_count;
-    const uint32_t lane = threadIdx.x & 31u;
-    const uint32_t K = p.K, N = p.N, groups = K / 64;
-    const uint32_t word = blockIdx.x * words_per_group + threadIdx.x;
-    if (threadIdx.x == 0) found_count = 0;
-    __syncthreads();
+    __shared__ uint32_t expert_s[kPatchRows];
+    static_assert(WIDTH * BITS >= 32);
+    const uint32_t tid = threadIdx.x, lane = tid & 31u, K = p.K, N = p.N, groups = K / 64, pieces = K / 8, blocks = K / WIDTH, row_words = N / 32u;
+    float* sums = reinterpret_cast<float*>(patch_x + rows_per * pieces);
+    using Found = std::conditional_t<GATED, uint32_t, uint16_t>;
+    Found* found = reinterpret_cast<Found*>(sums + rows_per * blocks);
     // Only the map words of covered positions were written by the product kernel: a word past them holds whatever the
     // buffer held before.  N is a multiple of 32, so a word never straddles two positions.
-    const uint32_t positions = p.near_words / (N / 32u);
+    const uint32_t positions = p.near_words / ((GATED ? 2 : 1) * row_words);
     const uint32_t covered = p.covered ? min(uint32_t(max(*p.covered, 0)), positions) : positions;
-    uint32_t marks = (threadIdx.x < words_per_group && word < p.near_words && word / (N / 32u) < covered) ? p.near_bits[word] : 0u;
-    if (marks) {
-        uint32_t at = atomicAdd(&found_count, uint32_t(__popc(marks)));
-        while (marks) { found[at++] = uint16_t(threadIdx.x * 32 + (__ffs(marks) - 1)); marks &= marks - 1; }
+    const uint32_t first = blockIdx.x * rows_per;
+    if (first >= covered) return;
+    const uint32_t rows = min(rows_per, covered - first);
+    const uint32_t mark_row = tid / row_words, mark_word = tid - mark_row * row_words;
+    uint32_t marks[2] = {0, 0};
+    if (mark_row < rows)
+#pragma unroll
+        for (int proj = 0; proj < (GATED ? 2 : 1); ++proj) marks[proj] = p.near_bits[((first + mark_row) * (GATED ? 2 : 1) + proj) * row_words + mark_word];
+    if (tid == 0) found_count = 0;
+    if (tid < rows) expert_s[tid] = p.ids ? uint32_t(p.ids[p.slots[first + tid]]) : 0u;
+    // (a block of sixteen is two pieces: they stand turned by their block, so that sixteen lanes' reads meet all banks)
+    auto place = [](uint32_t piece) { return WIDTH == 16 ? piece ^ (piece >> 4 & 1u) : piece; };
+    for (uint32_t i0 = tid; i0 < rows * pieces; i0 += 1024) {
+        uint4 v[4];
+        uint32_t at[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const uint32_t i = min(i0 + 256 * u, rows * pieces - 1), r = i / pieces, c = i - r * pieces;
+            const uint32_t a_row = p.a_rows ? uint32_t(p.a_rows[first + r]) : first + r;
+            v[u] = reinterpret_cast<const uint4*>(p.a_plain + uint64_t(a_row) * K)[c];
+            at[u] = r * pieces + place(c);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const uint32_t i = i0 + 256 * u, w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+            const bool inside = i < rows * pieces;
+            float x[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) x[k] = __uint_as_float((k & 1) ? w[k / 2] & 0xffff0000u : w[k / 2] << 16);
+            if (inside) patch_x[at[u]] = v[u];
+            if constexpr (BITS == 4) {
+                const float low = bf(bf(bf(x[0] + x[1]) + x[2]) + x[3]), high = bf(bf(bf(x[4] + x[5]) + x[6]) + x[7]);
+                const float half = (0.0f + low) + high;
+                if constexpr (WIDTH == 8) { if (inside) sums[i] = half; }
+                else {   // (a row has an even number of pieces: a block's two are neighbouring lanes')
+                    const float before = __shfl_xor(half, 1);
+                    if (inside && (i & 1u)) sums[i / 2] = (before + low) + high;
+                }
+            } else if constexpr (WIDTH == 8) {
+                float sum = 0;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) sum += x[k];
+                if (inside) sums[i] = sum;
+            } else {
+                float low = 0, high = 0;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) { low += x[k]; high += x[4 + k]; }
+                if (inside) { sums[2 * i] = low; sums[2 * i + 1] = high; }
+            }
+        }
+    }
+    __syncthreads();
+    if (uint32_t either = marks[0] | marks[1]) {
+        const uint32_t base = mark_row << 12 | mark_word * 32u;
+        uint32_t at = atomicAdd(&found_count, uint32_t(__popc(either)));
+        for (; either; either &= either - 1) {
+            const uint32_t bit = uint32_t(__ffs(either) - 1);
+            if constexpr (GATED) found[at++] = (base + bit) | (marks[0] >> bit & 1u) << 16 | (marks[1] >> bit & 1u) << 17;
+            else found[at++] = Found(base + bit);
+        }
     }
     __syncthreads();
     const uint32_t listed = found_count;
-  for (uint32_t item = threadIdx.x >> 5; item < listed; item += 8) {
-    const uint32_t code = blockIdx.x * (words_per_group * 32u) + found[item], pos = code / N, n = code % N;
-    const uint32_t expert = p.ids ? uint32_t(p.ids[p.slots[pos]]) : 0u;
-    if (p.ids && expert >= p.experts) continue;   // an id the router could not give (reported through the status word)
-    const uint8_t* record = p.records + uint64_t(expert) * p.stride;
-    const uint32_t a_row = p.a_rows ? uint32_t(p.a_rows[pos]) : pos;
-    const uint16_t* xr = p.a_plain + uint64_t(a_row) * K;
-    static_assert(WIDTH * BITS >= 32 && !(TABLED && BITS == 8), "a block is whole code words; the table holds Q4 chain sums");
-    constexpr int DW = WIDTH * BITS / 32, XV = WIDTH >= 8 ? WIDTH / 8 : 1, kAhead = 4;   // a lane's next four blocks are fetched together: one memory latency, not four
-    float result[2] = {0, 0};
-    const uint32_t blocks = K / WIDTH;
-    for (uint32_t b0 = lane; b0 < blocks; b0 += 32 * kAhead) {
-        uint4 xv[kAhead][XV];
-        uint32_t words[kAhead][GATED ? 2 : 1][DW];
-        uint16_t scale_bits[kAhead][GATED ? 2 : 1], bias_bits[kAhead][GATED ? 2 : 1];
-        // the block's BF16-rounded chain sum depends on the row only: with 16-element blocks it comes from the table the
-        // row kernels left (the same additions in the same order)
-        constexpr bool tabled = TABLED;   // a compile-time choice: with both forms in one kernel the registers of either stay live
-        float chain[kAhead];
+    for (uint32_t item = tid >> 5; item < listed; item += 8) {
+        const uint32_t element = found[item], row = element >> 12 & 15u, n = element & 4095u, pos = first + row, expert = expert_s[row];
+        if (p.ids && expert >= p.experts) continue;   // an id the router could not give (reported through the status word)
+        const uint8_t* record = p.records + uint64_t(expert) * p.stride;
+        constexpr int DW = WIDTH * BITS / 32;
+        auto lanes_sum = [&](const uint64_t* off) {
+        float result = 0;
+        for (uint32_t b0 = lane; b0 < blocks; b0 += 32 * AHEAD) {
+            uint32_t words[AHEAD][DW];
+            uint16_t scale_bits[AHEAD], bias_bits[AHEAD];
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u) {
-            const uint32_t b = min(b0 + 32u * u, blocks - 1);   // past the end: the last block again, not used
-            if constexpr (WIDTH >= 8) {
+            for (int u = 0; u < AHEAD; ++u) {
+                const uint32_t b = min(b0 + 32u * u, blocks - 1);   // past the end: the last block again, not used
+                const uint32_t g = n * groups + (b * WIDTH) / 64;
+                const uint32_t* src = reinterpret_cast<const uint32_t*>(record + off[0] + uint64_t(n) * (K * BITS / 8)) + b * DW;
 #pragma unroll
-                for (int i = 0; i < WIDTH / 8; ++i) xv[u][i] = *reinterpret_cast<const uint4*>(xr + b * WIDTH + 8 * i);
-            } else {
-                const uint2 v = *reinterpret_cast<const uint2*>(xr + b * WIDTH);   // four inputs
-                xv[u][0] = make_uint4(v.x, v.y, 0, 0);
-            }
-            chain[u] = tabled ? p.asum16[uint64_t(a_row) * (K / 16) + b] : 0.0f;
-            const uint32_t g = n * groups + (b * WIDTH) / 64;
-#pragma unroll
-            for (int proj = 0; proj < (GATED ? 2 : 1); ++proj) {
-                const uint32_t* src = reinterpret_cast<const uint32_t*>(record + p.off[proj * 3] + uint64_t(n) * (K * BITS / 8)) + b * DW;
-#pragma unroll
-                for (int i = 0; i < DW; ++i) words[u][proj][i] = src[i];
-                scale_bits[u][proj] = reinterpret_cast<const uint16_t*>(record + p.off[proj * 3 + 1])[g];
-                bias_bits[u][proj] = reinterpret_cast<const uint16_t*>(record + p.off[proj * 3 + 2])[g];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kAhead; ++u) {
-            if (b0 + 32u * u >= blocks) break;
-            float xb[WIDTH];
-#pragma unroll
-            for (int i = 0; i < WIDTH; i += 2) {
-                const uint4 v = xv[u][i / 8];
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-                xb[i] = __uint_as_float(w[(i % 8) / 2] << 16); xb[i + 1] = __uint_as_float(w[(i % 8) / 2] & 0xffff0000u);
-            }
-            float sum = chain[u];
-            if constexpr (BITS == 8) {
-#pragma unroll
-                for (int i = 0; i < WIDTH; ++i) sum += xb[i];
-            } else if (!tabled) {
-#pragma unroll
-                for (int i = 0; i < WIDTH; i += 4) sum += bf(bf(bf(xb[i] + xb[i + 1]) + xb[i + 2]) + xb[i + 3]);
+                for (int i = 0; i < DW; ++i) words[u][i] = src[i];
+                scale_bits[u] = reinterpret_cast<const uint16_t*>(record + off[1])[g];
+                bias_bits[u] = reinterpret_cast<const uint16_t*>(record + off[2])[g];
             }
 #pragma unroll
-            for (int proj = 0; proj < (GATED ? 2 : 1); ++proj) {
+            for (int u = 0; u < AHEAD; ++u) {
+                const uint32_t b = b0 + 32u * u;
+                if (b >= blocks) break;
+                uint32_t xw[WIDTH / 2];   // the block's inputs, two a word
+                if constexpr (WIDTH >= 8) {
+#pragma unroll
+                    for (int i = 0; i < WIDTH / 8; ++i) {
+                        const uint4 v = patch_x[row * pieces + place(b * (WIDTH / 8) + uint32_t(i))];
+                        xw[4 * i] = v.x; xw[4 * i + 1] = v.y; xw[4 * i + 2] = v.z; xw[4 * i + 3] = v.w;
+                    }
+                } else {
+                    const uint2 v = reinterpret_cast<const uint2*>(patch_x)[row * (2 * pieces) + b];
+                    xw[0] = v.x; xw[1] = v.y;
+                }
+                float x[WIDTH];
+#pragma unroll
+                for (int i = 0; i < WIDTH; ++i) x[i] = __uint_as_float((i & 1) ? xw[i / 2] & 0xffff0000u : xw[i / 2] << 16);
                 float dot = 0;
                 if constexpr (BITS == 8) {
                     // (a BF16 value times a byte code is exact in fp32: the fused multiply-add rounds as the reference's multiply and add)
 #pragma unroll
-                    for (int i = 0; i < WIDTH; ++i) dot = __builtin_fmaf(xb[i], float((words[u][proj][i / 4] >> (8 * (i % 4))) & 0xffu), dot);
+                    for (int i = 0; i < WIDTH; ++i) dot = __builtin_fmaf(x[i], float((words[u][i / 4] >> (8 * (i % 4))) & 0xffu), dot);
                 } else
 #pragma unroll
                 for (int i = 0; i < WIDTH; i += 8) {
                     // nibble j of a word is element j: the even ones and the odd ones as bytes, each converted by one byte-to-float instruction
-                    const uint32_t even = words[u][proj][i / 8] & 0x0f0f0f0fu, odd = (words[u][proj][i / 8] >> 4) & 0x0f0f0f0fu;
+                    const uint32_t even = words[u][i / 8] & 0x0f0f0f0fu, odd = (words[u][i / 8] >> 4) & 0x0f0f0f0fu;
                     // (a BF16 value times a 4-bit code is exact in fp32, so a fused multiply-add rounds as the reference's
                     // multiply and add do: ((p0 + p1) + p2) + p3, then onto the block's sum)
-                    dot += __builtin_fmaf(xb[i + 3], float((odd >> 8) & 0xffu), __builtin_fmaf(xb[i + 2], float((even >> 8) & 0xffu),
-                           __builtin_fmaf(xb[i + 1], float(odd & 0xffu), xb[i] * float(even & 0xffu))));
-                    dot += __builtin_fmaf(xb[i + 7], float(odd >> 24), __builtin_fmaf(xb[i + 6], float(even >> 24),
-                           __builtin_fmaf(xb[i + 5], float((odd >> 16) & 0xffu), xb[i + 4] * float((even >> 16) & 0xffu))));
+                    dot += __builtin_fmaf(x[i + 3], float((odd >> 8) & 0xffu), __builtin_fmaf(x[i + 2], float((even >> 8) & 0xffu),
+                           __builtin_fmaf(x[i + 1], float(odd & 0xffu), x[i] * float(even & 0xffu))));
+                    dot += __builtin_fmaf(x[i + 7], float(odd >> 24), __builtin_fmaf(x[i + 6], float(even >> 24),
+                           __builtin_fmaf(x[i + 5], float((odd >> 16) & 0xffu), x[i + 4] * float((even >> 16) & 0xffu))));
                 }
-                result[proj] += b16(scale_bits[u][proj]) * dot + sum * b16(bias_bits[u][proj]);
+                result += b16(scale_bits[u]) * dot + sums[row * blocks + b] * b16(bias_bits[u]);
+            }
+        }
+        return lane_sum32(result);
+        };
+        if constexpr (GATED) {
+            uint16_t* out = p.out_b + uint64_t(pos) * N + n;
+            const bool up_first = !(element >> 16 & 1u);
+            float other = b16(*out);
+            const float marked = lanes_sum(p.off + (up_first ? 3 : 0));
+            if (element >> 16 == 3u) other = lanes_sum(p.off + 3);
+            if (lane == 0) *out = uint16_t(__float_as_uint(up_first ? swiglu_bf(other, marked) : swiglu_bf(marked, other)) >> 16);
+        } else {
+            const float value = bf(lanes_sum(p.off));
+            if (lane == 0) {
+                const uint64_t at = uint64_t(p.out_rows ? uint32_t(p.out_rows[pos]) : pos) * N + n;
+                if (p.out_h) p.out_h[at] = uint16_t(__float_as_uint(value) >> 16); else p.out_f[at] = value;
             }
         }
     }
-    result[0] = lane_sum32(result[0]);
-    if constexpr (GATED) result[1] = lane_sum32(result[1]);
-    if (lane == 0) {
-        if constexpr (GATED) p.out_b[uint64_t(pos) * N + n] = uint16_t(__float_as_uint(swiglu_bf(result[0], result[1])) >> 16);
-        else {
-            const uint64_t at = uint64_t(p.out_rows ? uint32_t(p.out_rows[pos]) : pos) * N + n;
-            if (p.out_h) p.out_h[at] = uint16_t(__float_as_uint(bf(result[0])) >> 16); else p.out_f[at] = bf(result[0]);
-        }
-    }
-  }
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
@@ -956,11 +1002,11 @@ void launch_prefill_router(hipStream_t s, const float* x, const uint16_t* xb, co
     hipLaunchKernelGGL(router_refine_kernel, dim3((T + 3) / 4), dim3(256), 4 * K * 2, s, xb, wb, offsets, norms, T, E, K, topk, logits, ids, weights);
 }
 
-void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain, float* sums16, int32_t* status) {
-    hipLaunchKernelGGL((prefill_rows_kernel<true>), dim3((rows * (K / 4) + 255) / 256), dim3(256), 0, s, x, rows, K, xb, xp, planes, plain, sums16, status);
+void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain, int32_t* status) {
+    hipLaunchKernelGGL((prefill_rows_kernel<true>), dim3((rows * (K / 4) + 255) / 256), dim3(256), 0, s, x, rows, K, xb, xp, planes, plain, status);
 }
-void launch_prefill_acts(hipStream_t s, const uint16_t* xb, uint32_t rows, uint32_t K, uint16_t* xp, uint16_t* planes, uint16_t* plain, float* sums16) {
-    hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3((rows * (K / 4) + 255) / 256), dim3(256), 0, s, xb, rows, K, nullptr, xp, planes, plain, sums16, nullptr);
+void launch_prefill_acts(hipStream_t s, const uint16_t* xb, uint32_t rows, uint32_t K, uint16_t* xp, uint16_t* planes, uint16_t* plain) {
+    hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3((rows * (K / 4) + 255) / 256), dim3(256), 0, s, xb, rows, K, nullptr, xp, planes, plain, nullptr);
 }
 void launch_prefill_tiles(hipStream_t s, const int32_t* offsets, uint32_t experts, uint32_t rows, int32_t* tile_expert, int32_t* tile_first,
                           int32_t* tile_rows, int32_t* tile_count) {
@@ -991,16 +1037,23 @@ void launch_prefill_gemm(hipStream_t s, const PrefillGemm& p, bool gated, uint32
     }
 }
 void launch_prefill_patch(hipStream_t s, const PrefillGemm& p, bool gated) {
-    const bool wide = p.K % 512 == 0 && p.N % 8 == 0;     // the reference's lane-width rule (metal.mm:649-674)
-    const uint32_t per = p.near_words >= kPatchWordsMax * 1024u ? kPatchWordsMax : 64u;   // words of the map per workgroup
-    const dim3 grid((p.near_words + per - 1) / per);
-    const bool tabled = wide && p.asum16 && p.bits == 4;  // the table holds the Q4 chain sums of 16-element blocks
-#define ZC_PATCH(W, G, T, B) hipLaunchKernelGGL((prefill_patch_kernel<W, G, T, B>), grid, dim3(256), 0, s, p, per)
-    if (p.bits == 8) {   // the Q8 lanes are half as wide (metal.mm:649-674)
-        if (gated) { if (wide) ZC_PATCH(8, true, false, 8); else ZC_PATCH(4, true, false, 8); }
-        else { if (wide) ZC_PATCH(8, false, false, 8); else ZC_PATCH(4, false, false, 8); }
-    } else if (gated) { if (tabled) ZC_PATCH(16, true, true, 4); else if (wide) ZC_PATCH(16, true, false, 4); else ZC_PATCH(8, true, false, 4); }
-    else { if (tabled) ZC_PATCH(16, false, true, 4); else if (wide) ZC_PATCH(16, false, false, 4); else ZC_PATCH(8, false, false, 4); }
+    const bool wide = p.K % 512 == 0 && p.N % 8 == 0;     // the reference's lane-width rule (metal.mm:649-674); the Q8 lanes are half as wide
+    const uint32_t width = (wide ? 16 : 8) / (p.bits / 4), row_bytes = 2 * p.K + 4 * (p.K / width);
+    const uint32_t rows = std::max(1u, std::min({(gated ? 2048u : 8192u) / p.N, kPatchRows, kPatchLds / row_bytes}));
+    const uint32_t lds = rows * (row_bytes + (gated ? 4 : 2) * p.N), positions = p.near_words / (p.N / 32 * (gated ? 2 : 1));
+    const dim3 grid((positions + rows - 1) / rows);
+    // (a lane's blocks in as few turns as four at a time allow, no more of them a turn than that takes)
+    const uint32_t each = (p.K / width + 31) / 32, turns = (each + 3) / 4, ahead = (each + turns - 1) / turns;
+#define ZC_PATCH(W, G, B, A) hipLaunchKernelGGL((prefill_patch_kernel<W, G, B, A>), grid, dim3(256), lds, s, p, rows)
+#define ZC_PATCH4(W, G) do { if (ahead == 1) ZC_PATCH(W, G, 4, 1); else if (ahead == 2) ZC_PATCH(W, G, 4, 2); else if (ahead == 3) ZC_PATCH(W, G, 4, 3); else ZC_PATCH(W, G, 4, 4); } while (0)
+#define ZC_PATCH8(W, G) do { if (ahead <= 2) ZC_PATCH(W, G, 8, 2); else ZC_PATCH(W, G, 8, 4); } while (0)
+    if (p.bits == 8) {
+        if (gated) { if (wide) ZC_PATCH8(8, true); else ZC_PATCH8(4, true); }
+        else { if (wide) ZC_PATCH8(8, false); else ZC_PATCH8(4, false); }
+    } else if (gated) { if (wide) ZC_PATCH4(16, true); else ZC_PATCH4(8, true); }
+    else { if (wide) ZC_PATCH4(16, false); else ZC_PATCH4(8, false); }
+#undef ZC_PATCH8
+#undef ZC_PATCH4
 #undef ZC_PATCH
 }
 // (hidden and intermediate sizes up to 4096: the margins of the recomputation are measured up to there)
