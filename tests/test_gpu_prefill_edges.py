@@ -34,3 +34,25 @@ def test_prefill_matches_the_exact_layer(ctx, hidden, inter, bits, T):
     assert np.mean(fast.view(np.uint32) == exact.view(np.uint32)) > 0.9999
     for b in (weights.router, weights.shared_gate, weights.shared_record, weights.records, x):
         ctx.free(b)
+
+
+# the dispatch sort in one launch: just enough slots for it, one more step of slots than is in flight, a partly filled last stretch, more
+# and fewer experts than a workgroup's wavefronts
+@pytest.mark.parametrize("experts,topk,T", [(1024, 10, 103), (1024, 10, 2200), (1021, 7, 2927), (5, 2, 4100), (17, 4, 333)])
+def test_prefill_dispatch_of_many_slots(ctx, experts, topk, T):
+    cfg = workload.tiny_config(128, experts, topk, 128)
+    weights = workload.LayerWeights(ctx, cfg, 19, ("zipf", 1.1))
+    x, outs = workload.hidden_rows(ctx, T, 128, 20), []
+    for call, size in ((ctx.moe_forward, ctx.moe_workspace_bytes), (ctx.moe_prefill, ctx.moe_prefill_workspace_bytes)):
+        out, ws, ids = ctx.alloc(T * 128 * 4), ctx.alloc(size(cfg, T)), ctx.alloc(T * topk * 4)
+        call(cfg, weights.layer, x, T, out, ws, z.Trace(None, ids.ptr, None, None, None, None))
+        ctx.moe_check()
+        outs.append((out.numpy(f32).copy(), ids.numpy(np.int32).tobytes()))
+        for b in (out, ws, ids):
+            ctx.free(b)
+    (exact, exact_ids), (fast, fast_ids) = outs
+    assert fast_ids == exact_ids
+    assert np.max(np.abs(fast - exact)) <= 2e-3 * np.max(np.abs(exact))
+    assert np.mean(fast.view(np.uint32) == exact.view(np.uint32)) > 0.9999
+    for b in (weights.router, weights.shared_gate, weights.shared_record, weights.records, x, weights.offsets):
+        ctx.free(b)

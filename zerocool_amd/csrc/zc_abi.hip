@@ -746,7 +746,7 @@ struct PrefillSpace {
     uint32_t max_tiles, max_shared_tiles;
     uint32_t* near_bits;      // one bit per product element: recompute exactly
     uint32_t* shared_near_bits;   // the same for the shared expert's products, which run beside the routed ones
-    float* norms;             // |row| of the inputs and of the router's rows (the router on bounds)
+    float* norms;             // |row| of the router's rows (the router on bounds)
     uint64_t bytes;
 };
 PrefillSpace carve_prefill(const zc_moe_config* c, uint32_t T, void* base) {
@@ -765,15 +765,15 @@ PrefillSpace carve_prefill(const zc_moe_config* c, uint32_t T, void* base) {
     w.stile_expert = (int32_t*)take(w.max_shared_tiles * 4ull); w.stile_first = (int32_t*)take(w.max_shared_tiles * 4ull);
     w.stile_rows = (int32_t*)take(w.max_shared_tiles * 4ull); w.stile_count = (int32_t*)take(4);
     w.near_bits = (uint32_t*)take(n * std::max(c->hidden, 2 * c->inter) / 8);
-    w.norms = (float*)take((uint64_t(T) + c->experts) * 4);
+    w.norms = (float*)take(uint64_t(c->experts) * 4);
     w.xplain = (uint16_t*)take(T * xpitch);
     w.shared_near_bits = (uint32_t*)take(uint64_t(T) * std::max(c->hidden, 2 * c->inter) / 8);
     w.bytes = at;
     return w;
 }
 // From here on the router on bounds is ahead: the exact one's chains fill the chip, where the other's short kernels leave room for the
-// shared expert beside them.  us a layer, exact logits / bounds: hidden 2048 without router skew, 200 tokens 318 / 350, 400 352 / 365, 700 393 / 406, 2048
-// 637 / 626; hidden 3072 with Zipf(1.1) offsets, 128 tokens 259 / 304, 300 392 / 420, 700 669 / 672, 1500 1187 / 1169.
+// shared expert beside them.  us a layer, exact logits / bounds: hidden 2048 without router skew, 200 tokens 300 / 322, 400 328 / 344, 700 372 / 377, 1024
+// 418 / 419, 1400 475 / 469; hidden 3072 with Zipf(1.1) offsets, 300 tokens 356 / 380, 500 467 / 480, 700 587 / 588, 1000 754 / 747.
 constexpr uint32_t kPrefillBoundsTokens = 768;
 bool prefill_config(const zc_moe_config* c) {
     // every projection affine Q4 or affine Q8 (the mixed 4/8-bit artifact: Q4 routed gate/up, Q8 down and shared expert)
@@ -814,13 +814,14 @@ zc_status zc_hip_moe_prefill(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
     const bool bounds = T >= kPrefillBoundsTokens && !(trace && trace->logits);
     const bool x_q4 = c->bits_gate_up == 4 || c->shared_bits_gate_up == 4, x_q8 = c->bits_gate_up == 8 || c->shared_bits_gate_up == 8;
     auto rows_on = [&](hipStream_t t) {
-        zc::launch_prefill_rows(t, x, T, H, w.xb, w.xp, x_q4 ? w.xplanes : nullptr, x_q8 ? w.xplain : nullptr, ctx->moe_status);
+        zc::launch_prefill_rows(t, x, T, H, w.xb, w.xp, x_q4 ? w.xplanes : nullptr, x_q8 ? w.xplain : nullptr, ctx->moe_status,
+                                l->router, bounds ? E : 0u, w.norms);
     };
     if (bounds) rows_on(s);
     ZC_HIP(hipEventRecord(ctx->fork, s)); ZC_HIP(hipStreamWaitEvent(s2, ctx->fork, 0));
     if (bounds) {
         const bool select = k <= 64;   // the refinement's wavefront selects its token's experts too
-        zc::launch_prefill_router(s, x, w.xb, l->router, l->router_offsets, T, H, E, k, w.norms, w.base.logits, select ? w.base.ids : nullptr, select ? w.base.weights : nullptr);
+        zc::launch_prefill_router(s, w.xb, l->router, l->router_offsets, T, H, E, k, w.norms, w.base.logits, select ? w.base.ids : nullptr, select ? w.base.weights : nullptr);
         if (!select) zc::launch_route(s, w.base.logits, T, E, k, w.base.ids, w.base.weights);
     } else {
         rows_on(s2);

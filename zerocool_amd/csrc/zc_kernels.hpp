@@ -180,11 +180,12 @@ struct PrefillGemm {
 // magnitude, so that one element in some millions may differ there by a step, which the path's tolerance allows.
 constexpr float prefill_margin(uint32_t K) { return K / 64 < 8 ? 0x1p-22f : (K / 64 <= 32 ? 0x1p-23f : float(K / 64) * 0x1p-28f); }
 constexpr uint32_t prefill_pitch(uint32_t K) { return (K / 64 + 7) / 8 * 8; }   // of a piece's row: sixteen-byte loads
-void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain, int32_t* status);
+void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain, int32_t* status,
+                         const void* norm_of, uint32_t norm_rows, float* norms);   // norm_rows, optional: |row| of as many bf16 rows
 void launch_prefill_acts(hipStream_t s, const uint16_t* xb, uint32_t rows, uint32_t K, uint16_t* xp, uint16_t* planes, uint16_t* plain);
 // ids / weights not null (topk <= 64): the selection runs in the same launch and the logits are not written
-void launch_prefill_router(hipStream_t s, const float* x, const uint16_t* xb, const void* w, const float* offsets, uint32_t T, uint32_t K,
-                           uint32_t E, uint32_t topk, float* norms, float* logits, int32_t* ids, float* weights);
+void launch_prefill_router(hipStream_t s, const uint16_t* xb, const void* w, const float* offsets, uint32_t T, uint32_t K,
+                           uint32_t E, uint32_t topk, const float* norms, float* logits, int32_t* ids, float* weights);
 void launch_prefill_dispatch(hipStream_t s, const int32_t* ids, uint32_t tokens, uint32_t topk, uint32_t E, int32_t* offsets, int32_t* slots, int32_t* rows,
                              int32_t* status, int32_t* tile_expert, int32_t* tile_first, int32_t* tile_rows, int32_t* tile_count);
 bool prefill_dispatch_fits(const int32_t* ids, uint32_t tokens, uint32_t topk, uint32_t E);

@@ -65,10 +65,40 @@ __device__ __forceinline__ void store_pieces(uint16_t* at, uint32_t pitch, float
     const uint32_t mid = __float_as_uint(rest) & 0xffff0000u;
     at[0] = uint16_t(hi >> 16); at[pitch] = uint16_t(mid >> 16); at[2 * pitch] = uint16_t(__float_as_uint(rest - __uint_as_float(mid)) >> 16);
 }
+//
+// The workgroups behind the rows', if norm_rows is not 0, leave |row| of the router's rows for the router on bounds, one wavefront a row.
+// |row| is rounded up a little.  A row so small that its squares leave the normal range has no usable norm: +inf makes the router
+// recompute everything.
+__device__ __forceinline__ float squares_of(uint4 v, float sum) {
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const float lo = __uint_as_float(w[q] << 16), hi = __uint_as_float(w[q] & 0xffff0000u);
+        sum = __builtin_fmaf(lo, lo, sum); sum = __builtin_fmaf(hi, hi, sum);
+    }
+    return sum;
+}
+__device__ __forceinline__ float row_norm(float lane_squares) {
+#pragma unroll
+    for (int o = 32; o; o >>= 1) lane_squares += __shfl_xor(lane_squares, o);
+    return lane_squares < 0x1p-100f ? __uint_as_float(0x7f800000u) : sqrtf(lane_squares) * 1.0001f;
+}
 template <bool F32>
 __global__ __launch_bounds__(256) void prefill_rows_kernel(const void* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain,
-                                                           int32_t* status) {
+                                                           int32_t* status, const uint16_t* norm_of, uint32_t norm_rows, float* norms) {
     const uint32_t quads = K / 4, i = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63u;
+    if constexpr (F32) {
+        const uint32_t before = (rows * quads + 255) / 256;
+        if (blockIdx.x >= before) {
+            const uint32_t row = (blockIdx.x - before) * 4 + threadIdx.x / 64;
+            if (row >= norm_rows) return;
+            float sum = 0;
+            for (uint32_t k = lane * 8; k < K; k += 512) sum = squares_of(ldg_u4(norm_of + uint64_t(row) * K + k), sum);
+            const float norm = row_norm(sum);
+            if (lane == 0) norms[row] = norm;
+            return;
+        }
+    }
     if (i >= rows * quads) return;               // (whole groups of sixteen lanes: K is a multiple of 128)
     const uint32_t r = i / quads, c = i % quads, pitch = prefill_pitch(K);
     float v[4];
@@ -147,42 +177,42 @@ __global__ __launch_bounds__(1024) void prefill_tiles_kernel(const int32_t* offs
 
 // The dispatch sort of a long batch and the routed experts' work list in ONE launch (the decode path's three dispatch
 // kernels and prefill_tiles_kernel hold the same steps as four launches in a row, each of them short: what they cost was
-// the four launches).  A workgroup = four experts (one per wave) x one of kDispatchParts stretches of the slots.  Every
+// the four launches).  A workgroup = sixteen experts (one per wave) x one of kDispatchParts stretches of the slots.  Every
 // workgroup counts ALL the slots' experts, per stretch, into a table in LDS and keeps its own stretch of the ids there;
 // it scans the table (sorted offsets and tile counts of every expert), and each wave then places its expert's slots of
 // the workgroup's stretch in ascending slot order, starting where the earlier stretches' slots of that expert end.  The
 // workgroups of the first stretch also write their experts' tiles, workgroup (0, 0) the offsets.  Same results as
 // launch_dispatch followed by launch_prefill_tiles; the list of selected experts is not written (nothing here reads it).
+// (Workgroups of sixteen waves and not of four: 20480 slots 23 -> 17.6 us beside the shared expert's product, 17.4 -> 13.2 alone.)
 // ids sixteen-byte aligned; stretch: slots per stretch, a multiple of 1024.
-constexpr uint32_t kDispatchParts = 4;
-__global__ __launch_bounds__(256) void prefill_dispatch_kernel(const int32_t* __restrict__ ids, uint32_t n, uint32_t topk, uint32_t E, uint32_t stretch,
+constexpr uint32_t kDispatchParts = 4, kDispatchThreads = 1024;
+__global__ __launch_bounds__(kDispatchThreads) void prefill_dispatch_kernel(const int32_t* __restrict__ ids, uint32_t n, uint32_t topk, uint32_t E, uint32_t stretch,
                                                                int32_t* __restrict__ offsets, int32_t* __restrict__ slots, int32_t* __restrict__ rows, int32_t* status,
                                                                int32_t* tile_expert, int32_t* tile_first, int32_t* tile_rows, int32_t* tile_count) {
     extern __shared__ __align__(16) int32_t table[];   // [parts][E] counts, [E + 1] offsets, [E + 1] tiles before, then the stretch's ids
-    __shared__ int32_t wave_sum[2][4];
+    __shared__ int32_t wave_sum[2][kDispatchThreads / 64];
     int32_t* cnt = table; int32_t* off = table + kDispatchParts * E; int32_t* tiles_before = off + E + 1;
     int32_t* copy = table + ((kDispatchParts + 2) * E + 2 + 3) / 4 * 4;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, part = blockIdx.y, first = part * stretch;
-    for (uint32_t i = tid; i < kDispatchParts * E; i += 256) cnt[i] = 0;
+    for (uint32_t i = tid; i < kDispatchParts * E; i += kDispatchThreads) cnt[i] = 0;
     __syncthreads();
     {
         int bad = 0;
-        uint32_t at = 0, until = stretch;   // the stretch of slot p: counted up as p goes
-        for (uint32_t b0 = 0; b0 < n; b0 += 8 * 1024) {   // eight steps' loads in flight
-            int4 batch[8];
+        constexpr int kSteps = 5;                                       // steps' loads in flight: 20480 slots in one go
+        for (uint32_t b0 = 0; b0 < n; b0 += kSteps * 4 * kDispatchThreads) {
+            int4 batch[kSteps];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const uint32_t p = b0 + u * 1024 + 4 * tid;
+            for (int u = 0; u < kSteps; ++u) {
+                const uint32_t p = b0 + (u * kDispatchThreads + tid) * 4;
                 int4 v = make_int4(-1, -1, -1, -1);   // (-1: past the end)
                 if (p + 3 < n) v = *reinterpret_cast<const int4*>(ids + p);
                 else { if (p < n) v.x = ids[p]; if (p + 1 < n) v.y = ids[p + 1]; if (p + 2 < n) v.z = ids[p + 2]; }
                 batch[u] = v;
             }
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const uint32_t p0 = b0 + u * 1024, p = p0 + 4 * tid;
-                if (p0 >= n) break;
-                if (p0 >= until) { ++at; until += stretch; }
+            for (int u = 0; u < kSteps; ++u) {
+                const uint32_t p = b0 + (u * kDispatchThreads + tid) * 4, at = (p >= stretch ? 1u : 0u) + (p >= 2 * stretch ? 1u : 0u) + (p >= 3 * stretch ? 1u : 0u);   // its stretch
+                if (p >= (n + 255) / 256 * 256) break;   // (the last 256 slots are looked at as a whole: -1 past the end)
                 const int32_t four[4] = {batch[u].x, batch[u].y, batch[u].z, batch[u].w};
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
@@ -196,14 +226,12 @@ __global__ __launch_bounds__(256) void prefill_dispatch_kernel(const int32_t* __
     }
     __syncthreads();
     auto count_of = [&](uint32_t e) { int32_t c = 0; for (uint32_t q = 0; q < kDispatchParts; ++q) c += cnt[q * E + e]; return c; };
-    {   // exclusive scans over the experts: thread t owns experts t * per .. t * per + per - 1
-        const uint32_t per = (E + 255) / 256;
+    {   // exclusive scans over the experts, one a thread
         auto tiles_of = [](int32_t count) {
             const int32_t whole = count / int32_t(kTileRows), left = count % int32_t(kTileRows);
             return count == 0 ? 0 : (whole == 0 ? 1 : whole + (left > int32_t(kTileRowsMax - kTileRows) ? 1 : 0));
         };
-        int32_t mine[2] = {0, 0};
-        for (uint32_t i = 0; i < per; ++i) { const uint32_t e = tid * per + i; if (e < E) { const int32_t c = count_of(e); mine[0] += c; mine[1] += tiles_of(c); } }
+        const int32_t c = tid < E ? count_of(tid) : 0, mine[2] = {c, tiles_of(c)};
         int32_t incl[2] = {mine[0], mine[1]};
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1)
@@ -211,21 +239,21 @@ __global__ __launch_bounds__(256) void prefill_dispatch_kernel(const int32_t* __
             for (int v = 0; v < 2; ++v) { const int32_t up = __shfl_up(incl[v], o); if (int(lane) >= o) incl[v] += up; }
         if (lane == 63) { wave_sum[0][wave] = incl[0]; wave_sum[1][wave] = incl[1]; }
         __syncthreads();
-        int32_t at[2];
 #pragma unroll
-        for (int v = 0; v < 2; ++v) { at[v] = incl[v] - mine[v]; for (uint32_t w = 0; w < wave; ++w) at[v] += wave_sum[v][w]; }
-        for (uint32_t i = 0; i < per; ++i) {
-            const uint32_t e = tid * per + i;
-            if (e < E) { const int32_t c = count_of(e); off[e] = at[0]; tiles_before[e] = at[1]; at[0] += c; at[1] += tiles_of(c); }
+        for (int v = 0; v < 2; ++v) {
+            int32_t at = incl[v] - mine[v];
+            for (uint32_t w = 0; w < wave; ++w) at += wave_sum[v][w];
+            int32_t* to = v ? tiles_before : off;
+            if (tid < E) to[tid] = at;
+            if (tid + 1 == E) to[E] = at + mine[v];
         }
-        if (tid == 255) { off[E] = at[0]; tiles_before[E] = at[1]; }
         __syncthreads();
     }
     if (blockIdx.x == 0 && part == 0) {
-        for (uint32_t e = tid; e <= E; e += 256) offsets[e] = off[e];
+        for (uint32_t e = tid; e <= E; e += kDispatchThreads) offsets[e] = off[e];
         if (tid == 0) *tile_count = tiles_before[E];
     }
-    const uint32_t e = blockIdx.x * 4 + wave;
+    const uint32_t e = blockIdx.x * (kDispatchThreads / 64) + wave;
     if (e >= E) return;
     const int32_t count = count_of(e);
     if (count == 0) return;
@@ -803,26 +831,6 @@ __global__ __launch_bounds__(256) void prefill_patch_kernel(PrefillGemm p, uint3
 // expert whose upper bound is below that cannot be among the top k, ties included.  A token with a logit that is not
 // finite has every expert recomputed.
 // ---------------------------------------------------------------------------------------------------------------------
-// |row| of bf16 rows, rounded up a little: one wavefront per row; rows [0, rows_a) come from a, the rest from b.
-__global__ __launch_bounds__(256) void row_norms_kernel(const uint16_t* a, uint32_t rows_a, const uint16_t* b, uint32_t rows_b, uint32_t K, float* norms) {
-    const uint32_t row = blockIdx.x * 4 + threadIdx.x / 64, lane = threadIdx.x & 63u;
-    if (row >= rows_a + rows_b) return;
-    const uint16_t* src = row < rows_a ? a + uint64_t(row) * K : b + uint64_t(row - rows_a) * K;
-    float sum = 0;
-    for (uint32_t i = lane * 8; i < K; i += 512) {
-        const uint4 v = *reinterpret_cast<const uint4*>(src + i);
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const float lo = __uint_as_float(w[q] << 16), hi = __uint_as_float(w[q] & 0xffff0000u);
-            sum = __builtin_fmaf(lo, lo, sum); sum = __builtin_fmaf(hi, hi, sum);
-        }
-    }
-#pragma unroll
-    for (int o = 32; o; o >>= 1) sum += __shfl_xor(sum, o);
-    // (a row so small that its squares leave the normal range has no usable norm: +inf makes the caller recompute everything)
-    if (lane == 0) norms[row] = sum < 0x1p-100f ? __uint_as_float(0x7f800000u) : sqrtf(sum) * 1.0001f;
-}
 constexpr uint32_t kRouterPitch = 72;   // in bf16 elements (144 bytes)
 // approx[t][e] = sum_k a[t][k] b[e][k] (+ offsets[e]): 64 tokens x 64 experts per workgroup, a wave a 32 x 32 block on
 // v_mfma_f32_32x32x16_bf16, K in steps of 64 through LDS (rows padded to 144 bytes), the next step's rows in registers.
@@ -830,7 +838,10 @@ __global__ __launch_bounds__(256) void router_product_kernel(const uint16_t* a, 
                                                              const float* offsets, float* approx) {
     __shared__ __align__(16) uint16_t a_s[2][64 * kRouterPitch], b_s[2][64 * kRouterPitch];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, m = lane & 31u, h = lane >> 5;
-    const uint32_t t0 = blockIdx.y * 64, e0 = blockIdx.x * 64;
+    // Every die gets one stretch of the (token block, expert block) list: neighbours on it share their token rows in the die's L2.
+    const uint32_t columns = (E + 63) / 64, blocks = (T + 63) / 64 * columns, share = (blocks + 7) / 8, block = blockIdx.x % 8 * share + blockIdx.x / 8;
+    if (blockIdx.x / 8 >= share || block >= blocks) return;
+    const uint32_t t0 = block / columns * 64, e0 = block % columns * 64;
     const uint32_t r = tid >> 3, c8 = tid & 7u;   // a thread moves rows r and r + 32, sixteen bytes each, of both operands
     const uint16_t* a_src0 = a + uint64_t(min(t0 + r, T - 1)) * K + c8 * 8;
     const uint16_t* a_src1 = a + uint64_t(min(t0 + r + 32, T - 1)) * K + c8 * 8;
@@ -877,21 +888,35 @@ __global__ __launch_bounds__(256) void router_product_kernel(const uint16_t* a, 
 // row it holds in LDS (route_token, the selection of the decode kernels: the same ids and weights as route_kernel's), and
 // the row itself is not written out.
 constexpr int kRefinePerLane = 16;   // experts <= 1024
+struct RefineLds { uint32_t x, w, row, list, bytes; };   // bytes from the start, of one wavefront's share
+__host__ __device__ inline RefineLds refine_lds(uint32_t K, uint32_t E) {
+    RefineLds l{};
+    l.w = 2 * (K + 128); l.row = l.w + 8192; l.list = l.row + (E + 3) / 4 * 16; l.bytes = l.list + (E + 7) / 8 * 16;
+    return l;
+}
 __global__ __launch_bounds__(256) void router_refine_kernel(const uint16_t* xb, const uint16_t* w, const float* offsets, const float* norms,
                                                             uint32_t T, uint32_t E, uint32_t K, uint32_t topk, float* logits,
                                                             int32_t* ids, float* weights) {
-    __shared__ float row_s[4][1024];
-    __shared__ uint16_t list_s[4][1024];
     __shared__ uint32_t pick_s[4][128];                      // route_token's scratch
     __shared__ int32_t ids_s[4][64]; __shared__ float weights_s[4][64];
-    extern __shared__ __align__(16) uint16_t x_s[];   // the four tokens' input rows (BF16-valued, so the bf16 copy is the input)
-    const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x & 63u, t = blockIdx.x * 4 + wave;
+    extern __shared__ __align__(16) uint8_t refine_s[];
+    const uint32_t wave = threadIdx.x / 64, lane = threadIdx.x & 63u, t = blockIdx.x * 4 + wave, P = K / 16;
     if (t >= T) return;
-    uint16_t* x_row = x_s + wave * K;
-    for (uint32_t i = lane * 8; i < K; i += 512) *reinterpret_cast<uint4*>(x_row + i) = *reinterpret_cast<const uint4*>(xb + uint64_t(t) * K + i);
+    const RefineLds at_s = refine_lds(K, E);
+    uint8_t* mine_s = refine_s + wave * at_s.bytes;
+    uint16_t* x_row = reinterpret_cast<uint16_t*>(mine_s);   // the token's input row (BF16-valued, so the bf16 copy is the input), eight elements behind every partition
+    uint4* w_s = reinterpret_cast<uint4*>(mine_s + at_s.w);  // 64 elements of every partition of four experts
+    float* row_s = reinterpret_cast<float*>(mine_s + at_s.row);
+    uint16_t* list_s = reinterpret_cast<uint16_t*>(mine_s + at_s.list);
+    float squares = 0;
+    for (uint32_t i = lane * 8; i < K; i += 512) {
+        const uint4 v = ldg_u4(xb + uint64_t(t) * K + i);
+        *reinterpret_cast<uint4*>(x_row + i + i / P * 8) = v;
+        squares = squares_of(v, squares);
+    }
     const float ninf = __uint_as_float(0xff800000u);
     float* row = logits + uint64_t(t) * E;
-    const float reach = float(K) * 0x1p-22f * norms[t];
+    const float reach = float(K) * 0x1p-22f * row_norm(squares);
     float upper[kRefinePerLane], best_lower = ninf;
     bool strange = false;
 #pragma unroll
@@ -899,7 +924,7 @@ __global__ __launch_bounds__(256) void router_refine_kernel(const uint16_t* xb, 
         const uint32_t e = lane + 64u * uint32_t(i);
         upper[i] = ninf;
         if (e < E) {
-            const float a = row[e], bound = reach * norms[T + e] + 0x1p-22f * fabsf(a);
+            const float a = row[e], bound = reach * norms[e] + 0x1p-22f * fabsf(a);
             strange = strange || !(fabsf(a) < __uint_as_float(0x7f800000u)) || !(bound < __uint_as_float(0x7f800000u));
             upper[i] = a + bound;
             best_lower = fmaxf(best_lower, a - bound);
@@ -911,9 +936,7 @@ __global__ __launch_bounds__(256) void router_refine_kernel(const uint16_t* xb, 
     {
         float mine = best_lower;
         for (uint32_t j = 0; j < topk && !all; ++j) {
-            float top = mine;
-#pragma unroll
-            for (int o = 32; o; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
+            const float top = wave_max_f32(mine);
             if (!(top > ninf)) { all = true; break; }
             threshold = top;
             const uint64_t holders = __ballot(mine == top);
@@ -927,62 +950,70 @@ __global__ __launch_bounds__(256) void router_refine_kernel(const uint16_t* xb, 
         const uint32_t e = lane + 64u * uint32_t(i);
         const bool take = e < E && (all || upper[i] >= threshold);
         const uint64_t takers = __ballot(take);
-        if (take) list_s[wave][count + uint32_t(__popcll(takers & ((1ull << lane) - 1)))] = uint16_t(e);
+        if (take) list_s[count + uint32_t(__popcll(takers & ((1ull << lane) - 1)))] = uint16_t(e);
         count += uint32_t(__popcll(takers));
-        if (e < E) row_s[wave][e] = ninf;
+        if (e < E) row_s[e] = ninf;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // four experts at a time: sixteen lanes run an expert's sixteen partition chains (router_kernel's arithmetic).  Eight weight
-    // pieces = 64 elements are requested together, and the next eight -- of this expert or of the next four's -- before the
-    // current ones are used.
-    const uint32_t split = lane % 16, P = K / 16, base = lane & ~15u;
-    const uint16_t* xr = x_row + split * P;
+    // four experts at a time: sixteen lanes run an expert's sixteen partition chains (router_kernel's arithmetic), 64 elements of every
+    // partition after the other.  Eight lanes fetch the 128 bytes of one partition, so that a load looks eight lines up and not 64, and the pieces
+    // change lanes in LDS, turned by their partition so that sixteen lanes' reads meet all banks.  The next 64 elements -- of these experts
+    // or of the next four -- are requested before the current ones are used.
+    const uint32_t split = lane % 16, base = lane & ~15u;
+    const uint16_t* xr = x_row + split * (P + 8);
     const uint32_t batches = (P + 63) / 64, total = (count + 3) / 4 * batches;
-    auto request = [&](uint32_t index, uint4 (&piece)[8]) {
-        const uint32_t at = min(index / batches * 4 + lane / 16, count - 1), i0 = index % batches * 64;
-        const uint16_t* wr = w + uint64_t(list_s[wave][at]) * K + split * P;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) piece[q] = *reinterpret_cast<const uint4*>(wr + min(i0 + 8 * uint32_t(q), P - 8));
-    };
     uint4 ahead[8];
-    if (total) request(0, ahead);
+    auto request = [&](uint32_t index) {
+        const uint32_t i = min(index % batches * 64 + lane % 8 * 8, P - 8);   // (past a partition's end: its last piece again, not used)
+#pragma unroll
+        for (uint32_t q = 0; q < 8; ++q) {
+            const uint32_t e = uint32_t(__builtin_amdgcn_readfirstlane(int(list_s[min(index / batches * 4 + q / 2, count - 1)])));
+            ahead[q] = ldg_u4(w + uint64_t(e) * K + (q % 2 * 8 + lane / 8) * P + i);
+        }
+    };
+    if (total) request(0);
     float c = 0;
     for (uint32_t index = 0; index < total; ++index) {
-        uint4 piece[8];
 #pragma unroll
-        for (int q = 0; q < 8; ++q) piece[q] = ahead[q];
-        if (index + 1 < total) request(index + 1, ahead);
+        for (uint32_t q = 0; q < 8; ++q) w_s[(q * 8 + lane / 8) * 8 + (lane + (q * 8 + lane / 8) % 16 / 2) % 8] = ahead[q];
+        if (index + 1 < total) request(index + 1);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         const uint32_t i0 = index % batches * 64;
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
-            if (i0 + 8 * uint32_t(q) >= P) break;
-            const uint4 xv4 = *reinterpret_cast<const uint4*>(xr + i0 + 8 * q);
-            const uint32_t ww[4] = {piece[q].x, piece[q].y, piece[q].z, piece[q].w}, xw[4] = {xv4.x, xv4.y, xv4.z, xv4.w};
+        for (uint32_t q = 0; q < 8; ++q) {
+            if (i0 + 8 * q >= P) break;
+            const uint4 xv4 = *reinterpret_cast<const uint4*>(xr + i0 + 8 * q), wv4 = w_s[lane * 8 + (q + split / 2) % 8];
+            const uint32_t ww[4] = {wv4.x, wv4.y, wv4.z, wv4.w}, xw[4] = {xv4.x, xv4.y, xv4.z, xv4.w};
 #pragma unroll
             for (int k = 0; k < 8; ++k)
                 c = __builtin_fmaf(__uint_as_float((k & 1) ? (xw[k / 2] & 0xffff0000u) : (xw[k / 2] << 16)),
                                    __uint_as_float((k & 1) ? (ww[k / 2] & 0xffff0000u) : (ww[k / 2] << 16)), c);
         }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         if (index % batches + 1 == batches) {   // the expert's chains are complete: partials added 0..15, then the offset
             const uint32_t at = index / batches * 4 + lane / 16;
             float sum = 0;
             for (uint32_t sidx = 0; sidx < 16; ++sidx) sum += __shfl(c, base + sidx);
-            if (split == 0 && at < count) { const uint32_t e = list_s[wave][at]; row_s[wave][e] = offsets ? sum + offsets[e] : sum; }
+            if (split == 0 && at < count) { const uint32_t e = list_s[at]; row_s[e] = offsets ? sum + offsets[e] : sum; }
             c = 0;
         }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (!ids) { for (uint32_t e = lane; e < E; e += 64) row[e] = row_s[wave][e]; return; }
+    if (!ids) { for (uint32_t e = lane; e < E; e += 64) row[e] = row_s[e]; return; }
     auto fetch = [&](auto& cand, uint32_t per) {
         constexpr int PER = int(sizeof(cand) / sizeof(float));
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
             const uint32_t e = lane * per + uint32_t(i);
-            cand[i] = (uint32_t(i) < per && e < E) ? row_s[wave][e] : ninf;
+            cand[i] = (uint32_t(i) < per && e < E) ? row_s[e] : ninf;
         }
     };
     if (E == 512) route_token<8>(fetch, E, topk, lane, ids_s[wave], weights_s[wave], pick_s[wave], []() {}, []() {});
@@ -993,20 +1024,23 @@ __global__ __launch_bounds__(256) void router_refine_kernel(const uint16_t* xb, 
     if (lane < topk) { ids[uint64_t(t) * topk + lane] = ids_s[wave][lane]; weights[uint64_t(t) * topk + lane] = weights_s[wave][lane]; }
 }
 // Router logits for the selection that follows: exact where it can matter, -inf elsewhere.  xb: the inputs as bf16 rows;
-// norms: rows + experts floats of scratch.  K % 128 == 0, experts <= 1024.
-void launch_prefill_router(hipStream_t s, const float* x, const uint16_t* xb, const void* w, const float* offsets, uint32_t T, uint32_t K,
-                           uint32_t E, uint32_t topk, float* norms, float* logits, int32_t* ids, float* weights) {
+// norms: those of the router's rows (launch_prefill_rows).  K % 128 == 0, experts <= 1024.
+void launch_prefill_router(hipStream_t s, const uint16_t* xb, const void* w, const float* offsets, uint32_t T, uint32_t K,
+                           uint32_t E, uint32_t topk, const float* norms, float* logits, int32_t* ids, float* weights) {
     const uint16_t* wb = static_cast<const uint16_t*>(w);
-    hipLaunchKernelGGL(row_norms_kernel, dim3((T + E + 3) / 4), dim3(256), 0, s, xb, T, wb, E, K, norms);
-    hipLaunchKernelGGL(router_product_kernel, dim3((E + 63) / 64, (T + 63) / 64), dim3(256), 0, s, xb, wb, T, E, K, offsets, logits);
-    hipLaunchKernelGGL(router_refine_kernel, dim3((T + 3) / 4), dim3(256), 4 * K * 2, s, xb, wb, offsets, norms, T, E, K, topk, logits, ids, weights);
+    const uint32_t blocks = ((E + 63) / 64) * ((T + 63) / 64), lds = 4 * refine_lds(K, E).bytes;
+    hipLaunchKernelGGL(router_product_kernel, dim3((blocks + 7) / 8 * 8), dim3(256), 0, s, xb, wb, T, E, K, offsets, logits);
+    if (lds > 48 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(router_refine_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    hipLaunchKernelGGL(router_refine_kernel, dim3((T + 3) / 4), dim3(256), lds, s, xb, wb, offsets, norms, T, E, K, topk, logits, ids, weights);
 }
 
-void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain, int32_t* status) {
-    hipLaunchKernelGGL((prefill_rows_kernel<true>), dim3((rows * (K / 4) + 255) / 256), dim3(256), 0, s, x, rows, K, xb, xp, planes, plain, status);
+void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain, int32_t* status,
+                         const void* norm_of, uint32_t norm_rows, float* norms) {
+    hipLaunchKernelGGL((prefill_rows_kernel<true>), dim3((rows * (K / 4) + 255) / 256 + (norm_rows + 3) / 4), dim3(256), 0, s, x, rows, K, xb, xp, planes, plain, status,
+                       static_cast<const uint16_t*>(norm_of), norm_rows, norms);
 }
 void launch_prefill_acts(hipStream_t s, const uint16_t* xb, uint32_t rows, uint32_t K, uint16_t* xp, uint16_t* planes, uint16_t* plain) {
-    hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3((rows * (K / 4) + 255) / 256), dim3(256), 0, s, xb, rows, K, nullptr, xp, planes, plain, nullptr);
+    hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3((rows * (K / 4) + 255) / 256), dim3(256), 0, s, xb, rows, K, nullptr, xp, planes, plain, nullptr, nullptr, 0u, nullptr);
 }
 void launch_prefill_tiles(hipStream_t s, const int32_t* offsets, uint32_t experts, uint32_t rows, int32_t* tile_expert, int32_t* tile_first,
                           int32_t* tile_rows, int32_t* tile_count) {
@@ -1017,7 +1051,7 @@ void launch_prefill_dispatch(hipStream_t s, const int32_t* ids, uint32_t tokens,
     const uint32_t n = tokens * topk, stretch = ((n + kDispatchParts - 1) / kDispatchParts + 1023) / 1024 * 1024;
     const size_t lds = size_t(((kDispatchParts + 2) * E + 2 + 3) / 4 * 4 + stretch) * 4;
     if (lds > 48 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_dispatch_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
-    hipLaunchKernelGGL(prefill_dispatch_kernel, dim3((E + 3) / 4, kDispatchParts), dim3(256), lds, s, ids, n, topk, E, stretch, offsets, slots, rows, status,
+    hipLaunchKernelGGL(prefill_dispatch_kernel, dim3((E + kDispatchThreads / 64 - 1) / (kDispatchThreads / 64), kDispatchParts), dim3(kDispatchThreads), lds, s, ids, n, topk, E, stretch, offsets, slots, rows, status,
                        tile_expert, tile_first, tile_rows, tile_count);
 }
 // whether launch_prefill_dispatch takes this batch (else: launch_dispatch and launch_prefill_tiles)
