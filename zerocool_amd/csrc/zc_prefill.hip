@@ -576,14 +576,18 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
         if constexpr (!GATED) { if (p.out_rows) out_row[rb] = ldg_u32(p.out_rows, pos); }
     }
     add_bias_sizes();
-    // epilogue: row m of the tile is sorted position first + m.  A sum close to a BF16 rounding boundary could round
-    // the other way under the reference's order of additions: such elements are listed for exact recomputation.  v rounds to
-    // r; the boundary next to r is half a BF16 step from it, the step that of the smallest magnitude v - e that the sum
-    // could have.  (A magnitude that is not finite, of a row or group that left the operand's range, marks the element.)
+    // epilogue: row m of the tile is sorted position first + m.  A sum v close to a BF16 rounding boundary could round
+    // the other way under the reference's order of additions: it is marked for exact recomputation if v - e and v + e round apart, e
+    // the margin and what forming v - e and v + e may lose.  Where they do not, both are v's BF16 value.  (A magnitude that is not
+    // finite, of a row or group that left the operand's range, marks the sum.)
+    // (Seven instructions a sum; a rounding of its own and the distance from it were sixteen, a layer of 2048 tokens of hidden 2048 582 -> 572 us,
+    // 1500 of hidden 3072 1053 -> 1043.)
     const float margin = p.near_margin;
-    auto near_boundary = [margin](float v, float r, float m) {
-        const float e = m * margin, least = fabsf(v) - e;
-        return !(least > 0.0f) || fabsf(v - r) + e >= __uint_as_float(__float_as_uint(least) & 0x7f800000u) * 0x1p-8f;
+    auto round_both = [margin](float v, float m, bool& near) {
+        const float e = __builtin_fmaf(fabsf(v), 0x1p-24f, m * margin), low = v - e, high = v + e;
+        const uint32_t both = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{low, high}, bf16x2));
+        near = !(low <= high) || (both & 0xffffu) != both >> 16;
+        return both << 16;
     };
     // Outputs and marks (one bit per sum: [sorted position][gate, up][N / 32] words, or [sorted position][N / 32]) cross through LDS, so that they leave in
     // whole pieces of a row: two-byte stores straight from the accumulators' lanes took longer than the walk of a short row.
@@ -597,13 +601,13 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
 #pragma unroll
             for (int q = 0; q < (GATED ? 1 : 2); ++q) {
                 const uint32_t col = GATED ? wave * 16 : (2 * wave + uint32_t(q)) * 16;
-                float value = bf(total[rb][q][r]);
-                const bool near = near_boundary(total[rb][q][r], value, mag[rb][q][r]);
+                bool near;
+                float value = __uint_as_float(round_both(total[rb][q][r], mag[rb][q][r], near));
                 const uint64_t marks = __ballot(near);
                 if (j == 0) marks_s[m * 8 + col / 16] = uint16_t(marks >> (16 * g4));
                 if constexpr (GATED) {   // where one of the two is marked the other waits in the output's place
-                    const float up = bf(total[rb][1][r]);
-                    const bool up_near = near_boundary(total[rb][1][r], up, mag[rb][1][r]);
+                    bool up_near;
+                    const float up = __uint_as_float(round_both(total[rb][1][r], mag[rb][1][r], up_near));
                     const uint64_t up_marks = __ballot(up_near);
                     if (j == 0) marks_s[m * 8 + 4 + col / 16] = uint16_t(up_marks >> (16 * g4));
                     value = near ? up : up_near ? value : swiglu_rounded(value, up);
