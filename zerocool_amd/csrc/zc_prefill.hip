@@ -787,14 +787,15 @@ __global__ __launch_bounds__(256) void prefill_patch_kernel(PrefillGemm p, uint3
                 } else
 #pragma unroll
                 for (int i = 0; i < WIDTH; i += 8) {
-                    // nibble j of a word is element j: the even ones and the odd ones as bytes, each converted by one byte-to-float instruction
+                    // nibble j of a word is element j: the even ones and the odd ones as bytes, which are 8-bit floats of code * 2^-9: two
+                    // converted by one instruction
                     const uint32_t even = words[u][i / 8] & 0x0f0f0f0fu, odd = (words[u][i / 8] >> 4) & 0x0f0f0f0fu;
+                    const f32x2 c02 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(even, 512.0f, false), c46 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(even, 512.0f, true);
+                    const f32x2 c13 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(odd, 512.0f, false), c57 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(odd, 512.0f, true);
                     // (a BF16 value times a 4-bit code is exact in fp32, so a fused multiply-add rounds as the reference's
                     // multiply and add do: ((p0 + p1) + p2) + p3, then onto the block's sum)
-                    dot += __builtin_fmaf(x[i + 3], float((odd >> 8) & 0xffu), __builtin_fmaf(x[i + 2], float((even >> 8) & 0xffu),
-                           __builtin_fmaf(x[i + 1], float(odd & 0xffu), x[i] * float(even & 0xffu))));
-                    dot += __builtin_fmaf(x[i + 7], float(odd >> 24), __builtin_fmaf(x[i + 6], float(even >> 24),
-                           __builtin_fmaf(x[i + 5], float((odd >> 16) & 0xffu), x[i + 4] * float((even >> 16) & 0xffu))));
+                    dot += __builtin_fmaf(x[i + 3], c13.y, __builtin_fmaf(x[i + 2], c02.y, __builtin_fmaf(x[i + 1], c13.x, x[i] * c02.x)));
+                    dot += __builtin_fmaf(x[i + 7], c57.y, __builtin_fmaf(x[i + 6], c46.y, __builtin_fmaf(x[i + 5], c57.x, x[i + 4] * c46.x)));
                 }
                 result += b16(scale_bits[u]) * dot + sums[row * blocks + b] * b16(bias_bits[u]);
             }
