@@ -741,7 +741,7 @@ namespace {
 struct PrefillSpace {
     Workspace base;
     // rows of the products: as bf16, as the matrix-core operand, their group sums in pieces (xplain: for affine Q8 gate/up 
-    uint16_t *xb, *actb, *sactb, *xp, *actp, *sactp, *xplanes, *xplain, *aplanes, *splanes;
+    uint16_t *xb, *xp, *actp, *sactp, *xplanes, *xplain, *aplanes, *splanes;
     int32_t *tile_expert, *tile_first, *tile_rows, *tile_count, *stile_expert, *stile_first, *stile_rows, *stile_count;
     uint32_t max_tiles, max_shared_tiles;
     uint32_t* near_bits;      // one bit per product element: recompute exactly
@@ -758,8 +758,8 @@ PrefillSpace carve_prefill(const zc_moe_config* c, uint32_t T, void* base) {
     w.max_tiles = (uint32_t(n / 32 + c->experts) + 7) / 8 * 8; w.max_shared_tiles = ((T + 31) / 32 + 7) / 8 * 8;   // (the product kernel deals tiles out eight at a time)
     const uint64_t xpitch = 3 * 2 * zc::prefill_pitch(c->hidden), apitch = 3 * 2 * zc::prefill_pitch(c->inter);
     w.xb = (uint16_t*)take(uint64_t(T) * c->hidden * 2); w.xp = (uint16_t*)take(uint64_t(T) * c->hidden * 2); w.xplanes = (uint16_t*)take(T * xpitch);
-    w.actb = (uint16_t*)take(n * c->inter * 2); w.actp = (uint16_t*)take(n * c->inter * 2); w.aplanes = (uint16_t*)take(n * apitch);
-    w.sactb = (uint16_t*)take(uint64_t(T) * c->inter * 2); w.sactp = (uint16_t*)take(uint64_t(T) * c->inter * 2); w.splanes = (uint16_t*)take(T * apitch);
+    w.actp = (uint16_t*)take(n * c->inter * 2); w.aplanes = (uint16_t*)take(n * apitch);
+    w.sactp = (uint16_t*)take(uint64_t(T) * c->inter * 2); w.splanes = (uint16_t*)take(T * apitch);
     w.tile_expert = (int32_t*)take(w.max_tiles * 4ull); w.tile_first = (int32_t*)take(w.max_tiles * 4ull); w.tile_rows = (int32_t*)take(w.max_tiles * 4ull);
     w.tile_count = (int32_t*)take(4);
     w.stile_expert = (int32_t*)take(w.max_shared_tiles * 4ull); w.stile_first = (int32_t*)take(w.max_shared_tiles * 4ull);
@@ -814,7 +814,7 @@ zc_status zc_hip_moe_prefill(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
     const bool bounds = T >= kPrefillBoundsTokens && !(trace && trace->logits);
     const bool x_q4 = c->bits_gate_up == 4 || c->shared_bits_gate_up == 4, x_q8 = c->bits_gate_up == 8 || c->shared_bits_gate_up == 8;
     auto rows_on = [&](hipStream_t t) {
-        zc::launch_prefill_rows(t, x, T, H, w.xb, w.xp, x_q4 ? w.xplanes : nullptr, x_q8 ? w.xplain : nullptr, ctx->moe_status,
+        zc::launch_prefill_rows(t, x, T, H, bounds ? w.xb : nullptr, w.xp, x_q4 ? w.xplanes : nullptr, x_q8 ? w.xplain : nullptr, ctx->moe_status,
                                 l->router, bounds ? E : 0u, w.norms);
     };
     if (bounds) rows_on(s);
@@ -848,18 +848,18 @@ zc_status zc_hip_moe_prefill(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
     {   // routed gate/up + SwiGLU on gathered rows (pipeline.cpp:18-24), then down scattered to the slots (pipeline.cpp:25-29)
         zc::PrefillGemm g{};
         g.bits = c->bits_gate_up;
-        g.a = w.xp; g.a_plain = w.xb; g.planes = g.bits == 4 ? w.xplanes : w.xplain; g.a_rows = w.base.rows; g.out_rows = nullptr;
+        g.a = w.xp; g.planes = g.bits == 4 ? w.xplanes : w.xplain; g.a_rows = w.base.rows; g.out_rows = nullptr;
         g.records = static_cast<const uint8_t*>(l->expert_records); g.stride = l->record_stride; offsets_of(l->expert_records, 0, g.off, 0, 2);
         g.tile_expert = w.tile_expert; g.tile_first = w.tile_first; g.tile_rows = w.tile_rows; g.tile_count = w.tile_count;
-        g.K = H; g.N = I; g.out_b = w.actb;
+        g.K = H; g.N = I; g.out_b = w.actp;
         g.near_bits = w.near_bits; g.near_words = uint32_t(uint64_t(n) * I / 16); g.near_margin = zc::prefill_margin(g.K); g.ids = w.base.ids; g.slots = w.base.slots;
         g.covered = w.base.offsets + E; g.experts = E;
         zc::launch_prefill_gemm(s, g, true, w.max_tiles);
         zc::launch_prefill_patch(s, g, true);
         zc::PrefillGemm d{};
         d.bits = c->bits_down;
-        zc::launch_prefill_acts(s, w.actb, uint32_t(n), I, w.actp, d.bits == 4 ? w.aplanes : nullptr, d.bits == 8 ? w.aplanes : nullptr);
-        d.a = w.actp; d.a_plain = w.actb; d.planes = w.aplanes; d.a_rows = nullptr; d.out_rows = w.base.slots;
+        zc::launch_prefill_acts(s, w.actp, uint32_t(n), I, d.bits == 4 ? w.aplanes : nullptr, d.bits == 8 ? w.aplanes : nullptr);
+        d.a = w.actp; d.planes = w.aplanes; d.a_rows = nullptr; d.out_rows = w.base.slots;
         d.records = g.records; d.stride = g.stride; offsets_of(l->expert_records, 0, d.off, 2, 1);
         d.tile_expert = w.tile_expert; d.tile_first = w.tile_first; d.tile_rows = w.tile_rows; d.tile_count = w.tile_count;
         d.K = I; d.N = H;
@@ -873,17 +873,17 @@ zc_status zc_hip_moe_prefill(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
     {   // shared expert (model.cpp:482-485): one group of all the tokens, beside the routed experts
         zc::PrefillGemm g{};
         g.bits = c->shared_bits_gate_up;
-        g.a = w.xp; g.a_plain = w.xb; g.planes = g.bits == 4 ? w.xplanes : w.xplain; g.a_rows = nullptr;
+        g.a = w.xp; g.planes = g.bits == 4 ? w.xplanes : w.xplain; g.a_rows = nullptr;
         g.records = static_cast<const uint8_t*>(l->shared_record); g.stride = 0; offsets_of(l->shared_record, 1, g.off, 0, 2);
         g.tile_expert = w.stile_expert; g.tile_first = w.stile_first; g.tile_rows = w.stile_rows; g.tile_count = w.stile_count;
-        g.K = H; g.N = I; g.out_b = w.sactb;
+        g.K = H; g.N = I; g.out_b = w.sactp;
         g.near_bits = w.shared_near_bits; g.near_words = uint32_t(uint64_t(T) * I / 16); g.near_margin = zc::prefill_margin(g.K); g.ids = nullptr; g.slots = nullptr;
         zc::launch_prefill_gemm(s2, g, true, w.max_shared_tiles);
         zc::launch_prefill_patch(s2, g, true);
         zc::PrefillGemm d{};
         d.bits = c->shared_bits_down;
-        zc::launch_prefill_acts(s2, w.sactb, T, I, w.sactp, d.bits == 4 ? w.splanes : nullptr, d.bits == 8 ? w.splanes : nullptr);
-        d.a = w.sactp; d.a_plain = w.sactb; d.planes = w.splanes; d.a_rows = nullptr; d.out_rows = nullptr;
+        zc::launch_prefill_acts(s2, w.sactp, T, I, d.bits == 4 ? w.splanes : nullptr, d.bits == 8 ? w.splanes : nullptr);
+        d.a = w.sactp; d.planes = w.splanes; d.a_rows = nullptr; d.out_rows = nullptr;
         d.records = g.records; d.stride = 0; offsets_of(l->shared_record, 1, d.off, 2, 1);
         d.tile_expert = w.stile_expert; d.tile_first = w.stile_first; d.tile_rows = w.stile_rows; d.tile_count = w.stile_count;
         d.K = I; d.N = H; d.out_f = w.base.shared;

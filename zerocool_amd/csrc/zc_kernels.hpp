@@ -145,7 +145,6 @@ hipError_t decode_wide_occupancy(uint32_t lds_bytes, int* blocks_per_cu);
 // ---- prefill: sorted-token grouped GEMM on the bf16 matrix cores (zc_prefill.hip)
 struct PrefillGemm {
     const uint16_t* a;        // rows [.][K] as the product kernel reads them (prefill_rows_kernel's xp)
-    const uint16_t* a_plain;  // the same rows as bf16 in their own order (read by the recomputation)
     const uint16_t* planes;   // per (row, group of 64): the input sum in three bf16 pieces
     const int32_t* a_rows;    // row of `a` for sorted position pos: a_rows ? a_rows[pos] : pos   (gate/up; down: null)
     const int32_t* out_rows;  // output row for sorted position pos: out_rows ? out_rows[pos] : pos   (down projection)
@@ -154,7 +153,7 @@ struct PrefillGemm {
     const int32_t *tile_expert, *tile_first, *tile_rows, *tile_count;
     uint32_t K, N;            // reduction length, rows of ONE projection
     uint32_t bits;            // 4: nibble codes, planes of the Q4 lanes' BF16-rounded sum-of-four chains; 8: byte codes, planes of the Q8 lanes' plain sums
-    uint16_t* out_b;          // gate/up: SwiGLU activations as bf16 [sorted position][N]
+    uint16_t* out_b;          // gate/up: SwiGLU activations as bf16 [sorted position][N], every eight in the order that `a` has them in
     float* out_f;             // down: BF16-rounded fp32 [output row][N]
     uint16_t* out_h;          // down, instead of out_f when not null: the same values as bf16 (what the combine reads is half as long)
     // Sums that land within near_margin * (sum of term magnitudes) of a BF16 rounding boundary are marked in a bit map
@@ -182,7 +181,7 @@ constexpr float prefill_margin(uint32_t K) { return K / 64 < 8 ? 0x1p-22f : (K /
 constexpr uint32_t prefill_pitch(uint32_t K) { return (K / 64 + 7) / 8 * 8; }   // of a piece's row: sixteen-byte loads
 void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t K, uint16_t* xb, uint16_t* xp, uint16_t* planes, uint16_t* plain, int32_t* status,
                          const void* norm_of, uint32_t norm_rows, float* norms);   // norm_rows, optional: |row| of as many bf16 rows
-void launch_prefill_acts(hipStream_t s, const uint16_t* xb, uint32_t rows, uint32_t K, uint16_t* xp, uint16_t* planes, uint16_t* plain);
+void launch_prefill_acts(hipStream_t s, const uint16_t* xp, uint32_t rows, uint32_t K, uint16_t* planes, uint16_t* plain);
 // ids / weights not null (topk <= 64): the selection runs in the same launch and the logits are not written
 void launch_prefill_router(hipStream_t s, const uint16_t* xb, const void* w, const float* offsets, uint32_t T, uint32_t K,
                            uint32_t E, uint32_t topk, const float* norms, float* logits, int32_t* ids, float* weights);

@@ -52,9 +52,10 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 constexpr uint32_t kTileRows = 32, kTileRowsMax = 48, kPitch = 136;   // LDS row pitch in bf16 elements: 128 elements of a row, sixteen rows on different banks
 
 // What the matrix-core products and the recomputation need of their token rows, from fp32 rows holding BF16 values (F32)
-// or from bf16 rows (the SwiGLU activations): a thread takes four neighbouring elements, so loads and stores are whole runs.
-//   xb      the row as bf16 (F32 only)
-//   xp      the row as bf16, every eight elements in the order 0 2 4 6 1 3 5 7: the matrix-core operand
+// or from bf16 rows in the operand's order (the SwiGLU activations): a thread takes four neighbouring elements, so loads and stores are whole runs.
+//   xb      the row as bf16 (F32 only, and only for the router on bounds)
+//   xp      the row as bf16, every eight elements in the order 0 2 4 6 1 3 5 7: the matrix-core operand (F32 only: the product kernel leaves the
+//           activations in that order)
 //   planes  per (row, group of 64) the group's input sum as three bf16 pieces, [row][piece][prefill_pitch(K)]: the four
 //           blocks' BF16-rounded sum-of-four chains (Q4 lanes), NaN where the group leaves the operand's exact range
 //   plain   the same of the plain fp32 sums (Q8 lanes, qwen.metal:112-125: sum += v, element by element in blocks of eight)
@@ -111,10 +112,12 @@ __global__ __launch_bounds__(256) void prefill_rows_kernel(const void* x, uint32
         if (low) atomicOr(status, 4);
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] = __uint_as_float(__float_as_uint(v[k]) & 0xffff0000u);
-        reinterpret_cast<uint2*>(xb)[i] = make_uint2((__float_as_uint(v[0]) >> 16) | __float_as_uint(v[1]), (__float_as_uint(v[2]) >> 16) | __float_as_uint(v[3]));
+        if (xb) reinterpret_cast<uint2*>(xb)[i] = make_uint2((__float_as_uint(v[0]) >> 16) | __float_as_uint(v[1]), (__float_as_uint(v[2]) >> 16) | __float_as_uint(v[3]));
     } else {
-        const uint2 q = reinterpret_cast<const uint2*>(x)[i];
-        v[0] = __uint_as_float(q.x << 16); v[1] = __uint_as_float(q.x & 0xffff0000u); v[2] = __uint_as_float(q.y << 16); v[3] = __uint_as_float(q.y & 0xffff0000u);
+        const uint2 q = reinterpret_cast<const uint2*>(x)[i];   // a pair's even lane: elements 0 2 | 4 6, the odd one 1 3 | 5 7
+        const bool odd = lane & 1u;
+        const uint32_t other = uint32_t(__shfl_xor(int(odd ? q.x : q.y), 1)), even = odd ? other : q.x, uneven = odd ? q.y : other;
+        v[0] = __uint_as_float(even << 16); v[1] = __uint_as_float(uneven << 16); v[2] = __uint_as_float(even & 0xffff0000u); v[3] = __uint_as_float(uneven & 0xffff0000u);
     }
     uint32_t largest = 0;
 #pragma unroll
@@ -122,7 +125,7 @@ __global__ __launch_bounds__(256) void prefill_rows_kernel(const void* x, uint32
 #pragma unroll
     for (int o = 1; o < 16; o <<= 1) largest = max(largest, uint32_t(__shfl_xor(int(largest), o)));
     const bool strange = largest >= 0x71800000u || (largest != 0 && largest < 0x21800000u);   // 2^100, 2^-60
-    {   // lane 2m of a pair holds elements 0..3, lane 2m + 1 elements 4..7: 0 2 4 6 | 1 3 5 7
+    if constexpr (F32) {   // lane 2m of a pair holds elements 0..3, lane 2m + 1 elements 4..7: 0 2 4 6 | 1 3 5 7
         const uint32_t even = (__float_as_uint(v[0]) >> 16) | __float_as_uint(v[2]), uneven = (__float_as_uint(v[1]) >> 16) | __float_as_uint(v[3]);
         const bool odd = lane & 1u;
         const uint32_t other = uint32_t(__shfl_xor(int(odd ? even : uneven), 1));
@@ -623,7 +626,9 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
         const uint32_t pos = first + m;
         const uint4 v = *reinterpret_cast<const uint4*>(out_s + m * kOutPitch + c * 8);
         if constexpr (GATED) {
-            *reinterpret_cast<uint4*>(p.out_b + uint64_t(pos) * N + n0 + c * 8) = v;
+            *reinterpret_cast<uint4*>(p.out_b + uint64_t(pos) * N + n0 + c * 8) =   // in the operand's order
+                make_uint4(__builtin_amdgcn_perm(v.y, v.x, 0x05040100u), __builtin_amdgcn_perm(v.w, v.z, 0x05040100u),
+                           __builtin_amdgcn_perm(v.y, v.x, 0x07060302u), __builtin_amdgcn_perm(v.w, v.z, 0x07060302u));
             if (c < 2) *reinterpret_cast<uint2*>(p.near_bits + (uint64_t(pos) * 2 * N + c * N + n0) / 32) = *reinterpret_cast<const uint2*>(marks_s + m * 8 + c * 4);
         } else {
             const uint64_t at = uint64_t(out_row[i]) * N + n0 + c * 8;   // (a piece's row is the thread's row of block i)
@@ -697,7 +702,9 @@ __global__ __launch_bounds__(256) void prefill_patch_kernel(PrefillGemm p, uint3
         for (uint32_t u = 0; u < 4; ++u) {
             const uint32_t i = min(i0 + 256 * u, rows * pieces - 1), r = i / pieces, c = i - r * pieces;
             const uint32_t a_row = p.a_rows ? uint32_t(p.a_rows[first + r]) : first + r;
-            v[u] = reinterpret_cast<const uint4*>(p.a_plain + uint64_t(a_row) * K)[c];
+            const uint4 q = reinterpret_cast<const uint4*>(p.a + uint64_t(a_row) * K)[c];   // 0 2 | 4 6 | 1 3 | 5 7
+            v[u] = make_uint4(__builtin_amdgcn_perm(q.z, q.x, 0x05040100u), __builtin_amdgcn_perm(q.z, q.x, 0x07060302u),
+                              __builtin_amdgcn_perm(q.w, q.y, 0x05040100u), __builtin_amdgcn_perm(q.w, q.y, 0x07060302u));
             at[u] = r * pieces + place(c);
         }
 #pragma unroll
@@ -803,7 +810,7 @@ __global__ __launch_bounds__(256) void prefill_patch_kernel(PrefillGemm p, uint3
         return lane_sum32(result);
         };
         if constexpr (GATED) {
-            uint16_t* out = p.out_b + uint64_t(pos) * N + n;
+            uint16_t* out = p.out_b + uint64_t(pos) * N + ((n & ~7u) | (n & 1u) << 2 | (n & 7u) >> 1);   // in the operand's order
             const bool up_first = !(element >> 16 & 1u);
             float other = b16(*out);
             const float marked = lanes_sum(p.off + (up_first ? 3 : 0));
@@ -1044,8 +1051,8 @@ void launch_prefill_rows(hipStream_t s, const float* x, uint32_t rows, uint32_t 
     hipLaunchKernelGGL((prefill_rows_kernel<true>), dim3((rows * (K / 4) + 255) / 256 + (norm_rows + 3) / 4), dim3(256), 0, s, x, rows, K, xb, xp, planes, plain, status,
                        static_cast<const uint16_t*>(norm_of), norm_rows, norms);
 }
-void launch_prefill_acts(hipStream_t s, const uint16_t* xb, uint32_t rows, uint32_t K, uint16_t* xp, uint16_t* planes, uint16_t* plain) {
-    hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3((rows * (K / 4) + 255) / 256), dim3(256), 0, s, xb, rows, K, nullptr, xp, planes, plain, nullptr, nullptr, 0u, nullptr);
+void launch_prefill_acts(hipStream_t s, const uint16_t* xp, uint32_t rows, uint32_t K, uint16_t* planes, uint16_t* plain) {
+    hipLaunchKernelGGL((prefill_rows_kernel<false>), dim3((rows * (K / 4) + 255) / 256), dim3(256), 0, s, xp, rows, K, nullptr, nullptr, planes, plain, nullptr, nullptr, 0u, nullptr);
 }
 void launch_prefill_tiles(hipStream_t s, const int32_t* offsets, uint32_t experts, uint32_t rows, int32_t* tile_expert, int32_t* tile_first,
                           int32_t* tile_rows, int32_t* tile_count) {
