@@ -302,9 +302,9 @@ __global__ __launch_bounds__(kDispatchThreads) void prefill_dispatch_kernel(cons
 // 1.5 ns; the listing of the loop: 54 and 342 per two pairs),
 // which overlap only in part -- weights and rows read from a warm cache leave the time of the walk unchanged.  A wave
 // alone issues one vector instruction every five clocks, so the registers are kept to what three waves per SIMD allow
-// (Q4: 165 and 168 of 168; with a second set of token rows or four pairs of weights in flight two waves fit, and the layer of
-// hidden 2048 took 680 us at 2048 tokens instead of 621).  At that size the routed gate/up product takes 239 us, the down product
-// 157 us (369 and 258 with a run-time number of row blocks, codes converted one by one and the scales staged through LDS).
+// (Q4: 156 and 160 of 168; with a second set of token rows or four pairs of weights in flight two waves fit, and the layer of
+// hidden 2048 took 680 us at 2048 tokens instead of 621).  At that size the routed gate/up product takes 240 us, the down product
+// 150 us (369 and 258 with a run-time number of row blocks, codes converted one by one and the scales staged through LDS).
 template <bool GATED, int BITS, int NB>
 __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s, uint16_t* marks_s, uint16_t* bias_s, uint32_t expert, uint32_t first, uint32_t rows, uint32_t n0) {
     constexpr int kAhead = 2, kRegs = BITS;       // pairs of groups in flight; dwords of a column tile's pair per lane
