@@ -56,3 +56,28 @@ def test_prefill_dispatch_of_many_slots(ctx, experts, topk, T):
     assert np.mean(fast.view(np.uint32) == exact.view(np.uint32)) > 0.9999
     for b in (weights.router, weights.shared_gate, weights.shared_record, weights.records, x, weights.offsets):
         ctx.free(b)
+
+
+# down rows of 512: five and nine blocks of weight rows, one to three blocks of token rows and several tiles, codes of either width
+@pytest.mark.parametrize("hidden,bits", [(640, (4, 4, 4, 4)), (1152, (4, 8, 8, 8)), (128, (8, 8, 4, 4))])
+@pytest.mark.parametrize("T", [1, 16, 20, 33, 48, 65, 130])
+def test_prefill_down_rows_of_512(ctx, hidden, bits, T):
+    cfg = workload.tiny_config(hidden, 2, 2, 512, bits=bits)      # both experts have every token
+    weights = workload.LayerWeights(ctx, cfg, 23 + T, ("normal", 0.5))
+    x, n, outs = workload.hidden_rows(ctx, T, hidden, 24), T * 2, []
+    for call, size in ((ctx.moe_forward, ctx.moe_workspace_bytes), (ctx.moe_prefill, ctx.moe_prefill_workspace_bytes)):
+        out, ws, eo, sh = ctx.alloc(T * hidden * 4), ctx.alloc(size(cfg, T)), ctx.alloc(n * hidden * 4), ctx.alloc(T * hidden * 4)
+        call(cfg, weights.layer, x, T, out, ws, z.Trace(None, None, None, eo.ptr, sh.ptr, None))
+        ctx.moe_check()
+        outs.append([b.numpy(f32).copy() for b in (out, eo, sh)])
+        if call == ctx.moe_prefill:                               # outputs of the slots as bf16
+            call(cfg, weights.layer, x, T, out, ws)
+            assert out.numpy(f32).tobytes() == outs[1][0].tobytes()
+        for b in (out, ws, eo, sh):
+            ctx.free(b)
+    for exact, fast in zip(*outs):
+        assert np.max(np.abs(fast - exact)) <= 2.0 ** -7 * np.max(np.abs(exact))
+        assert np.mean(fast.view(np.uint32) == exact.view(np.uint32)) > 0.9999
+    assert np.max(np.abs(outs[1][0] - outs[0][0])) <= 2e-3 * np.max(np.abs(outs[0][0]))
+    for b in (weights.router, weights.shared_gate, weights.shared_record, weights.records, x):
+        ctx.free(b)

@@ -293,6 +293,31 @@ __global__ __launch_bounds__(kDispatchThreads) void prefill_dispatch_kernel(cons
     }
 }
 
+// codes -> matrix-core operand, element order 0 2 4 6 1 3 5 7: eight nibbles of a word, or eight bytes of two words
+__device__ __forceinline__ bf16x8 nibble_operand(uint32_t word) {
+    const uint32_t even = word & 0x0f0f0f0fu, odd = (word >> 4) & 0x0f0f0f0fu;
+    auto two = [](bf16x2 v) { return __builtin_bit_cast(uint32_t, v); };
+    return __builtin_bit_cast(bf16x8, make_uint4(two(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, false)), two(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, true)),
+                                                 two(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, false)), two(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, true))));
+}
+__device__ __forceinline__ bf16x8 byte_operand(uint32_t lo, uint32_t hi) {
+    auto two = [](uint32_t word, int i) {   // bytes i and i + 2: whole numbers up to 255 have all their bits in a float's upper half
+        return __builtin_amdgcn_perm(__float_as_uint(float((word >> (8 * i + 16)) & 0xffu)), __float_as_uint(float((word >> (8 * i)) & 0xffu)), 0x07060302u);
+    };
+    return __builtin_bit_cast(bf16x8, make_uint4(two(lo, 0), two(hi, 0), two(lo, 1), two(hi, 1)));
+}
+// A sum v, terms of magnitude m, close to a BF16 rounding boundary could round
+// the other way under the reference's order of additions: it is marked for exact recomputation if v - e and v + e round apart, e
+// the margin and what forming v - e and v + e may lose.  Where they do not, both are v's BF16 value.  (A magnitude that is not
+// finite, of a row or group that left the operand's range, marks the sum.)
+// (Seven instructions a sum; a rounding of its own and the distance from it were sixteen, a layer of 2048 tokens of hidden 2048 582 -> 572 us,
+// 1500 of hidden 3072 1053 -> 1043.)
+__device__ __forceinline__ uint32_t prefill_round(float v, float m, float margin, bool& near) {
+    const float e = __builtin_fmaf(fabsf(v), 0x1p-24f, m * margin), low = v - e, high = v + e;
+    const uint32_t both = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{low, high}, bf16x2));
+    near = !(low <= high) || (both & 0xffffu) != both >> 16;
+    return both << 16;
+}
 // One tile: up to 16 NB rows of one expert x 128 weight rows.  BITS: 4 (nibble codes) or 8 (byte codes; the planes are then
 // the plain sums of the Q8 lanes).  The number of row blocks is a compile-time value, so that the walk over K is straight-line
 // code: as a run-time bound it cut every step into short blocks that each waited for its own LDS reads.
@@ -471,19 +496,6 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
 #pragma unroll
                 for (int r = 0; r < 4; ++r) mag[rb][q][r] *= 1.0078125f;
     };
-    // codes -> matrix-core operand, element order 0 2 4 6 1 3 5 7: eight nibbles of a word, or eight bytes of two words
-    auto nibbles = [](uint32_t word) {
-        const uint32_t even = word & 0x0f0f0f0fu, odd = (word >> 4) & 0x0f0f0f0fu;
-        auto two = [](bf16x2 v) { return __builtin_bit_cast(uint32_t, v); };
-        return __builtin_bit_cast(bf16x8, make_uint4(two(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, false)), two(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, true)),
-                                                     two(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, false)), two(__builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, true))));
-    };
-    auto bytes = [](uint32_t lo, uint32_t hi) {
-        auto two = [](uint32_t word, int i) {   // bytes i and i + 2: whole numbers up to 255 have all their bits in a float's upper half
-            return __builtin_amdgcn_perm(__float_as_uint(float((word >> (8 * i + 16)) & 0xffu)), __float_as_uint(float((word >> (8 * i)) & 0xffu)), 0x07060302u);
-        };
-        return __builtin_bit_cast(bf16x8, make_uint4(two(lo, 0), two(hi, 0), two(lo, 1), two(hi, 1)));
-    };
     // elements of a group that lane (j, g4) multiplies, from this one on: sixteen of them.  Q4: a load brings the four
     // lanes of a row the four quarters of two groups; a swap between the half waves gives every lane its share of either
     const uint32_t koff = BITS == 4 ? (g4 & 1u) * 32u + (g4 >> 1) * 16u : g4 * 16u;
@@ -518,8 +530,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
             for (int q = 0; q < 2; ++q)
 #pragma unroll
                 for (int kk = 0; kk < 2; ++kk) {
-                    if constexpr (BITS == 4) b[q][kk] = nibbles(codes[q][2 * h + kk]);
-                    else b[q][kk] = bytes(codes[q][4 * h + 2 * kk], codes[q][4 * h + 2 * kk + 1]);
+                    if constexpr (BITS == 4) b[q][kk] = nibble_operand(codes[q][2 * h + kk]);
+                    else b[q][kk] = byte_operand(codes[q][4 * h + 2 * kk], codes[q][4 * h + 2 * kk + 1]);
                 }
             float scale[2];
 #pragma unroll
@@ -579,19 +591,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
         if constexpr (!GATED) { if (p.out_rows) out_row[rb] = ldg_u32(p.out_rows, pos); }
     }
     add_bias_sizes();
-    // epilogue: row m of the tile is sorted position first + m.  A sum v close to a BF16 rounding boundary could round
-    // the other way under the reference's order of additions: it is marked for exact recomputation if v - e and v + e round apart, e
-    // the margin and what forming v - e and v + e may lose.  Where they do not, both are v's BF16 value.  (A magnitude that is not
-    // finite, of a row or group that left the operand's range, marks the sum.)
-    // (Seven instructions a sum; a rounding of its own and the distance from it were sixteen, a layer of 2048 tokens of hidden 2048 582 -> 572 us,
-    // 1500 of hidden 3072 1053 -> 1043.)
+    // epilogue: row m of the tile is sorted position first + m
     const float margin = p.near_margin;
-    auto round_both = [margin](float v, float m, bool& near) {
-        const float e = __builtin_fmaf(fabsf(v), 0x1p-24f, m * margin), low = v - e, high = v + e;
-        const uint32_t both = __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{low, high}, bf16x2));
-        near = !(low <= high) || (both & 0xffffu) != both >> 16;
-        return both << 16;
-    };
     // Outputs and marks (one bit per sum: [sorted position][gate, up][N / 32] words, or [sorted position][N / 32]) cross through LDS, so that they leave in
     // whole pieces of a row: two-byte stores straight from the accumulators' lanes took longer than the walk of a short row.
     constexpr uint32_t kCols = GATED ? 64u : 128u, kOutPitch = kPitch;
@@ -605,12 +606,12 @@ __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s
             for (int q = 0; q < (GATED ? 1 : 2); ++q) {
                 const uint32_t col = GATED ? wave * 16 : (2 * wave + uint32_t(q)) * 16;
                 bool near;
-                float value = __uint_as_float(round_both(total[rb][q][r], mag[rb][q][r], near));
+                float value = __uint_as_float(prefill_round(total[rb][q][r], mag[rb][q][r], margin, near));
                 const uint64_t marks = __ballot(near);
                 if (j == 0) marks_s[m * 8 + col / 16] = uint16_t(marks >> (16 * g4));
                 if constexpr (GATED) {   // where one of the two is marked the other waits in the output's place
                     bool up_near;
-                    const float up = __uint_as_float(round_both(total[rb][1][r], mag[rb][1][r], up_near));
+                    const float up = __uint_as_float(prefill_round(total[rb][1][r], mag[rb][1][r], margin, up_near));
                     const uint64_t up_marks = __ballot(up_near);
                     if (j == 0) marks_s[m * 8 + 4 + col / 16] = uint16_t(up_marks >> (16 * g4));
                     value = near ? up : up_near ? value : swiglu_rounded(value, up);
@@ -655,6 +656,219 @@ __global__ __launch_bounds__(256, BITS == 4 ? 3 : 2) void prefill_gemm_kernel(Pr
     if (rows <= 16) prefill_tile<GATED, BITS, 1>(p, a_s, marks_s, bias_s, expert, first, rows, n0);
     else if (rows <= 32) prefill_tile<GATED, BITS, 2>(p, a_s, marks_s, bias_s, expert, first, rows, n0);
     else prefill_tile<GATED, BITS, 3>(p, a_s, marks_s, bias_s, expert, first, rows, n0);
+}
+
+// The down product of rows of 512.  prefill_tile walks four pairs of groups there, and a workgroup is mostly its requests
+// before the walk and its epilogue behind it (60 of 145 us at 2048 tokens).  Here a workgroup stages its tile's rows once, whole, and takes several
+// blocks of 128 weight rows in turn: a wave multiplies its 32 weight rows of a block without waiting for any other, and asks for the next
+// block's codes, scales and biases as it uses up this one's, so that loads are in flight during the epilogue too.  Sums, marks and outputs are
+// prefill_tile's, added in the same order.  2048 weight rows, routed product alone: 2048 tokens 141 -> 123 us, 300 tokens with byte codes 130 ->
+// 108; a layer 551 -> 534 and 332 -> 320.  (Rows of 640, whose LDS and registers leave as many waves: a layer of 300 tokens of hidden 2560 408 -> 402 us, but
+// 600 503 -> 509 and 1000 612 -> 621.  Longer rows leave one workgroup a compute unit.)
+constexpr uint32_t kShortK = 512, kShortPitch = kShortK + 8, kShortOutPitch = 40;   // pitches in bf16 elements: sixteen rows on different banks
+constexpr uint32_t kShortLds = 2 * (8 + kTileRowsMax * (kShortPitch + 3 * prefill_pitch(kShortK)) + 4 * 16 * kShortOutPitch);
+template <int BITS, int NB>
+__device__ __forceinline__ void prefill_short_tile(const PrefillGemm& p, uint16_t* lds, uint32_t expert, uint32_t first, uint32_t rows, uint32_t block0, uint32_t block1) {
+    constexpr uint32_t K = kShortK, groups = K / 64, pitch = prefill_pitch(K), kPitchX = kShortPitch;
+    constexpr int PAIRS = K / 128, kRegs = BITS, kQuads = groups / 4;   // kRegs: dwords of a column tile's pair per lane; kQuads: loads of four groups' scales
+    static_assert(groups == 8 && pitch == groups);
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, j = lane & 15u, g4 = lane >> 4, N = p.N;
+    const uint8_t* record = p.records + uint64_t(expert) * p.stride;
+    const uint8_t *codes_of = record + p.off[0], *scales_of = record + p.off[1], *biases_of = record + p.off[2];
+    uint16_t *zeros_s = lds, *planes_s = lds + 8, *x_s = planes_s + kTileRowsMax * 3 * pitch, *out_s = x_s + kTileRowsMax * kPitchX + wave * (16 * kShortOutPitch);
+    // (Bases are the same in every lane, lanes add 32-bit offsets; past the last block: it again, not used.)
+    auto lane_row = [&](int q) { return (2 * wave + uint32_t(q)) * 16 + j; };
+    u32x4 ring[PAIRS][2][kRegs / 4];
+    auto fetch_b = [&](uint32_t block, int pair, uint32_t none) {
+        const uint8_t* from = codes_of + uint64_t(min(block, block1 - 1)) * (128 * (K * BITS / 8));
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int h = 0; h < kRegs / 4; ++h) ring[pair][q][h] = *as_global<u32x4>(from + (lane_row(q) * (K * BITS / 8) + g4 * 16 + none + uint32_t(pair) * (16 * BITS) + 64u * uint32_t(h)));
+    };
+    uint2 scales_next[2][kQuads], biases_next[2][kQuads];
+    auto fetch_s = [&](uint32_t block, uint32_t none) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int i = 0; i < kQuads; ++i) {
+                const uint64_t from = uint64_t(min(block, block1 - 1)) * (128 * groups * 2);
+                const uint32_t at = (lane_row(q) * groups + 4u * uint32_t(i)) * 2 + none;
+                scales_next[q][i] = ldg_u2_by_words(scales_of + from + at); biases_next[q][i] = ldg_u2_by_words(biases_of + from + at);
+            }
+    };
+    // the tile's rows and their chain sums; rows past the end repeat the last one (never stored)
+    uint4 row[NB][PAIRS], sums[NB];
+#pragma unroll
+    for (int rb = 0; rb < NB; ++rb) {
+        const uint32_t pos = first + min(16 * uint32_t(rb) + (tid >> 4), rows - 1);
+        sums[rb] = ldg_u4(p.planes + uint64_t(pos) * (3 * pitch) + min(tid & 15u, 3 * pitch / 8 - 1) * 8);
+#pragma unroll
+        for (int i = 0; i < PAIRS; ++i) row[rb][i] = ldg_u4(p.a + uint64_t(pos) * K + ((tid & 15u) + 16 * uint32_t(i)) * 8);
+    }
+    fetch_s(block0, 0);
+#pragma unroll
+    for (int u = 0; u < PAIRS; ++u) fetch_b(block0, u, 0);
+    uint32_t out_row[NB];
+#pragma unroll
+    for (int rb = 0; rb < NB; ++rb) {
+        const uint32_t pos = first + min(16 * uint32_t(rb) + lane / 4, rows - 1);
+        out_row[rb] = p.out_rows ? ldg_u32(p.out_rows, pos) : pos;
+    }
+    if (tid < 4) reinterpret_cast<uint32_t*>(zeros_s)[tid] = 0;
+#pragma unroll
+    for (int rb = 0; rb < NB; ++rb) {
+        const uint32_t r = 16 * uint32_t(rb) + (tid >> 4), c = tid & 15u;
+        if (c < 3 * pitch / 8)
+            *reinterpret_cast<uint4*>(planes_s + r * (3 * pitch) + c * 8) = sums[rb];
+#pragma unroll
+        for (int i = 0; i < PAIRS; ++i) *reinterpret_cast<uint4*>(x_s + r * kPitchX + (c + 16 * uint32_t(i)) * 8) = row[rb][i];
+    }
+    lds_barrier();
+    const uint32_t koff = BITS == 4 ? (g4 & 1u) * 32u + (g4 >> 1) * 16u : g4 * 16u;   // (as in prefill_tile)
+    const uint16_t* x_lane = x_s + j * kPitchX + koff;
+    const uint16_t* sums_at = g4 < 3 ? planes_s + (j * 3 + g4) * pitch : zeros_s;
+    const uint32_t sums_rb = g4 < 3 ? 48 * pitch : 0u, sums_g = g4 < 3 ? 1u : 0u;
+    for (uint32_t block = block0; block < block1; ++block) {
+        uint32_t none = 0;                       // (a zero that the compiler does not know: it would form every address and read the rows once, in front of the loop, into registers that are not there)
+        asm volatile("" : "+v"(none));
+        uint2 scales[2][kQuads], biases[2][kQuads];
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int i = 0; i < kQuads; ++i) { scales[q][i] = scales_next[q][i]; biases[q][i] = biases_next[q][i]; }
+        fetch_s(block + 1, none);
+        f32x4 total[NB][2], mag[NB][2];
+#pragma unroll
+        for (int rb = 0; rb < NB; ++rb)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) total[rb][q] = mag[rb][q] = f32x4{0, 0, 0, 0};
+        auto add_biases = [&](int i) {           // of the groups 4 i .. 4 i + 3
+#pragma unroll
+            for (uint32_t rb = 0; rb < NB; ++rb) {
+                const s16x4 piece = *reinterpret_cast<const s16x4*>(sums_at + (rb * sums_rb + sums_g * 4 * uint32_t(i) + none));
+#pragma unroll
+                for (int q = 0; q < 2; ++q) total[rb][q] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(piece, __builtin_bit_cast(s16x4, biases[q][i]), total[rb][q], 0, 0, 0);
+            }
+        };
+#pragma unroll
+        for (int pair = 0; pair < PAIRS; ++pair) {
+            uint32_t codes[2][kRegs];
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int w = 0; w < kRegs; ++w) codes[q][w] = ring[pair][q][w / 4][w % 4];
+            if constexpr (BITS == 4) {
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int w = 0; w < 2; ++w) {
+                        const auto both = __builtin_amdgcn_permlane32_swap(codes[q][w], codes[q][w + 2], false, false);
+                        codes[q][w] = both[0]; codes[q][w + 2] = both[1];
+                    }
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                bf16x8 b[2][2];
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int kk = 0; kk < 2; ++kk) {
+                        if constexpr (BITS == 4) b[q][kk] = nibble_operand(codes[q][2 * h + kk]);
+                        else b[q][kk] = byte_operand(codes[q][4 * h + 2 * kk], codes[q][4 * h + 2 * kk + 1]);
+                    }
+                float scale[2];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const uint32_t two = pair % 2 ? scales[q][pair / 2].y : scales[q][pair / 2].x;
+                    scale[q] = __uint_as_float(h ? two & 0xffff0000u : two << 16);
+                }
+#pragma unroll
+                for (int rb = 0; rb < NB; ++rb) {
+                    bf16x8 a[2];
+#pragma unroll
+                    for (int kk = 0; kk < 2; ++kk) a[kk] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(x_lane + (none + 16 * uint32_t(rb) * kPitchX + 128 * uint32_t(pair) + 64 * uint32_t(h) + 8 * uint32_t(kk))));
+                    f32x4 dot[2];
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) dot[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[q][0], f32x4{0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) dot[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[q][1], dot[q], 0, 0, 0);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            total[rb][q][r] = __builtin_fmaf(scale[q], dot[q][r], total[rb][q][r]);
+                            mag[rb][q][r] = __builtin_fmaf(fabsf(scale[q]), fabsf(dot[q][r]), mag[rb][q][r]);
+                        }
+                }
+            }
+            fetch_b(block + 1, pair, none);
+            if (pair % 2 == 0) add_biases(pair / 2);
+            // (the pair is done here: the compiler would put its last multiply-adds off to where the sums are used, and keep all dots until then)
+#pragma unroll
+            for (int rb = 0; rb < NB; ++rb)
+#pragma unroll
+                for (int q = 0; q < 2; ++q) asm volatile("" : "+v"(total[rb][q]), "+v"(mag[rb][q]));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // the biases' share of the magnitudes: the operand's first quarter holds the eight groups, the others zeros
+        const uint32_t M = g4 == 0 ? 0x7fff7fffu : 0u;
+        bf16x8 size[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) size[q] = __builtin_bit_cast(bf16x8, make_uint4(biases[q][0].x & M, biases[q][0].y & M, biases[q][1].x & M, biases[q][1].y & M));
+        const uint32_t n0 = block * 128 + wave * 32;
+#pragma unroll
+        for (uint32_t rb = 0; rb < NB; ++rb) {
+            const uint4 v = *reinterpret_cast<const uint4*>(planes_s + ((rb * 16 + j) * 3 * pitch + none));
+            const bf16x8 sums_of = __builtin_bit_cast(bf16x8, make_uint4(v.x & M, v.y & M, v.z & M, v.w & M));
+#pragma unroll
+            for (int q = 0; q < 2; ++q) mag[rb][q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(sums_of, size[q], mag[rb][q], 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t m = 4 * g4 + uint32_t(r), pos = first + 16 * rb + m + none;
+                uint64_t marks[2];
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    bool near;
+                    const uint32_t value = prefill_round(total[rb][q][r], mag[rb][q][r] * 1.0078125f, p.near_margin, near);
+                    marks[q] = __ballot(near);
+                    out_s[m * kShortOutPitch + uint32_t(q) * 16 + j] = uint16_t(value >> 16);
+                }
+                if (j == 0 && 16 * rb + m < rows) p.near_bits[(uint64_t(pos) * N + n0) / 32] = (uint32_t(marks[0] >> (16 * g4)) & 0xffffu) | uint32_t(marks[1] >> (16 * g4)) << 16;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            const uint4 o = *reinterpret_cast<const uint4*>(out_s + lane / 4 * kShortOutPitch + lane % 4 * 8);
+            if (16 * rb + lane / 4 < rows) {
+                const uint64_t at = uint64_t(out_row[rb] + none) * N + n0 + lane % 4 * 8;
+                if (p.out_h) *reinterpret_cast<uint4*>(p.out_h + at) = o;
+                else {
+                    *reinterpret_cast<float4*>(p.out_f + at) = make_float4(__uint_as_float(o.x << 16), __uint_as_float(o.x & 0xffff0000u), __uint_as_float(o.y << 16), __uint_as_float(o.y & 0xffff0000u));
+                    *reinterpret_cast<float4*>(p.out_f + at + 4) = make_float4(__uint_as_float(o.z << 16), __uint_as_float(o.z & 0xffff0000u), __uint_as_float(o.w << 16), __uint_as_float(o.w & 0xffff0000u));
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+    }
+}
+template <int BITS>
+__global__ __launch_bounds__(256, 2) void prefill_short_kernel(PrefillGemm p, uint32_t share) {   // share: blocks of a workgroup
+    extern __shared__ __align__(16) uint16_t short_lds[];
+    const uint32_t blocks = p.N / 128u, shares = (blocks + share - 1) / share, turn = blockIdx.x / 8u;   // (a tile's workgroups on one die, as in prefill_gemm_kernel)
+    const uint32_t tile = turn / shares * 8u + blockIdx.x % 8u, block0 = turn % shares * share, block1 = min(block0 + share, blocks);
+    const uint32_t count = uint32_t(*p.tile_count), expert = uint32_t(p.tile_expert[tile]), first = uint32_t(p.tile_first[tile]), rows = uint32_t(p.tile_rows[tile]);
+    if (tile >= count) return;
+    if (rows <= 16) prefill_short_tile<BITS, 1>(p, short_lds, expert, first, rows, block0, block1);
+    else if (rows <= 32) prefill_short_tile<BITS, 2>(p, short_lds, expert, first, rows, block0, block1);
+    else if constexpr (BITS == 4) prefill_short_tile<BITS, 3>(p, short_lds, expert, first, rows, block0, block1);
+    else {   // (three blocks of rows beside twice the codes do not fit the registers)
+        prefill_short_tile<BITS, 2>(p, short_lds, expert, first, 32, block0, block1);
+        lds_barrier();
+        prefill_short_tile<BITS, 1>(p, short_lds, expert, first + 32, rows - 32, block0, block1);
+    }
 }
 
 // Exact recomputation of the marked elements: one group of 32 lanes plays the reference's 32 lanes for one element
@@ -1072,6 +1286,19 @@ bool prefill_dispatch_fits(const int32_t* ids, uint32_t tokens, uint32_t topk, u
     return reinterpret_cast<uintptr_t>(ids) % 16 == 0 && n > 1024 && n < (1u << 24) && E <= 1024 && n / kDispatchParts + 1024 <= 24 * 1024;
 }
 void launch_prefill_gemm(hipStream_t s, const PrefillGemm& p, bool gated, uint32_t max_tiles) {
+    if (!gated && p.K == kShortK) {
+        // (four blocks a workgroup where that leaves the chip two workgroups a compute unit: a shared expert's few tiles need more of them)
+        const uint32_t tiles = (max_tiles + 7) / 8 * 8, blocks = p.N / 128;
+        uint32_t share = 4;
+        while (share > 1 && tiles * ((blocks + share - 1) / share) < 512) share /= 2;
+        const dim3 grid(tiles * ((blocks + share - 1) / share));
+        auto go = [&](auto kernel) {
+            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(kShortLds));
+            hipLaunchKernelGGL(kernel, grid, dim3(256), kShortLds, s, p, share);
+        };
+        if (p.bits == 8) go(prefill_short_kernel<8>); else go(prefill_short_kernel<4>);
+        return;
+    }
     const dim3 grid((max_tiles + 7) / 8 * 8 * (gated ? p.N / 64 : p.N / 128));
     const uint32_t lds = (8 + (kTileRowsMax * 3 + 128) * prefill_pitch(p.K)) * 2;
     if (p.bits == 8) {
