@@ -1256,7 +1256,8 @@ void launch_prefill_router(hipStream_t s, const uint16_t* xb, const void* w, con
     const uint16_t* wb = static_cast<const uint16_t*>(w);
     const uint32_t blocks = ((E + 63) / 64) * ((T + 63) / 64), lds = 4 * refine_lds(K, E).bytes;
     hipLaunchKernelGGL(router_product_kernel, dim3((blocks + 7) / 8 * 8), dim3(256), 0, s, xb, wb, T, E, K, offsets, logits);
-    if (lds > 48 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(router_refine_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    // (the most that any shape asks for: the same whoever calls)
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(router_refine_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(4 * refine_lds(4096, 1024).bytes));
     hipLaunchKernelGGL(router_refine_kernel, dim3((T + 3) / 4), dim3(256), lds, s, xb, wb, offsets, norms, T, E, K, topk, logits, ids, weights);
 }
 
