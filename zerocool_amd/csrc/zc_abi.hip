@@ -4,8 +4,8 @@
 // of error before anything reaches the GPU.
 #include "../../include/zc_hip.h"
 #include "zc_kernels.hpp"
+#include "zc_answers.hpp"
 #include <algorithm>
-#include <atomic>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -43,7 +43,6 @@ bool overlaps(const void* a, uint64_t an, const void* b, uint64_t bn) {
     const auto x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
     return a && b && x < y + bn && y < x + an;
 }
-constexpr uint32_t kAnswers = 64;
 uint64_t align_up(uint64_t v, uint64_t a) { return (v + a - 1) / a * a; }
 }  // namespace
 
@@ -56,8 +55,7 @@ struct zc_hip_ctx {
     std::vector<hipEvent_t> tickets;   // live tickets: ticket t -> tickets[t - retired - 1]
     uint64_t retired = 0;              // tickets known complete and destroyed
     int32_t* moe_status = nullptr;     // device flag: an id outside [0,E) was seen
-    uint32_t* answers = nullptr;       // pinned words in which kernels answer gather checks, one per call in turn (calls of several threads may wait at once)
-    std::atomic<uint32_t> asked{0};
+    zc::AnswerWords answers;           // pinned words in which kernels answer gather checks (calls of several threads may wait at once)
     hipEvent_t timer[2] = {nullptr, nullptr};
     // The prefill layer runs its shared expert beside the router, the selection and the dispatch sort, which are chains of
     // small kernels: a second stream of default priority, forked from and joined to `stream` by two events per call.
@@ -140,10 +138,11 @@ zc_status zc_hip_create(int device, uint64_t budget_bytes, zc_hip_ctx** out) {
     if (hipMalloc(&ctx->moe_status, 256) != hipSuccess || hipMemsetAsync(ctx->moe_status, 0, 256, ctx->stream) != hipSuccess) {
         hipStreamDestroy(ctx->stream); delete ctx; return fail(ZC_RUNTIME_ERROR, "HIP execution: cannot allocate status word");
     }
-    if (hipHostMalloc(reinterpret_cast<void**>(&ctx->answers), kAnswers * 4, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
+    uint32_t* answers = nullptr;
+    if (hipHostMalloc(reinterpret_cast<void**>(&answers), zc::AnswerWords::kWords * 4, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess) {
         hipFree(ctx->moe_status); hipStreamDestroy(ctx->stream); delete ctx; return fail(ZC_RUNTIME_ERROR, "HIP execution: cannot allocate answer words");
     }
-    std::memset(ctx->answers, 0, kAnswers * 4);
+    ctx->answers.use(answers);
     *out = ctx;
     return ZC_OK;
 }
@@ -157,7 +156,7 @@ zc_status zc_hip_destroy(zc_hip_ctx* ctx) {
     for (auto& b : ctx->blocks) hipFree(b.first);
     for (auto& b : ctx->host_blocks) hipHostFree(b.first);
     hipFree(ctx->moe_status);
-    hipHostFree(ctx->answers);
+    hipHostFree(ctx->answers.words());
     if (ctx->beside) { hipStreamSynchronize(ctx->beside); hipStreamDestroy(ctx->beside); }
     for (hipEvent_t e : {ctx->fork, ctx->rows_ready, ctx->join}) if (e) hipEventDestroy(e);
     hipStreamDestroy(ctx->stream);
@@ -455,20 +454,32 @@ zc_status zc_hip_router_logits(zc_hip_ctx* ctx, const void* w, const float* x, u
     return ZC_OK;
 }
 // Waits for the answer of a kernel that is on the stream.  The word is polled: waiting for the kernel's end would take the product's time too.
-static zc_status await_answer(zc_hip_ctx* ctx, const zc::GatherCheck& check) {
-    for (uint32_t polls = 1;; ++polls) {
-        const uint32_t word = __atomic_load_n(check.slot, __ATOMIC_ACQUIRE);
-        if ((word & ~1u) == check.answer) {
-            ZC_REQUIRE(!(word & 1u), "fused gate/up row outside input");
-            return ZC_OK;
-        }
+static zc_status await_answer(zc_hip_ctx* ctx, const zc::AnswerWords::Question& question) {
+    using Answer = zc::AnswerWords::Answer;
+    Answer answer = Answer::none;
+    for (uint32_t polls = 1; (answer = zc::AnswerWords::look(question)) == Answer::none; ++polls) {
         __builtin_ia32_pause();
         if (polls % 4096) continue;
         const hipError_t state = hipStreamQuery(ctx->stream);   // (an error on the stream ends the wait; a stream that is done has stored the word)
         if (state == hipErrorNotReady) { (void)hipGetLastError(); continue; }
         ZC_HIP(state);
-        if ((__atomic_load_n(check.slot, __ATOMIC_ACQUIRE) & ~1u) != check.answer) return fail(ZC_RUNTIME_ERROR, "HIP execution: a gather's rows were not checked");
+        if ((answer = zc::AnswerWords::look(question)) == Answer::none) return fail(ZC_RUNTIME_ERROR, "HIP execution: a gather's rows were not checked");
+        break;
     }
+    ctx->answers.give_back(question);
+    ZC_REQUIRE(answer == Answer::yes, "fused gate/up row outside input");
+    return ZC_OK;
+}
+// The same of a caller who finds every word taken: the list is copied, and the host looks.
+static zc_status look_at_rows(zc_hip_ctx* ctx, const int32_t* rows, uint32_t n, uint32_t x_rows) {
+    int32_t piece[2048];
+    for (uint64_t at = 0; at < n; at += std::size(piece)) {
+        const uint64_t count = std::min<uint64_t>(n - at, std::size(piece));
+        ZC_HIP(hipMemcpyAsync(piece, rows + at, count * 4, hipMemcpyDeviceToHost, ctx->stream));
+        ZC_HIP(hipStreamSynchronize(ctx->stream));
+        for (uint64_t i = 0; i < count; ++i) ZC_REQUIRE(piece[i] >= 0 && uint32_t(piece[i]) < x_rows, "fused gate/up row outside input");
+    }
+    return ZC_OK;
 }
 zc_status zc_hip_gated_linear(zc_hip_ctx* ctx, const zc_linear* gate, const zc_linear* up, const float* x, uint32_t x_rows,
                               uint32_t tokens, const int32_t* rows, float* out) {
@@ -490,13 +501,13 @@ zc_status zc_hip_gated_linear(zc_hip_ctx* ctx, const zc_linear* gate, const zc_l
         hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
         ZC_HIP(hipStreamIsCapturing(ctx->stream, &capturing));
         if (capturing != hipStreamCaptureStatusNone) return fail(ZC_RUNTIME_ERROR, "HIP execution: a gather's rows cannot be checked while the stream is captured");
-        const uint32_t turn = ctx->asked.fetch_add(1, std::memory_order_relaxed);
-        zc::GatherCheck check; check.slot = ctx->answers + turn % kAnswers; check.answer = (turn << 1) | 1u << 31; check.x_rows = x_rows;
-        const bool together = !xint && tokens <= zc::kGatherInKernel;
+        const zc::AnswerWords::Question question = ctx->answers.ask();
+        const zc::GatherCheck check{question.slot, question.answer, x_rows};
+        const bool together = question.slot && !xint && tokens <= zc::kGatherInKernel;
         if (together) { a.check = check; zc::launch_affine(ctx->stream, a); }
-        else zc::launch_gather_check(ctx->stream, rows, tokens, check);
-        ZC_LAUNCHED();
-        if (const zc_status s = await_answer(ctx, check)) return s;
+        else if (question.slot) zc::launch_gather_check(ctx->stream, rows, tokens, check);
+        ZC_LAUNCHED();   // (a launch that failed leaves its word taken: something may still store to it)
+        if (const zc_status s = question.slot ? await_answer(ctx, question) : look_at_rows(ctx, rows, tokens, x_rows)) return s;
         if (together) return ZC_OK;
     }
     if (xint) zc::launch_affine_xint(ctx->stream, a);

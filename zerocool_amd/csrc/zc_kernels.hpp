@@ -20,7 +20,7 @@ struct AffineDesc {
     float* out = nullptr;
     uint32_t tokens = 0;
     uint32_t float_output = 0;
-    GatherCheck check;           // literal lane arithmetic, at most kGatherInKernel rows
+    GatherCheck check;           // gate/up with in_rows, at most kGatherInKernel of them
 };
 void launch_affine(hipStream_t s, const AffineDesc& a);          // literal lane arithmetic, any shape
 bool xint_supported(const zc_linear& l);                          // wide affine Q4, group 64, 16-byte aligned
