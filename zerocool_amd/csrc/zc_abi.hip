@@ -5,6 +5,7 @@
 #include "../../include/zc_hip.h"
 #include "zc_kernels.hpp"
 #include "zc_answers.hpp"
+#include "zc_prefill_tiles.hpp"
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
@@ -766,7 +767,7 @@ PrefillSpace carve_prefill(const zc_moe_config* c, uint32_t T, void* base) {
     uint64_t at = w.base.bytes;
     auto take = [&](uint64_t bytes) { void* p = base ? static_cast<uint8_t*>(base) + at : nullptr; at += align_up(bytes, 256); return p; };
     const uint64_t n = uint64_t(T) * c->topk;
-    w.max_tiles = (uint32_t(n / 32 + c->experts) + 7) / 8 * 8; w.max_shared_tiles = ((T + 31) / 32 + 7) / 8 * 8;   // (the product kernel deals tiles out eight at a time)
+    w.max_tiles = (zc::prefill_max_tiles(n, c->experts) + 7) / 8 * 8; w.max_shared_tiles = ((T + 31) / 32 + 7) / 8 * 8;   // (the product kernel deals tiles out eight at a time)
     const uint64_t xpitch = 3 * 2 * zc::prefill_pitch(c->hidden), apitch = 3 * 2 * zc::prefill_pitch(c->inter);
     w.xb = (uint16_t*)take(uint64_t(T) * c->hidden * 2); w.xp = (uint16_t*)take(uint64_t(T) * c->hidden * 2); w.xplanes = (uint16_t*)take(T * xpitch);
     w.actp = (uint16_t*)take(n * c->inter * 2); w.aplanes = (uint16_t*)take(n * apitch);

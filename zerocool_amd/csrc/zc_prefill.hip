@@ -37,6 +37,7 @@
 #include <algorithm>
 #include <type_traits>
 #include "zc_kernels.hpp"
+#include "zc_prefill_tiles.hpp"
 #include "zc_device.hpp"
 #include "zc_decode_common.hpp"   // lds_barrier; route_token: top-k + softmax of one token by one wavefront
 
@@ -49,7 +50,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
-constexpr uint32_t kTileRows = 32, kTileRowsMax = 48, kPitch = 136;   // LDS row pitch in bf16 elements: 128 elements of a row, sixteen rows on different banks
+constexpr uint32_t kPitch = 136;   // LDS row pitch in bf16 elements: 128 elements of a row, sixteen rows on different banks
 
 // What the matrix-core products and the recomputation need of their token rows, from fp32 rows holding BF16 values (F32)
 // or from bf16 rows in the operand's order (the SwiGLU activations): a thread takes four neighbouring elements, so loads and stores are whole runs.
@@ -159,9 +160,7 @@ __global__ __launch_bounds__(1024) void prefill_tiles_kernel(const int32_t* offs
     __shared__ int32_t scan[1024];
     const uint32_t e = threadIdx.x;
     const int32_t first = offsets ? (e < experts ? offsets[e] : 0) : 0, count = offsets ? (e < experts ? offsets[e + 1] - offsets[e] : 0) : (e == 0 ? int32_t(rows) : 0);
-    // whole tiles of 32 rows; what is left joins the last of them when that gives at most 48 rows, else it is a tile of its own
-    const int32_t whole = count / int32_t(kTileRows), left = count % int32_t(kTileRows);
-    const int32_t tiles = count == 0 ? 0 : (whole == 0 ? 1 : whole + (left > int32_t(kTileRowsMax - kTileRows) ? 1 : 0));
+    const int32_t tiles = prefill_tiles_of(count);
     scan[e] = tiles;
     __syncthreads();
     for (uint32_t step = 1; step < 1024; step <<= 1) {
@@ -230,11 +229,7 @@ __global__ __launch_bounds__(kDispatchThreads) void prefill_dispatch_kernel(cons
     __syncthreads();
     auto count_of = [&](uint32_t e) { int32_t c = 0; for (uint32_t q = 0; q < kDispatchParts; ++q) c += cnt[q * E + e]; return c; };
     {   // exclusive scans over the experts, one a thread
-        auto tiles_of = [](int32_t count) {
-            const int32_t whole = count / int32_t(kTileRows), left = count % int32_t(kTileRows);
-            return count == 0 ? 0 : (whole == 0 ? 1 : whole + (left > int32_t(kTileRowsMax - kTileRows) ? 1 : 0));
-        };
-        const int32_t c = tid < E ? count_of(tid) : 0, mine[2] = {c, tiles_of(c)};
+        const int32_t c = tid < E ? count_of(tid) : 0, mine[2] = {c, prefill_tiles_of(c)};
         int32_t incl[2] = {mine[0], mine[1]};
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1)
@@ -1288,10 +1283,8 @@ bool prefill_dispatch_fits(const int32_t* ids, uint32_t tokens, uint32_t topk, u
 }
 void launch_prefill_gemm(hipStream_t s, const PrefillGemm& p, bool gated, uint32_t max_tiles) {
     if (!gated && p.K == kShortK) {
-        // (four blocks a workgroup where that leaves the chip two workgroups a compute unit: a shared expert's few tiles need more of them)
-        const uint32_t tiles = (max_tiles + 7) / 8 * 8, blocks = p.N / 128;
-        uint32_t share = 4;
-        while (share > 1 && tiles * ((blocks + share - 1) / share) < 512) share /= 2;
+        // (a shared expert's few tiles, and a short batch's, need more workgroups than four blocks each leave)
+        const uint32_t tiles = (max_tiles + 7) / 8 * 8, blocks = p.N / 128, share = prefill_short_share(tiles, blocks);
         const dim3 grid(tiles * ((blocks + share - 1) / share));
         auto go = [&](auto kernel) {
             (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, int(kShortLds));
