@@ -253,7 +253,8 @@ def test_prefill_full_size_unskewed(ctx):
         ctx.free(b)
 
 
-@pytest.mark.parametrize("T", [70, 300])   # 300 tokens: the router on bounds with the selection in its launch, and the one-launch dispatch sort
+# 300 tokens: the one-launch dispatch sort; 800: the router on bounds too, with the selection in its launch
+@pytest.mark.parametrize("T", [70, 300, 800])
 def test_prefill_reports_unroutable_rows(ctx, T):
     # A NaN row gives that token no selectable expert (ids -1): its sorted positions are not covered by any tile.  The
     # call must end normally and the check must report "invalid router output", as the exact path does.
@@ -297,9 +298,10 @@ def test_prefill_rejects_what_it_cannot_run(ctx):
         ctx.moe_prefill(odd, weights.layer, x, T, out, ws)
 
 
+@pytest.mark.parametrize("T", [200, 800])   # below 768 tokens: exact logits
 @pytest.mark.parametrize("skew", [None, ("zipf", 1.1)])
-def test_prefill_router_on_bounds_picks_the_exact_ids(ctx, skew):
-    """From 128 tokens on (and when the logits themselves are not asked for) the prefill router forms every logit with a
+def test_prefill_router_on_bounds_picks_the_exact_ids(ctx, skew, T):
+    """From 768 tokens on (and when the logits themselves are not asked for) the prefill router forms every logit with a
     bf16 matrix-core product, bounds its distance from the reference's chains, and recomputes exactly only the experts that
     can be among the top k.  Ids and softmax weights must be the exact path's bits, also where logits tie exactly (router
     rows repeated, an all-zero input row), nearly tie (a row that differs from another in one element's last bit), where an
@@ -307,7 +309,7 @@ def test_prefill_router_on_bounds_picks_the_exact_ids(ctx, skew):
     untouched)."""
     cfg = workload.tiny_config(1024, 128, 8, 128)
     weights = workload.LayerWeights(ctx, cfg, 301, skew)
-    E, H, T = cfg.experts, cfg.hidden, 200
+    E, H = cfg.experts, cfg.hidden
     router = weights.router.numpy(np.uint16).reshape(E, H).copy()
     router[17] = router[5]; router[90] = router[5]; router[33] = router[64]      # exact ties
     router[70] = router[12]; router[70, 100] ^= 1                                  # one element differs by its last bit
