@@ -56,12 +56,14 @@ def test_prefill_logits(ctx, T, H, E):
         ctx.free(b)
 
 
-@pytest.mark.parametrize("T", [767, 768, 1025])   # exact logits, and from 768 tokens on those that the selection can see
-def test_prefill_selection_of_long_batches(ctx, T):
+# Exact logits, and from 768 tokens on those that the selection can see.  There: partitions of two, three and four steps of 64 elements, the
+# longest rows of the most experts (91 KB of LDS a workgroup), and more picks than the refinement selects itself
+@pytest.mark.parametrize("T,H,E,topk", [(767, 1152, 72, 8), (768, 1152, 72, 8), (1025, 1152, 72, 8), (770, 3072, 80, 10), (769, 4096, 1024, 10), (771, 512, 128, 70)])
+def test_prefill_selection_of_long_batches(ctx, T, H, E, topk):
     """Rows that tie exactly or nearly, zero, huge, tiny, not finite: ids and softmax weights are the exact layer's bits."""
-    cfg = workload.tiny_config(1152, 72, 8, 128)
+    cfg = workload.tiny_config(H, E, topk, 128)
     weights = workload.LayerWeights(ctx, cfg, 303, ("normal", 0.5))
-    E, H, n = cfg.experts, cfg.hidden, T * cfg.topk
+    n = T * topk
     router = weights.router.numpy(np.uint16).reshape(E, H).copy()
     router[17] = router[5]; router[61] = router[5]; router[33] = router[64]
     router[70] = router[12]; router[70, 100] ^= 1
