@@ -58,15 +58,10 @@ def test_prefill_dispatch_of_many_slots(ctx, experts, topk, T):
         ctx.free(b)
 
 
-# down rows of 512: five and nine blocks of weight rows, one to three blocks of token rows and several tiles, codes of either width
-@pytest.mark.parametrize("hidden,bits", [(640, (4, 4, 4, 4)), (1152, (4, 8, 8, 8)), (128, (8, 8, 4, 4))])
-@pytest.mark.parametrize("T", [1, 16, 20, 33, 48, 65, 130])
-def test_prefill_down_rows_of_512(ctx, hidden, bits, T):
-    cfg = workload.tiny_config(hidden, 2, 2, 512, bits=bits)      # both experts have every token
-    weights = workload.LayerWeights(ctx, cfg, 23 + T, ("normal", 0.5))
-    x, n, outs = workload.hidden_rows(ctx, T, hidden, 24), T * 2, []
+def down_rows_of_512(ctx, cfg, weights, T):
+    x, n, outs = workload.hidden_rows(ctx, T, cfg.hidden, 24), T * cfg.topk, []
     for call, size in ((ctx.moe_forward, ctx.moe_workspace_bytes), (ctx.moe_prefill, ctx.moe_prefill_workspace_bytes)):
-        out, ws, eo, sh = ctx.alloc(T * hidden * 4), ctx.alloc(size(cfg, T)), ctx.alloc(n * hidden * 4), ctx.alloc(T * hidden * 4)
+        out, ws, eo, sh = ctx.alloc(T * cfg.hidden * 4), ctx.alloc(size(cfg, T)), ctx.alloc(n * cfg.hidden * 4), ctx.alloc(T * cfg.hidden * 4)
         call(cfg, weights.layer, x, T, out, ws, z.Trace(None, None, None, eo.ptr, sh.ptr, None))
         ctx.moe_check()
         outs.append([b.numpy(f32).copy() for b in (out, eo, sh)])
@@ -79,5 +74,27 @@ def test_prefill_down_rows_of_512(ctx, hidden, bits, T):
         assert np.max(np.abs(fast - exact)) <= 2.0 ** -7 * np.max(np.abs(exact))
         assert np.mean(fast.view(np.uint32) == exact.view(np.uint32)) > 0.9999
     assert np.max(np.abs(outs[1][0] - outs[0][0])) <= 2e-3 * np.max(np.abs(outs[0][0]))
-    for b in (weights.router, weights.shared_gate, weights.shared_record, weights.records, x):
+    for b in (weights.router, weights.shared_gate, weights.shared_record, weights.records, weights.offsets, x):
         ctx.free(b)
+
+
+# down rows of 512, a workgroup a block of weight rows: one to three blocks of token rows and several tiles, codes of either width
+@pytest.mark.parametrize("hidden,bits", [(640, (4, 4, 4, 4)), (1152, (4, 8, 8, 8)), (128, (8, 8, 4, 4))])
+@pytest.mark.parametrize("T", [1, 16, 20, 33, 48, 65, 130])
+def test_prefill_down_rows_of_512(ctx, hidden, bits, T):
+    cfg = workload.tiny_config(hidden, 2, 2, 512, bits=bits)      # both experts have every token
+    down_rows_of_512(ctx, cfg, workload.LayerWeights(ctx, cfg, 23 + T, ("normal", 0.5)), T)
+
+
+# The same with several blocks a workgroup, the last workgroup with fewer of them: five blocks by two (2 2 1; at 20 tokens) and by four (4 1), nine by four (4 4 1).
+# Three experts have every token (tiles of 20 and 33 to 48 rows, and of 32 and 18), the others a few.
+@pytest.mark.parametrize("hidden", [640, 1152])
+@pytest.mark.parametrize("bits", [(4, 4, 4, 4), (4, 8, 8, 8)])
+@pytest.mark.parametrize("T", [20, 33, 48, 50])
+def test_prefill_down_rows_of_512_several_blocks_a_workgroup(ctx, hidden, bits, T):
+    cfg = workload.tiny_config(hidden, 512, 10, 512, bits=bits)
+    weights = workload.LayerWeights(ctx, cfg, 29 + T, ("normal", 0.5))
+    offsets = weights.offsets.numpy(f32).copy()
+    offsets[[3, 200, 511]] += 40                                   # (logits are N(0, 1) and their offsets)
+    ctx.upload(offsets, into=weights.offsets)
+    down_rows_of_512(ctx, cfg, weights, T)
