@@ -1,5 +1,6 @@
 """The gather's row check of the fused gate/up operator: a refused call leaves the output alone, an accepted one is the oracle's.
-Lists up to 256 rows are looked at by the product's own kernel (lanes, and from 48 rows on matrix cores), longer ones in front of it."""
+Lists up to 256 rows are looked at by the product's own kernel (the lanes', or the matrix cores' where the product has a wave for every SIMD: 64 outputs
+from 253 rows on, 256 from 61), longer ones in front of it."""
 import threading
 import numpy as np
 import pytest
@@ -12,7 +13,7 @@ f32 = np.float32
 
 
 @pytest.mark.parametrize("n", [1, 2, 47, 64, 65, 255, 256, 257, 1030])
-@pytest.mark.parametrize("K,N", [(320, 7), (512, 64)])
+@pytest.mark.parametrize("K,N", [(320, 7), (512, 64), (512, 256)])
 def test_gathered_rows_are_checked_whichever_kernel_looks(ctx, n, K, N):
     T, rng = 9, np.random.RandomState(n)
     w = rng.randint(0, 2 ** 32, N * K // 8, dtype=np.uint32)
