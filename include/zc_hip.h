@@ -107,7 +107,9 @@ zc_status zc_hip_linear_into(zc_hip_ctx* ctx, const zc_linear* layer, const floa
 zc_status zc_hip_router_logits(zc_hip_ctx* ctx, const void* w_bf16, const float* x, uint32_t tokens,
                                uint32_t hidden, uint32_t experts, const float* offsets, float* logits);
 /* Metal::gated_linear (metal.mm:845-880; qwen.metal:71-81, 134-144). rows may be NULL.
- * x_rows is the number of rows x holds (bounds for the gather). */
+ * x_rows is the number of rows x holds (bounds for the gather).  With rows the call waits until the GPU has looked at the list, which
+ * work in front of it on the stream may write; a row outside x is an error, and nothing is written then.  Threads that share the context
+ * may wait at once.  Not while the stream is being captured. */
 zc_status zc_hip_gated_linear(zc_hip_ctx* ctx, const zc_linear* gate, const zc_linear* up,
                               const float* x, uint32_t x_rows, uint32_t tokens,
                               const int32_t* rows, float* out);

@@ -59,7 +59,8 @@ struct zc_hip_ctx {
     zc::AnswerWords answers;           // pinned words in which kernels answer gather checks (calls of several threads may wait at once)
     hipEvent_t timer[2] = {nullptr, nullptr};
     // The prefill layer runs its shared expert beside the router, the selection and the dispatch sort, which are chains of
-    // small kernels: a second stream of default priority, forked from and joined to `stream` by two events per call.
+    // small kernels: a second stream of default priority, forked from and joined to `stream` by two events per call, and a third where
+    // the products' rows are made there (a batch with exact logits): the routed products wait for those.
     hipStream_t beside = nullptr; hipEvent_t fork = nullptr, rows_ready = nullptr, join = nullptr;
     // 0 literal lane kernels, 1 exact-integer matrix-core kernels where possible, 2 the lanes except where prefers_xint() says otherwise.
     uint32_t affine_policy = 2;
@@ -649,6 +650,8 @@ uint64_t zc_hip_moe_workspace_bytes(const zc_moe_config* cfg, uint32_t tokens) {
 //   1024 x 512, 64 experts, 2, 6, 12, 16 tokens 28.6 -> 32.4, 40.3 -> 49.2, 49.0 -> 51.6, 54.6 -> 53.4 / 29.5 -> 33.7, 37.7 -> 39.1, 46.5 -> 43.5, 52 -> 54
 //   2048 x 512, 512 experts, 4, 12, 24 tokens   56 -> 67, 108 -> 114, 178 -> 175 / 43 -> 47, 73 -> 72, 109 -> 95
 //   4096 x 2048, 128 experts, 2, 4, 8 tokens    128 -> 129, 233 -> 229, 360 -> 357 / 103 -> 103, 181 -> 150, 245 -> 202
+// (The matrix cores' side as it was before MatrixPace and the slots in place, which made batches of two to five tokens up to 5 % faster and
+// larger ones 4 to 13 %: the lines may lie a little high.)
 static bool matrix_preferred(const zc_moe_config& c, uint32_t T) {
     const uint64_t weights = uint64_t(c.hidden) * c.inter;
     if (c.bits_gate_up == 8) return weights >= 1u << 23 ? T >= 4 : T >= 12 && 2ull * T * c.topk >= c.experts;
@@ -752,11 +755,12 @@ zc_status zc_hip_moe_forward(zc_hip_ctx* ctx, const zc_moe_config* c, const zc_m
 namespace {
 struct PrefillSpace {
     Workspace base;
-    // rows of the products: as bf16, as the matrix-core operand, their group sums in pieces (xplain: for affine Q8 gate/up 
+    // the inputs as bf16 rows (for the router on bounds only); inputs, activations and the shared expert's activations as the matrix-core operand; their
+    // group sums in pieces (xplain: the inputs' for affine Q8 gate/up)
     uint16_t *xb, *xp, *actp, *sactp, *xplanes, *xplain, *aplanes, *splanes;
     int32_t *tile_expert, *tile_first, *tile_rows, *tile_count, *stile_expert, *stile_first, *stile_rows, *stile_count;
     uint32_t max_tiles, max_shared_tiles;
-    uint32_t* near_bits;      // one bit per product element: recompute exactly
+    uint32_t* near_bits;      // one bit per sum (two for an element of gate/up, one for one of down): recompute exactly
     uint32_t* shared_near_bits;   // the same for the shared expert's products, which run beside the routed ones
     float* norms;             // |row| of the router's rows (the router on bounds)
     uint64_t bytes;
@@ -1197,6 +1201,8 @@ static zc_status launch_piece(zc_hip_ctx* ctx, zc_hip_stack* st, const float* x,
 // gain from: 31 -> 24 and 38 -> 34.  That kernel's Q8 rows are walked a row at a time: one, two, six and sixteen mixed layers of hidden 2048
 // 37 -> 24, 35 -> 25, 33 -> 25, 37 -> 27, Q8 only in the shared expert 33 -> 24, 30 -> 24, 29 -> 24; of hidden 3072 69 -> 40, 61 -> 37, 68 -> 41,
 // 66 -> 41, and 48 -> 37, 43 -> 35, 42 -> 38.
+// (Layer by layer as it was before MatrixPace and the slots in place, which made batches of two to five tokens up to 5 % faster and larger
+// ones 4 to 13 %: further on its side.)
 // (Above sixty-four tokens the rule says nothing: the inputs' check for BF16 values is the short router's, which ends there.)
 static bool layers_preferred(const zc_hip_stack* st, uint32_t tokens) {
     if (tokens > 64 || st->store || st->wait_limit != kWaitPolls) return false;

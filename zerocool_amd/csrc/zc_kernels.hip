@@ -250,6 +250,8 @@ static dim3 affine_grid(uint32_t x, uint32_t jobs) { const uint32_t y = std::min
 // Q8: gate/up at 48, 64 and 128, 2048 x 512 14.7 -> 13.9, 18.9 -> 14.2, 30 -> 23; 3072 x 1024 at 48 and 128 33 -> 24, 71 -> 53; down at 128
 // and 192, 512 x 2048 16.8 -> 12.4, 22.6 -> 18.3; 1024 x 3072 37 -> 26, 52 -> 39.  Q4 rows of half steps: gate/up at 48 and 128, 640 x 2560 25.6 -> 15.2, 56 -> 27;
 // 1920 x 640 18.4 -> 12.6, 36 -> 28; down at 128, 640 x 2560 26.8 -> 17.5, 1920 x 2560 59 -> 37.
+// (All of it, and the figures below, with the matrix cores' side as it was before MatrixPace and the slots in place, which took up to a sixth off
+// an expert phase of 32 to 64 tokens: the lines may lie a little high.)
 constexpr uint32_t kMatrixFrom[2] = {128, 48};   // plain, gate/up
 // And from a wave a SIMD on (two where a matrix has less than a workgroup's tiles), since with fewer the call lasts as long as one workgroup's chain,
 // which is longer there.  Gate/up with 512, 768, 1024 and 2048 waves: 2048 x 64 7.6 -> 10.0, 9.0 -> 9.9, 10.4 -> 10.1, 17.4 -> 12.8; down 2048 x 128 7.2 -> 9.6, 8.5 ->

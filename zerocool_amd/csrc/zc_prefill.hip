@@ -323,8 +323,8 @@ __device__ __forceinline__ uint32_t prefill_round(float v, float m, float margin
 // which overlap only in part -- weights and rows read from a warm cache leave the time of the walk unchanged.  A wave
 // alone issues one vector instruction every five clocks, so the registers are kept to what three waves per SIMD allow
 // (Q4: 156 and 160 of 168; with a second set of token rows or four pairs of weights in flight two waves fit, and the layer of
-// hidden 2048 took 680 us at 2048 tokens instead of 621).  At that size the routed gate/up product takes 240 us, the down product
-// 150 us (369 and 258 with a run-time number of row blocks, codes converted one by one and the scales staged through LDS).
+// hidden 2048 took 680 us at 2048 tokens where it took 621 then).  At that size the routed gate/up product takes 240 us (369 with a run-time number of
+// row blocks, codes converted one by one and the scales staged through LDS); the down product of its rows of 512 is prefill_short_tile's.
 template <bool GATED, int BITS, int NB>
 __device__ __forceinline__ void prefill_tile(const PrefillGemm& p, uint16_t* a_s, uint16_t* marks_s, uint16_t* bias_s, uint32_t expert, uint32_t first, uint32_t rows, uint32_t n0) {
     constexpr int kAhead = 2, kRegs = BITS;       // pairs of groups in flight; dwords of a column tile's pair per lane
@@ -659,7 +659,8 @@ __global__ __launch_bounds__(256, BITS == 4 ? 3 : 2) void prefill_gemm_kernel(Pr
 // block's codes, scales and biases as it uses up this one's, so that loads are in flight during the epilogue too.  Sums, marks and outputs are
 // prefill_tile's, added in the same order.  2048 weight rows, routed product alone: 2048 tokens 141 -> 123 us, 300 tokens with byte codes 130 ->
 // 108; a layer 551 -> 534 and 332 -> 320.  (Rows of 640, whose LDS and registers leave as many waves: a layer of 300 tokens of hidden 2560 408 -> 402 us, but
-// 600 503 -> 509 and 1000 612 -> 621.  Longer rows leave one workgroup a compute unit.)
+// 600 503 -> 509 and 1000 612 -> 621.  Longer rows, where a tile has three blocks of them, leave one workgroup a compute unit.  Rows of 128 to 384 have not been
+// tried.)
 constexpr uint32_t kShortK = 512, kShortPitch = kShortK + 8, kShortOutPitch = 40;   // pitches in bf16 elements: sixteen rows on different banks
 constexpr uint32_t kShortLds = 2 * (8 + kTileRowsMax * (kShortPitch + 3 * prefill_pitch(kShortK)) + 4 * 16 * kShortOutPitch);
 template <int BITS, int NB>
